@@ -103,10 +103,11 @@ enum Slot : int {
 // (filled with vertex 0) so vectorised edge loads may run past m.
 constexpr int64_t kEdgePad = 4096;
 
-// Tables of the pull PageRank sweep over the transpose, built once per graph.
+// Tables of the row sweep (rowsweep.hpp) over one row-offset array, built once
+// per graph.
 struct PullPlan {
   bool ready = false;
-  int64_t ntiles = 0;
+  int64_t full = 0;  // rows with edges
   DevBuf buf;
 };
 

@@ -24,15 +24,12 @@
 //  - The pull runs over the transpose in degree order (vertices relabelled
 //    by out-degree, descending), so the most-gathered y entries share cache
 //    lines; results are mapped back to the caller's ids at the end.
-//  - The row sums are the merge-path tile sweep of rowsweep.hpp: tiles of a
-//    fixed number of row ends + edges, columns staged with 16-byte loads,
-//    every gather of a tile in flight at once, per-lane walks in LDS, and
-//    coalesced per-row finalisation (x', y' = x'/outdeg, residual, dangling
-//    mass).  Rows spanning tiles are completed by a second small launch.
-//  - FP32 mode: compensated (Neumaier) row sums in registers and
-//    TwoSum-merged wave reductions; x and y stored in FP32; the residual and
-//    dangling mass are accumulated in FP64 per workgroup and reduced in a
-//    fixed order (deterministic).
+//  - The row sums are the tile sweep of rowsweep.hpp: a wavefront per 512
+//    edges, FP64 sums, coalesced per-row finalisation (x', y' = x'/outdeg,
+//    residual, dangling mass).  Rows spanning chunks of tiles are completed by
+//    a second small launch.
+//  - The residual and dangling mass are accumulated in FP64 per workgroup and
+//    reduced in a fixed order (deterministic).
 //  - Iterations are enqueued in batches with no host round trip: each sweep
 //    reads a device `converged` flag and returns at once when it is set, so
 //    surplus launches after convergence are no-ops.
@@ -51,7 +48,6 @@ using namespace gx;
 
 namespace {
 
-using rs::Acc;
 using rs::block_sum;
 using rs::kBlock;
 using rs::kSweepGrid;
@@ -71,10 +67,9 @@ struct PrState {
 
 template <class Real>
 struct PrSrc {
+  static constexpr bool kCol = true;
   const Real* __restrict__ y;
   __device__ __forceinline__ Real operator()(int64_t, int32_t c) const { return y[c]; }
-  __device__ __forceinline__ Real load(int32_t c) const { return y[c]; }
-  __device__ __forceinline__ Real apply(int64_t, Real v) const { return v; }
 };
 
 // FP32 update x' = base + alpha*(s_hi + s_lo) with base and alpha carried as
@@ -122,14 +117,14 @@ struct PrFin {
   __device__ __forceinline__ Pre pre(uint32_t r) const {
     return Pre{rs::ld_stream(&x_old[r]), part ? rs::ld_stream(&part[r]) : Real(0), rs::ld_stream(&outdeg[r])};
   }
-  __device__ __forceinline__ void operator()(uint32_t r, Real sum, const Pre& p, double& resid, double& dang) const {
+  __device__ __forceinline__ void operator()(uint32_t r, double sum, const Pre& p, double& resid, double& dang) const {
     Real xn;
+    sum += static_cast<double>(p.pa);
     if constexpr (std::is_same<Real, float>::value) {
-      float sh, sl;
-      two_sum(p.pa, sum, sh, sl);
-      xn = pr_update_f32(bp, ap, sh, sl);
+      const F32Pair sp = split_f64(sum);
+      xn = pr_update_f32(bp, ap, sp.hi, sp.lo);
     } else {
-      xn = base + alpha * (p.pa + sum);
+      xn = base + alpha * sum;
     }
     resid += fabs(static_cast<double>(xn) - static_cast<double>(p.xo));
     __builtin_nontemporal_store(xn, &x_new[r]);
@@ -150,8 +145,8 @@ struct PartFin {
   struct Pre {};
   __device__ __forceinline__ void load() {}
   __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
-  __device__ __forceinline__ void operator()(uint32_t r, Real sum, const Pre&, double&, double&) const {
-    __builtin_nontemporal_store(sum, &part[r]);
+  __device__ __forceinline__ void operator()(uint32_t r, double sum, const Pre&, double&, double&) const {
+    __builtin_nontemporal_store(static_cast<Real>(sum), &part[r]);
   }
 };
 
@@ -414,7 +409,7 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   }
   const PbLayout& L = D.pb;
   Real* part = hot > 0 ? g->scratch<Real>(WS_V3, n) : nullptr;
-  Real* carryA = hot > 0 ? g->scratch<Real>(WS_V4, 3 * PA.ntiles) : nullptr;
+  double* carryA = hot > 0 ? g->scratch<double>(WS_V4, 2 * PA.nchunks) : nullptr;
   double* partsA = hot > 0 ? g->scratch<double>(WS_V5, 2 * rs::kParts) : nullptr;
   const uint32_t* outdeg = D.outdeg.as<uint32_t>();
   Real* xb = g->scratch<Real>(WS_V0, 2 * n);
@@ -425,7 +420,7 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   double* parts = g->scratch<double>(WS_REDUCE, 2 * nparts);
   double* part_resid = parts;
   double* part_dang = parts + nparts;
-  Real* carry = blocked ? nullptr : g->scratch<Real>(WS_V2, 3 * P.ntiles);
+  double* carry = blocked ? nullptr : g->scratch<double>(WS_V2, 2 * P.nchunks);
   PrState* state = g->scratch<PrState>(WS_COUNTERS, 1);
   PrState* host = static_cast<PrState*>(g->host_pinned(sizeof(PrState)));
 
@@ -470,16 +465,11 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
       PrFin<Real> fin{state, x[cur], x[nxt], y[nxt], outdeg, part, Real(0), Real(0)};
       ktimer.begin();
       if (hot > 0) {
-        rs::launch_sweep<Real, rs::HotCache<Real>::kHot>(PA, src, PartFin<Real>{part}, &state->converged, partsA,
-                                                         partsA + rs::kParts, carryA, s, nullptr);
+        rs::launch_sweep<Real>(PA, src, PartFin<Real>{part}, &state->converged, partsA, partsA + rs::kParts, carryA, s,
+                               nullptr);
         launches += 2;
       }
-      // Degree order puts the most-gathered sources first: cache them in LDS
-      // (only the single pass / hot pass; the cold pass has no such prefix).
-      const int np = hot > 0 ? rs::launch_sweep<Real>(P, src, fin, &state->converged, part_resid, part_dang,
-                                                      carry, s, nullptr)
-                             : rs::launch_sweep<Real, rs::HotCache<Real>::kHot>(
-                                   P, src, fin, &state->converged, part_resid, part_dang, carry, s, nullptr);
+      const int np = rs::launch_sweep<Real>(P, src, fin, &state->converged, part_resid, part_dang, carry, s, nullptr);
       ktimer.end();
       pr_reduce_kernel<<<1, kBlock, 0, s>>>(state, part_resid, part_dang, np, static_cast<unsigned>(nxt));
       GX_LAUNCHED("pr_reduce_kernel");

@@ -45,17 +45,25 @@ struct AdState {
   unsigned max_iter;
 };
 
-// Per-row inverse weight sums (0 marks a dangling row), FP64 accumulation.
+// Per-row inverse weight sums (0 marks a dangling row): a row sweep over the
+// weights alone, summed in FP64.  A lane per row instead, hubs and all, took
+// 18.2 ms on 4.2M rows with 67M edges.
 template <class Real>
-__global__ void inv_rowsum_kernel(const int32_t* __restrict__ row, const float* __restrict__ w, int64_t n,
-                                  Real* __restrict__ inv_s) {
-  for (int64_t u = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; u < n;
-       u += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    double s = 0;
-    for (int32_t e = row[u]; e < row[u + 1]; ++e) s += w[e];
-    inv_s[u] = s > 0 ? static_cast<Real>(1.0 / s) : Real(0);
+struct RowWeights {
+  static constexpr bool kCol = false;
+  const float* __restrict__ w;
+  __device__ __forceinline__ Real operator()(int64_t e, int32_t) const { return static_cast<Real>(rs::ld_stream(&w[e])); }
+};
+template <class Real>
+struct InvFin {
+  Real* __restrict__ inv_s;
+  struct Pre {};
+  __device__ __forceinline__ void load() {}
+  __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
+  __device__ __forceinline__ void operator()(uint32_t r, double sum, const Pre&, double&, double&) const {
+    inv_s[r] = sum > 0 ? static_cast<Real>(1.0 / sum) : Real(0);
   }
-}
+};
 
 // Weights in transpose order: wt[j] = w[tperm[j]].
 template <class Real>
@@ -76,6 +84,7 @@ __global__ void convert_weights_kernel(const float* __restrict__ w, int64_t m, R
 
 template <class Real>
 struct WSrc {  // value of edge slot e = y[c] * w[e]
+  static constexpr bool kCol = true;
   const Real* __restrict__ y;
   const Real* __restrict__ w;
   __device__ __forceinline__ Real operator()(int64_t e, int32_t c) const { return y[c] * w[e]; }
@@ -101,8 +110,8 @@ struct FwdFin {
     Real is, xo;
   };
   __device__ __forceinline__ Pre pre(uint32_t r) const { return Pre{t[r], inv_s[r], x_old[r]}; }
-  __device__ __forceinline__ void operator()(uint32_t r, Real sum, const Pre& p, double& resid, double& dang) const {
-    const Real xn = (Real(1) - alpha) * static_cast<Real>(p.t) + base + alpha * sum;
+  __device__ __forceinline__ void operator()(uint32_t r, double sum, const Pre& p, double& resid, double& dang) const {
+    const Real xn = (Real(1) - alpha) * static_cast<Real>(p.t) + base + alpha * static_cast<Real>(sum);
     resid += fabs(static_cast<double>(xn) - static_cast<double>(p.xo));
     x_new[r] = xn;
     const Real is = p.is;
@@ -140,9 +149,9 @@ struct AdjFin {
     }
     return q;
   }
-  __device__ __forceinline__ void operator()(uint32_t r, Real sum, const Pre& q, double& resid, double& tot) const {
+  __device__ __forceinline__ void operator()(uint32_t r, double sum, const Pre& q, double& resid, double& tot) const {
     const Real is = q.is;
-    const Real p = (is == Real(0)) ? base : sum * is;
+    const Real p = (is == Real(0)) ? base : static_cast<Real>(sum) * is;
     if (final_pass) {
       pl[r] = p;
       return;
@@ -320,6 +329,7 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
   hipStream_t s = g->stream;
   build_transpose(g);
   const rs::RowPlan P = rs::build_plan(g, g->trow(), g->tcol(), n, m, g->csc_plan);
+  const rs::RowPlan W = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);  // row sums of the weights
   Real* inv_s = g->scratch<Real>(WS_V4, n);
   Real* wt = g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
   Real* xb = g->scratch<Real>(WS_V0, 2 * n);
@@ -328,13 +338,13 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
   Real* ys[2] = {yb, yb + n};
   const int nparts = rs::kParts;
   double* parts = g->scratch<double>(WS_REDUCE, 2 * nparts);
-  Real* carry = g->scratch<Real>(WS_V2, 3 * P.ntiles);
+  double* carry = g->scratch<double>(WS_V2, std::max<int64_t>(2 * P.nchunks, 1));
   AdState* state = g->scratch<AdState>(WS_COUNTERS, 1);
   AdState* host = static_cast<AdState*>(g->host_pinned(sizeof(AdState)));
   RegionTimer region(s);
   KernelTimer ktimer(s);
-  uint32_t launches = 6;
-  inv_rowsum_kernel<Real><<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(g->row, w, n, inv_s);
+  uint32_t launches = 7;
+  rs::launch_sweep<Real>(W, RowWeights<Real>{w}, InvFin<Real>{inv_s}, nullptr, parts, parts + nparts, carry, s, nullptr);
   if (m) permute_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, g->tperm(), m, wt);
   ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / n, max_iter);
   fwd_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(xs[0], ys[0], inv_s, n, parts);
@@ -374,7 +384,7 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   Real* lam[2] = {lb, lb + n};
   const int nparts = rs::kParts;
   double* parts = g->scratch<double>(WS_REDUCE, 2 * nparts);
-  Real* carry = g->scratch<Real>(WS_V2, 3 * P.ntiles);
+  double* carry = g->scratch<double>(WS_V2, std::max<int64_t>(2 * P.nchunks, 1));
   uint32_t* hubq = g->scratch<uint32_t>(WS_Q2, n);
   unsigned* hubc = g->scratch<unsigned>(WS_Q3, 4);
   uint32_t* hub_off = g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n));
@@ -382,8 +392,8 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   AdState* host = static_cast<AdState*>(g->host_pinned(sizeof(AdState)));
   RegionTimer region(s);
   KernelTimer ktimer(s);
-  uint32_t launches = 5;
-  inv_rowsum_kernel<Real><<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(g->row, w, n, inv_s);
+  uint32_t launches = 6;
+  rs::launch_sweep<Real>(P, RowWeights<Real>{w}, InvFin<Real>{inv_s}, nullptr, parts, parts + nparts, carry, s, nullptr);
   if (m) convert_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, m, wr);
   ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / n, max_iter);
   adj_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(lam[0], c, n, parts);

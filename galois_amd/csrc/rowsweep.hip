@@ -1,6 +1,5 @@
-// Plan table of the row sweep (rowsweep.hpp): the merge-path coordinates
-// (first row, first edge) of every tile.  Built once per row-offset array and
-// cached in the graph.
+// Plan tables of the row sweep (rowsweep.hpp), built once per row-offset array
+// and cached in the graph.
 #include <algorithm>
 
 #include "rowsweep.hpp"
@@ -9,50 +8,105 @@ namespace gx {
 namespace rs {
 namespace {
 
-// Item d of the merge path (row ends and edges of a sequential CSR walk, a
-// row's end after its last edge): rows ended before item d = the largest r
-// with r == 0 or rowoff[r] + r <= d; edges before it = d - r.
-__global__ void tile_coords_kernel(const int32_t* __restrict__ rowoff, int64_t n, int64_t m, int64_t ntiles,
-                                   int32_t* __restrict__ tile_row, int32_t* __restrict__ tile_edge) {
-  int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (; t <= ntiles; t += stride) {
-    const int64_t d = std::min<int64_t>(t * kTile, n + m);
-    int64_t lo = std::max<int64_t>(0, d - m), hi = std::min<int64_t>(d, n);
-    while (lo < hi) {
-      const int64_t mid = (lo + hi + 1) >> 1;
-      if (static_cast<int64_t>(rowoff[mid]) + mid <= d) lo = mid; else hi = mid - 1;
+__global__ void full_flag_kernel(const int32_t* __restrict__ rowoff, int64_t n, uint32_t* __restrict__ flag) {
+  for (int64_t r = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; r <= n;
+       r += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    flag[r] = r < n && rowoff[r + 1] > rowoff[r] ? 1u : 0u;
+}
+
+// pos: rows with edges before each row (n + 1 entries).
+__global__ void rid_kernel(const uint32_t* __restrict__ pos, int64_t n, uint32_t* __restrict__ rid) {
+  const uint32_t full = pos[n];
+  for (int64_t r = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; r < n;
+       r += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const uint32_t p = pos[r];
+    rid[pos[r + 1] > p ? p : full + static_cast<uint32_t>(r) - p] = static_cast<uint32_t>(r);
+  }
+}
+
+// Index in rid of the row that holds edge e (e < m).
+__device__ __forceinline__ uint32_t row_index(const int32_t* __restrict__ rowoff, const uint32_t* __restrict__ rid,
+                                              uint32_t full, int64_t e) {
+  uint32_t lo = 0, hi = full - 1;  // last row with rowoff <= e
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo + 1) / 2;
+    if (rowoff[rid[mid]] <= e) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
+__global__ void tile_row_kernel(const int32_t* __restrict__ rowoff, const uint32_t* __restrict__ rid, uint32_t full,
+                                int64_t m, int64_t ntiles, uint32_t* __restrict__ tile_row) {
+  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t <= ntiles;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    tile_row[t] = t * kTile < m ? row_index(rowoff, rid, full, t * kTile) : full;
+}
+
+__global__ void lane_info_kernel(const int32_t* __restrict__ rowoff, const uint32_t* __restrict__ rid, uint32_t full,
+                                 int64_t m, int64_t ntiles, const uint32_t* __restrict__ tile_row,
+                                 uint32_t* __restrict__ info) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < ntiles * kWave;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t e0 = i * kItems;
+    uint32_t word = 0;
+    if (e0 < m) {
+      uint32_t k = row_index(rowoff, rid, full, e0);
+      word = (k - tile_row[i / kWave]) << 8;
+      int64_t end = rowoff[rid[k] + 1];
+      for (int u = 0; u < kItems && e0 + u < m; ++u) {
+        if (e0 + u + 1 != end) continue;
+        word |= 1u << u;
+        if (++k < full) end = rowoff[rid[k] + 1];
+      }
     }
-    tile_row[t] = static_cast<int32_t>(lo);
-    tile_edge[t] = static_cast<int32_t>(d - lo);
+    info[i] = word;
   }
 }
 
 }  // namespace
 
-// Table layout in cache.buf: tile_row[ntiles+1] | tile_edge[ntiles+1].
+// Layout of cache.buf (words): rid[n] | tile_row[ntiles + 1] | lane_info[64 * ntiles].
 RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64_t n, int64_t m, PullPlan& cache) {
   GX_REQUIRE(n > 0, "row sweep over an empty graph");
-  const int64_t ntiles = (n + m + kTile - 1) / kTile;
+  const int64_t ntiles = (m + kTile - 1) / kTile;
   auto view = [&]() {
     RowPlan P{};
     P.rowoff = rowoff;
     P.col = col;
     P.n = n;
     P.len = m;
-    P.tile_row = cache.buf.as<int32_t>();
-    P.tile_edge = P.tile_row + (ntiles + 1);
+    P.rid = cache.buf.as<uint32_t>();
+    P.full = cache.full;
+    P.tile_row = P.rid + n;
+    P.lane_info = P.tile_row + ntiles + 1;
     P.ntiles = ntiles;
+    P.kt = tiles_per_chunk(ntiles);
+    P.nchunks = (ntiles + P.kt - 1) / P.kt;
     return P;
   };
   if (cache.ready) return view();
-  cache.buf.ensure(2 * (ntiles + 1) * sizeof(int32_t));
-  RowPlan P = view();
-  tile_coords_kernel<<<grid_for(ntiles + 1, kBlock, 4096), kBlock, 0, g->stream>>>(rowoff, n, m, ntiles, P.tile_row,
-                                                                                  P.tile_edge);
-  GX_LAUNCHED("tile_coords_kernel");
-  GX_HIP(hipStreamSynchronize(g->stream));
-  cache.ntiles = ntiles;
+  hipStream_t s = g->stream;
+  cache.buf.ensure((n + ntiles + 1 + ntiles * kWave) * sizeof(uint32_t));
+  uint32_t* rid = cache.buf.as<uint32_t>();
+  uint32_t* tile_row = rid + n;
+  DevBuf pos;
+  pos.ensure((n + 1) * sizeof(uint32_t));
+  full_flag_kernel<<<grid_for(n + 1, kBlock, 8192), kBlock, 0, s>>>(rowoff, n, pos.as<uint32_t>());
+  GX_LAUNCHED("full_flag_kernel");
+  exclusive_scan_u32(pos.as<uint32_t>(), pos.as<uint32_t>(), n + 1, s);
+  rid_kernel<<<grid_for(n, kBlock, 8192), kBlock, 0, s>>>(pos.as<uint32_t>(), n, rid);
+  GX_LAUNCHED("rid_kernel");
+  uint32_t full = 0;
+  read_bytes(g, &full, pos.as<uint32_t>() + n, sizeof(full));
+  cache.full = full;
+  tile_row_kernel<<<grid_for(ntiles + 1, kBlock, 8192), kBlock, 0, s>>>(rowoff, rid, full, m, ntiles, tile_row);
+  GX_LAUNCHED("tile_row_kernel");
+  if (ntiles > 0) {
+    lane_info_kernel<<<grid_for(ntiles * kWave, kBlock, 16384), kBlock, 0, s>>>(rowoff, rid, full, m, ntiles, tile_row,
+                                                                                tile_row + ntiles + 1);
+    GX_LAUNCHED("lane_info_kernel");
+  }
+  GX_HIP(hipStreamSynchronize(s));
   cache.ready = true;
   return view();
 }

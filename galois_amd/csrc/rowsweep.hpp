@@ -2,39 +2,49 @@
 // value(e, col[e]) for every row, the pull step of PageRank (over the
 // transpose) and of its adjoint (over the CSR).
 //
-// Layout (merge path).  A sequential CSR walk visits n row ends and m edges
-// in one interleaved order; that sequence is cut into tiles of kTile items,
-// so every tile holds exactly kTile row ends + edges whatever the degree mix
-// (empty rows, hubs and everything between cost the same per item).  The
-// plan stores each tile's first row and first edge.
+// Layout.  The edges are cut into tiles of kTile = 512 (8 per lane of one
+// wavefront); `kt` consecutive tiles are a chunk, which one wavefront sums
+// from front to back.  A static plan holds, per lane and tile, which of the
+// lane's 8 edges end a row and how many rows of the tile end before them
+// (one word), per tile the index of its first row among the rows that have
+// edges, and those rows' ids in order.  Rows without edges are listed behind
+// them and finalised in a pass of their own, so that a tile costs the same
+// whatever the degrees.
 //
-// Tile work (one 512-lane workgroup, two resident per CU).
-//  1. Stage: a software pipeline keeps the next tile's gathers, row ends and
-//     finalisation operands, and the columns of the tile after it, in
-//     flight while a tile is processed (consecutive lanes on consecutive
-//     edges; values of the hottest sources come from an LDS cache).  A
-//     tile's values and row ends are then stored to LDS.
-//  2. Walk: lane t takes merge-path items [t*kUnits, (t+1)*kUnits), finds its
-//     starting (row, edge) by binary search in LDS and walks them in order,
-//     adding edge values and emitting a row sum at every row end.
-//  3. Carries: the partial of the row left open at the end of each lane is
-//     combined by a segmented scan over lanes (fixed tree order); the lane
-//     that emits a row adds the carries of the earlier lanes of that row.
-//  4. Finalise: the tile's row sums are written to LDS and finalised by
-//     consecutive lanes, so the per-row loads and stores are coalesced.
-// A row that began in an earlier tile is not finalised in the tile where it
-// ends: that tile stores its partial (head) and every tile stores the partial
-// of the row open at its end (tail); a second small launch adds the tails of
-// the earlier tiles to the head, in tile order, and finalises those rows.
-// Sums are compensated (Neumaier) in FP32 and plain in FP64; every reduction
-// has a fixed order, so results are bit-reproducible run to run.
+// Tile work (one wavefront, no workgroup barrier).
+//  1. The columns of the tile are loaded with consecutive lanes on consecutive
+//     edges (gathers of neighbouring sources then share cache lines), the
+//     values gathered and laid down in LDS.
+//  2. Each lane reads its 8 consecutive values and sums what follows its last
+//     row end; a segmented scan of those sums over the lanes (DPP, fixed
+//     order) gives every lane the open sum it continues.
+//  3. The lane walks its values once more from that sum and stores a row sum
+//     to LDS at each row end.
+//  4. Consecutive lanes finalise consecutive rows.
+// The sum left open at a tile's end is carried in a register to the next tile
+// of the chunk.  A row that began in an earlier chunk is not finalised where
+// it ends: the chunk stores its part (head), every chunk stores the sum of
+// the row open at its end (tail), and a second launch adds the tails of the
+// earlier chunks and the head, in a fixed order, and finalises those rows.
+// Sums are FP64 for both precisions (the FP32 values are summed in FP64, which
+// on this GPU takes one conversion and one addition where a compensated FP32
+// sum takes six operations); every order is fixed, so results are
+// bit-reproducible run to run.
 //
-// Src  : __device__ Real operator()(int64_t e, int32_t c) const  (value of
+// Bound: the gathers.  One request per edge reaches the L2 at about 130 G/s
+// whatever the occupancy (67M edges, 4.2M rows, FP32 with weights: 555 us;
+// 20.6M edges, 1.5M rows, FP64: 156 us, where a version with 512-lane
+// workgroups, a merge-path search per lane and workgroup barriers took 172 us
+// and 15 wavefronts fewer per CU), so what is left to save here is the fixed
+// cost of a small sweep.
+//
+// Src  : static constexpr bool kCol (false: the value does not need the column)
+//        __device__ Real operator()(int64_t e, int32_t c) const  (value of
 //        edge slot e whose column id is c)
 // Fin  : __device__ void load()  (read per-sweep scalars, once per thread)
 //        struct Pre; __device__ Pre pre(uint32_t r) const  (per-row operands,
 //        loaded early so their latency overlaps the tile's gathers)
-//        __device__ void operator()(uint32_t r, Real sum, const Pre&,
+//        __device__ void operator()(uint32_t r, double sum, const Pre&,
 //        double& a0, double& a1) const  (finalise row r; two FP64
 //        per-workgroup accumulators, e.g. residual and dangling mass)
 #pragma once
@@ -49,52 +59,13 @@
 namespace gx {
 namespace rs {
 
-constexpr int kBlock = 256;                 // generic kernels (reductions, spanning rows)
-constexpr int kSweepBlock = 512;            // tile workgroup: 8 wavefronts, two per CU with the LDS cache
-constexpr int kUnits = 8;                   // merge-path items per lane
-constexpr int kTile = kSweepBlock * kUnits; // items (row ends + edges) per tile
-constexpr int kWaves = kSweepBlock / kWave;
-constexpr int kSweepGrid = 256 * 8;         // upper bound of the persistent tile launch
-constexpr int kFixGrid = 256;               // workgroups of the spanning-row launch
+constexpr int kBlock = 256;          // 4 wavefronts
+constexpr int kWaves = kBlock / kWave;
+constexpr int kItems = 8;            // edges per lane and tile
+constexpr int kTile = kWave * kItems;
+constexpr int kSweepGrid = 256 * 8;  // workgroups of the sweep: 8 per CU
+constexpr int kFixGrid = 256;        // most workgroups of the spanning-row launch
 constexpr int kParts = kSweepGrid + kFixGrid;
-constexpr int kItems = kTile / kSweepBlock; // edges per lane at most (a tile has <= kTile edges)
-// LDS cache of the gathered vector for sources [0, kHot) (the hottest ones
-// in degree order), sized to what the tile leaves of the 160 KB of LDS.
-template <class Real>
-struct HotCache {
-  static constexpr int kHot = sizeof(Real) == 4 ? 11264 : 1024;
-};
-
-template <class Real>
-struct Acc;
-
-template <>
-struct Acc<float> {
-  float s = 0.f, c = 0.f;
-  __device__ __forceinline__ void add(float x) {
-    const float t = s + x;
-    if (fabsf(s) >= fabsf(x))
-      c += (s - t) + x;
-    else
-      c += (x - t) + s;
-    s = t;
-  }
-  __device__ __forceinline__ void merge(float os, float oc) {
-    add(os);
-    c += oc;
-  }
-  __device__ __forceinline__ float value() const { return s + c; }
-  __device__ __forceinline__ float comp() const { return c; }
-};
-
-template <>
-struct Acc<double> {
-  double s = 0.0;
-  __device__ __forceinline__ void add(double x) { s += x; }
-  __device__ __forceinline__ void merge(double os, double) { s += os; }
-  __device__ __forceinline__ double value() const { return s; }
-  __device__ __forceinline__ double comp() const { return 0.0; }
-};
 
 // Workgroup sum of one double per lane in a fixed order (valid in lane 0);
 // NT = threads of the workgroup, lds holds NT / 64 doubles.
@@ -115,320 +86,223 @@ template <class T>
 __device__ __forceinline__ T ld_stream(const T* p) {
   return __builtin_nontemporal_load(p);
 }
-typedef int v4i __attribute__((ext_vector_type(4)));
 
 struct RowPlan {
-  const int32_t* rowoff;  // n+1
-  const int32_t* col;     // len
-  int64_t n;              // rows
-  int64_t len;            // edges
-  int32_t* tile_row;      // ntiles+1: row of each tile's first item
-  int32_t* tile_edge;     // ntiles+1: edge of each tile's first item
-  int64_t ntiles;
+  const int32_t* rowoff;      // n+1
+  const int32_t* col;         // len
+  int64_t n;                  // rows
+  int64_t len;                // edges
+  const uint32_t* rid;        // rows with edges, ascending, then the rows without
+  int64_t full;               // rows with edges
+  const uint32_t* tile_row;   // ntiles+1: index in rid of the row of each tile's first edge
+  const uint32_t* lane_info;  // ntiles*64: bits 0..7 row ends, bits 8.. rows of the tile ended before
+  int64_t ntiles, nchunks;
+  int kt;                     // tiles per chunk
 };
 
 // Builds (or returns the cached) plan of a row-offset array; defined in
 // rowsweep.hip.
 RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64_t n, int64_t m, PullPlan& cache);
 
-// LDS index with one pad word per kUnits: lanes walk items kUnits apart, and
-// the pad spreads them over the banks.
-__device__ __forceinline__ int pad8(int j) { return j + j / kUnits; }
+// Tiles per chunk.
+inline int tiles_per_chunk(int64_t ntiles) {
+  return static_cast<int>(std::min<int64_t>(8, std::max<int64_t>(1, ntiles / (4 * kSweepGrid * kWaves))));
+}
 
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// Inclusive sum over lanes first..lane (first <= lane, the same for every lane
+// of a segment).  Fixed order: within rows of 16 lanes by shifts, then across
+// rows by broadcasts of their last lanes.
+__device__ __forceinline__ double wave_seg_scan(double v, int first, int lane) {
+  const int in_row = lane & 15;
+  double o;
+  o = dpp_f64<0x111, 0xf>(v);
+  if (in_row >= 1 && lane - 1 >= first) v += o;
+  o = dpp_f64<0x112, 0xf>(v);
+  if (in_row >= 2 && lane - 2 >= first) v += o;
+  o = dpp_f64<0x114, 0xf>(v);
+  if (in_row >= 4 && lane - 4 >= first) v += o;
+  o = dpp_f64<0x118, 0xf>(v);
+  if (in_row >= 8 && lane - 8 >= first) v += o;
+  o = dpp_f64<0x142, 0xa>(v);  // lane 15 of rows 0 and 2 to rows 1 and 3
+  if ((lane & 16) && (lane | 15) - 16 >= first) v += o;
+  o = dpp_f64<0x143, 0xc>(v);  // lane 31 to rows 2 and 3
+  if ((lane & 32) && 31 >= first) v += o;
+  return v;
+}
+
+// One LDS area per wavefront: first the tile's values (one pad word per kItems,
+// which spreads the lanes' reads over the banks), then its row sums.
 template <class Real>
-struct TileShared {
-  Real val[kTile + kTile / kUnits];          // edge values (padded index)
-  alignas(16) char rows[kTile * sizeof(Real)];  // relative row ends, then row sums
-  Real ws[kWaves], wc[kWaves];               // per-wave tail segment of the carries
-  int wkey[kWaves], wfirst[kWaves];          // its key; key of the wave's lane 0
-  Real ts[kWaves], tc[kWaves];               // tile tail partial per wave
+union WaveShared {
+  Real val[kTile + kTile / kItems];
+  double sum[kTile];
 };
 
-// Inclusive scan of (s, c) over the lanes of a wavefront, restarted wherever
-// `key` changes (equal keys are contiguous).  Fixed tree order.
-template <class Real>
-__device__ __forceinline__ Acc<Real> wave_seg_scan(int key, Acc<Real> a) {
-  const int lane = static_cast<int>(lane_id());
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const Real os = __shfl_up(a.s, off);
-    const Real oc = __shfl_up(a.comp(), off);
-    const int ok = __shfl_up(key, off);
-    if (lane >= off && ok == key) a.merge(os, oc);
-  }
-  return a;
-}
-
-struct TileCoord {
-  int32_t r0, r1, e0, e1;
-  bool defer0;  // row r0 began in an earlier tile and ends in this one
-};
-
-__device__ __forceinline__ TileCoord tile_coord(const RowPlan& P, int64_t T) {
-  TileCoord c;
-  c.r0 = P.tile_row[T];
-  c.r1 = P.tile_row[T + 1];
-  c.e0 = P.tile_edge[T];
-  c.e1 = P.tile_edge[T + 1];
-  c.defer0 = c.r1 > c.r0 && P.rowoff[c.r0] < c.e0;
-  return c;
-}
-
-// Columns of a tile: edge e0 + tid + i*kSweepBlock in cc[i].  Consecutive lanes
-// hold consecutive edges, so the gathers of one wavefront instruction hit
-// runs of neighbouring sources (rows in degree order have ascending, and for
-// heavy rows dense, source ids) that the texture unit coalesces into few
-// cache lines.
-__device__ __forceinline__ void tile_cols(const RowPlan& P, const TileCoord& tc, int32_t (&cc)[kItems]) {
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < kItems; ++i) {
-    const int64_t q = static_cast<int64_t>(tc.e0) + tid + i * kSweepBlock;
-    cc[i] = q < tc.e1 ? ld_stream(&P.col[q]) : 0;
-  }
-}
-
-// The loads of one tile, issued ahead of the tile's processing: columns
-// (two tiles ahead), then gathered values, the lane's first row end and the
-// finalisation operands of the lane's first row (one tile ahead).
-template <class Real, class Fin>
-struct Stage {
-  TileCoord tc;
-  bool valid;
-  int32_t cc[kItems];
-  Real v[kItems];
-  int32_t rend;
-  typename Fin::Pre pre;
-};
-
-template <class Real, class Fin>
-__device__ __forceinline__ void stage_cols(const RowPlan& P, int64_t T, Stage<Real, Fin>& st) {
-  st.valid = T < P.ntiles;
-  if (st.valid) {
-    st.tc = tile_coord(P, T);
-    tile_cols(P, st.tc, st.cc);
-  }
-}
-
-template <class Real, int HOT, class Src, class Fin>
-__device__ __forceinline__ void stage_gather(const RowPlan& P, const Src& src, const Fin& fin, const Real* hot,
-                                             Stage<Real, Fin>& st) {
-  if (!st.valid) return;
-  const int tid = threadIdx.x;
-  const int32_t e0 = st.tc.e0, e1 = st.tc.e1;
-#pragma unroll
-  for (int i = 0; i < kItems; ++i) {
-    const int64_t q = static_cast<int64_t>(e0) + tid + i * kSweepBlock;
-    if constexpr (HOT > 0)
-      st.v[i] = q < e1 ? src.apply(q, st.cc[i] < HOT ? hot[st.cc[i]] : src.load(st.cc[i])) : Real(0);
-    else
-      st.v[i] = q < e1 ? src(q, st.cc[i]) : Real(0);
-  }
-  const int nre = st.tc.r1 - st.tc.r0;
-  st.rend = tid < nre ? ld_stream(&P.rowoff[st.tc.r0 + 1 + tid]) : 0;
-  st.pre = tid < nre ? fin.pre(static_cast<uint32_t>(st.tc.r0 + tid)) : typename Fin::Pre{};
-}
-
-// One tile (see the file comment); its loads were issued by stage_gather
-// one tile earlier.
+// One launch over every chunk (chunk c on wavefront c mod the grid's) and the
+// rows without edges.  Workgroup partials of the two accumulators go to
+// part0/part1[blockIdx.x].  Returns at once when *skip is non-zero (a
+// converged iteration loop).  carry: 2 * nchunks.
 template <class Real, class Src, class Fin>
-__device__ __forceinline__ void sweep_tile(int64_t T, const RowPlan& P, const Fin& fin, TileShared<Real>& sh,
-                                           Real* __restrict__ carry, const Stage<Real, Fin>& st, double& a0,
-                                           double& a1) {
-  const int tid = threadIdx.x;
-  const int lane = static_cast<int>(lane_id());
-  const int wid = tid / kWave;
-  const TileCoord& tc = st.tc;
-  const int32_t r0 = tc.r0, e0 = tc.e0, e1 = tc.e1;
-  const int nre = tc.r1 - r0;  // row ends in this tile
-  const int ned = e1 - e0;     // edges in this tile
-  const int L = nre + ned;
-  const bool defer0 = tc.defer0;
-  int32_t* s_end = reinterpret_cast<int32_t*>(sh.rows);
-  Real* s_sum = reinterpret_cast<Real*>(sh.rows);
-  const typename Fin::Pre& pre0 = st.pre;
-
-  // 1. Values and row ends to LDS.
-  if (tid < nre) s_end[tid] = st.rend - e0;
-  for (int j = tid + kSweepBlock; j < nre; j += kSweepBlock) s_end[j] = ld_stream(&P.rowoff[r0 + 1 + j]) - e0;
-#pragma unroll
-  for (int i = 0; i < kItems; ++i) {
-    const int j = tid + i * kSweepBlock;
-    if (j < ned) sh.val[pad8(j)] = st.v[i];
-  }
-  __syncthreads();
-
-  // 2. Walk this lane's merge-path items.
-  const int d = tid * kUnits;
-  int rr = 0, ee = 0;
-  if (d < L) {
-    int lo = max(0, d - ned), hi = min(d, nre);  // rows ended before item d
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (s_end[mid - 1] + mid <= d) lo = mid; else hi = mid - 1;
-    }
-    rr = lo;
-    ee = d - lo;
-  }
-  Acc<Real> acc, first;
-  Real em[kUnits];
-  uint32_t emask = 0;
-  int rstart = 0;
-#pragma unroll
-  for (int u = 0; u < kUnits; ++u) {
-    em[u] = Real(0);
-    if (d + u < L) {
-      if (rr < nre && ee >= s_end[rr]) {
-        if (emask == 0) {
-          first = acc;
-          rstart = rr;
-        }
-        em[u] = acc.value();
-        emask |= 1u << u;
-        acc = Acc<Real>();
-        ++rr;
-      } else {
-        acc.add(sh.val[pad8(ee)]);
-        ++ee;
-      }
-    }
-  }
-
-  // 3. Carries: key = the row left open by this lane.
-  const int key = (d < L) ? rr : INT_MAX;
-  const Acc<Real> seg = wave_seg_scan(key, acc);
-  const Real prev_s = __shfl_up(seg.s, 1);
-  const Real prev_c = __shfl_up(seg.comp(), 1);
-  const int prev_key = __shfl_up(key, 1);
-  const int key0 = __shfl(key, 0);
-  if (lane == kWave - 1) {
-    sh.ws[wid] = seg.s;
-    sh.wc[wid] = seg.comp();
-    sh.wkey[wid] = key;
-  }
-  if (lane == 0) sh.wfirst[wid] = key;
-  // Tile tail: the carries of the row open at the tile's end (local nre).
-  Acc<Real> tail;
-  if (key == nre) tail = acc;
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const Real os = __shfl_xor(tail.s, off);
-    const Real oc = __shfl_xor(tail.comp(), off);
-    tail.merge(os, oc);
-  }
-  if (lane == 0) {
-    sh.ts[wid] = tail.s;
-    sh.tc[wid] = tail.comp();
-  }
-  __syncthreads();  // walk done: s_end may now be overwritten by row sums
-
-  if (emask) {
-    Acc<Real> f = first;
-    if (lane > 0 && prev_key == rstart) f.merge(prev_s, prev_c);
-    if (key0 == rstart || lane == 0) {
-      // The run of this row reaches lane 0: add earlier wavefronts whose
-      // trailing segment belongs to it.
-      for (int w = wid - 1; w >= 0 && sh.wkey[w] == rstart; --w) {
-        f.merge(sh.ws[w], sh.wc[w]);
-        if (sh.wfirst[w] != rstart) break;
-      }
-    }
-    const Real fval = f.value();
-    int k = 0;
-#pragma unroll
-    for (int u = 0; u < kUnits; ++u) {
-      if ((emask >> u) & 1u) {
-        const int r = rstart + k;
-        const Real val = (k == 0) ? fval : em[u];
-        if (r == 0 && defer0)
-          carry[T] = val;  // head of a row that began in an earlier tile
-        else
-          s_sum[r] = val;
-        ++k;
-      }
-    }
-  }
-  if (tid == 0) {
-    Acc<Real> t;
-    for (int w = 0; w < kWaves; ++w) t.merge(sh.ts[w], sh.tc[w]);
-    carry[P.ntiles + T] = t.s;
-    carry[2 * P.ntiles + T] = t.comp();
-  }
-  __syncthreads();
-
-  // 4. Finalise the rows that end here (coalesced).
-  if (tid < nre && (tid > 0 || !defer0)) fin(static_cast<uint32_t>(r0 + tid), s_sum[tid], pre0, a0, a1);
-  for (int j = tid + kSweepBlock; j < nre; j += kSweepBlock)
-    fin(static_cast<uint32_t>(r0 + j), s_sum[j], fin.pre(static_cast<uint32_t>(r0 + j)), a0, a1);
-  __syncthreads();
-}
-
-// One launch over every tile (persistent workgroups; tile T runs on
-// workgroup T mod gridDim.x).  Workgroup partials of the two accumulators
-// go to part0/part1[blockIdx.x].  Returns at once when *skip is non-zero (a
-// converged iteration loop).  With HOT > 0 the gathered vector of sources
-// [0, HOT) is first copied to LDS (src.load(c) is the gathered value,
-// src.apply(e, value) the edge's term).
-template <class Real, int HOT, class Src, class Fin>
-__global__ void __launch_bounds__(kSweepBlock) sweep_kernel(RowPlan P, Src src, Fin fin,
-                                                            const unsigned* __restrict__ skip,
-                                                            double* __restrict__ part0, double* __restrict__ part1,
-                                                            Real* __restrict__ carry) {
+__global__ void __launch_bounds__(kBlock) sweep_kernel(RowPlan P, Src src, Fin fin, const unsigned* __restrict__ skip,
+                                                       double* __restrict__ part0, double* __restrict__ part1,
+                                                       double* __restrict__ carry) {
   if (skip && *skip) return;
   fin.load();
-  __shared__ TileShared<Real> sh;
+  __shared__ WaveShared<Real> shared[kWaves];
   __shared__ double red[kWaves];
-  __shared__ Real hot[HOT > 0 ? HOT : 1];
-  if constexpr (HOT > 0) {
-    const int64_t nh = P.n < HOT ? P.n : HOT;
-    for (int64_t i = threadIdx.x; i < nh; i += kSweepBlock) hot[i] = src.load(static_cast<int32_t>(i));
-    __syncthreads();
-  }
+  const int lane = static_cast<int>(lane_id());
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  WaveShared<Real>& sh = shared[wid];
   double a0 = 0, a1 = 0;
-  // Software pipeline: tile T is processed while the gathers of tile
-  // T + grid and the columns of tile T + 2*grid are in flight.
-  const int64_t G = gridDim.x;
-  int64_t T = blockIdx.x;
-  Stage<Real, Fin> cur, nxt;
-  stage_cols(P, T, cur);
-  stage_gather<Real, HOT>(P, src, fin, hot, cur);
-  stage_cols(P, T + G, nxt);
-  for (; T < P.ntiles; T += G) {
-    stage_gather<Real, HOT>(P, src, fin, hot, nxt);
-    Stage<Real, Fin> after;
-    stage_cols(P, T + 2 * G, after);
-    sweep_tile<Real, Src>(T, P, fin, sh, carry, cur, a0, a1);
-    cur = nxt;
-    nxt = after;
+  const int64_t nwaves = static_cast<int64_t>(gridDim.x) * kWaves;
+  for (int64_t c = static_cast<int64_t>(blockIdx.x) * kWaves + wid; c < P.nchunks; c += nwaves) {
+    const int64_t T0 = c * P.kt, T1 = T0 + P.kt < P.ntiles ? T0 + P.kt : P.ntiles;
+    uint32_t k0 = P.tile_row[T0];
+    // The chunk's first row began in an earlier chunk.
+    bool defer = P.rowoff[P.rid[k0]] < T0 * kTile;
+    double open = 0;  // sum of the row open at the start of the tile (uniform)
+    for (int64_t T = T0; T < T1; ++T) {
+      const int64_t e0 = T * kTile;
+      const int ned = static_cast<int>(P.len - e0 < kTile ? P.len - e0 : kTile);
+      const uint32_t k1 = P.tile_row[T + 1];
+      const int nrow = static_cast<int>(k1 - k0);  // rows that end in this tile
+      int32_t cc[kItems];
+      if constexpr (Src::kCol) {
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+          const int j = lane + i * kWave;
+          cc[i] = j < ned ? ld_stream(&P.col[e0 + j]) : 0;
+        }
+      }
+      const uint32_t info = ld_stream(&P.lane_info[T * kWave + lane]);
+      const uint32_t row = lane < nrow ? P.rid[k0 + lane] : 0u;
+      const typename Fin::Pre pre = lane < nrow ? fin.pre(row) : typename Fin::Pre{};
+      Real v[kItems];
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {
+        const int j = lane + i * kWave;
+        v[i] = j < ned ? src(e0 + j, Src::kCol ? cc[i] : 0) : Real(0);
+      }
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {
+        const int j = lane + i * kWave;
+        sh.val[j + j / kItems] = v[i];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) v[u] = sh.val[lane * (kItems + 1) + u];
+      // Sum after the lane's last row end, scanned over the lanes.
+      const uint32_t ends = info & 0xffu;
+      double tail = 0;
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) {
+        tail += static_cast<double>(v[u]);
+        if ((ends >> u) & 1u) tail = 0;
+      }
+      const uint64_t heads = __ballot(ends != 0);
+      const uint64_t upto = heads & (~0ull >> (63 - lane));
+      const double seg = wave_seg_scan(tail, upto ? 63 - __builtin_clzll(upto) : 0, lane);
+      double acc = __shfl_up(seg, 1);
+      if (lane == 0) acc = 0;
+      if ((heads & ((1ull << lane) - 1)) == 0) acc += open;
+      const double last = __shfl(seg, kWave - 1);
+      open = heads ? last : open + last;
+      // Row sums (the values are in registers: the LDS area is free).
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      uint32_t slot = info >> 8;
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) {
+        acc += static_cast<double>(v[u]);
+        if ((ends >> u) & 1u) {
+          sh.sum[slot++] = acc;
+          acc = 0;
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (lane < nrow) {
+        const double s = sh.sum[lane];
+        if (lane == 0 && defer)
+          carry[c] = s;  // head of a row that began in an earlier chunk
+        else
+          fin(row, s, pre, a0, a1);
+      }
+      for (int j = lane + kWave; j < nrow; j += kWave) {
+        const uint32_t r = P.rid[k0 + j];
+        fin(r, sh.sum[j], fin.pre(r), a0, a1);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (nrow > 0) defer = false;
+      k0 = k1;
+    }
+    if (lane == 0) carry[P.nchunks + c] = open;
   }
-  a0 = block_sum<kSweepBlock>(a0, red);
-  a1 = block_sum<kSweepBlock>(a1, red);
+  // Rows without edges.
+  for (int64_t i = P.full + static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < P.n;
+       i += static_cast<int64_t>(gridDim.x) * kBlock) {
+    const uint32_t r = P.rid[i];
+    fin(r, 0.0, fin.pre(r), a0, a1);
+  }
+  a0 = block_sum(a0, red);
+  a1 = block_sum(a1, red);
   if (threadIdx.x == 0) {
     part0[blockIdx.x] = a0;
     part1[blockIdx.x] = a1;
   }
 }
 
-// Rows that span tiles: head of the tile where the row ends plus the tails
-// of the earlier tiles, latest first.
-template <class Real, class Fin>
+// Rows that span chunks: the tails of the chunks before the one where the row
+// ends, then that chunk's head.  A lane per chunk looks for such a row; the
+// wavefront then sums each found row's tails together (a hub spans thousands).
+template <class Fin>
 __global__ void __launch_bounds__(kBlock) span_finalize_kernel(RowPlan P, Fin fin, const unsigned* __restrict__ skip,
-                                                               const Real* __restrict__ carry,
+                                                               const double* __restrict__ carry,
                                                                double* __restrict__ part0,
                                                                double* __restrict__ part1) {
   if (skip && *skip) return;
   fin.load();
-  __shared__ double red[kBlock / kWave];
+  __shared__ double red[kWaves];
+  const int lane = static_cast<int>(lane_id());
+  const int64_t chunk_edges = static_cast<int64_t>(P.kt) * kTile;
   double a0 = 0, a1 = 0;
-  for (int64_t T = blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x; T < P.ntiles;
-       T += static_cast<int64_t>(gridDim.x) * kBlock) {
-    const int32_t r0 = P.tile_row[T];
-    if (r0 >= P.tile_row[T + 1] || P.rowoff[r0] >= P.tile_edge[T]) continue;
-    Acc<Real> a;
-    a.merge(carry[T], Real(0));
-    for (int64_t t2 = T - 1; t2 >= 0 && P.tile_row[t2 + 1] == r0; --t2)
-      a.merge(carry[P.ntiles + t2], carry[2 * P.ntiles + t2]);
-    fin(static_cast<uint32_t>(r0), a.value(), fin.pre(static_cast<uint32_t>(r0)), a0, a1);
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
+  for (int64_t b = static_cast<int64_t>(blockIdx.x) * kBlock + (threadIdx.x & ~(kWave - 1)); b < P.nchunks;
+       b += stride) {
+    const int64_t c = b + lane;
+    uint32_t r = 0;
+    int32_t first = 0;
+    bool spans = false;
+    if (c > 0 && c < P.nchunks) {
+      r = P.rid[P.tile_row[c * P.kt]];
+      const int32_t rb = P.rowoff[r], re = P.rowoff[r + 1];
+      spans = rb < c * chunk_edges && re <= (c + 1) * chunk_edges;
+      first = static_cast<int32_t>(rb / chunk_edges);
+    }
+    double sum = 0;
+    // Short spans by their own lane, long ones by the whole wavefront.
+    constexpr int kAlone = 8;
+    if (spans && c - first <= kAlone)
+      for (int64_t t = first; t < c; ++t) sum += carry[P.nchunks + t];
+    for (uint64_t todo = __ballot(spans && c - first > kAlone); todo; todo &= todo - 1) {
+      const int i = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+      const int64_t f = __shfl(first, i), e = b + i;
+      double s = 0;
+      for (int64_t t = f + lane; t < e; t += kWave) s += carry[P.nchunks + t];
+      s = wave_sum(s);
+      if (lane == i) sum = s;
+    }
+    if (spans) fin(r, sum + carry[c], fin.pre(r), a0, a1);
   }
   a0 = block_sum(a0, red);
   a1 = block_sum(a1, red);
@@ -439,30 +313,22 @@ __global__ void __launch_bounds__(kBlock) span_finalize_kernel(RowPlan P, Fin fi
 }
 
 // Host: one full sweep (tile launch + spanning-row launch) on stream s.
-// part0/part1 hold kParts entries each and carry 3 * P.ntiles; returns the
+// part0/part1 hold kParts entries each and carry 2 * P.nchunks; returns the
 // number of partials written (at most kParts, contiguous from 0).  `timer`
-// brackets the tile launch.  HOT > 0 caches the gathered values of sources
-// [0, HOT) in LDS (only worth it when the lowest ids are the most gathered,
-// as in the degree-ordered PageRank pull).
-template <class Real, int HOT = 0, class Src, class Fin>
+// brackets the tile launch.
+template <class Real, class Src, class Fin>
 int launch_sweep(const RowPlan& P, const Src& src, const Fin& fin, const unsigned* skip, double* part0,
-                 double* part1, Real* carry, hipStream_t s, KernelTimer* timer) {
-  // Persistent grid: every workgroup resident at once (occupancy x CUs).
-  static const int grid = [] {
-    int per_cu = 0, dev = 0, cus = 0;
-    GX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sweep_kernel<Real, HOT, Src, Fin>, kSweepBlock,
-                                                        0));
-    GX_HIP(hipGetDevice(&dev));
-    GX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    return std::max(1, std::min(kSweepGrid, per_cu * cus));
-  }();
+                 double* part1, double* carry, hipStream_t s, KernelTimer* timer) {
+  const int64_t items = std::max<int64_t>(P.nchunks * kWave, P.n - P.full);
+  const int grid = static_cast<int>(grid_for(items, kBlock, kSweepGrid));
   if (timer) timer->begin();
-  sweep_kernel<Real, HOT, Src, Fin><<<grid, kSweepBlock, 0, s>>>(P, src, fin, skip, part0, part1, carry);
+  sweep_kernel<Real, Src, Fin><<<grid, kBlock, 0, s>>>(P, src, fin, skip, part0, part1, carry);
   if (timer) timer->end();
   GX_LAUNCHED("sweep_kernel");
-  span_finalize_kernel<Real, Fin><<<kFixGrid, kBlock, 0, s>>>(P, fin, skip, carry, part0 + grid, part1 + grid);
+  const int fix = static_cast<int>(grid_for(P.nchunks, kBlock, kFixGrid));
+  span_finalize_kernel<Fin><<<fix, kBlock, 0, s>>>(P, fin, skip, carry, part0 + grid, part1 + grid);
   GX_LAUNCHED("span_finalize_kernel");
-  return grid + kFixGrid;
+  return grid + fix;
 }
 
 }  // namespace rs

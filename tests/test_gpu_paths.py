@@ -53,3 +53,81 @@ def test_cc_orders_and_components(gx, oracle, n, m, order):
     exp = oracle.cc(row, col)
     for _ in range(3):  # scratch of an earlier call
         assert np.array_equal(u32(gx.connected_components(G)[0]), exp)
+
+
+def weighted_csr(n, m, seed, hub_rows=0):
+    """Directed CSR with float32 weights; the first hub_rows rows hold half of
+    the edges, so that rows span several tiles and chunks of tiles."""
+    rng = np.random.default_rng(seed)
+    u = rng.integers(0, n, m)
+    if hub_rows:
+        u[:m // 2] = rng.integers(0, hub_rows, m // 2)
+    v = rng.integers(0, n, m)
+    key = np.unique(u.astype(np.int64) * n + v)
+    u, v = key // n, key % n
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=n), out=row[1:])
+    w = rng.lognormal(size=len(u)).astype(np.float32)
+    return row, v.astype(np.int32), w
+
+
+def weighted_reference(row, col, w, t, c, alpha=0.85, tol=1e-15, iters=300):
+    """Forward vector, weight gradients and teleport gradients in FP64 (numpy
+    sums pairwise: the oracle adds 200,000 dangling terms one after another,
+    which alone is 1.2e-12 off)."""
+    import scipy.sparse as sp
+    n = len(row) - 1
+    A = sp.csr_matrix((w.astype(np.float64), col, row), shape=(n, n))
+    s = np.asarray(A.sum(1)).ravel()
+    none = s == 0
+    inv = np.divide(1.0, s, out=np.zeros(n), where=~none)
+    At = sp.csr_matrix(A.T)
+
+    def fixed_point(step, x):
+        for _ in range(iters):
+            new = step(x)
+            done = np.abs(new - x).sum() < tol
+            x = new
+            if done:
+                break
+        return x
+
+    t, c = t.astype(np.float64), c.astype(np.float64)
+    x = fixed_point(lambda x: alpha * (At @ (x * inv) + x[none].sum() / n) + (1 - alpha) * t, np.full(n, 1.0 / n))
+    below = lambda lam: (A @ lam) * inv + none * (lam.sum() / n)  # noqa: E731
+    lam = fixed_point(lambda v: c + alpha * below(v), c)
+    src = np.repeat(np.arange(n), np.diff(row))
+    # The terms whose difference a weight's gradient is, for its error's scale.
+    terms = (alpha * np.abs(x[src]) * np.abs(lam).max() * inv[src]).max()
+    return x, alpha * x[src] * (lam[col] - below(lam)[src]) * inv[src], (1 - alpha) * lam, terms
+
+
+# (vertices, edges drawn, hub rows): one edge; one tile less one, full and plus
+# one edge; rows over several tiles; one row over every chunk; mostly empty rows.
+SWEEPS = [(2, 1, 0), (600, 511, 0), (600, 513, 0), (5000, 20000, 3), (3000, 9000, 1), (200003, 60000, 2),
+          (40001, 700000, 1)]
+
+
+@pytest.mark.parametrize("n,m,hubs", SWEEPS)
+def test_row_sweep_shapes(gx, n, m, hubs):
+    """Weighted forward and adjoint in FP64 (FP64 sums of FP64 products: 1e-12
+    relative to the largest value) and FP32 (1e-5 of it: 40-odd iterations of
+    FP32 rounding) over shapes at the edges of tiles and chunks.  A weight's
+    gradient is a difference (lambda_v - (P lambda)_u) scaled by x_u / s_u, zero
+    for the only edge of a row: its errors are relative to the terms."""
+    import torch
+    row, col, w = weighted_csr(n, m, n + m, hubs)
+    rng = np.random.default_rng(1)
+    t = rng.random(n).astype(np.float32)
+    t /= t.sum()
+    c = (rng.standard_normal(n) / n).astype(np.float32)
+    print(f"row sweep n={n} m={len(col)}", flush=True)
+    G = gx.Graph.from_csr(row, col, w)
+    tt, cc, ww = torch.from_numpy(t).cuda(), torch.from_numpy(c).cuda(), torch.from_numpy(w).cuda()
+    x_ref, gw_ref, gt_ref, terms = weighted_reference(row, col, w, t, c)
+    for prec, rel in (("fp64", 1e-12), ("fp32", 1e-5)):
+        x, _ = gx.pagerank_weighted(G, ww, tt, tol=1e-15, max_iter=300, precision=prec)
+        gw, gt, _ = gx.pagerank_adjoint(G, ww, x, cc, tol=1e-15, max_iter=300, precision=prec)
+        for got, ref, scale in ((x, x_ref, np.abs(x_ref).max()), (gw, gw_ref, terms), (gt, gt_ref, np.abs(gt_ref).max())):
+            got = got.cpu().numpy().astype(np.float64)
+            assert np.abs(got - ref).max() <= rel * scale, (prec, np.abs(got - ref).max(), scale)
