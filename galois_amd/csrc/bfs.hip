@@ -17,9 +17,13 @@
 //    frontier.hpp (degree above frontier.hub_degree, 128 by default, goes
 //    to a grid-wide hub pass).  Discovery is
 //    an atomicCAS on the level word, so each vertex enters the next frontier
-//    once.  New vertices are staged in an LDS queue and moved to the global
-//    frontier with one atomic per workgroup flush; per-lane counters are
-//    reduced once per workgroup.
+//    once.  New vertices are staged per wavefront in LDS; a workgroup takes
+//    room for what is left at its end, and adds the degrees of what it found,
+//    with one atomic on one packed word (see frontier.hpp: with 2048
+//    workgroups and two words, two thirds of an RMAT-18 level went into
+//    them; RMAT-18 375 -> 286 us, direction-optimising RMAT-24 1209 -> 1004
+//    us, 4096 vertices 248 -> 153 us, most of the last from spreading small
+//    frontiers over more workgroups).
 //  - gx_bfs drives its levels on the device: each level is a fixed kernel
 //    sequence (begin, expand, hubs, end) that reads the frontier size from a
 //    device state word; levels are captured in HIP graphs (7 for the first
@@ -38,15 +42,14 @@ using namespace gx;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kQCap = 2048;
+constexpr int kQCap = 4096;  // bitmap_to_queue_kernel
 constexpr uint32_t kInf = GX_DIST_INFINITY;
 constexpr uint32_t kNoParent = 0xffffffffu;
-constexpr int kGrid = 256 * 8;
 // Graphs without hubs (maximum degree at or below the hub threshold, such as
-// road-like grids) have small frontiers per step and many steps; a quarter
-// of the workgroups per launch costs less there (2048-grid SSSP 26.4 ->
-// 21.7 ms, BFS 2.03 -> 1.57 ms), while RMAT frontiers need the full grid.
-constexpr int kGridNoHubs = 512;
+// road-like grids) have small frontiers per level and many levels: a quarter
+// of the workgroups start faster.
+constexpr int kGridNoHubs = 128;
+constexpr int kHubLanes = 256;  // lanes per step of the hub pass
 constexpr int kLevelsPerGraph = 8;
 constexpr int kLevelsFirst = 7;  // first replay: power-law graphs need 5-6 levels plus the empty one
 
@@ -58,8 +61,10 @@ struct BfsState {
   unsigned level;         // level being written
   unsigned active;        // this level has a frontier
   unsigned done;
-  unsigned found;         // vertices found by a pull step
-  unsigned pad;
+  // Vertices discovered this level (low 32 bits: also the end of the queue a
+  // push fills) and their degree sum (high 32 bits; it is at most m < 2^31),
+  // so that a workgroup adds both with one atomic.
+  unsigned long long app;
   unsigned long long scout;  // degree sum of the vertices discovered this level
   unsigned long long edges;  // degree sum of every discovered vertex
   unsigned long long items;
@@ -107,7 +112,7 @@ __global__ void bfs_reset_kernel(BfsState* S, uint32_t* q0, uint32_t src, uint32
     S->level = 0;
     S->active = 0;
     S->done = 0;
-    S->found = 0;
+    S->app = 0;
     S->scout = 0;
     S->edges = 0;
     S->items = 1;
@@ -123,14 +128,15 @@ __device__ __forceinline__ void level_begin(BfsState* S) {
   }
   S->active = 1;
   S->level += 1;
-  S->count[S->q ^ 1] = 0;
+  S->app = 0;
   S->hub_count = 0;
-  S->scout = 0;
 }
 
 __device__ __forceinline__ void level_end(BfsState* S) {
   if (!S->active) return;
   S->q ^= 1;
+  S->count[S->q] = static_cast<unsigned>(S->app);
+  S->scout = S->app >> 32;
   S->items += S->count[S->q];
   S->edges += S->scout;
   S->active = 0;
@@ -162,82 +168,91 @@ struct TdOp {
   uint32_t* level;
   uint32_t* parent;
   uint32_t* qout;
-  unsigned* qcount;
   unsigned cap;
   BfsState* S;
-  LdsQueue<kQCap>* sq;
+  WaveQueue<kWaveQCap> wq;
   uint32_t nl;
   unsigned long long scout;  // this lane's degree sum of discovered vertices
   uint32_t* vis;
   // With a visited bitmap (n/8 bytes, mostly cache-resident) an edge to an
   // already discovered vertex is dropped without the random read of its
   // level word; a bit set late only sends the edge on to the level check.
-  __device__ __forceinline__ void operator()(bool valid, uint32_t u, int32_t e) {
-    bool won = false;
-    uint32_t v = 0;
-    if (valid) {
-      v = static_cast<uint32_t>(col[e]);
-      const bool seen = vis && ((vis[v >> 5] >> (v & 31)) & 1u);
-      if (!seen && level[v] == kInf && atomicCAS(&level[v], kInf, nl) == kInf) {
-        won = true;
-        if (vis) atomicOr(&vis[v >> 5], 1u << (v & 31));
-        if (parent) parent[v] = u;
-        scout += static_cast<unsigned long long>(row[v + 1] - row[v]);
+  template <int U>
+  __device__ __forceinline__ void run(const bool (&valid)[U], const uint32_t (&u)[U], const int32_t (&e)[U]) {
+    bool won[U];
+    uint32_t v[U], lv[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = static_cast<uint32_t>(col[e[k]]);
+    if (vis) {
+#pragma unroll
+      for (int k = 0; k < U; ++k) won[k] = valid[k] && !((vis[v[k] >> 5] >> (v[k] & 31)) & 1u);
+#pragma unroll
+      for (int k = 0; k < U; ++k) lv[k] = won[k] ? level[v[k]] : 0u;
+    } else {
+#pragma unroll
+      for (int k = 0; k < U; ++k) lv[k] = level[v[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      won[k] = valid[k] && lv[k] == kInf && atomicCAS(&level[v[k]], kInf, nl) == kInf;
+      if (won[k]) {
+        if (vis) atomicOr(&vis[v[k] >> 5], 1u << (v[k] & 31));
+        if (parent) parent[v[k]] = u[k];
+        scout += static_cast<unsigned long long>(row[v[k] + 1] - row[v[k]]);
       }
     }
-    lq_push(*sq, won, v);
+    wq.push(won, v);
   }
-  __device__ __forceinline__ void after_step() { lq_flush(*sq, qout, qcount, cap, &S->overflow, false); }
+  // Room in the next queue, and the degree sum of what was found, with one atomic.
+  __device__ __forceinline__ void after_step() {
+    if (!wq.full(kWideStep)) return;
+    unsigned base = 0;
+    if (lane_id() == 0) base = static_cast<unsigned>(atomicAdd(&S->app, static_cast<unsigned long long>(wq.count)));
+    wq.store(__builtin_amdgcn_readfirstlane(base), qout, cap, &S->overflow);
+  }
+  // Workgroup-uniform: what is left, for all wavefronts at once.
+  __device__ __forceinline__ void finish() {
+    __shared__ unsigned long long s_sum[kWideWaves + 1];
+    unsigned long long total;
+    const unsigned long long before =
+        waves_exclusive_sum<kWideBlock>(wq.count | (wave_sum(scout) << 32), s_sum, &total);
+    if (threadIdx.x == 0) s_sum[kWideWaves] = total ? atomicAdd(&S->app, total) : 0ull;
+    __syncthreads();
+    wq.store(static_cast<unsigned>(s_sum[kWideWaves]) + static_cast<unsigned>(before), qout, cap, &S->overflow);
+  }
 };
 
-__device__ __forceinline__ TdOp make_td(const Bufs& B, LdsQueue<kQCap>* sq) {
+__device__ __forceinline__ TdOp make_td(const Bufs& B, uint32_t (&stage)[kWideWaves][kWaveQCap]) {
   BfsState* S = B.S;
-  const unsigned nq = S->q ^ 1;
-  return TdOp{B.row, B.col, S->level_out, S->parent_out, B.q[nq], &S->count[nq], B.cap, S, sq, S->level, 0ull, B.vis};
+  return TdOp{B.row, B.col, S->level_out, S->parent_out, B.q[S->q ^ 1], B.cap, S, {stage[threadIdx.x / kWave]},
+              S->level, 0ull, B.vis};
 }
 
-// Workgroup-uniform: the scout count is summed over the workgroup, so the
-// state word takes one atomic per workgroup rather than one per wavefront.
-__device__ __forceinline__ void td_finish(TdOp& op) {
-  lq_flush(*op.sq, op.qout, op.qcount, op.cap, &op.S->overflow, true);
-  __shared__ unsigned long long s_sc[kBlock / kWave];
-  const unsigned long long sc = wave_sum(op.scout);
-  if (lane_id() == 0) s_sc[threadIdx.x / kWave] = sc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    for (int i = 0; i < kBlock / kWave; ++i) t += s_sc[i];
-    if (t) atomicAdd(&op.S->scout, t);
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) td_expand_kernel(Bufs B) {
+__global__ void __launch_bounds__(kWideBlock) td_expand_kernel(Bufs B) {
   BfsState* S = B.S;
   if (!S->active) return;
-  __shared__ LdsQueue<kQCap> sq;
-  lq_init(sq);
-  TdOp op = make_td(B, &sq);
-  expand_queue<kBlock>(B.row, B.q[S->q], S->count[S->q], B.hub, B.hubq, &S->hub_count, B.cap, &S->overflow, op);
-  td_finish(op);
+  __shared__ uint32_t stage[kWideWaves][kWaveQCap];
+  TdOp op = make_td(B, stage);
+  expand_queue<kWideBlock, TdOp, false, kWideEdges>(B.row, B.q[S->q], S->count[S->q], B.hub, B.hubq, &S->hub_count, B.cap, &S->overflow, op);
+  op.finish();
 }
 
-__global__ void __launch_bounds__(kBlock) td_hubs_kernel(Bufs B) {
+__global__ void __launch_bounds__(kWideBlock) td_hubs_kernel(Bufs B) {
   BfsState* S = B.S;
   if (!S->active || S->hub_count == 0) return;
-  __shared__ LdsQueue<kQCap> sq;
-  lq_init(sq);
-  TdOp op = make_td(B, &sq);
-  expand_hubs<kBlock>(B.row, B.hubq, S->hub_count, B.cap, B.hub_off, op);
-  td_finish(op);
+  __shared__ uint32_t stage[kWideWaves][kWaveQCap];
+  TdOp op = make_td(B, stage);
+  expand_hubs<kWideBlock, TdOp, kHubLanes, kWideEdges>(B.row, B.hubq, S->hub_count, B.cap, B.hub_off, op);
+  op.finish();
 }
 
 // Expansion of one level.  `hubs` false: no vertex exceeds the hub
 // threshold, so the hub list stays empty and its two launches are left out.
 void enqueue_expand(const Bufs& B, bool hubs, hipStream_t s) {
-  td_expand_kernel<<<hubs ? kGrid : kGridNoHubs, kBlock, 0, s>>>(B);
+  td_expand_kernel<<<hubs ? kWideGrid : kGridNoHubs, kWideBlock, 0, s>>>(B);
   if (hubs) {
-    launch_hub_offsets<kBlock>(B.row, B.hubq, &B.S->hub_count, B.cap, B.hub_off, s);
-    td_hubs_kernel<<<kGrid, kBlock, 0, s>>>(B);
+    launch_hub_offsets<kHubLanes * kWideEdges>(B.row, B.hubq, &B.S->hub_count, B.cap, B.hub_off, s);
+    td_hubs_kernel<<<kWideGrid, kWideBlock, 0, s>>>(B);
   }
 }
 
@@ -274,15 +289,14 @@ __global__ void queue_to_bitmap_kernel(const uint32_t* __restrict__ q, const uns
 }
 
 // Every unreached vertex looks for a frontier in-neighbour.
-__global__ void __launch_bounds__(kBlock) bu_step_kernel(const int32_t* __restrict__ trow,
+__global__ void __launch_bounds__(kWideBlock) bu_step_kernel(const int32_t* __restrict__ trow,
                                                          const int32_t* __restrict__ tcol,
                                                          const int32_t* __restrict__ row,
                                                          uint32_t* __restrict__ level, uint32_t* __restrict__ parent,
                                                          const uint32_t* __restrict__ front,
                                                          uint32_t* __restrict__ next, BfsState* S, int64_t n,
                                                          uint32_t nl) {
-  __shared__ unsigned long long red[kBlock / kWave];
-  __shared__ unsigned redc[kBlock / kWave];
+  __shared__ unsigned long long red[kWideWaves];
   unsigned long long deg = 0;
   unsigned found = 0;
   for (int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; v < n;
@@ -300,28 +314,13 @@ __global__ void __launch_bounds__(kBlock) bu_step_kernel(const int32_t* __restri
       }
     }
   }
-  deg = wave_sum(deg);
-  found = wave_sum(found);
-  if (lane_id() == 0) {
-    red[threadIdx.x / kWave] = deg;
-    redc[threadIdx.x / kWave] = found;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long d = 0;
-    unsigned f = 0;
-    for (int i = 0; i < kBlock / kWave; ++i) {
-      d += red[i];
-      f += redc[i];
-    }
-    if (f) {
-      atomicAdd(&S->found, f);
-      atomicAdd(&S->scout, d);
-    }
-  }
+  // Degree sum and count in one word, as the pushes add them.
+  unsigned long long both;
+  waves_exclusive_sum<kWideBlock>(wave_sum((deg << 32) | found), red, &both);
+  if (threadIdx.x == 0 && both) atomicAdd(&S->app, both);
 }
 
-__global__ void __launch_bounds__(kBlock) bitmap_to_queue_kernel(const uint32_t* __restrict__ bm, int64_t n,
+__global__ void __launch_bounds__(kWideBlock) bitmap_to_queue_kernel(const uint32_t* __restrict__ bm, int64_t n,
                                                                  uint32_t* __restrict__ q, unsigned* count,
                                                                  unsigned cap, unsigned* overflow) {
   __shared__ LdsQueue<kQCap> sq;
@@ -338,8 +337,7 @@ __global__ void __launch_bounds__(kBlock) bitmap_to_queue_kernel(const uint32_t*
 
 __global__ void do_pull_begin_kernel(BfsState* S) {
   if (threadIdx.x == 0) {
-    S->found = 0;
-    S->scout = 0;
+    S->app = 0;
   }
 }
 
@@ -355,6 +353,7 @@ __global__ void do_to_queue_begin_kernel(BfsState* S) {
 }
 
 unsigned sweep_grid(int64_t n) { return grid_for(n, kBlock, 256 * 16); }
+unsigned wide_grid(int64_t n) { return grid_for(n, kWideBlock, kWideGrid); }
 
 }  // namespace
 
@@ -529,20 +528,20 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
         fill_kernel<uint32_t><<<sweep_grid(words), kBlock, 0, s>>>(bm[b ^ 1], 0u, words);
         do_pull_begin_kernel<<<1, 64, 0, s>>>(B.S);
         ktimer.begin();
-        bu_step_kernel<<<sweep_grid(n), kBlock, 0, s>>>(trow, tcol, row, B.level, B.parent, bm[b], bm[b ^ 1], B.S,
+        bu_step_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(trow, tcol, row, B.level, B.parent, bm[b], bm[b ^ 1], B.S,
                                                         n, lvl);
         ktimer.end();
         GX_LAUNCHED("bu_step_kernel");
         launches += 3;
         read_state();
-        work = host->found;
-        items += host->found;
-        edges_visited += host->scout;
+        work = static_cast<uint32_t>(host->app);
+        items += work;
+        edges_visited += host->app >> 32;
         b ^= 1;
       } while (work > 0 && (work >= old_work || work > static_cast<uint64_t>(n) / beta));
       // Bitmap -> queue for the next push level.
       do_to_queue_begin_kernel<<<1, 64, 0, s>>>(B.S);
-      bitmap_to_queue_kernel<<<sweep_grid(n), kBlock, 0, s>>>(bm[b], n, B.q[0], &B.S->count[0], cap,
+      bitmap_to_queue_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(bm[b], n, B.q[0], &B.S->count[0], cap,
                                                               &B.S->overflow);
       GX_LAUNCHED("bitmap_to_queue_kernel");
       launches += 2;

@@ -1,30 +1,58 @@
 // Load-balanced neighbour expansion shared by the frontier-driven kernels
 // (BFS, SSSP, k-core, CC hooking, BC forward).
 //
-// A workgroup of BLOCK lanes takes BLOCK frontier vertices, exclusive-scans
-// their degrees in LDS and walks the concatenated edge list with all lanes;
-// the owning vertex of edge slot e is found by binary search over the LDS
-// offsets.  Vertices whose degree exceeds `hub_thresh` are not expanded here:
+// A workgroup of BLOCK lanes takes up to BLOCK frontier vertices (fewer when the
+// frontier has fewer than that for every workgroup of the launch, see
+// batch_vertices), exclusive-scans their degrees in LDS and walks the
+// concatenated edge list with all lanes; the owning vertex of edge slot e is
+// found by binary search over the LDS offsets.  Vertices whose degree exceeds `hub_thresh` are not expanded here:
 // they are appended to a hub queue and their edges are later spread over the
 // whole grid by expand_hubs.  This gives three effective tiers — short
 // adjacencies packed many-per-wavefront, medium ones spread over the
 // workgroup, hubs spread over the grid.
 //
 // The per-edge operation is called by every lane of the workgroup the same
-// number of times (with `valid` false for padding lanes), so it may use
-// wavefront-collective operations (ballot, shuffles).  After every step of
-// BLOCK edges, every lane calls op.after_step() (workgroup-uniform), where an
-// operation may flush its LDS-staged output (LdsQueue below).
+// number of times (with `valid` false and edge 0 for padding lanes), so it may
+// use wavefront-collective operations (ballot, shuffles).  With U > 1 a lane
+// takes U edges of a step at once (op.run), so that their loads are in flight
+// together.  After every step of BLOCK * U edges, every lane calls
+// op.after_step() (workgroup-uniform), where an operation may flush its
+// LDS-staged output (LdsQueue below).
+//
+// Counters shared by a whole launch (queue ends, sums) are single words, and
+// atomics on one word are served one after another, about 12 ns each on this
+// GPU whether or not the result is used (256 workgroups: 3 us, 2048: 25 us).
+// So the operations count per workgroup first, a workgroup's counts go out in
+// one packed 64-bit atomic where they can, and the launches with the most such
+// traffic use few wide workgroups (kWideBlock lanes, kWideGrid workgroups).
 #pragma once
 
 #include "gx_device.hpp"
 
 namespace gx {
 
+constexpr int kWideBlock = 1024;
+constexpr int kWideGrid = 256 * 2;
+constexpr int kWideWaves = kWideBlock / kWave;
+constexpr int kWideEdges = 4;                       // edges per lane and step of the wide launches
+constexpr int kWideStep = kWave * kWideEdges;       // most items a wavefront pushes per step
+constexpr int kWaveQCap = 2 * kWideStep;            // items a wavefront stages
+
+// Frontier vertices a workgroup takes at a time: an equal share of the frontier
+// between kBatchMin and BLOCK.  With whole blocks a frontier of a few thousand
+// vertices kept a dozen workgroups busy, each walking up to 32K edges alone
+// (BFS on 4096 vertices, 97K edges: one level 77 us).
+constexpr unsigned kBatchMin = 4;
+template <int BLOCK>
+__device__ __forceinline__ unsigned batch_vertices(unsigned qcount) {
+  const unsigned share = (qcount + gridDim.x - 1) / gridDim.x;
+  return share < kBatchMin ? kBatchMin : (share < BLOCK ? share : BLOCK);
+}
+
 // Identity frontier (q null): vertex first + i for i in [0, count).
 // Otherwise q[i].  With ADMIT, op.admit(v) is asked once per frontier vertex
 // and a vertex it rejects contributes no edges (a fused filter).
-template <int BLOCK, class Op, bool ADMIT = false>
+template <int BLOCK, class Op, bool ADMIT = false, int U = 1>
 __device__ __forceinline__ void expand_queue(const int32_t* __restrict__ row, const uint32_t* __restrict__ q,
                                              unsigned qcount, uint32_t hub_thresh, uint32_t* __restrict__ hubq,
                                              unsigned* hub_count, unsigned cap, unsigned* overflow, Op& op,
@@ -35,12 +63,14 @@ __device__ __forceinline__ void expand_queue(const int32_t* __restrict__ row, co
   __shared__ uint64_t s_scan[BLOCK / kWave + 1];
   __shared__ unsigned s_hub_base;
   const unsigned tid = threadIdx.x;
-  for (unsigned base = blockIdx.x * BLOCK; base < qcount; base += gridDim.x * BLOCK) {
-    const unsigned i = base + tid;
+  const unsigned per = batch_vertices<BLOCK>(qcount);
+  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * per; base < qcount;
+       base += static_cast<uint64_t>(gridDim.x) * per) {
+    const unsigned i = static_cast<unsigned>(base) + tid;
     uint32_t v = 0, deg = 0;
     int32_t start = 0;
     bool hub = false;
-    if (i < qcount) {
+    if (tid < per && i < qcount) {
       v = q ? q[i] : first + i;
       bool in = true;
       if constexpr (ADMIT) in = op.admit(v);
@@ -74,21 +104,28 @@ __device__ __forceinline__ void expand_queue(const int32_t* __restrict__ row, co
       else
         atomicOr(overflow, 1u);
     }
-    for (uint32_t e0 = 0; e0 < total; e0 += BLOCK) {
-      const uint32_t e = e0 + tid;
-      const bool valid = e < total;
-      uint32_t u = 0;
-      int32_t edge = 0;
-      if (valid) {
-        int lo = 0, hi = BLOCK - 1;
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if (s_off[mid] <= e) lo = mid; else hi = mid - 1;
+    for (uint32_t e0 = 0; e0 < total; e0 += BLOCK * U) {
+      bool valid[U];
+      uint32_t u[U];
+      int32_t edge[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const uint32_t e = e0 + k * BLOCK + tid;
+        valid[k] = e < total;
+        u[k] = 0;
+        edge[k] = 0;
+        if (valid[k]) {
+          int lo = 0, hi = static_cast<int>(per) - 1;
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (s_off[mid] <= e) lo = mid; else hi = mid - 1;
+          }
+          u[k] = s_src[lo];
+          edge[k] = s_start[lo] + static_cast<int32_t>(e - s_off[lo]);
         }
-        u = s_src[lo];
-        edge = s_start[lo] + static_cast<int32_t>(e - s_off[lo]);
       }
-      op(valid, u, edge);
+      if constexpr (U == 1) op(valid[0], u[0], edge[0]);
+      else op.run(valid, u, edge);
       op.after_step();
     }
     __syncthreads();
@@ -150,17 +187,20 @@ inline void launch_hub_offsets(const int32_t* row, const uint32_t* hubq, const u
   hub_offsets_kernel<BLOCK><<<kHubSlices, kHubScanThreads, 0, s>>>(row, hubq, hub_count, cap, off);
 }
 
-// Edges of the hub vertices hubq[0..hubs), cut into BLOCK-edge steps (a
-// hub's steps are consecutive).  Each workgroup takes a contiguous range of
-// steps: one binary search over the hub offsets (those of hub_offsets_kernel
-// plus the scanned slice totals) finds the hub of its first step, and the
-// following steps advance to the next hub when they pass its first step, so
-// a step costs no search.
-template <int BLOCK, class Op>
+// Edges of the hub vertices hubq[0..hubs), cut into steps of LANES * U edges
+// (a hub's steps are consecutive; hub_offsets_kernel<LANES * U> counted them).
+// Each workgroup takes a contiguous range of steps, BLOCK / LANES at a time,
+// one per group of LANES lanes: one binary search over the hub offsets (those
+// of hub_offsets_kernel plus the scanned slice totals) finds the hub of a
+// group's first step, and the following steps advance to the next hubs when
+// they pass their first steps, so a step costs no search.
+template <int BLOCK, class Op, int LANES = BLOCK, int U = 1>
 __device__ __forceinline__ void expand_hubs(const int32_t* __restrict__ row, const uint32_t* __restrict__ hubq,
                                             unsigned hub_count, unsigned cap, const uint32_t* __restrict__ off,
                                             Op& op) {
   static_assert(BLOCK >= kHubSlices, "one slice total per lane");
+  static_assert(BLOCK % LANES == 0 && LANES % kWave == 0, "groups are whole wavefronts");
+  constexpr uint32_t kGroups = BLOCK / LANES;
   __shared__ uint32_t s_base[kHubSlices];
   __shared__ uint32_t s_scan[BLOCK / kWave + 1];
   __shared__ uint32_t s_total;
@@ -180,29 +220,44 @@ __device__ __forceinline__ void expand_hubs(const int32_t* __restrict__ row, con
   const uint32_t c0 = static_cast<uint32_t>(min(static_cast<uint64_t>(blockIdx.x) * per, static_cast<uint64_t>(total)));
   const uint32_t c1 = static_cast<uint32_t>(min(static_cast<uint64_t>(c0) + per, static_cast<uint64_t>(total)));
   if (c0 >= c1) return;
+  const uint32_t group = threadIdx.x / LANES, lane = threadIdx.x % LANES;
   auto first_step = [&](unsigned h) { return off[h] + s_base[h >> sh]; };
-  unsigned lo = 0, hi = hubs - 1;  // last h with first_step(h) <= c0 (steps >= 1 per hub: increasing)
+  const uint32_t mine = min(c0 + group, total - 1);  // a step that exists, for the search
+  unsigned lo = 0, hi = hubs - 1;  // last h with first_step(h) <= mine (steps >= 1 per hub: increasing)
   while (lo < hi) {
     const unsigned mid = (lo + hi + 1) >> 1;
-    if (first_step(mid) <= c0) lo = mid; else hi = mid - 1;
+    if (first_step(mid) <= mine) lo = mid; else hi = mid - 1;
   }
   unsigned h = lo;
   uint32_t first = first_step(h);
   uint32_t next = h + 1 < hubs ? first_step(h + 1) : total;
   uint32_t v = hubq[h];
   int64_t rb = row[v], re = row[v + 1];
-  for (uint32_t c = c0; c < c1; ++c) {
-    if (c >= next) {  // workgroup-uniform; the next hub has >= 1 step
-      ++h;
-      first = next;
-      next = h + 1 < hubs ? first_step(h + 1) : total;
+  for (uint32_t base = c0; base < c1; base += kGroups) {  // workgroup-uniform
+    const uint32_t c = base + group;
+    const bool live = c < c1;
+    if (live && c >= next) {  // uniform in the group; every hub has >= 1 step
+      do {
+        ++h;
+        first = next;
+        next = h + 1 < hubs ? first_step(h + 1) : total;
+      } while (c >= next);
       v = hubq[h];
       rb = row[v];
       re = row[v + 1];
     }
-    const int64_t e = rb + static_cast<int64_t>(c - first) * BLOCK + threadIdx.x;
-    const bool valid = e < re;
-    op(valid, v, valid ? static_cast<int32_t>(e) : 0);
+    bool valid[U];
+    uint32_t u[U];
+    int32_t edge[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int64_t e = rb + static_cast<int64_t>(c - first) * (LANES * U) + k * LANES + lane;
+      valid[k] = live && e < re;
+      u[k] = v;
+      edge[k] = valid[k] ? static_cast<int32_t>(e) : 0;
+    }
+    if constexpr (U == 1) op(valid[0], u[0], edge[0]);
+    else op.run(valid, u, edge);
     op.after_step();
   }
 }
@@ -259,6 +314,60 @@ __device__ __forceinline__ void lq_flush(LdsQueue<CAP>& q, uint32_t* __restrict_
   __syncthreads();
   if (threadIdx.x == 0) q.count = 0;
   __syncthreads();
+}
+
+// Output queue of one wavefront in LDS, its length in a register: a push costs
+// no LDS atomic and a flush no workgroup barrier, so the wavefronts of a
+// workgroup run on at their own pace between two batches of vertices.
+template <int CAP>
+struct WaveQueue {
+  uint32_t* items;     // CAP words of LDS of this wavefront
+  unsigned count = 0;  // wavefront-uniform
+  // U items per lane; room for kWave * U is the caller's to see to.
+  template <int U>
+  __device__ __forceinline__ void push(const bool (&pred)[U], const uint32_t (&v)[U]) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const uint64_t mask = __ballot(pred[k]);
+      if (pred[k]) items[count + lanes_below(mask)] = v[k];
+      count += static_cast<unsigned>(__popcll(mask));
+    }
+  }
+  __device__ __forceinline__ bool full(unsigned step) const { return count + step > CAP; }
+  // Stores the items to gq[base, base + count), bounded by cap.
+  __device__ __forceinline__ void store(unsigned base, uint32_t* __restrict__ gq, unsigned cap, unsigned* overflow) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (unsigned i = lane_id(); i < count; i += kWave) {
+      if (base + i < cap)
+        gq[base + i] = items[i];
+      else
+        atomicOr(overflow, 1u);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    count = 0;
+  }
+};
+
+// Workgroup-uniform: the sum of one wavefront-uniform value per wavefront and
+// the sum of those of earlier wavefronts.  lds: BLOCK / kWave + 1 words.
+template <int BLOCK>
+__device__ __forceinline__ unsigned long long waves_exclusive_sum(unsigned long long v, unsigned long long* lds,
+                                                                  unsigned long long* total) {
+  constexpr int kW = BLOCK / kWave;
+  const unsigned w = threadIdx.x / kWave;
+  if (lane_id() == 0) lds[w] = v;
+  __syncthreads();
+  unsigned long long before = 0, all = 0;
+#pragma unroll
+  for (int i = 0; i < kW; ++i) {
+    const unsigned long long x = lds[i];
+    before += static_cast<unsigned>(i) < w ? x : 0ull;
+    all += x;
+  }
+  *total = all;
+  return before;
 }
 
 // Segmented inclusive sum across a wavefront where equal `key`s form

@@ -14,8 +14,11 @@
 // Design (gfx950): the dead frontier is expanded with the load-balanced
 // workgroup expansion of frontier.hpp (hubs spread over the grid); each
 // decrement is one atomicSub on the degree word, and the `old == k` winner
-// appends the neighbour to the next frontier through the workgroup's LDS
-// queue.  On the degree-ordered copy the decrements of the hub ids are
+// appends the neighbour to the next frontier through the wavefront's LDS
+// queue.  Random atomics run at 27 G/s on this GPU, which is what the first
+// round's decrements take; the passes over all vertices count per workgroup
+// (init 53 -> 17 us, membership 171 -> 12 us on RMAT-22; the call 908 -> 722
+// us).  On the degree-ordered copy the decrements of the hub ids are
 // counted in LDS first (kHot below).
 #include <algorithm>
 
@@ -57,7 +60,8 @@ __global__ void kcore_reset_kernel(KcoreCounters* c) {
   }
 }
 
-constexpr int kQCap = 2048;
+constexpr int kQCap = 4096;  // kcore_init_kernel
+constexpr int kHubLanes = 256;  // lanes per step of the hub pass
 // On the degree-ordered copy the hubs are the smallest ids (and on graphs
 // whose generator gives small ids the high degrees, such as RMAT without a
 // relabelling, too), and in the first round (every vertex below k dies at
@@ -75,7 +79,7 @@ constexpr int kRoundsFirst = 2;  // first replay: many graphs need one round (pl
 // (staged in LDS, one global append per workgroup flush).  Vertices without
 // edges are dead from the start but decrement no one, so they are left out
 // of it (on RMAT graphs they are a large share of the vertices).
-__global__ void __launch_bounds__(kBlock) kcore_init_kernel(const int32_t* __restrict__ row,
+__global__ void __launch_bounds__(kWideBlock) kcore_init_kernel(const int32_t* __restrict__ row,
                                                             uint32_t* __restrict__ degree, int64_t n, uint32_t k,
                                                             uint32_t* __restrict__ q, KcoreCounters* c,
                                                             unsigned cap) {
@@ -103,29 +107,46 @@ struct PeelOp {
   uint32_t* degree;
   uint32_t* qout;
   KcoreCounters* c;
-  LdsQueue<kQCap>* sq;
+  WaveQueue<kWaveQCap> wq;
   uint32_t k;
   unsigned out;
   unsigned cap;
   uint32_t hub;   // frontier.hub_degree
   uint32_t* hot;  // LDS counters of the ids below nhot (nhot = 0: none)
   uint32_t nhot;
-  __device__ __forceinline__ void operator()(bool valid, uint32_t, int32_t e) {
-    bool dies = false;
-    uint32_t v = 0;
-    if (valid) {
-      v = static_cast<uint32_t>(col[e]);
-      if (v < nhot)
-        atomicAdd(&hot[v], 1u);
-      else
-        dies = atomicSub(&degree[v], 1u) == k;
+  template <int U>
+  __device__ __forceinline__ void run(const bool (&valid)[U], const uint32_t (&)[U], const int32_t (&e)[U]) {
+    bool dies[U];
+    uint32_t v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = static_cast<uint32_t>(col[e[k]]);
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      dies[k] = false;
+      if (valid[k]) {
+        if (v[k] < nhot)
+          atomicAdd(&hot[v[k]], 1u);
+        else
+          dies[k] = atomicSub(&degree[v[k]], 1u) == this->k;
+      }
     }
-    lq_push(*sq, dies, v);
+    wq.push(dies, v);
   }
-  __device__ __forceinline__ void flush(bool force) {
-    lq_flush(*sq, qout, &c->count[out], cap, &c->overflow, force);
+  __device__ __forceinline__ void after_step() {
+    if (!wq.full(kWideStep)) return;
+    unsigned base = 0;
+    if (lane_id() == 0) base = atomicAdd(&c->count[out], wq.count);
+    wq.store(__builtin_amdgcn_readfirstlane(base), qout, cap, &c->overflow);
   }
-  __device__ __forceinline__ void after_step() { flush(false); }
+  // Workgroup-uniform: what is left, for all wavefronts with one atomic.
+  __device__ __forceinline__ void finish() {
+    __shared__ unsigned long long s_sum[kWideWaves + 1];
+    unsigned long long total;
+    const unsigned long long before = waves_exclusive_sum<kWideBlock>(wq.count, s_sum, &total);
+    if (threadIdx.x == 0) s_sum[kWideWaves] = total ? atomicAdd(&c->count[out], static_cast<unsigned>(total)) : 0u;
+    __syncthreads();
+    wq.store(static_cast<unsigned>(s_sum[kWideWaves] + before), qout, cap, &c->overflow);
+  }
 };
 
 struct KcoreBufs {
@@ -142,14 +163,15 @@ struct KcoreBufs {
   uint32_t hub;
 };
 
-__device__ __forceinline__ PeelOp make_peel(const KcoreBufs& B, LdsQueue<kQCap>* sq, uint32_t* hot, uint32_t nhot) {
+__device__ __forceinline__ PeelOp make_peel(const KcoreBufs& B, uint32_t (&stage)[kWideWaves][kWaveQCap], uint32_t* hot,
+                                            uint32_t nhot) {
   const unsigned out = B.c->in ^ 1u;
-  return PeelOp{B.col, B.degree, out ? B.q1 : B.q0, B.c, sq, B.k, out, B.cap, B.hub, hot, nhot};
+  return PeelOp{B.col, B.degree, out ? B.q1 : B.q0, B.c, {stage[threadIdx.x / kWave]}, B.k, out, B.cap, B.hub, hot, nhot};
 }
 
 // Workgroup-uniform.  Clears the LDS counters of the hot ids.
 __device__ __forceinline__ void hot_clear(uint32_t* hot) {
-  for (uint32_t i = threadIdx.x; i < kHot; i += kBlock) hot[i] = 0;
+  for (uint32_t i = threadIdx.x; i < kHot; i += kWideBlock) hot[i] = 0;
   __syncthreads();
 }
 
@@ -157,46 +179,45 @@ __device__ __forceinline__ void hot_clear(uint32_t* hot) {
 // ids (ids at or above n are never counted).
 __device__ __forceinline__ void hot_apply(PeelOp& op) {
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < kHot; i += kBlock) {
+  for (uint32_t i = threadIdx.x; i < kHot; i += kWideBlock) {
     const uint32_t cnt = op.hot[i];
-    bool dies = false;
+    bool dies[1] = {false};
+    const uint32_t id[1] = {i};
     if (cnt) {
       const uint32_t old = atomicSub(&op.degree[i], cnt);
-      dies = old >= op.k && old - cnt < op.k;
+      dies[0] = old >= op.k && old - cnt < op.k;
     }
-    lq_push(*op.sq, dies, i);
-    op.flush(false);
+    op.wq.push(dies, id);
+    op.after_step();
   }
 }
 
 template <bool kAgg>
-__global__ void __launch_bounds__(kBlock) kcore_peel_kernel(KcoreBufs B) {
+__global__ void __launch_bounds__(kWideBlock) kcore_peel_kernel(KcoreBufs B) {
   KcoreCounters* c = B.c;
   if (!c->active) return;
-  __shared__ LdsQueue<kQCap> sq;
+  __shared__ uint32_t stage[kWideWaves][kWaveQCap];
   __shared__ uint32_t hot[kAgg ? kHot : 1];
-  lq_init(sq);
   if constexpr (kAgg) hot_clear(hot);
-  PeelOp op = make_peel(B, &sq, hot, kAgg ? kHot : 0u);
+  PeelOp op = make_peel(B, stage, hot, kAgg ? kHot : 0u);
   const unsigned in = c->in;
-  expand_queue<kBlock>(B.row, in ? B.q1 : B.q0, c->count[in], B.hub, B.hubq, &c->hub_count, B.cap, &c->overflow,
+  expand_queue<kWideBlock, PeelOp, false, kWideEdges>(B.row, in ? B.q1 : B.q0, c->count[in], B.hub, B.hubq, &c->hub_count, B.cap, &c->overflow,
                        op);
   if constexpr (kAgg) hot_apply(op);
-  op.flush(true);
+  op.finish();
 }
 
 template <bool kAgg>
-__global__ void __launch_bounds__(kBlock) kcore_hubs_kernel(KcoreBufs B) {
+__global__ void __launch_bounds__(kWideBlock) kcore_hubs_kernel(KcoreBufs B) {
   KcoreCounters* c = B.c;
   if (!c->active || c->hub_count == 0) return;
-  __shared__ LdsQueue<kQCap> sq;
+  __shared__ uint32_t stage[kWideWaves][kWaveQCap];
   __shared__ uint32_t hot[kAgg ? kHot : 1];
-  lq_init(sq);
   if constexpr (kAgg) hot_clear(hot);
-  PeelOp op = make_peel(B, &sq, hot, kAgg ? kHot : 0u);
-  expand_hubs<kBlock>(B.row, B.hubq, c->hub_count, B.cap, B.hub_off, op);
+  PeelOp op = make_peel(B, stage, hot, kAgg ? kHot : 0u);
+  expand_hubs<kWideBlock, PeelOp, kHubLanes, kWideEdges>(B.row, B.hubq, c->hub_count, B.cap, B.hub_off, op);
   if constexpr (kAgg) hot_apply(op);
-  op.flush(true);
+  op.finish();
 }
 
 // Round bracket, driven by the device state: a round runs while the dead
@@ -235,7 +256,7 @@ __global__ void kcore_round_turn_kernel(KcoreCounters* c) {
   round_begin(c);
 }
 
-__global__ void __launch_bounds__(kBlock) kcore_finish_kernel(const uint32_t* __restrict__ degree,
+__global__ void __launch_bounds__(kWideBlock) kcore_finish_kernel(const uint32_t* __restrict__ degree,
                                                               uint8_t* __restrict__ alive, int64_t n, uint32_t k,
                                                               KcoreCounters* c) {
   int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
@@ -246,8 +267,17 @@ __global__ void __launch_bounds__(kBlock) kcore_finish_kernel(const uint32_t* __
     if (alive) alive[v] = a ? 1 : 0;
     cnt += a ? 1ull : 0ull;
   }
+  // One atomic per workgroup, few workgroups: with one per wavefront 65,536
+  // of them met at one word (RMAT-22: 171 us, 10 us this way).
+  __shared__ unsigned long long s_cnt[kWideBlock / kWave];
   cnt = wave_sum(cnt);
-  if (lane_id() == 0 && cnt) atomicAdd(&c->alive, cnt);
+  if (lane_id() == 0) s_cnt[threadIdx.x / kWave] = cnt;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (int i = 0; i < kWideBlock / kWave; ++i) t += s_cnt[i];
+    if (t) atomicAdd(&c->alive, t);
+  }
 }
 
 }  // namespace
@@ -299,7 +329,7 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
           8.0 * static_cast<double>(kHot) * static_cast<double>(g->m);
   }
   kcore_reset_kernel<<<1, 64, 0, s>>>(c);
-  kcore_init_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(B.row, B.degree, n, k, q[0], c, cap);
+  kcore_init_kernel<<<grid_for(n, kWideBlock, kWideGrid), kWideBlock, 0, s>>>(B.row, B.degree, n, k, q[0], c, cap);
   GX_LAUNCHED("kcore_init_kernel");
   uint64_t key = 0;
   for (const void* p : {(const void*)B.row, (const void*)B.col, (const void*)B.degree, (const void*)B.q0,
@@ -314,15 +344,15 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
       kcore_round_begin_kernel<<<1, 64, 0, cs>>>(c);
       for (int i = 0; i < nr; ++i) {
         if (agg)
-          kcore_peel_kernel<true><<<256 * 8, kBlock, 0, cs>>>(B);
+          kcore_peel_kernel<true><<<kWideGrid, kWideBlock, 0, cs>>>(B);
         else
-          kcore_peel_kernel<false><<<256 * 8, kBlock, 0, cs>>>(B);
+          kcore_peel_kernel<false><<<kWideGrid, kWideBlock, 0, cs>>>(B);
         if (hubs) {
-          launch_hub_offsets<kBlock>(B.row, B.hubq, &c->hub_count, cap, B.hub_off, cs);
+          launch_hub_offsets<kHubLanes * kWideEdges>(B.row, B.hubq, &c->hub_count, cap, B.hub_off, cs);
           if (agg)
-            kcore_hubs_kernel<true><<<256 * 8, kBlock, 0, cs>>>(B);
+            kcore_hubs_kernel<true><<<kWideGrid, kWideBlock, 0, cs>>>(B);
           else
-            kcore_hubs_kernel<false><<<256 * 8, kBlock, 0, cs>>>(B);
+            kcore_hubs_kernel<false><<<kWideGrid, kWideBlock, 0, cs>>>(B);
         }
         if (i + 1 < nr)
           kcore_round_turn_kernel<<<1, 64, 0, cs>>>(c);
@@ -347,7 +377,7 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
     unpermute_u32(B.degree, g->relab.new_of_old.as<uint32_t>(), degree, n, s);
     launches += 1;
   }
-  kcore_finish_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(degree, alive, n, k, c);
+  kcore_finish_kernel<<<grid_for(n, kWideBlock, kWideGrid), kWideBlock, 0, s>>>(degree, alive, n, k, c);
   GX_LAUNCHED("kcore_finish_kernel");
   launches += 1;
   GX_HIP(hipMemcpyAsync(host, c, sizeof(KcoreCounters), hipMemcpyDeviceToHost, s));

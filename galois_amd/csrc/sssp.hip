@@ -15,8 +15,11 @@
 //    round's queue once (stamp word per vertex).  A vertex is expanded only
 //    if its distance changed since it was last expanded (`done` word), the
 //    GPU form of the reference's stale-item test (SSSP.cpp:138).
-//  - far pile: vertices improved to a later bucket; each vertex is in the far
-//    pile at most once (farmark word), so the pile is bounded by n.  A
+//  - far pile: vertices whose distance lies in a later bucket.  A vertex joins
+//    it when it is first reached there and stays until a split takes it out
+//    or finds it settled, so each is in the pile at most once and no mark is
+//    needed (an atomic per improvement less; random atomics run at 27 G/s
+//    on this GPU, a fifth of the gathers).  A
 //    running minimum of the far buckets (every improvement into a later
 //    bucket, and every item a split keeps) names the next bucket; when the
 //    near frontier drains, one pass moves that bucket into the near frontier
@@ -51,6 +54,10 @@
 //    own once the near frontier drains.  The extra steps pay on large
 //    power-law graphs only, so the default enables it from 2^24 vertices
 //    on.
+//  - Shared words: a workgroup takes room in both queues with one atomic on
+//    one packed word, lowers a minimum only when a read shows it would, and
+//    counts edges and items in a pair of its own (RMAT-22 5.16 -> 4.20 ms
+//    with these, the wavefronts' own queues and the hub order by edges).
 //  - Locality: on graphs with hubs (knob frontier.relabel) the kernels run
 //    on the degree-ordered copy of the CSR (gx_graph::relab): the hubs and
 //    the vertices most often relaxed get the smallest ids, so their
@@ -79,14 +86,13 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr uint32_t kInf = GX_DIST_INFINITY;
-constexpr int kGrid = 256 * 8;
 // Graphs without hubs (maximum degree at or below the hub threshold, such as
-// road-like grids) have small frontiers per step and many steps; a quarter
-// of the workgroups per launch costs less there (2048-grid SSSP 26.4 ->
-// 21.7 ms, BFS 2.03 -> 1.57 ms), while RMAT frontiers need the full grid.
-constexpr int kGridNoHubs = 512;
+// road-like grids) have small frontiers per step and many steps: a quarter of
+// the workgroups start faster and meet less at the step's counters.
+constexpr int kGridNoHubs = 128;
+constexpr int kHubLanes = 256;  // lanes per step of the hub pass
 constexpr int kStepsPerGraph = 16;
-constexpr int kHubSelectGrid = 256;
+constexpr int kHubSelectGrid = 128;
 // Bucket merging thresholds (items admitted per phase).
 constexpr unsigned long long kMergeLow = 1ull << 14;
 constexpr unsigned long long kMergeHigh = 1ull << 17;
@@ -96,6 +102,9 @@ enum Mode : unsigned { kIdle = 0, kRelax = 1, kAdvance = 2, kHubs = 3 };
 struct SsspState {
   unsigned near_count[2];  // near queues (double buffered by q)
   unsigned far_count[2];   // far piles (double buffered by far_sel)
+  // Ends of the queues a step fills: near (low 32 bits) and far (high 32 bits),
+  // so that a workgroup gets room in both with one atomic.
+  unsigned long long app;
   unsigned hub_count;
   unsigned overflow;
   unsigned far_min;        // running minimum of the far buckets
@@ -116,11 +125,11 @@ struct SsspState {
   unsigned hub_step;       // this step selects and expands pending hubs
   uint32_t near_min;       // smallest distance in the near queue the step reads
   uint32_t near_min_next;  // the same for the near queue the step fills
-  unsigned long long phase_items0;  // items admitted before the current phase
+  unsigned long long phase_items;  // items queued in the current phase
   unsigned round;
   unsigned phase;
   unsigned steps;
-  unsigned long long edges;
+  unsigned long long edges;  // sums of the workgroups' counts at the end of a batch
   unsigned long long items;
   // Output of the current call, read by the captured step kernels.
   uint32_t* dist_out;
@@ -132,7 +141,6 @@ struct Bufs {
   const uint32_t* w;
   uint32_t* dist;
   uint32_t* stamp;
-  uint32_t* farmark;
   uint32_t* done;
   uint32_t* hubmark;  // generation of the pending hub list a hub is in
   uint32_t* nearq[2];
@@ -140,6 +148,9 @@ struct Bufs {
   uint32_t* hubq[2];  // pending hub lists (hq); without deferral hubq[0] holds the step's hubs
   uint32_t* hubx;     // hubs a hub step expands
   SsspState* S;
+  // Edges relaxed and items expanded, per workgroup index: every kernel of the
+  // run adds to its own workgroup's pair, and only the batch's end sums them.
+  unsigned long long* tally;
   uint32_t shift;
   unsigned cap;
   uint32_t* hub_off;
@@ -151,26 +162,27 @@ struct Bufs {
 };
 
 __global__ void sssp_init_kernel(uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp,
-                                 uint32_t* __restrict__ farmark, uint32_t* __restrict__ done,
+                                 uint32_t* __restrict__ done,
                                  uint32_t* __restrict__ hubmark, int64_t n, uint32_t src) {
   int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
   int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (; v < n; v += stride) {
     dist[v] = (v == src) ? 0u : kInf;
     stamp[v] = 0xffffffffu;
-    farmark[v] = 0xffffffffu;
     done[v] = kInf;
     hubmark[v] = 0xffffffffu;
   }
 }
 
-__global__ void sssp_reset_kernel(SsspState* S, uint32_t* nearq0, uint32_t src, uint32_t* dist,
-                                  unsigned max_width) {
+__global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint32_t* nearq0, uint32_t src,
+                                  uint32_t* dist, unsigned max_width) {
+  for (int i = threadIdx.x; i < 2 * kWideGrid; i += blockDim.x) tally[i] = 0;
   if (threadIdx.x == 0) {
     S->dist_out = dist;
     S->near_count[0] = 1;
     S->near_count[1] = 0;
     S->far_count[0] = S->far_count[1] = 0;
+    S->app = 0;
     S->hub_count = 0;
     S->overflow = 0;
     S->far_min = 0xffffffffu;
@@ -189,7 +201,7 @@ __global__ void sssp_reset_kernel(SsspState* S, uint32_t* nearq0, uint32_t src, 
     S->hub_step = 0;
     S->near_min = 0;  // the source
     S->near_min_next = 0xffffffffu;
-    S->phase_items0 = 0;
+    S->phase_items = 0;
     S->round = 0;
     S->phase = 0;
     S->steps = 0;
@@ -212,14 +224,14 @@ __device__ __forceinline__ void close_step(SsspState* S) {
     S->hub_min = S->hub_min_next;
     S->hub_step = 0;
   }
-  if (S->mode == kRelax || S->mode == kHubs) {
-    S->q ^= 1;
-  } else if (S->mode == kAdvance) {
+  if (S->mode == kAdvance) {
     S->far_count[S->far_sel] = 0;
     S->far_sel ^= 1;
-    S->q ^= 1;
   }
   if (S->mode != kIdle) {
+    S->q ^= 1;
+    S->near_count[S->q] = static_cast<unsigned>(S->app);
+    S->far_count[S->far_sel] = static_cast<unsigned>(S->app >> 32);
     S->near_min = S->near_min_next;
     S->near_min_next = 0xffffffffu;
   }
@@ -247,12 +259,13 @@ __global__ void step_kernel(SsspState* S, uint32_t defer, uint32_t hub_span) {
   close_step(S);
   if (S->done || S->overflow) return;
   S->round += 1;
-  S->near_count[S->q ^ 1] = 0;
+  S->app = static_cast<unsigned long long>(S->far_count[S->far_sel]) << 32;
   if (!defer) S->hub_count = 0;  // hubs of a relax step are expanded in that step
   const uint32_t span_limit =
       (hub_span == 0 || S->hub_min >= 0xffffffffu - hub_span) ? 0xffffffffu : S->hub_min + (hub_span - 1u);
   if (S->near_count[S->q] > 0) {
     S->mode = kRelax;
+    S->phase_items += S->near_count[S->q];
     // With hub slices, the pending hubs at or below every near distance are
     // expanded in the same step as the near frontier: nothing left to
     // expand can still lower them (weights are positive).
@@ -263,16 +276,15 @@ __global__ void step_kernel(SsspState* S, uint32_t defer, uint32_t hub_span) {
     begin_hub_step(S, span_limit);
   } else if (S->far_count[S->far_sel] > 0 && S->far_min != 0xffffffffu) {
     S->mode = kAdvance;
-    const unsigned long long admitted = S->items - S->phase_items0;
-    if (admitted < kMergeLow && S->width < S->max_width)
+    if (S->phase_items < kMergeLow && S->width < S->max_width)
       S->width = min(2 * S->width, S->max_width);
-    else if (admitted > kMergeHigh && S->width > 1)
+    else if (S->phase_items > kMergeHigh && S->width > 1)
       S->width >>= 1;
-    S->phase_items0 = S->items;
+    S->phase_items = 0;
     S->phase += 1;
     S->bucket = S->far_min;
     S->far_min = 0xffffffffu;
-    S->far_count[S->far_sel ^ 1] = 0;
+    S->app = 0;  // the kept far items fill the other pile
   } else {
     S->done = 1;
     return;
@@ -280,14 +292,76 @@ __global__ void step_kernel(SsspState* S, uint32_t defer, uint32_t hub_span) {
   S->steps += 1;
 }
 
-// Last kernel of a captured batch: closes its last step, so the state is
-// whole when the host reads it.
-__global__ void batch_end_kernel(SsspState* S) {
+// Last kernel of a captured batch (one workgroup of kBlock lanes): closes its
+// last step and sums the workgroups' counts, so the state is whole when the
+// host reads it.
+__global__ void __launch_bounds__(kBlock) batch_end_kernel(SsspState* S, const unsigned long long* tally) {
+  __shared__ unsigned long long s_sum[2][kBlock / kWave];
+  unsigned long long e = 0, t = 0;
+  for (int i = threadIdx.x; i < kWideGrid; i += kBlock) {
+    e += tally[2 * i];
+    t += tally[2 * i + 1];
+  }
+  e = wave_sum(e);
+  t = wave_sum(t);
+  if (lane_id() == 0) {
+    s_sum[0][threadIdx.x / kWave] = e;
+    s_sum[1][threadIdx.x / kWave] = t;
+  }
+  __syncthreads();
   if (threadIdx.x != 0) return;
+  S->edges = S->items = 0;
+  for (int i = 0; i < kBlock / kWave; ++i) {
+    S->edges += s_sum[0][i];
+    S->items += s_sum[1][i];
+  }
   close_step(S);
 }
 
-constexpr int kQCap = 2048;
+// Lowers *word to v.  Most workgroups bring nothing below what is there: a
+// read at agent scope spares them the atomic.
+__device__ __forceinline__ void lower(uint32_t* word, uint32_t v) {
+  if (v < __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(word, v);
+}
+
+using Stage = uint32_t[kWideWaves][kWaveQCap];
+
+// The two queues a step fills, staged per wavefront: nearer items go to nq,
+// later ones to fq, room in both taken with one atomic.
+struct PairQueue {
+  WaveQueue<kWaveQCap> near, far;
+  uint32_t* nq;
+  uint32_t* fq;
+  SsspState* S;
+  unsigned cap;
+  __device__ __forceinline__ PairQueue(SsspState* s, Stage& sn, Stage& sf, uint32_t* n, uint32_t* f, unsigned c)
+      : near{sn[threadIdx.x / kWave]}, far{sf[threadIdx.x / kWave]}, nq(n), fq(f), S(s), cap(c) {}
+  __device__ __forceinline__ unsigned long long counts() const {
+    return near.count | (static_cast<unsigned long long>(far.count) << 32);
+  }
+  __device__ __forceinline__ void store(unsigned long long base) {
+    near.store(static_cast<unsigned>(base), nq, cap, &S->overflow);
+    far.store(static_cast<unsigned>(base >> 32), fq, cap, &S->overflow);
+  }
+  // After every step of at most `step` items a wavefront and queue.
+  __device__ __forceinline__ void after_step(unsigned step) {
+    if (!near.full(step) && !far.full(step)) return;
+    unsigned long long base = 0;
+    if (lane_id() == 0) base = atomicAdd(&S->app, counts());
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32));
+    store((static_cast<unsigned long long>(hi) << 32) | lo);
+  }
+  // Workgroup-uniform: what is left, for all wavefronts at once.
+  __device__ __forceinline__ void finish() {
+    __shared__ unsigned long long s_sum[kWideWaves + 1];
+    unsigned long long total;
+    const unsigned long long before = waves_exclusive_sum<kWideBlock>(counts(), s_sum, &total);
+    if (threadIdx.x == 0) s_sum[kWideWaves] = total ? atomicAdd(&S->app, total) : 0ull;
+    __syncthreads();
+    store(s_sum[kWideWaves] + before);
+  }
+};
 
 // Holds the output pointer read from the device state: the kernel-argument
 // Bufs stays unmodified (a modified copy of it, with its runtime-indexed
@@ -295,13 +369,8 @@ constexpr int kQCap = 2048;
 struct RelaxOp {
   Bufs B;
   uint32_t* dist;
-  LdsQueue<kQCap>* qn;  // staged near pushes
-  LdsQueue<kQCap>* qf;  // staged far pushes
-  uint32_t* nearq_out;
-  unsigned* near_out_count;
-  uint32_t* farq;
-  unsigned* far_count;
-  uint32_t bucket_end, round, phase, hub_gen;  // bucket_end: last bucket of the phase
+  PairQueue q;
+  uint32_t bucket_end, round, hub_gen;  // bucket_end: last bucket of the phase
   uint32_t far_min = 0xffffffffu;  // this lane's smallest far bucket improved into
   uint32_t hub_min = 0xffffffffu;  // this lane's smallest distance of a hub it listed
   uint32_t near_min = 0xffffffffu;  // this lane's smallest distance improved into the near range
@@ -325,42 +394,41 @@ struct RelaxOp {
     items += 1;
     return true;
   }
-  __device__ __forceinline__ void operator()(bool valid, uint32_t u, int32_t e) {
-    bool to_near = false, to_far = false;
-    uint32_t v = 0;
-    if (valid) {
-      v = static_cast<uint32_t>(B.col[e]);
-      const uint32_t nd = dist[u] + B.w[e];
-      if (nd < dist[v]) {
-        const uint32_t old = atomicMin(&dist[v], nd);
-        if (nd < old) {
-          const uint32_t nb = nd >> B.shift;
-          if (nb <= bucket_end) {
-            near_min = min(near_min, nd);
-            to_near = atomicExch(&B.stamp[v], round) != round;
-          } else {
-            to_far = atomicExch(&B.farmark[v], phase) != phase;
-            far_min = min(far_min, nb);
-          }
-        }
+  template <int U>
+  __device__ __forceinline__ void run(const bool (&valid)[U], const uint32_t (&u)[U], const int32_t (&e)[U]) {
+    bool to_near[U], to_far[U];
+    uint32_t v[U], nd[U], dv[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      v[k] = static_cast<uint32_t>(B.col[e[k]]);
+      nd[k] = dist[u[k]] + B.w[e[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) dv[k] = dist[v[k]];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      to_near[k] = to_far[k] = false;
+      if (!valid[k] || nd[k] >= dv[k]) continue;
+      const uint32_t old = atomicMin(&dist[v[k]], nd[k]);
+      if (nd[k] >= old) continue;
+      const uint32_t nb = nd[k] >> B.shift;
+      if (nb > bucket_end) {
+        far_min = min(far_min, nb);
+        to_far[k] = old == kInf;  // reached before: it is in the far pile
+      } else {
+        near_min = min(near_min, nd[k]);
+        to_near[k] = atomicExch(&B.stamp[v[k]], round) != round;
       }
     }
-    lq_push(*qn, to_near, v);
-    lq_push(*qf, to_far, v);
+    q.near.push(to_near, v);
+    q.far.push(to_far, v);
   }
-  __device__ __forceinline__ void flush(bool force) {
-    lq_flush(*qn, nearq_out, near_out_count, B.cap, &B.S->overflow, force);
-    lq_flush(*qf, farq, far_count, B.cap, &B.S->overflow, force);
-  }
-  __device__ __forceinline__ void after_step() { flush(false); }
-  // End of a launch: queues flushed, far minimum and filter counts reduced
-  // once per wavefront.
-  // Workgroup-uniform.  The minima and counts are reduced over the
-  // workgroup first, so the state words (one cache line) take one atomic
-  // per workgroup rather than one per wavefront.
+  __device__ __forceinline__ void after_step() { q.after_step(kWideStep); }
+  // End of a launch, workgroup-uniform: queues flushed, minima and counts
+  // reduced over the workgroup; the counts go to the workgroup's own pair.
   __device__ __forceinline__ void finish() {
-    flush(true);
-    constexpr int kW = kBlock / kWave;
+    q.finish();
+    constexpr int kW = kWideBlock / kWave;
     __shared__ uint32_t s_min[3][kW];
     __shared__ unsigned long long s_sum[2][kW];
     const uint32_t fm = wave_min(far_min), hm = wave_min(hub_min), nm = wave_min(near_min);
@@ -384,39 +452,43 @@ struct RelaxOp {
         e += s_sum[0][i];
         t += s_sum[1][i];
       }
-      if (f != 0xffffffffu) atomicMin(&B.S->far_min, f);
-      if (h != 0xffffffffu) atomicMin(&B.S->hub_min, h);
-      if (nn != 0xffffffffu && B.hub_span) atomicMin(&B.S->near_min_next, nn);  // read only with hub slices
-      if (e) atomicAdd(&B.S->edges, e);  // hub steps count edges in every workgroup, items in one
-      if (t) atomicAdd(&B.S->items, t);
+      if (f != 0xffffffffu) lower(&B.S->far_min, f);
+      if (h != 0xffffffffu) lower(&B.S->hub_min, h);
+      if (nn != 0xffffffffu && B.hub_span) lower(&B.S->near_min_next, nn);  // read only with hub slices
+      if (e | t) {
+        B.tally[2 * blockIdx.x] += e;  // hub steps count edges in every workgroup, items in one
+        B.tally[2 * blockIdx.x + 1] += t;
+      }
     }
   }
 };
 
-__device__ __forceinline__ RelaxOp make_relax(const Bufs& B, LdsQueue<kQCap>* qn, LdsQueue<kQCap>* qf) {
+__device__ __forceinline__ RelaxOp make_relax(const Bufs& B, Stage& sn, Stage& sf) {
   SsspState* S = B.S;
   const unsigned q = S->q, fs = S->far_sel;
-  return RelaxOp{B, S->dist_out, qn, qf, B.nearq[q ^ 1], &S->near_count[q ^ 1], B.farq[fs], &S->far_count[fs],
-                 S->bucket + (S->width - 1), S->round, S->phase, S->hub_gen};
+  return RelaxOp{B, S->dist_out, PairQueue(S, sn, sf, B.nearq[q ^ 1], B.farq[fs], B.cap), S->bucket + (S->width - 1),
+                 S->round, S->hub_gen};
 }
 
 // Relax operation over hub edges: counts every valid edge it relaxes.
 template <class Op>
 struct HubCount {
   Op& op;
-  __device__ __forceinline__ void operator()(bool valid, uint32_t u, int32_t e) {
-    op.edges += valid ? 1ull : 0ull;
-    op(valid, u, e);
+  template <int U>
+  __device__ __forceinline__ void run(const bool (&valid)[U], const uint32_t (&u)[U], const int32_t (&e)[U]) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) op.edges += valid[k] ? 1ull : 0ull;
+    op.run(valid, u, e);
   }
   __device__ __forceinline__ void after_step() { op.after_step(); }
 };
 
 // Relax step: expand the near items that pass the stale-item filter.
-__device__ __forceinline__ void relax_step(const Bufs& B, LdsQueue<kQCap>& qn, LdsQueue<kQCap>& qf) {
+__device__ __forceinline__ void relax_step(const Bufs& B, Stage& sn, Stage& sf) {
   SsspState* S = B.S;
-  RelaxOp op = make_relax(B, &qn, &qf);
+  RelaxOp op = make_relax(B, sn, sf);
   const unsigned q = S->q;
-  expand_queue<kBlock, RelaxOp, true>(B.row, B.nearq[q], S->near_count[q], B.hub, B.hubq[S->hq], &S->hub_count, B.cap,
+  expand_queue<kWideBlock, RelaxOp, true, kWideEdges>(B.row, B.nearq[q], S->near_count[q], B.hub, B.hubq[S->hq], &S->hub_count, B.cap,
                                       &S->overflow, op);
   op.finish();
 }
@@ -424,58 +496,70 @@ __device__ __forceinline__ void relax_step(const Bufs& B, LdsQueue<kQCap>& qn, L
 // The hubs of a relax step (hub_count), or with deferral the pending hubs
 // of a hub step (hub_expand, 0 outside hub steps), spread over the grid;
 // hub_offsets ran over the same count.
-__global__ void __launch_bounds__(kBlock) hubs_kernel(Bufs B) {
+__global__ void __launch_bounds__(kWideBlock) hubs_kernel(Bufs B) {
   SsspState* S = B.S;
   const unsigned hubs = B.defer ? (S->hub_step ? S->hub_expand : 0u) : (S->mode == kRelax ? S->hub_count : 0u);
   if (hubs == 0) return;
-  __shared__ LdsQueue<kQCap> qn, qf;
-  lq_init(qn);
-  lq_init(qf);
-  RelaxOp op = make_relax(B, &qn, &qf);
+  __shared__ Stage sn, sf;
+  RelaxOp op = make_relax(B, sn, sf);
   HubCount<RelaxOp> hc{op};
-  expand_hubs<kBlock>(B.row, B.defer ? B.hubx : B.hubq[0], hubs, B.cap, B.hub_off, hc);
+  expand_hubs<kWideBlock, HubCount<RelaxOp>, kHubLanes, kWideEdges>(B.row, B.defer ? B.hubx : B.hubq[0], hubs, B.cap, B.hub_off, hc);
   if (blockIdx.x == 0 && threadIdx.x == 0) op.items += min(hubs, B.cap);
   op.finish();
 }
 
 // Advance step: far items of the new bucket go to the near queue, later
-// ones are kept (one copy per vertex, their buckets fold into the running far
-// minimum), settled ones are dropped.
-__device__ __forceinline__ void far_split_step(const Bufs& B, LdsQueue<kQCap>& qn, LdsQueue<kQCap>& qk) {
+// ones are kept (their buckets fold into the running far minimum), settled ones
+// are dropped.
+__device__ __forceinline__ void far_split_step(const Bufs& B, Stage& sn, Stage& sk) {
   SsspState* S = B.S;
   const uint32_t* __restrict__ dist = S->dist_out;
   const uint32_t next = S->bucket, last = S->bucket + (S->width - 1);
   const unsigned fs = S->far_sel, q = S->q;
   const unsigned cnt = S->far_count[fs];
   const uint32_t* farq = B.farq[fs];
-  const uint32_t round = S->round, phase = S->phase;
+  const uint32_t round = S->round;
   uint32_t kept_min = 0xffffffffu, near_min = 0xffffffffu;
-  for (unsigned b0 = blockIdx.x * kBlock; b0 < cnt; b0 += gridDim.x * kBlock) {
-    const unsigned i = b0 + threadIdx.x;
-    bool to_near = false, keep = false;
-    uint32_t v = 0;
+  PairQueue out(S, sn, sk, B.nearq[q ^ 1], B.farq[fs ^ 1], B.cap);
+  for (uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kWideBlock; b0 < cnt;
+       b0 += static_cast<uint64_t>(gridDim.x) * kWideBlock) {
+    const unsigned i = static_cast<unsigned>(b0) + threadIdx.x;
+    bool to_near[1] = {false}, keep[1] = {false};
+    uint32_t v[1] = {0};
     if (i < cnt) {
-      v = farq[i];
-      const uint32_t dv = dist[v], b = dv >> B.shift;
+      v[0] = farq[i];
+      const uint32_t dv = dist[v[0]], b = dv >> B.shift;
       if (b >= next && b <= last) {
         near_min = min(near_min, dv);
-        to_near = atomicExch(&B.stamp[v], round) != round;
+        B.stamp[v[0]] = round;
+        to_near[0] = true;
       } else if (b > last) {
-        keep = atomicExch(&B.farmark[v], phase) != phase;
+        keep[0] = true;
         kept_min = min(kept_min, b);
       }
     }
-    lq_push(qn, to_near, v);
-    lq_push(qk, keep, v);
-    lq_flush(qn, B.nearq[q ^ 1], &S->near_count[q ^ 1], B.cap, &S->overflow, false);
-    lq_flush(qk, B.farq[fs ^ 1], &S->far_count[fs ^ 1], B.cap, &S->overflow, false);
+    out.near.push(to_near, v);
+    out.far.push(keep, v);
+    out.after_step(kWave);
   }
-  lq_flush(qn, B.nearq[q ^ 1], &S->near_count[q ^ 1], B.cap, &S->overflow, true);
-  lq_flush(qk, B.farq[fs ^ 1], &S->far_count[fs ^ 1], B.cap, &S->overflow, true);
+  out.finish();
+  constexpr int kW = kWideBlock / kWave;
+  __shared__ uint32_t s_min[2][kW];
   kept_min = wave_min(kept_min);
   near_min = wave_min(near_min);
-  if (lane_id() == 0 && kept_min != 0xffffffffu) atomicMin(&S->far_min, kept_min);
-  if (lane_id() == 0 && near_min != 0xffffffffu && B.hub_span) atomicMin(&S->near_min_next, near_min);
+  if (lane_id() == 0) {
+    s_min[0][threadIdx.x / kWave] = kept_min;
+    s_min[1][threadIdx.x / kWave] = near_min;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kW; ++i) {
+      kept_min = min(kept_min, s_min[0][i]);
+      near_min = min(near_min, s_min[1][i]);
+    }
+    if (kept_min != 0xffffffffu) lower(&S->far_min, kept_min);
+    if (near_min != 0xffffffffu && B.hub_span) lower(&S->near_min_next, near_min);
+  }
 }
 
 // Hub step, first part: the pending hubs at or below hub_limit go to the
@@ -486,9 +570,10 @@ __device__ __forceinline__ void far_split_step(const Bufs& B, LdsQueue<kQCap>& q
 // The two lists are staged in LDS and moved out with one global atomic per
 // flush, not one per wavefront: the pending list can hold millions of hubs,
 // and every selecting step passes over it.
-__global__ void __launch_bounds__(kBlock) hub_select_kernel(Bufs B) {
+__global__ void __launch_bounds__(kWideBlock) hub_select_kernel(Bufs B) {
   SsspState* S = B.S;
   if (!S->hub_step) return;
+  constexpr int kQCap = 4096;
   __shared__ LdsQueue<kQCap> qs, qk;
   lq_init(qs);
   lq_init(qk);
@@ -497,8 +582,9 @@ __global__ void __launch_bounds__(kBlock) hub_select_kernel(Bufs B) {
   const uint32_t limit = S->hub_limit;
   const uint32_t* pending = B.hubq[hq];
   uint32_t kept_min = 0xffffffffu;
-  for (unsigned b0 = blockIdx.x * kBlock; b0 < cnt; b0 += gridDim.x * kBlock) {  // workgroup-uniform
-    const unsigned i = b0 + threadIdx.x;
+  for (uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kWideBlock; b0 < cnt;
+       b0 += static_cast<uint64_t>(gridDim.x) * kWideBlock) {  // workgroup-uniform
+    const unsigned i = static_cast<unsigned>(b0) + threadIdx.x;
     bool sel = false, keep = false;
     uint32_t h = 0;
     if (i < cnt) {
@@ -519,33 +605,31 @@ __global__ void __launch_bounds__(kBlock) hub_select_kernel(Bufs B) {
   lq_flush(qs, B.hubx, &S->hub_expand, B.cap, &S->overflow, true);
   lq_flush(qk, B.hubq[hq ^ 1], &S->hub_kept, B.cap, &S->overflow, true);
   kept_min = wave_min(kept_min);
-  if (lane_id() == 0 && kept_min != 0xffffffffu) atomicMin(&S->hub_min_next, kept_min);
+  if (lane_id() == 0 && kept_min != 0xffffffffu) lower(&S->hub_min_next, kept_min);
 }
 
 // The work of a step: a relax or an advance (the step's mode picks one; the
 // two never share a step, so one launch serves both).
-__global__ void __launch_bounds__(kBlock) work_kernel(Bufs B) {
+__global__ void __launch_bounds__(kWideBlock) work_kernel(Bufs B) {
   const unsigned mode = B.S->mode;
   if (mode != kRelax && mode != kAdvance) return;
-  __shared__ LdsQueue<kQCap> q0, q1;
-  lq_init(q0);
-  lq_init(q1);
+  __shared__ Stage s0, s1;
   if (mode == kRelax)
-    relax_step(B, q0, q1);
+    relax_step(B, s0, s1);
   else
-    far_split_step(B, q0, q1);
+    far_split_step(B, s0, s1);
 }
 
 // `hubs` false: no vertex exceeds the hub threshold, so the hub list stays
 // empty and its two launches are left out of the step.
 void enqueue_step(const Bufs& B, bool hubs, hipStream_t s) {
   step_kernel<<<1, 64, 0, s>>>(B.S, B.defer, B.hub_span);
-  work_kernel<<<hubs ? kGrid : kGridNoHubs, kBlock, 0, s>>>(B);
+  work_kernel<<<hubs ? kWideGrid : kGridNoHubs, kWideBlock, 0, s>>>(B);
   if (hubs) {
-    if (B.defer) hub_select_kernel<<<kHubSelectGrid, kBlock, 0, s>>>(B);
-    launch_hub_offsets<kBlock>(B.row, B.defer ? B.hubx : B.hubq[0], B.defer ? &B.S->hub_expand : &B.S->hub_count,
+    if (B.defer) hub_select_kernel<<<kHubSelectGrid, kWideBlock, 0, s>>>(B);
+    launch_hub_offsets<kHubLanes * kWideEdges>(B.row, B.defer ? B.hubx : B.hubq[0], B.defer ? &B.S->hub_expand : &B.S->hub_count,
                                B.cap, B.hub_off, s);
-    hubs_kernel<<<kGrid, kBlock, 0, s>>>(B);
+    hubs_kernel<<<kWideGrid, kWideBlock, 0, s>>>(B);
   }
   GX_LAUNCHED("sssp step");
 }
@@ -574,11 +658,11 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   B.hubq[0] = g->scratch<uint32_t>(WS_V0, cap);
   B.hubq[1] = g->scratch<uint32_t>(WS_BITMAP0, cap);
   B.hubx = g->scratch<uint32_t>(WS_BITMAP1, cap);
-  B.stamp = g->scratch<uint32_t>(WS_V1, cap);
-  B.farmark = g->scratch<uint32_t>(WS_V2, cap);
-  B.done = g->scratch<uint32_t>(WS_V3, cap);
-  B.hubmark = g->scratch<uint32_t>(WS_V4, cap);
+  B.stamp = g->scratch<uint32_t>(WS_V1, n);
+  B.done = g->scratch<uint32_t>(WS_V3, n);
+  B.hubmark = g->scratch<uint32_t>(WS_V4, n);
   B.S = g->scratch<SsspState>(WS_COUNTERS, 1);
+  B.tally = g->scratch<unsigned long long>(WS_REDUCE, 2 * kWideGrid);
   B.shift = shift;
   B.cap = cap;
   B.hub_off = g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(cap));
@@ -595,7 +679,7 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
     B.row = g->relab.row.as<int32_t>();
     B.col = g->relab.col.as<int32_t>();
     B.w = g->relab.w.as<uint32_t>();
-    B.dist = g->scratch<uint32_t>(WS_V5, cap);
+    B.dist = g->scratch<uint32_t>(WS_V5, n);
     run_src = read_scalar(g, g->relab.new_of_old.as<uint32_t>() + src);
   }
   SsspState* host = static_cast<SsspState*>(g->host_pinned(sizeof(SsspState)));
@@ -603,17 +687,16 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   RegionTimer region(s);
   KernelTimer ktimer(s);
   const unsigned max_width = static_cast<unsigned>(tune_effective("sssp.max_merge", n, g->m));
-  sssp_init_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(B.dist, B.stamp, B.farmark, B.done, B.hubmark, n,
+  sssp_init_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(B.dist, B.stamp, B.done, B.hubmark, n,
                                                                  run_src);
   GX_LAUNCHED("sssp_init_kernel");
-  sssp_reset_kernel<<<1, 64, 0, s>>>(B.S, B.nearq[0], run_src, B.dist, max_width);
+  sssp_reset_kernel<<<1, kBlock, 0, s>>>(B.S, B.tally, B.nearq[0], run_src, B.dist, max_width);
   GX_LAUNCHED("sssp_reset_kernel");
   uint64_t key = 0;
   for (const void* p : {(const void*)B.row, (const void*)B.col, (const void*)B.w,
                         (const void*)B.nearq[0], (const void*)B.nearq[1], (const void*)B.farq[0],
                         (const void*)B.farq[1], (const void*)B.hubq[0], (const void*)B.hubq[1], (const void*)B.hubx,
-                        (const void*)B.stamp, (const void*)B.farmark,
-                        (const void*)B.done, (const void*)B.hubmark, (const void*)B.S, (const void*)B.hub_off})
+                        (const void*)B.stamp, (const void*)B.done, (const void*)B.hubmark, (const void*)B.S, (const void*)B.tally, (const void*)B.hub_off})
     key = mix_key(key, reinterpret_cast<uintptr_t>(p));
   key = mix_key(mix_key(mix_key(mix_key(mix_key(mix_key(key, shift), cap), B.hub), hubs ? 1u : 0u), B.defer),
                 B.hub_span);
@@ -622,7 +705,7 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
     ktimer.begin();
     g->replay(g->sssp_batch, key, [&](hipStream_t cs) {
       for (int i = 0; i < kStepsPerGraph; ++i) enqueue_step(B, hubs, cs);
-      batch_end_kernel<<<1, 64, 0, cs>>>(B.S);
+      batch_end_kernel<<<1, kBlock, 0, cs>>>(B.S, B.tally);
       GX_LAUNCHED("batch_end_kernel");
     });
     ktimer.end();

@@ -131,3 +131,49 @@ def test_row_sweep_shapes(gx, n, m, hubs):
         for got, ref, scale in ((x, x_ref, np.abs(x_ref).max()), (gw, gw_ref, terms), (gt, gt_ref, np.abs(gt_ref).max())):
             got = got.cpu().numpy().astype(np.float64)
             assert np.abs(got - ref).max() <= rel * scale, (prec, np.abs(got - ref).max(), scale)
+
+
+def star_csr(degrees, n, seed):
+    """Symmetric weighted CSR: vertex i joined to `degrees[i]` others, and a path
+    through every vertex."""
+    rng = np.random.default_rng(seed)
+    u = [np.full(d, i) for i, d in enumerate(degrees)] + [np.arange(n - 1)]
+    v = [rng.choice(n, d, replace=False) for d in degrees] + [np.arange(1, n)]
+    u, v = np.concatenate(u), np.concatenate(v)
+    keep = u != v
+    u, v = u[keep], v[keep]
+    lo, hi = np.minimum(u, v), np.maximum(u, v)
+    key = np.unique(lo.astype(np.int64) * n + hi)
+    lo, hi = key // n, key % n
+    w = rng.integers(1, 60, len(lo)).astype(np.uint32)
+    u, v, w = np.concatenate([lo, hi]), np.concatenate([hi, lo]), np.concatenate([w, w])
+    o = np.lexsort((v, u))
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=n), out=row[1:])
+    return row, v[o].astype(np.int32), w[o]
+
+
+# Degrees around the hub threshold (128) and the edges a step of the hub pass and
+# of a workgroup take (1024, 4096); frontiers from one vertex to more than every
+# workgroup of a launch takes at once.
+@pytest.mark.parametrize("n,degrees", [(2, []), (130, [127, 128, 129]), (5000, [128, 129, 1023, 1024, 1025, 4096, 4097]),
+                                       (70001, [1, 1024, 60000] + [129] * 300), (600011, [200000] * 3 + [130] * 2000)])
+def test_frontier_shapes(gx, oracle, n, degrees):
+    row, col, w = star_csr(degrees, n, n)
+    G = gx.Graph.from_csr(row, col, w, symmetric=True)
+    for src in {0, n // 2, n - 1}:
+        print(f"frontier n={n} m={len(col)} src={src}", flush=True)
+        lv, dist = oracle.bfs(row, col, src), oracle.sssp(row, col, w, src, 4)
+        assert np.array_equal(u32(gx.bfs(G, src)[0]), lv)
+        assert np.array_equal(u32(gx.bfs_do(G, src)[0]), lv)
+        for refine in (0, 1):
+            gx.tune_set("sssp.hub_refine", refine)
+            try:
+                assert np.array_equal(u32(gx.sssp(G, src, 4)[0]), dist), refine
+            finally:
+                gx.tune_set("sssp.hub_refine", -1)
+    for k in (2, 3, 129):
+        deg, alive, count, _ = gx.kcore(G, k)
+        exp = oracle.kcore(row, col, k)
+        assert np.array_equal(u32(deg), exp) and count == int((exp >= k).sum())
+        assert np.array_equal(alive.cpu().numpy(), (exp >= k).astype(np.uint8))
