@@ -1,0 +1,376 @@
+// Layout of the blocked row sums (blocksum.hpp), built once per graph.
+//
+//  1. The edges, in row order, are sorted stably by chunk (a radix sort of a
+//     few bits, the edge id riding in the key's upper half): (chunk, row) order.
+//  2. Each chunk starts on a tile; every position gets its in-chunk index with
+//     the group-end flag, its row and (weighted) its edge id.
+//  3. Group ends counted per tile and scanned; every group gets its row.
+//  4. Bins: blocks of bin_rows rows, halved while they hold many groups, so that
+//     no wavefront of phase 2 sums much more than the others.
+//  5. Run starts marked and scanned, the runs sorted stably by bin.
+#include <algorithm>
+#include <vector>
+
+#include "blocksum.hpp"
+
+namespace gx {
+namespace bs {
+namespace {
+
+constexpr int kB = 256;
+constexpr double kAvgRun = 16.0;
+constexpr uint32_t kNone = 0xffffffffu;
+constexpr uint32_t kFirst = 1u << 31;  // grow: first group of a wavefront's range
+
+unsigned grid(int64_t n) { return grid_for(n, kB, 16384); }
+
+__global__ void key_kernel(const int32_t* __restrict__ col, int64_t m, int shift, uint64_t* __restrict__ key) {
+  for (int64_t e = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; e < m; e += static_cast<int64_t>(gridDim.x) * kB)
+    key[e] = (static_cast<uint64_t>(e) << 32) | (static_cast<uint32_t>(col[e]) >> shift);
+}
+
+// First position whose low word is >= c, for c in [0, count].
+__global__ void bounds_kernel(const uint64_t* __restrict__ key, int64_t len, int64_t count, uint32_t* __restrict__ off) {
+  for (int64_t c = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; c <= count;
+       c += static_cast<int64_t>(gridDim.x) * kB) {
+    int64_t lo = 0, hi = len;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (static_cast<uint32_t>(key[mid]) < static_cast<uint32_t>(c)) lo = mid + 1; else hi = mid;
+    }
+    off[c] = static_cast<uint32_t>(lo);
+  }
+}
+
+template <class T>
+__global__ void set_kernel(T* __restrict__ p, T v, int64_t n) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * kB)
+    p[i] = v;
+}
+
+__global__ void place_kernel(const uint64_t* __restrict__ key, const int32_t* __restrict__ col,
+                             const int32_t* __restrict__ perm, const uint32_t* __restrict__ esrc, int64_t m, int shift,
+                             const uint32_t* __restrict__ off, const uint32_t* __restrict__ tile0,
+                             uint16_t* __restrict__ idx16, uint32_t* __restrict__ prow, uint32_t* __restrict__ eid) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; i < m; i += static_cast<int64_t>(gridDim.x) * kB) {
+    const uint64_t k = key[i];
+    const uint32_t c = static_cast<uint32_t>(k), e = static_cast<uint32_t>(k >> 32);
+    const uint32_t rel = static_cast<uint32_t>(i) - off[c], row = esrc[e];
+    const int64_t p = static_cast<int64_t>(tile0[c]) * kTile + rel;
+    const bool end = static_cast<uint32_t>(i) + 1 == off[c + 1] || (rel + 1) % (kRangeTiles * kTile) == 0 ||
+                     esrc[static_cast<uint32_t>(key[i + 1] >> 32)] != row;
+    idx16[p] = static_cast<uint16_t>((static_cast<uint32_t>(col[e]) & ((1u << shift) - 1)) | (end ? kEnd : 0u));
+    prow[p] = row;
+    if (eid) eid[p] = perm ? static_cast<uint32_t>(perm[e]) : e;
+  }
+}
+
+// One wavefront per tile: group ends of the tile.
+__global__ void tile_count_kernel(const uint16_t* __restrict__ idx16, int64_t ntiles, uint32_t* __restrict__ cnt) {
+  const int64_t nw = static_cast<int64_t>(gridDim.x) * (kB / kWave);
+  for (int64_t T = blockIdx.x * static_cast<int64_t>(kB / kWave) + threadIdx.x / kWave; T <= ntiles; T += nw) {
+    uint32_t c = 0;
+    if (T < ntiles)
+      for (int i = 0; i < kItems; ++i) c += __popcll(__ballot((idx16[T * kTile + i * kWave + lane_id()] & kEnd) != 0));
+    if (lane_id() == 0) cnt[T] = c;
+  }
+}
+
+// One wavefront per tile: the rows of its groups; the first group of a range is
+// marked.  range_first: first tile of each tile's range is (T - its chunk's
+// first tile) % kRangeTiles == 0.
+__global__ void group_kernel(const uint16_t* __restrict__ idx16, const uint32_t* __restrict__ prow, int64_t ntiles,
+                             const uint32_t* __restrict__ tile_grp, const uint8_t* __restrict__ range_first,
+                             uint32_t* __restrict__ grow) {
+  const int64_t nw = static_cast<int64_t>(gridDim.x) * (kB / kWave);
+  for (int64_t T = blockIdx.x * static_cast<int64_t>(kB / kWave) + threadIdx.x / kWave; T < ntiles; T += nw) {
+    uint32_t g = tile_grp[T];
+    // The first group that ends in a range need not end in its first tile.
+    bool first = false;
+    for (int64_t t = T;; --t) {
+      if (range_first[t]) {
+        first = tile_grp[t] == g;
+        break;
+      }
+    }
+    for (int i = 0; i < kItems; ++i) {
+      const int64_t p = T * kTile + i * kWave + lane_id();
+      const bool end = (idx16[p] & kEnd) != 0;
+      const uint64_t mask = __ballot(end);
+      const unsigned before = lanes_below(mask);
+      if (end) grow[g + before] = prow[p] | (first && before == 0 ? kFirst : 0u);
+      if (mask) first = false;
+      g += static_cast<uint32_t>(__popcll(mask));
+    }
+  }
+}
+
+struct Bins {
+  const uint32_t* block_bin;  // first bin of every block of 2^block_shift rows
+  const uint8_t* block_shift; // log2 of the rows of its bins
+  int shift;                  // log2 of the rows of a block
+};
+__device__ __forceinline__ uint32_t bin_of(const Bins& B, uint32_t row) {
+  const uint32_t b = row >> B.shift;
+  return B.block_bin[b] + ((row & ((1u << B.shift) - 1)) >> B.block_shift[b]);
+}
+
+__global__ void run_flag_kernel(const uint32_t* __restrict__ grow, int64_t ng, Bins B, uint32_t* __restrict__ flag) {
+  for (int64_t g = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; g <= ng; g += static_cast<int64_t>(gridDim.x) * kB) {
+    if (g == ng) {
+      flag[g] = 0;
+      continue;
+    }
+    const uint32_t w = grow[g];
+    flag[g] = g == 0 || (w & kFirst) || bin_of(B, w & ~kFirst) != bin_of(B, grow[g - 1] & ~kFirst) ? 1u : 0u;
+  }
+}
+
+// pos: scanned flags of run_flag_kernel (group g is in run pos[g + 1] - 1);
+// cut: 1 on the first group of every run and every kWave groups on.
+__global__ void run_first_kernel(const uint32_t* __restrict__ pos, int64_t ng, uint32_t* __restrict__ run_g0) {
+  for (int64_t g = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; g < ng; g += static_cast<int64_t>(gridDim.x) * kB)
+    if (pos[g + 1] != pos[g]) run_g0[pos[g]] = static_cast<uint32_t>(g);
+}
+__global__ void run_cut_kernel(const uint32_t* __restrict__ pos, const uint32_t* __restrict__ run_g0, int64_t ng,
+                               uint32_t* __restrict__ cut) {
+  for (int64_t g = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; g <= ng; g += static_cast<int64_t>(gridDim.x) * kB)
+    cut[g] = g < ng && (static_cast<uint32_t>(g) - run_g0[pos[g + 1] - 1]) % kWave == 0 ? 1u : 0u;
+}
+
+__global__ void run_key_kernel(const uint32_t* __restrict__ grow, int64_t ng, Bins B, const uint32_t* __restrict__ pos,
+                               const uint32_t* __restrict__ bin_row, uint64_t* __restrict__ key,
+                               uint32_t* __restrict__ run_g0, uint16_t* __restrict__ row16) {
+  for (int64_t g = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; g < ng; g += static_cast<int64_t>(gridDim.x) * kB) {
+    const uint32_t row = grow[g] & ~kFirst, b = bin_of(B, row), p = pos[g];
+    row16[g] = static_cast<uint16_t>(row - bin_row[b]);
+    if (pos[g + 1] != p) {
+      key[p] = (static_cast<uint64_t>(p) << 32) | b;
+      run_g0[p] = static_cast<uint32_t>(g);
+    }
+  }
+}
+
+__global__ void run_table_kernel(const uint64_t* __restrict__ key, const uint32_t* __restrict__ run_g0, int64_t nruns,
+                                 uint32_t ng, uint2* __restrict__ runs) {
+  for (int64_t k = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; k < nruns;
+       k += static_cast<int64_t>(gridDim.x) * kB) {
+    const uint32_t r = static_cast<uint32_t>(key[k] >> 32);
+    const uint32_t a = run_g0[r], e = r + 1 < nruns ? run_g0[r + 1] : ng;
+    runs[k] = make_uint2(a, e - a);
+  }
+}
+
+__global__ void weights_kernel(const uint32_t* __restrict__ eid, const float* __restrict__ w, int64_t len,
+                               float* __restrict__ wt) {
+  for (int64_t p = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; p < len; p += static_cast<int64_t>(gridDim.x) * kB) {
+    const uint32_t e = eid[p];
+    wt[p] = e == kNone ? 0.0f : w[e];
+  }
+}
+
+__global__ void block_edges_kernel(const int32_t* __restrict__ rowoff, int64_t n, int shift, int64_t nblocks,
+                                   uint32_t* __restrict__ out) {
+  for (int64_t b = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; b < nblocks;
+       b += static_cast<int64_t>(gridDim.x) * kB) {
+    const int64_t r0 = b << shift, r1 = std::min<int64_t>(n, (b + 1) << shift);
+    out[b] = static_cast<uint32_t>(rowoff[r1] - rowoff[r0]);
+  }
+}
+
+int bits_for(uint64_t v) {  // bits that hold 0 .. v - 1
+  int b = 1;
+  while ((uint64_t(1) << b) < v) ++b;
+  return b;
+}
+
+}  // namespace
+
+// From 2M edges on: below, too few pieces keep the CUs busy.  Forward and
+// adjoint (FP32) / FP64 pull, row sweep against blocks: 1.1M edges 2.7 ms
+// against 4.6; 2.1M edges 0.66 ms against 0.63; 3.2M edges 5.4 ms against 4.1;
+// 4.1M edges 1.08 ms against 0.80; 20.6M edges 4.13 ms against 2.04; 67M edges
+// 75.0 ms against 30.7.
+bool pays(int64_t n, int64_t m) { return m >= (int64_t(1) << 21) && n >= (int64_t(1) << 15) && m < (int64_t(1) << 31); }
+
+void layout_weights(const Plan& P, const float* w, float* wt, hipStream_t s) {
+  weights_kernel<<<grid(P.ntiles * kTile), kB, 0, s>>>(P.eid, w, P.ntiles * kTile, wt);
+  GX_LAUNCHED("bs::weights_kernel");
+}
+
+Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t* perm, int64_t n, int64_t m,
+           int shift, bool weighted, BlockSums& L) {
+  auto view = [&]() {
+    Plan P{};
+    P.pieces = L.pieces.as<Piece>();
+    P.idx16 = L.idx16.as<uint16_t>();
+    P.tile_grp = L.tile_grp.as<uint32_t>();
+    P.eid = L.eid.as<uint32_t>();
+    P.row16 = L.row16.as<uint16_t>();
+    P.runs = L.runs.as<uint2>();
+    P.bins = L.bins.as<Bin>();
+    P.npieces = L.npieces;
+    P.ntiles = L.ntiles;
+    P.ngroups = L.ngroups;
+    P.nbins = L.nbins;
+    P.bin_rows = L.bin_rows;
+    return P;
+  };
+  if (L.ready && L.shift == shift) return view();
+  L.ready = false;
+  GX_REQUIRE(n > 0 && m > 0, "blocked row sums over an empty graph");
+  hipStream_t s = g->stream;
+  const int64_t nchunks = (n + (int64_t(1) << shift) - 1) >> shift;
+  // 1. (chunk, row) order.
+  DevBuf k0, key, esrc, off, tile0, prow;
+  k0.ensure(m * 8);
+  key.ensure((m + 1) * 8);
+  key_kernel<<<grid(m), kB, 0, s>>>(col, m, shift, k0.as<uint64_t>());
+  GX_LAUNCHED("bs::key_kernel");
+  sort_keys_u64(k0.as<uint64_t>(), key.as<uint64_t>(), m, bits_for(nchunks), s);
+  esrc.ensure(m * 4);
+  edge_sources(rowoff, n, m, esrc.as<uint32_t>(), s);
+  off.ensure((nchunks + 1) * 4);
+  bounds_kernel<<<grid(nchunks + 1), kB, 0, s>>>(key.as<uint64_t>(), m, nchunks, off.as<uint32_t>());
+  GX_LAUNCHED("bs::bounds_kernel");
+  std::vector<uint32_t> hoff(nchunks + 1), htile(nchunks + 1);
+  read_bytes(g, hoff.data(), off.p, hoff.size() * 4);
+  // 2. Tiles and pieces.  A piece has at least a range for every wavefront of
+  // its workgroup and at most 32 (64K edges, against which the staging of the
+  // chunk costs little), and about a thousand pieces spread a graph over the
+  // CUs.
+  const int64_t waves = shift == Shape<float>::kShift ? Shape<float>::kBlock / kWave : Shape<double>::kBlock / kWave;
+  const uint32_t kPieceTiles = static_cast<uint32_t>(
+      kRangeTiles * std::min<int64_t>(32, std::max<int64_t>(waves, m / (int64_t(1024) * kRangeTiles * kTile))));
+  std::vector<Piece> pieces;
+  uint32_t nt = 0;
+  for (int64_t c = 0; c < nchunks; ++c) {
+    htile[c] = nt;
+    const uint32_t t = (hoff[c + 1] - hoff[c] + kTile - 1) / kTile;
+    for (uint32_t a = 0; a < t; a += kPieceTiles)
+      pieces.push_back(Piece{static_cast<uint32_t>(c), nt + a, nt + std::min(t, a + kPieceTiles), 0});
+    nt += t;
+  }
+  htile[nchunks] = nt;
+  std::vector<uint8_t> hfirst(nt);
+  for (int64_t c = 0; c < nchunks; ++c)
+    for (uint32_t t = htile[c]; t < htile[c + 1]; ++t) hfirst[t] = (t - htile[c]) % kRangeTiles == 0;
+  // Largest first: the pieces' sizes differ where a chunk ends.
+  std::stable_sort(pieces.begin(), pieces.end(),
+                   [](const Piece& a, const Piece& b) { return a.tile1 - a.tile0 > b.tile1 - b.tile0; });
+  L.npieces = static_cast<int64_t>(pieces.size());
+  L.ntiles = nt;
+  const int64_t len = static_cast<int64_t>(nt) * kTile;
+  L.pieces.ensure(pieces.size() * sizeof(Piece));
+  tile0.ensure(htile.size() * 4);
+  DevBuf first;
+  first.ensure(hfirst.size());
+  GX_HIP(hipMemcpyAsync(L.pieces.p, pieces.data(), pieces.size() * sizeof(Piece), hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(tile0.p, htile.data(), htile.size() * 4, hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(first.p, hfirst.data(), hfirst.size(), hipMemcpyHostToDevice, s));
+  L.idx16.ensure(len * 2);
+  prow.ensure(len * 4);
+  set_kernel<uint16_t><<<grid(len), kB, 0, s>>>(L.idx16.as<uint16_t>(), uint16_t(0), len);
+  if (weighted) {
+    L.eid.ensure(len * 4);
+    set_kernel<uint32_t><<<grid(len), kB, 0, s>>>(L.eid.as<uint32_t>(), kNone, len);
+  }
+  place_kernel<<<grid(m), kB, 0, s>>>(key.as<uint64_t>(), col, perm, esrc.as<uint32_t>(), m, shift, off.as<uint32_t>(),
+                                      tile0.as<uint32_t>(), L.idx16.as<uint16_t>(), prow.as<uint32_t>(),
+                                      weighted ? L.eid.as<uint32_t>() : nullptr);
+  GX_LAUNCHED("bs::place_kernel");
+  // 3. Groups.
+  L.tile_grp.ensure((nt + 1) * 4);
+  tile_count_kernel<<<grid((nt + 1) * int64_t(kWave)), kB, 0, s>>>(L.idx16.as<uint16_t>(), nt, L.tile_grp.as<uint32_t>());
+  GX_LAUNCHED("bs::tile_count_kernel");
+  exclusive_scan_u32(L.tile_grp.as<uint32_t>(), L.tile_grp.as<uint32_t>(), nt + 1, s);
+  uint32_t ng = 0;
+  read_bytes(g, &ng, L.tile_grp.as<uint32_t>() + nt, 4);
+  L.ngroups = ng;
+  DevBuf grow;
+  grow.ensure(static_cast<size_t>(ng) * 4);
+  group_kernel<<<grid(nt * int64_t(kWave)), kB, 0, s>>>(L.idx16.as<uint16_t>(), prow.as<uint32_t>(), nt,
+                                                        L.tile_grp.as<uint32_t>(), first.as<uint8_t>(),
+                                                        grow.as<uint32_t>());
+  GX_LAUNCHED("bs::group_kernel");
+  // 4. Bins: rows per block so that a run holds about 16 groups (a quarter of
+  // a wavefront's lanes), between 512 and 4096 (4 and 32 KB of LDS sums).
+  int bshift = 9;
+  while (bshift < 12 && static_cast<double>(ng) * (int64_t(1) << bshift) < kAvgRun * static_cast<double>(nchunks) * n) ++bshift;
+  const int64_t nblocks = (n + (int64_t(1) << bshift) - 1) >> bshift;
+  DevBuf bedges;
+  bedges.ensure(nblocks * 4);
+  block_edges_kernel<<<grid(nblocks), kB, 0, s>>>(rowoff, n, bshift, nblocks, bedges.as<uint32_t>());
+  GX_LAUNCHED("bs::block_edges_kernel");
+  std::vector<uint32_t> hedges(nblocks), hbin(nblocks);
+  std::vector<uint8_t> hshift(nblocks);
+  read_bytes(g, hedges.data(), bedges.p, nblocks * 4);
+  std::vector<uint32_t> brow;
+  // A block is halved until its groups (at most its edges, and a row's at most
+  // the chunks) are within three times the average or 16 rows are left.
+  const double most = 3.0 * std::max(1.0, static_cast<double>(ng) / static_cast<double>(nblocks));
+  for (int64_t b = 0; b < nblocks; ++b) {
+    int sh = bshift;
+    double w = std::min<double>(hedges[b], static_cast<double>(nchunks) * (int64_t(1) << bshift));
+    while (sh > 4 && w > most) {
+      w /= 2;
+      --sh;
+    }
+    hbin[b] = static_cast<uint32_t>(brow.size());
+    hshift[b] = static_cast<uint8_t>(sh);
+    const int64_t r0 = b << bshift, r1 = std::min<int64_t>(n, (b + 1) << bshift);
+    for (int64_t r = r0; r < r1; r += int64_t(1) << sh) brow.push_back(static_cast<uint32_t>(r));
+  }
+  L.nbins = static_cast<int64_t>(brow.size());
+  brow.push_back(static_cast<uint32_t>(n));
+  L.bin_rows = 1 << bshift;
+  DevBuf drow;
+  drow.ensure(brow.size() * 4);
+  DevBuf dbin, dshift;
+  dbin.ensure(nblocks * 4);
+  dshift.ensure(nblocks);
+  GX_HIP(hipMemcpyAsync(drow.p, brow.data(), brow.size() * 4, hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(dbin.p, hbin.data(), nblocks * 4, hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(dshift.p, hshift.data(), nblocks, hipMemcpyHostToDevice, s));
+  const Bins B{dbin.as<uint32_t>(), dshift.as<uint8_t>(), bshift};
+  // 5. Runs, first as they lie, then cut.
+  DevBuf pos, cut, rkey, rsorted, rg0, boff;
+  pos.ensure((static_cast<size_t>(ng) + 1) * 4);
+  run_flag_kernel<<<grid(ng + int64_t(1)), kB, 0, s>>>(grow.as<uint32_t>(), ng, B, pos.as<uint32_t>());
+  GX_LAUNCHED("bs::run_flag_kernel");
+  exclusive_scan_u32(pos.as<uint32_t>(), pos.as<uint32_t>(), ng + int64_t(1), s);
+  rg0.ensure(static_cast<size_t>(ng) * 4);  // no more runs than groups
+  run_first_kernel<<<grid(ng), kB, 0, s>>>(pos.as<uint32_t>(), ng, rg0.as<uint32_t>());
+  cut.ensure((static_cast<size_t>(ng) + 1) * 4);
+  run_cut_kernel<<<grid(ng + int64_t(1)), kB, 0, s>>>(pos.as<uint32_t>(), rg0.as<uint32_t>(), ng, cut.as<uint32_t>());
+  GX_LAUNCHED("bs::run_cut_kernel");
+  exclusive_scan_u32(cut.as<uint32_t>(), cut.as<uint32_t>(), ng + int64_t(1), s);
+  uint32_t nr = 0;
+  read_bytes(g, &nr, cut.as<uint32_t>() + ng, 4);
+  rkey.ensure(static_cast<size_t>(nr) * 8);
+  rsorted.ensure(static_cast<size_t>(nr) * 8);
+  L.row16.ensure(static_cast<size_t>(ng) * 2);
+  L.runs.ensure(static_cast<size_t>(nr) * sizeof(uint2));
+  boff.ensure((L.nbins + 1) * 4);
+  run_key_kernel<<<grid(ng), kB, 0, s>>>(grow.as<uint32_t>(), ng, B, cut.as<uint32_t>(), drow.as<uint32_t>(),
+                                         rkey.as<uint64_t>(), rg0.as<uint32_t>(), L.row16.as<uint16_t>());
+  GX_LAUNCHED("bs::run_key_kernel");
+  sort_keys_u64(rkey.as<uint64_t>(), rsorted.as<uint64_t>(), nr, bits_for(L.nbins), s);
+  bounds_kernel<<<grid(L.nbins + 1), kB, 0, s>>>(rsorted.as<uint64_t>(), nr, L.nbins, boff.as<uint32_t>());
+  run_table_kernel<<<grid(nr), kB, 0, s>>>(rsorted.as<uint64_t>(), rg0.as<uint32_t>(), nr, ng, L.runs.as<uint2>());
+  GX_LAUNCHED("bs::run_table_kernel");
+  std::vector<uint32_t> hoffs(L.nbins + 1);
+  read_bytes(g, hoffs.data(), boff.p, hoffs.size() * 4);
+  std::vector<Bin> bins(L.nbins);
+  for (int64_t b = 0; b < L.nbins; ++b) bins[b] = Bin{brow[b], brow[b + 1] - brow[b], hoffs[b], hoffs[b + 1]};
+  std::stable_sort(bins.begin(), bins.end(), [](const Bin& a, const Bin& b) { return a.run1 - a.run0 > b.run1 - b.run0; });
+  L.bins.ensure(bins.size() * sizeof(Bin));
+  GX_HIP(hipMemcpyAsync(L.bins.p, bins.data(), bins.size() * sizeof(Bin), hipMemcpyHostToDevice, s));
+  GX_HIP(hipStreamSynchronize(s));  // the host tables above are read by then
+  L.shift = shift;
+  L.ready = true;
+  return view();
+}
+
+}  // namespace bs
+}  // namespace gx

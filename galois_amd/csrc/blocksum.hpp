@@ -1,0 +1,290 @@
+// Deterministic row sums over a CSR/CSC in two streaming phases, for vectors
+// whose gathers the row sweep (rowsweep.hpp) would send to the L2 one by one:
+// that sweep is bound by about 130 G gathers/s, while here an edge gathers
+// from LDS.
+//
+//   layout  edges sorted by (chunk of the gathered index, row): a chunk is
+//           2^shift gathered entries, staged in LDS.  A group is the edges of
+//           one row inside one chunk.  Rows are cut into bins; a run is the
+//           consecutive groups of one (chunk, bin) pair, cut after 64 groups
+//           and where the edges of one wavefront of phase 1 end, so that a row
+//           appears at most once in a run.  Built once per graph.
+//   phase 1 (gather_kernel) one workgroup per piece of a chunk: stages the
+//           chunk, then its wavefronts stream the edges (2 bytes of index per
+//           edge, bit 15 set on the last edge of a group; 4 bytes of weight
+//           where there are weights), add each group's products in FP64 and
+//           write one partial sum per group in layout order.
+//   phase 2 (sum_kernel) one wavefront per bin adds the bin's runs, in chunk
+//           order, to FP64 sums in LDS and finalises the bin's rows.
+//
+// Every order is fixed: a group is summed by one wavefront front to back, and
+// a row's partial sums are added by one wavefront, whose LDS additions are
+// served in order (no two lanes of one addition hold the same row).  So the
+// results are bit-reproducible run to run without exact sums, for any sign,
+// scale, infinity or NaN.
+//
+// Bytes per sweep: 2 per edge (6 with weights), 2R + 2 per group (R the size
+// of a partial sum: FP32 or FP64 as the vector), R + what the finaliser reads
+// and writes per row.
+//
+// Bound: phase 1 by memory (67M edges with weights, FP32: 0.50 GB in 130 us, 3.9
+// TB/s), phase 2 by the latency of its short runs (25M groups: 85-100 us).  One
+// such sweep took 510-555 us gather by gather; 20.6M edges in FP64 156 us, 38 +
+// 40 us here.
+#pragma once
+
+#include <algorithm>
+
+#include "gx_device.hpp"
+#include "gx_internal.hpp"
+#include "rowsweep.hpp"
+
+namespace gx {
+namespace bs {
+
+constexpr int kItems = 8;                // edges per lane and tile
+constexpr int kTile = kWave * kItems;    // 512
+constexpr int kRangeTiles = 4;           // tiles of one wavefront's range: a group never crosses its end
+constexpr uint32_t kEnd = 1u << 15;      // idx16 flag: last edge of a group
+constexpr int kSumGrid = 256 * 16;       // most wavefronts of phase 2
+
+// Gathered entries per chunk (64 KB of LDS) and lanes per workgroup of phase 1:
+// with the tiles' group sums both precisions then keep 16 wavefronts on a CU.
+template <class Real>
+struct Shape;
+template <>
+struct Shape<float> {
+  static constexpr int kShift = 14, kBlock = 512;
+};
+template <>
+struct Shape<double> {
+  static constexpr int kShift = 13, kBlock = 1024;
+};
+
+struct Piece {
+  uint32_t chunk, tile0, tile1, pad;
+};
+
+struct Bin {
+  uint32_t row0, rows, run0, run1;
+};
+
+struct Plan {
+  const Piece* pieces;
+  const uint16_t* idx16;     // ntiles * kTile
+  const uint32_t* tile_grp;  // ntiles + 1: first group of every tile
+  const uint32_t* eid;       // ntiles * kTile: edge id of every position, ~0 = padding (weighted layouts)
+  const uint16_t* row16;     // per group: row in its bin
+  const uint2* runs;         // per bin, in chunk order: first group, length (at most kWave)
+  const Bin* bins;           // nbins, most runs first
+  int64_t npieces, ntiles, ngroups, nbins;
+  int bin_rows;              // most rows of a bin (LDS sums)
+};
+
+// Whether the layout pays for and can be built for this shape (see blocksum.hip).
+bool pays(int64_t n, int64_t m);
+// Builds (or returns the cached) layout of the row offsets `rowoff` and gathered
+// indices `col`; perm != null: edge ids are perm[position] (CSC slot -> CSR
+// edge).  shift: Shape<Real>::kShift.
+Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t* perm, int64_t n, int64_t m,
+           int shift, bool weighted, BlockSums& cache);
+
+// wt[p] = w[eid[p]] (0 where padded).
+void layout_weights(const Plan& P, const float* w, float* wt, hipStream_t s);
+
+__device__ __forceinline__ uint32_t wave_exclusive_sum(uint32_t v, int lane) {
+  uint32_t x = v;
+  const int in_row = lane & 15;
+  uint32_t o;
+  o = __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += in_row >= 1 ? o : 0u;
+  o = __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += in_row >= 2 ? o : 0u;
+  o = __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += in_row >= 4 ? o : 0u;
+  o = __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += in_row >= 8 ? o : 0u;
+  o = __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += (lane & 16) ? o : 0u;
+  o = __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  x += (lane & 32) ? o : 0u;
+  return x - v;
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// The loads of one tile: 8 consecutive edges per lane.
+template <bool W>
+struct TileLoad {
+  u32x4 idx;
+  f32x4 w[W ? 2 : 1];
+  __device__ __forceinline__ void load(const uint16_t* __restrict__ idx16, const float* __restrict__ wt, int64_t T,
+                                       int lane) {
+    idx = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(idx16 + T * kTile) + lane);
+    if constexpr (W) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(wt + T * kTile) + 2 * lane;
+      w[0] = __builtin_nontemporal_load(p);
+      w[1] = __builtin_nontemporal_load(p + 1);
+    }
+  }
+};
+
+// Phase 1 (see the file comment).  y: n entries.
+template <class Real, bool W>
+__global__ void __launch_bounds__(Shape<Real>::kBlock) gather_kernel(Plan P, const float* __restrict__ wt,
+                                                                     const Real* __restrict__ y, int64_t n,
+                                                                     Real* __restrict__ partial,
+                                                                     const unsigned* __restrict__ skip) {
+  if (skip && *skip) return;
+  constexpr int kSpan = 1 << Shape<Real>::kShift, kBlock = Shape<Real>::kBlock, kWaves = kBlock / kWave;
+  __shared__ Real ys[kSpan];
+  __shared__ Real stage[kWaves][kTile];
+  const Piece pc = P.pieces[blockIdx.x];
+  const int64_t base = static_cast<int64_t>(pc.chunk) * kSpan;
+  const int cnt = static_cast<int>(n - base < kSpan ? n - base : kSpan);
+  for (int i = threadIdx.x; i < cnt; i += kBlock) ys[i] = y[base + i];
+  __syncthreads();
+  const int lane = static_cast<int>(lane_id());
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  Real* st = stage[wid];
+  for (int64_t r0 = pc.tile0 + wid * kRangeTiles; r0 < pc.tile1; r0 += kWaves * kRangeTiles) {
+    const int64_t r1 = r0 + kRangeTiles < pc.tile1 ? r0 + kRangeTiles : pc.tile1;
+    double open = 0;  // sum of the group open at the start of the tile (uniform)
+    TileLoad<W> cur, nxt;
+    cur.load(P.idx16, wt, r0, lane);
+    for (int64_t T = r0; T < r1; ++T) {
+      if (T + 1 < r1) nxt.load(P.idx16, wt, T + 1, lane);
+      const uint32_t g0 = P.tile_grp[T], g1 = P.tile_grp[T + 1];
+      double v[kItems];
+      uint32_t ends = 0;
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) {
+        const uint32_t word = (cur.idx[u / 2] >> (16 * (u & 1))) & 0xffffu;
+        ends |= (word >> 15) << u;
+        v[u] = static_cast<double>(ys[word & (kSpan - 1)]);
+        if constexpr (W) v[u] *= static_cast<double>(cur.w[u / 4][u & 3]);
+      }
+      double tail = 0;
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) {
+        tail += v[u];
+        if ((ends >> u) & 1u) tail = 0;
+      }
+      const uint64_t heads = __ballot(ends != 0);
+      const uint64_t upto = heads & (~0ull >> (63 - lane));
+      const double seg = rs::wave_seg_scan(tail, upto ? 63 - __builtin_clzll(upto) : 0, lane);
+      double acc = __shfl_up(seg, 1);
+      if (lane == 0) acc = 0;
+      if ((heads & ((1ull << lane) - 1)) == 0) acc += open;
+      const double last = __shfl(seg, kWave - 1);
+      open = heads ? last : open + last;
+      uint32_t slot = wave_exclusive_sum(static_cast<uint32_t>(__popc(ends)), lane);
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) {
+        acc += v[u];
+        if ((ends >> u) & 1u) {
+          st[slot++] = static_cast<Real>(acc);
+          acc = 0;
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (uint32_t j = lane; j < g1 - g0; j += kWave) partial[g0 + j] = st[j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      cur = nxt;
+    }
+  }
+}
+
+// Phase 2: one wavefront per workgroup, bin b on workgroup b mod the grid.  It
+// is a chain of short loads (a run is about half a wavefront's lanes), so 16
+// runs are in flight at a time and the next 64 runs' descriptors are loaded
+// ahead: with 4 in flight it took 2-3 times as long.
+template <class Real, class Fin>
+__global__ void __launch_bounds__(kWave) sum_kernel(Plan P, const Real* __restrict__ partial, Fin fin,
+                                                    double* __restrict__ part0, double* __restrict__ part1,
+                                                    const unsigned* __restrict__ skip) {
+  if (skip && *skip) return;
+  fin.load();
+  extern __shared__ double acc[];
+  const int lane = static_cast<int>(lane_id());
+  double a0 = 0, a1 = 0;
+  constexpr int kRuns = 16;
+  for (int64_t b = blockIdx.x; b < P.nbins; b += gridDim.x) {
+    const Bin bin = P.bins[b];
+    const uint32_t row0 = bin.row0, q0 = bin.run0, q1 = bin.run1;
+    const int rows = static_cast<int>(bin.rows);
+    uint2 next{0, 0};
+    if (q0 + lane < q1) next = P.runs[q0 + lane];
+    for (int i = lane; i < rows; i += kWave) acc[i] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t q = q0; q < q1; q += kWave) {
+      const uint2 mine = next;  // lanes past the last run: length 0
+      next = make_uint2(0, 0);
+      if (q + kWave + lane < q1) next = P.runs[q + kWave + lane];
+      const int nr = static_cast<int>(q1 - q < kWave ? q1 - q : kWave);
+      for (int i = 0; i < nr; i += kRuns) {
+        uint32_t r[kRuns];
+        Real x[kRuns];
+#pragma unroll
+        for (int k = 0; k < kRuns; ++k) {
+          const uint32_t g = __builtin_amdgcn_readlane(mine.x, i + k), len = __builtin_amdgcn_readlane(mine.y, i + k);
+          r[k] = 0;
+          x[k] = Real(0);
+          if (static_cast<uint32_t>(lane) < len) {
+            r[k] = P.row16[g + lane];
+            x[k] = partial[g + lane];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kRuns; ++k)
+          if (static_cast<uint32_t>(lane) < static_cast<uint32_t>(__builtin_amdgcn_readlane(mine.y, i + k)))
+            atomicAdd(&acc[r[k]], static_cast<double>(x[k]));
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    constexpr int kU = 4;
+    for (int i = lane; i < rows; i += kU * kWave) {
+      typename Fin::Pre pre[kU];
+#pragma unroll
+      for (int k = 0; k < kU; ++k)
+        if (i + k * kWave < rows) pre[k] = fin.pre(row0 + i + k * kWave);
+#pragma unroll
+      for (int k = 0; k < kU; ++k)
+        if (i + k * kWave < rows) fin(row0 + i + k * kWave, acc[i + k * kWave], pre[k], a0, a1);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  a0 = wave_sum(a0);
+  a1 = wave_sum(a1);
+  if (lane == 0) {
+    part0[blockIdx.x] = a0;
+    part1[blockIdx.x] = a1;
+  }
+}
+
+// Host: one sweep; wt null: unweighted.  Returns the number of partials
+// written to part0/part1 (at most kSumGrid).
+template <class Real, class Fin>
+int launch(const Plan& P, const float* wt, const Real* y, int64_t n, Real* partial, const Fin& fin,
+           const unsigned* skip, double* part0, double* part1, hipStream_t s) {
+  if (P.npieces > 0) {
+    if (wt)
+      gather_kernel<Real, true><<<static_cast<unsigned>(P.npieces), Shape<Real>::kBlock, 0, s>>>(P, wt, y, n, partial, skip);
+    else
+      gather_kernel<Real, false><<<static_cast<unsigned>(P.npieces), Shape<Real>::kBlock, 0, s>>>(P, wt, y, n, partial, skip);
+    GX_LAUNCHED("bs::gather_kernel");
+  }
+  const int grid = static_cast<int>(std::min<int64_t>(P.nbins, kSumGrid));
+  sum_kernel<Real, Fin><<<grid, kWave, P.bin_rows * sizeof(double), s>>>(P, partial, fin, part0, part1, skip);
+  GX_LAUNCHED("bs::sum_kernel");
+  return grid;
+}
+
+}  // namespace bs
+}  // namespace gx

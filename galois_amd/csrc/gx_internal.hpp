@@ -135,6 +135,15 @@ struct PbLayout {
   DevBuf gsrc16, dst16, vals, pieces, jobs, tasks, multi, gacc;
 };
 
+// Layout of the blocked row sums (blocksum.hpp) over one CSR/CSC for chunks of
+// 2^shift gathered entries, built once per graph.
+struct BlockSums {
+  bool ready = false;
+  int shift = 0, bin_rows = 0;
+  int64_t npieces = 0, ntiles = 0, ngroups = 0, nbins = 0;
+  DevBuf pieces, idx16, eid, tile_grp, row16, runs, bins;
+};
+
 struct DegreeOrder {
   bool ready = false;
   DevBuf new_of_old, old_of_new, trow, tcol, outdeg;
@@ -144,6 +153,7 @@ struct DegreeOrder {
   DevBuf rowA, colA, rowB, colB;
   PullPlan planA, planB;
   PbLayout pb;
+  BlockSums sums;  // transpose, FP64 pull
 };
 
 // Degree-ordered copy of a weighted CSR for the frontier kernels: vertices
@@ -200,6 +210,7 @@ struct gx_graph {
   int64_t max_deg = -1;  // largest out-degree, computed on demand (gx::max_degree)
   gx::PullPlan pull_plan;            // degree-ordered transpose (PageRank pull)
   gx::PullPlan csc_plan, csr_plan;   // plain transpose / CSR (weighted PageRank and adjoint)
+  gx::BlockSums csc_sums[2], csr_sums[2];  // the same sums in blocks, FP32 and FP64 (weighted PageRank and adjoint)
   gx::DegreeOrder degree_order;
   gx::Relabeled relab;
   std::shared_ptr<void> bc_cache;  // batched-BC tables (bc.hip)

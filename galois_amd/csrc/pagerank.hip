@@ -27,7 +27,9 @@
 //  - The row sums are the tile sweep of rowsweep.hpp: a wavefront per 512
 //    edges, FP64 sums, coalesced per-row finalisation (x', y' = x'/outdeg,
 //    residual, dangling mass).  Rows spanning chunks of tiles are completed by
-//    a second small launch.
+//    a second small launch.  FP64 on 2M edges and more goes through the
+//    blocked sums of blocksum.hpp instead, as deterministic and not bound by
+//    the gathers.
 //  - The residual and dangling mass are accumulated in FP64 per workgroup and
 //    reduced in a fixed order (deterministic).
 //  - Iterations are enqueued in batches with no host round trip: each sweep
@@ -38,6 +40,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "blocksum.hpp"
 #include "frontier.hpp"
 #include "gx_device.hpp"
 #include "gx_internal.hpp"
@@ -396,8 +399,14 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   DegreeOrder& D = g->degree_order;
   const bool blocked = use_blocking(g, sizeof(Real));
   const int64_t hot = blocked ? 0 : hot_sources(n, sizeof(Real));
+  // FP64 in one pass: the deterministic sums in blocks where they pay.
+  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && bs::pays(n, g->m);
   rs::RowPlan P{}, PA{};
-  if (blocked) {
+  bs::Plan S{};
+  if (sums) {
+    S = bs::build(g, D.trow.as<int32_t>(), D.tcol.as<int32_t>(), nullptr, n, g->m, bs::Shape<Real>::kShift, false,
+                  D.sums);
+  } else if (blocked) {
     pb::build_layout(g);
     D.pb.vals.ensure(D.pb.ngroups * sizeof(Real));  // grows once for FP64 contributions
   } else if (hot > 0) {
@@ -416,11 +425,13 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   Real* yb = g->scratch<Real>(WS_V1, 2 * n);
   Real* x[2] = {xb, xb + n};
   Real* y[2] = {yb, yb + n};
-  const int nparts = blocked ? static_cast<int>(std::max<int64_t>(L.ntasks + L.nmulti, rs::kParts)) : rs::kParts;
+  const int nparts = blocked ? static_cast<int>(std::max<int64_t>(L.ntasks + L.nmulti, rs::kParts))
+                             : std::max(rs::kParts, bs::kSumGrid);
   double* parts = g->scratch<double>(WS_REDUCE, 2 * nparts);
   double* part_resid = parts;
   double* part_dang = parts + nparts;
-  double* carry = blocked ? nullptr : g->scratch<double>(WS_V2, 2 * P.nchunks);
+  double* carry = blocked || sums ? nullptr : g->scratch<double>(WS_V2, 2 * P.nchunks);
+  Real* partial = sums ? g->scratch<Real>(WS_BC_SIGMA, S.ngroups) : nullptr;
   PrState* state = g->scratch<PrState>(WS_COUNTERS, 1);
   PrState* host = static_cast<PrState*>(g->host_pinned(sizeof(PrState)));
 
@@ -464,6 +475,15 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
       PrSrc<Real> src{y[cur]};
       PrFin<Real> fin{state, x[cur], x[nxt], y[nxt], outdeg, part, Real(0), Real(0)};
       ktimer.begin();
+      if (sums) {
+        const int np = bs::launch<Real>(S, nullptr, y[cur], n, partial, fin, &state->converged, part_resid, part_dang, s);
+        ktimer.end();
+        pr_reduce_kernel<<<1, kBlock, 0, s>>>(state, part_resid, part_dang, np, static_cast<unsigned>(nxt));
+        GX_LAUNCHED("pr_reduce_kernel");
+        launches += 3;
+        cur = nxt;
+        continue;
+      }
       if (hot > 0) {
         rs::launch_sweep<Real>(PA, src, PartFin<Real>{part}, &state->converged, partsA, partsA + rs::kParts, carryA, s,
                                nullptr);

@@ -13,12 +13,14 @@
 //   lambda = c + alpha*(P lambda + (sum(lambda)/n) d),
 //   dL/dt = (1-alpha)*lambda,
 //   dL/dw_uv = alpha * x_u * (lambda_v - (P lambda)_u) / s_u.
-// Both solves are Jacobi iterations on the row sweep of rowsweep.hpp (FP32
-// compensated or FP64), stopping at sum|change| < tol or max_iter.  The
+// Both solves are Jacobi iterations on the row sweep of rowsweep.hpp or, from 2M
+// edges on, the blocked row sums of blocksum.hpp (the weights are put into the
+// layout's order once per call), stopping at sum|change| < tol or max_iter.  The
 // backward pass needs only the converged forward vector x.
 #include <algorithm>
 #include <cmath>
 
+#include "blocksum.hpp"
 #include "frontier.hpp"
 #include "gx_device.hpp"
 #include "gx_internal.hpp"
@@ -328,31 +330,46 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
   const int64_t n = g->n, m = g->m;
   hipStream_t s = g->stream;
   build_transpose(g);
-  const rs::RowPlan P = rs::build_plan(g, g->trow(), g->tcol(), n, m, g->csc_plan);
+  const bool blocked = bs::pays(n, m);
+  const rs::RowPlan P = blocked ? rs::RowPlan{} : rs::build_plan(g, g->trow(), g->tcol(), n, m, g->csc_plan);
+  const bs::Plan L = blocked ? bs::build(g, g->trow(), g->tcol(), g->tperm(), n, m, bs::Shape<Real>::kShift, true,
+                                         g->csc_sums[sizeof(Real) == 8])
+                             : bs::Plan{};
   const rs::RowPlan W = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);  // row sums of the weights
   Real* inv_s = g->scratch<Real>(WS_V4, n);
-  Real* wt = g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
+  Real* wt = blocked ? nullptr : g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
+  float* wl = blocked ? g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile) : nullptr;
+  Real* partial = blocked ? g->scratch<Real>(WS_BC_SIGMA, L.ngroups) : nullptr;
   Real* xb = g->scratch<Real>(WS_V0, 2 * n);
   Real* yb = g->scratch<Real>(WS_V1, 2 * n);
   Real* xs[2] = {xb, xb + n};
   Real* ys[2] = {yb, yb + n};
-  const int nparts = rs::kParts;
+  const int nparts = std::max(rs::kParts, bs::kSumGrid);
   double* parts = g->scratch<double>(WS_REDUCE, 2 * nparts);
-  double* carry = g->scratch<double>(WS_V2, std::max<int64_t>(2 * P.nchunks, 1));
+  double* carry = g->scratch<double>(WS_V2, std::max<int64_t>(2 * std::max(P.nchunks, W.nchunks), 1));
   AdState* state = g->scratch<AdState>(WS_COUNTERS, 1);
   AdState* host = static_cast<AdState*>(g->host_pinned(sizeof(AdState)));
   RegionTimer region(s);
   KernelTimer ktimer(s);
   uint32_t launches = 7;
   rs::launch_sweep<Real>(W, RowWeights<Real>{w}, InvFin<Real>{inv_s}, nullptr, parts, parts + nparts, carry, s, nullptr);
-  if (m) permute_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, g->tperm(), m, wt);
+  if (blocked)
+    bs::layout_weights(L, w, wl, s);
+  else if (m)
+    permute_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, g->tperm(), m, wt);
   ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / n, max_iter);
   fwd_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(xs[0], ys[0], inv_s, n, parts);
   ad_init_reduce_kernel<<<1, kBlock, 0, s>>>(state, parts, kSweepGrid, 0);
   GX_LAUNCHED("forward init");
   auto sweep = [&](int cur, int nxt) {
-    WSrc<Real> src{ys[cur], wt};
     FwdFin<Real> fin{state, t, inv_s, xs[cur], xs[nxt], ys[nxt], Real(0), Real(0)};
+    if (blocked) {
+      ktimer.begin();
+      const int np = bs::launch<Real>(L, wl, ys[cur], n, partial, fin, &state->converged, parts, parts + nparts, s);
+      ktimer.end();
+      return np;
+    }
+    WSrc<Real> src{ys[cur], wt};
     return rs::launch_sweep<Real>(P, src, fin, &state->converged, parts, parts + nparts, carry, s,
                                   &ktimer);
   };
@@ -377,12 +394,17 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   const int64_t n = g->n, m = g->m;
   hipStream_t s = g->stream;
   const rs::RowPlan P = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);
+  const bool blocked = bs::pays(n, m);
+  const bs::Plan L =
+      blocked ? bs::build(g, g->row, g->col, nullptr, n, m, bs::Shape<Real>::kShift, true, g->csr_sums[sizeof(Real) == 8]) : bs::Plan{};
   Real* inv_s = g->scratch<Real>(WS_V4, n);
-  Real* wr = g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
+  Real* wr = blocked ? nullptr : g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
+  float* wl = blocked ? g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile) : nullptr;
+  Real* partial = blocked ? g->scratch<Real>(WS_BC_SIGMA, L.ngroups) : nullptr;
   Real* lb = g->scratch<Real>(WS_V0, 2 * n);
   Real* pl = g->scratch<Real>(WS_V1, n);
   Real* lam[2] = {lb, lb + n};
-  const int nparts = rs::kParts;
+  const int nparts = std::max(rs::kParts, bs::kSumGrid);
   double* parts = g->scratch<double>(WS_REDUCE, 2 * nparts);
   double* carry = g->scratch<double>(WS_V2, std::max<int64_t>(2 * P.nchunks, 1));
   uint32_t* hubq = g->scratch<uint32_t>(WS_Q2, n);
@@ -394,28 +416,34 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   KernelTimer ktimer(s);
   uint32_t launches = 6;
   rs::launch_sweep<Real>(P, RowWeights<Real>{w}, InvFin<Real>{inv_s}, nullptr, parts, parts + nparts, carry, s, nullptr);
-  if (m) convert_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, m, wr);
+  if (blocked)
+    bs::layout_weights(L, w, wl, s);
+  else if (m)
+    convert_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, m, wr);
   ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / n, max_iter);
   adj_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(lam[0], c, n, parts);
   ad_init_reduce_kernel<<<1, kBlock, 0, s>>>(state, parts, kSweepGrid, 1);
   GX_LAUNCHED("adjoint init");
-  const Real* wsrc = wr;
+  // One sweep over the vector lv, timed when it iterates.
+  auto sums = [&](const Real* lv, const AdjFin<Real>& fin, const unsigned* skip, KernelTimer* timer) {
+    if (blocked) {
+      if (timer) timer->begin();
+      const int np = bs::launch<Real>(L, wl, lv, n, partial, fin, skip, parts, parts + nparts, s);
+      if (timer) timer->end();
+      return np;
+    }
+    return rs::launch_sweep<Real>(P, WSrc<Real>{lv, wr}, fin, skip, parts, parts + nparts, carry, s, timer);
+  };
   auto sweep = [&](int cur, int nxt) {
-    WSrc<Real> src{lam[cur], wsrc};
-    AdjFin<Real> fin{state, c, inv_s, lam[cur], lam[nxt], pl, 0, Real(0), Real(0)};
-    return rs::launch_sweep<Real>(P, src, fin, &state->converged, parts, parts + nparts, carry, s,
-                                  &ktimer);
+    return sums(lam[cur], AdjFin<Real>{state, c, inv_s, lam[cur], lam[nxt], pl, 0, Real(0), Real(0)},
+                &state->converged, &ktimer);
   };
   const uint32_t iters = iterate(g, state, host, parts, parts + nparts, 1, max_iter, sweep, launches);
   const Real* lam_f = lam[host->final_buf];
   // (P lambda) at the converged lambda: one more sweep with final_pass set.
   // Its dangling value is sum(lambda)/n, which the last reduce stored in base.
-  {
-    WSrc<Real> src{lam_f, wsrc};
-    AdjFin<Real> fin{state, c, inv_s, lam_f, nullptr, pl, 1, Real(0), Real(0)};
-    rs::launch_sweep<Real>(P, src, fin, nullptr, parts, parts + nparts, carry, s, nullptr);
-    launches += 2;
-  }
+  sums(lam_f, AdjFin<Real>{state, c, inv_s, lam_f, nullptr, pl, 1, Real(0), Real(0)}, nullptr, nullptr);
+  launches += 2;
   zero_u32_kernel<<<1, 64, 0, s>>>(hubc, 2);
   GradOp<Real> op{g->col, x, lam_f, pl, inv_s, grad_w, static_cast<Real>(alpha)};
   grad_edges_kernel<Real><<<grid_for(n, kBlock, 256 * 16), kBlock, 0, s>>>(g->row, op, static_cast<unsigned>(n), hubq,

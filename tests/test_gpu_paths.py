@@ -108,7 +108,13 @@ SWEEPS = [(2, 1, 0), (600, 511, 0), (600, 513, 0), (5000, 20000, 3), (3000, 9000
           (40001, 700000, 1)]
 
 
-@pytest.mark.parametrize("n,m,hubs", SWEEPS)
+# The blocked sums' side of the size rule: few chunks and many, rows with edges in
+# every chunk and over many of a wavefront's ranges, mostly empty rows, a last
+# chunk of one vertex.
+BLOCKS = [(32768, 2300000, 0), (65537, 2600000, 2), (1 << 20, 2200000, 1), (300001, 5000000, 3)]
+
+
+@pytest.mark.parametrize("n,m,hubs", SWEEPS + BLOCKS)
 def test_row_sweep_shapes(gx, n, m, hubs):
     """Weighted forward and adjoint in FP64 (FP64 sums of FP64 products: 1e-12
     relative to the largest value) and FP32 (1e-5 of it: 40-odd iterations of
