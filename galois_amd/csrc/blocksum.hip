@@ -221,20 +221,44 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   GX_REQUIRE(n > 0 && m > 0, "blocked row sums over an empty graph");
   hipStream_t s = g->stream;
   const int64_t nchunks = (n + (int64_t(1) << shift) - 1) >> shift;
+  // Working memory, allocated and freed once (freeing waits for the device):
+  // five areas used again as the steps go on.  No more groups and runs than
+  // edges; every chunk pads its last tile.
+  const int64_t most_tiles = (m + kTile - 1) / kTile + nchunks;
+  const size_t area_a = (m + 2) * 8, area_b = (m + 2) * 8, area_c = (m + 2) * 4, area_d = most_tiles * kTile * 8,
+               area_e = (m + 2) * 4;
+  const int64_t most_blocks = n / 512 + 1, most_bins = n / 16 + most_blocks + 1;
+  const size_t tables = 2 * (nchunks + 1) * 4 + most_tiles + 9 * most_blocks + 8 * (most_bins + 1) + 16 * 256;
+  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+  DevBuf work;
+  work.ensure(up(area_a) + up(area_b) + up(area_c) + up(area_d) + up(area_e) + tables);
+  char* top = work.as<char>();
+  auto take = [&](size_t b) {
+    char* p = top;
+    top += up(b);
+    GX_REQUIRE(top <= work.as<char>() + work.bytes, "blocked row sums: working memory");
+    return p;
+  };
+  char* const wa = take(area_a);
+  char* const wb = take(area_b);
+  char* const wc = take(area_c);
+  char* const wd = take(area_d);
+  char* const we = take(area_e);
   // 1. (chunk, row) order.
-  DevBuf k0, key, esrc, off, tile0, prow;
-  k0.ensure(m * 8);
-  key.ensure((m + 1) * 8);
-  key_kernel<<<grid(m), kB, 0, s>>>(col, m, shift, k0.as<uint64_t>());
+  uint64_t* k0 = reinterpret_cast<uint64_t*>(wa);
+  uint64_t* key = reinterpret_cast<uint64_t*>(wb);
+  uint32_t* esrc = reinterpret_cast<uint32_t*>(wc);
+  uint32_t* prow = reinterpret_cast<uint32_t*>(wd);
+  uint32_t* off = reinterpret_cast<uint32_t*>(take((nchunks + 1) * 4));
+  uint32_t* tile0 = reinterpret_cast<uint32_t*>(take((nchunks + 1) * 4));
+  key_kernel<<<grid(m), kB, 0, s>>>(col, m, shift, k0);
   GX_LAUNCHED("bs::key_kernel");
-  sort_keys_u64(k0.as<uint64_t>(), key.as<uint64_t>(), m, bits_for(nchunks), s);
-  esrc.ensure(m * 4);
-  edge_sources(rowoff, n, m, esrc.as<uint32_t>(), s);
-  off.ensure((nchunks + 1) * 4);
-  bounds_kernel<<<grid(nchunks + 1), kB, 0, s>>>(key.as<uint64_t>(), m, nchunks, off.as<uint32_t>());
+  sort_keys_u64(k0, key, m, bits_for(nchunks), s);
+  edge_sources(rowoff, n, m, esrc, s);
+  bounds_kernel<<<grid(nchunks + 1), kB, 0, s>>>(key, m, nchunks, off);
   GX_LAUNCHED("bs::bounds_kernel");
   std::vector<uint32_t> hoff(nchunks + 1), htile(nchunks + 1);
-  read_bytes(g, hoff.data(), off.p, hoff.size() * 4);
+  read_bytes(g, hoff.data(), off, hoff.size() * 4);
   // 2. Tiles and pieces.  A piece has at least a range for every wavefront of
   // its workgroup and at most 32 (64K edges, against which the staging of the
   // chunk costs little), and about a thousand pieces spread a graph over the
@@ -262,21 +286,17 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   L.ntiles = nt;
   const int64_t len = static_cast<int64_t>(nt) * kTile;
   L.pieces.ensure(pieces.size() * sizeof(Piece));
-  tile0.ensure(htile.size() * 4);
-  DevBuf first;
-  first.ensure(hfirst.size());
+  uint8_t* first = reinterpret_cast<uint8_t*>(take(hfirst.size()));
   GX_HIP(hipMemcpyAsync(L.pieces.p, pieces.data(), pieces.size() * sizeof(Piece), hipMemcpyHostToDevice, s));
-  GX_HIP(hipMemcpyAsync(tile0.p, htile.data(), htile.size() * 4, hipMemcpyHostToDevice, s));
-  GX_HIP(hipMemcpyAsync(first.p, hfirst.data(), hfirst.size(), hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(tile0, htile.data(), htile.size() * 4, hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(first, hfirst.data(), hfirst.size(), hipMemcpyHostToDevice, s));
   L.idx16.ensure(len * 2);
-  prow.ensure(len * 4);
   set_kernel<uint16_t><<<grid(len), kB, 0, s>>>(L.idx16.as<uint16_t>(), uint16_t(0), len);
   if (weighted) {
     L.eid.ensure(len * 4);
     set_kernel<uint32_t><<<grid(len), kB, 0, s>>>(L.eid.as<uint32_t>(), kNone, len);
   }
-  place_kernel<<<grid(m), kB, 0, s>>>(key.as<uint64_t>(), col, perm, esrc.as<uint32_t>(), m, shift, off.as<uint32_t>(),
-                                      tile0.as<uint32_t>(), L.idx16.as<uint16_t>(), prow.as<uint32_t>(),
+  place_kernel<<<grid(m), kB, 0, s>>>(key, col, perm, esrc, m, shift, off, tile0, L.idx16.as<uint16_t>(), prow,
                                       weighted ? L.eid.as<uint32_t>() : nullptr);
   GX_LAUNCHED("bs::place_kernel");
   // 3. Groups.
@@ -287,24 +307,21 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   uint32_t ng = 0;
   read_bytes(g, &ng, L.tile_grp.as<uint32_t>() + nt, 4);
   L.ngroups = ng;
-  DevBuf grow;
-  grow.ensure(static_cast<size_t>(ng) * 4);
-  group_kernel<<<grid(nt * int64_t(kWave)), kB, 0, s>>>(L.idx16.as<uint16_t>(), prow.as<uint32_t>(), nt,
-                                                        L.tile_grp.as<uint32_t>(), first.as<uint8_t>(),
-                                                        grow.as<uint32_t>());
+  uint32_t* grow = reinterpret_cast<uint32_t*>(wc);  // the edges' rows are not needed any more
+  group_kernel<<<grid(nt * int64_t(kWave)), kB, 0, s>>>(L.idx16.as<uint16_t>(), prow, nt, L.tile_grp.as<uint32_t>(),
+                                                        first, grow);
   GX_LAUNCHED("bs::group_kernel");
   // 4. Bins: rows per block so that a run holds about 16 groups (a quarter of
   // a wavefront's lanes), between 512 and 4096 (4 and 32 KB of LDS sums).
   int bshift = 9;
   while (bshift < 12 && static_cast<double>(ng) * (int64_t(1) << bshift) < kAvgRun * static_cast<double>(nchunks) * n) ++bshift;
   const int64_t nblocks = (n + (int64_t(1) << bshift) - 1) >> bshift;
-  DevBuf bedges;
-  bedges.ensure(nblocks * 4);
-  block_edges_kernel<<<grid(nblocks), kB, 0, s>>>(rowoff, n, bshift, nblocks, bedges.as<uint32_t>());
+  uint32_t* bedges = reinterpret_cast<uint32_t*>(take(nblocks * 4));
+  block_edges_kernel<<<grid(nblocks), kB, 0, s>>>(rowoff, n, bshift, nblocks, bedges);
   GX_LAUNCHED("bs::block_edges_kernel");
   std::vector<uint32_t> hedges(nblocks), hbin(nblocks);
   std::vector<uint8_t> hshift(nblocks);
-  read_bytes(g, hedges.data(), bedges.p, nblocks * 4);
+  read_bytes(g, hedges.data(), bedges, nblocks * 4);
   std::vector<uint32_t> brow;
   // A block is halved until its groups (at most its edges, and a row's at most
   // the chunks) are within three times the average or 16 rows are left.
@@ -324,43 +341,39 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   L.nbins = static_cast<int64_t>(brow.size());
   brow.push_back(static_cast<uint32_t>(n));
   L.bin_rows = 1 << bshift;
-  DevBuf drow;
-  drow.ensure(brow.size() * 4);
-  DevBuf dbin, dshift;
-  dbin.ensure(nblocks * 4);
-  dshift.ensure(nblocks);
-  GX_HIP(hipMemcpyAsync(drow.p, brow.data(), brow.size() * 4, hipMemcpyHostToDevice, s));
-  GX_HIP(hipMemcpyAsync(dbin.p, hbin.data(), nblocks * 4, hipMemcpyHostToDevice, s));
-  GX_HIP(hipMemcpyAsync(dshift.p, hshift.data(), nblocks, hipMemcpyHostToDevice, s));
-  const Bins B{dbin.as<uint32_t>(), dshift.as<uint8_t>(), bshift};
+  uint32_t* drow = reinterpret_cast<uint32_t*>(take(brow.size() * 4));
+  uint32_t* dbin = reinterpret_cast<uint32_t*>(take(nblocks * 4));
+  uint8_t* dshift = reinterpret_cast<uint8_t*>(take(nblocks));
+  GX_HIP(hipMemcpyAsync(drow, brow.data(), brow.size() * 4, hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(dbin, hbin.data(), nblocks * 4, hipMemcpyHostToDevice, s));
+  GX_HIP(hipMemcpyAsync(dshift, hshift.data(), nblocks, hipMemcpyHostToDevice, s));
+  const Bins B{dbin, dshift, bshift};
   // 5. Runs, first as they lie, then cut.
-  DevBuf pos, cut, rkey, rsorted, rg0, boff;
-  pos.ensure((static_cast<size_t>(ng) + 1) * 4);
-  run_flag_kernel<<<grid(ng + int64_t(1)), kB, 0, s>>>(grow.as<uint32_t>(), ng, B, pos.as<uint32_t>());
+  uint32_t* pos = reinterpret_cast<uint32_t*>(wa);  // ng + 1
+  uint32_t* cut = pos + ng + 1;                       // ng + 1
+  uint32_t* rg0 = reinterpret_cast<uint32_t*>(we);
+  run_flag_kernel<<<grid(ng + int64_t(1)), kB, 0, s>>>(grow, ng, B, pos);
   GX_LAUNCHED("bs::run_flag_kernel");
-  exclusive_scan_u32(pos.as<uint32_t>(), pos.as<uint32_t>(), ng + int64_t(1), s);
-  rg0.ensure(static_cast<size_t>(ng) * 4);  // no more runs than groups
-  run_first_kernel<<<grid(ng), kB, 0, s>>>(pos.as<uint32_t>(), ng, rg0.as<uint32_t>());
-  cut.ensure((static_cast<size_t>(ng) + 1) * 4);
-  run_cut_kernel<<<grid(ng + int64_t(1)), kB, 0, s>>>(pos.as<uint32_t>(), rg0.as<uint32_t>(), ng, cut.as<uint32_t>());
+  exclusive_scan_u32(pos, pos, ng + int64_t(1), s);
+  run_first_kernel<<<grid(ng), kB, 0, s>>>(pos, ng, rg0);
+  run_cut_kernel<<<grid(ng + int64_t(1)), kB, 0, s>>>(pos, rg0, ng, cut);
   GX_LAUNCHED("bs::run_cut_kernel");
-  exclusive_scan_u32(cut.as<uint32_t>(), cut.as<uint32_t>(), ng + int64_t(1), s);
+  exclusive_scan_u32(cut, cut, ng + int64_t(1), s);
   uint32_t nr = 0;
-  read_bytes(g, &nr, cut.as<uint32_t>() + ng, 4);
-  rkey.ensure(static_cast<size_t>(nr) * 8);
-  rsorted.ensure(static_cast<size_t>(nr) * 8);
+  read_bytes(g, &nr, cut + ng, 4);
+  uint64_t* rkey = reinterpret_cast<uint64_t*>(wb);
+  uint64_t* rsorted = reinterpret_cast<uint64_t*>(wd);
   L.row16.ensure(static_cast<size_t>(ng) * 2);
   L.runs.ensure(static_cast<size_t>(nr) * sizeof(uint2));
-  boff.ensure((L.nbins + 1) * 4);
-  run_key_kernel<<<grid(ng), kB, 0, s>>>(grow.as<uint32_t>(), ng, B, cut.as<uint32_t>(), drow.as<uint32_t>(),
-                                         rkey.as<uint64_t>(), rg0.as<uint32_t>(), L.row16.as<uint16_t>());
+  uint32_t* boff = reinterpret_cast<uint32_t*>(take((L.nbins + 1) * 4));
+  run_key_kernel<<<grid(ng), kB, 0, s>>>(grow, ng, B, cut, drow, rkey, rg0, L.row16.as<uint16_t>());
   GX_LAUNCHED("bs::run_key_kernel");
-  sort_keys_u64(rkey.as<uint64_t>(), rsorted.as<uint64_t>(), nr, bits_for(L.nbins), s);
-  bounds_kernel<<<grid(L.nbins + 1), kB, 0, s>>>(rsorted.as<uint64_t>(), nr, L.nbins, boff.as<uint32_t>());
-  run_table_kernel<<<grid(nr), kB, 0, s>>>(rsorted.as<uint64_t>(), rg0.as<uint32_t>(), nr, ng, L.runs.as<uint2>());
+  sort_keys_u64(rkey, rsorted, nr, bits_for(L.nbins), s);
+  bounds_kernel<<<grid(L.nbins + 1), kB, 0, s>>>(rsorted, nr, L.nbins, boff);
+  run_table_kernel<<<grid(nr), kB, 0, s>>>(rsorted, rg0, nr, ng, L.runs.as<uint2>());
   GX_LAUNCHED("bs::run_table_kernel");
   std::vector<uint32_t> hoffs(L.nbins + 1);
-  read_bytes(g, hoffs.data(), boff.p, hoffs.size() * 4);
+  read_bytes(g, hoffs.data(), boff, hoffs.size() * 4);
   std::vector<Bin> bins(L.nbins);
   for (int64_t b = 0; b < L.nbins; ++b) bins[b] = Bin{brow[b], brow[b + 1] - brow[b], hoffs[b], hoffs[b + 1]};
   std::stable_sort(bins.begin(), bins.end(), [](const Bin& a, const Bin& b) { return a.run1 - a.run0 > b.run1 - b.run0; });

@@ -27,7 +27,7 @@
 //  - The row sums are the tile sweep of rowsweep.hpp: a wavefront per 512
 //    edges, FP64 sums, coalesced per-row finalisation (x', y' = x'/outdeg,
 //    residual, dangling mass).  Rows spanning chunks of tiles are completed by
-//    a second small launch.  FP64 on 2M edges and more goes through the
+//    a second small launch.  FP64 on 8M edges and more goes through the
 //    blocked sums of blocksum.hpp instead, as deterministic and not bound by
 //    the gathers.
 //  - The residual and dangling mass are accumulated in FP64 per workgroup and
@@ -399,8 +399,11 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   DegreeOrder& D = g->degree_order;
   const bool blocked = use_blocking(g, sizeof(Real));
   const int64_t hot = blocked ? 0 : hot_sources(n, sizeof(Real));
-  // FP64 in one pass: the deterministic sums in blocks where they pay.
-  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && bs::pays(n, g->m);
+  // FP64 in one pass: the deterministic sums in blocks where they pay.  A solve
+  // here is 20 to 40 sweeps, so that the layout has to pay for itself sooner
+  // than in a training loop: 4.1M edges 1.08 -> 0.80 ms a solve, but the first
+  // one 4.1 -> 6.3 ms; 20.6M edges 4.13 -> 2.04 ms, the first 9.4 -> 9.6 ms.
+  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && g->m >= (int64_t(1) << 23) && bs::pays(n, g->m);
   rs::RowPlan P{}, PA{};
   bs::Plan S{};
   if (sums) {
