@@ -222,6 +222,7 @@ __global__ void bc_plain_reset_kernel(const uint32_t* __restrict__ q, unsigned c
 // default kEdgeChunk).
 // Forward levels per captured replay of the batched BC.
 constexpr int kFwdLevels = 8;
+constexpr int kVisitGrid = 512;
 
 struct ChunkTable {
   uint32_t* vtx;     // owning vertex
@@ -388,8 +389,7 @@ __global__ void bcb_seed_kernel(const uint32_t* __restrict__ src, int count, Bat
 
 // Device state of the forward level loop.
 struct FwdState {
-  unsigned long long found;  // new (vertex, source) pairs of the level (forward count)
-  unsigned long long exact;  // the same, counted once per vertex by the visit kernel
+  unsigned long long exact;  // new (vertex, source) pairs of the level, counted by the visit kernel
   unsigned level;            // current level L (masks F[L] -> F[L + 1])
   unsigned done;             // set when a level finds nothing new; deepest = level
 };
@@ -417,7 +417,6 @@ __global__ void bcb_level_begin_kernel(FwdState* S, uint64_t* const* __restrict_
        i += static_cast<int64_t>(gridDim.x) * blockDim.x)
     Fn[i] = 0ull;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    S->found = 0;
     S->exact = 0;
   }
 }
@@ -428,6 +427,29 @@ __global__ void bcb_level_end_kernel(FwdState* S) {
   if (S->exact == 0) S->done = 1;
   else S->level += 1;
 }
+
+// The next kRows neighbours with a useful bit, in lane order: their rows of 64
+// values (256 or 512 contiguous bytes) are loaded together, where a loop over
+// single neighbours waited for each in turn.  Missing ones have an empty mask.
+constexpr int kRows = 4;
+struct Rows {
+  uint64_t mask[kRows];
+  uint32_t vtx[kRows];
+  // act: lanes whose neighbour is still to be taken; f, v: their masks and ids.
+  __device__ __forceinline__ void take(uint64_t& act, uint64_t f, uint32_t v) {
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+      mask[k] = 0;
+      vtx[k] = 0;
+      if (act) {  // wavefront-uniform
+        const int i = __ffsll(static_cast<unsigned long long>(act)) - 1;
+        act &= act - 1;
+        mask[k] = readlane64(f, i);
+        vtx[k] = __builtin_amdgcn_readlane(v, i);
+      }
+    }
+  }
+};
 
 // Forward pull for level L -> L+1 (L from the state).  slab: component label
 // of each lane's source, comp: component label of each vertex (null when
@@ -440,14 +462,12 @@ __global__ void __launch_bounds__(kBlock) bcb_forward_kernel(
   if (S->done) return;
   const uint64_t* __restrict__ FL = F[S->level];
   uint64_t* __restrict__ Fn = F[S->level + 1];
-  unsigned long long* newcount = &S->found;
   const unsigned lane = lane_id();
   const int64_t wave = (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x) / kWave;
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * blockDim.x / kWave;
   __shared__ GroupLds GL;
   load_ranges(R, D.groups, GL);
   const int64_t items = GL.istart[D.groups];
-  unsigned long long found = 0;
   for (int64_t it = wave; it < items; it += nwaves) {
     const int g = item_group(GL, D.groups, it);
     const int64_t c = GL.clo[g] + (it - GL.istart[g]);
@@ -471,12 +491,17 @@ __global__ void __launch_bounds__(kBlock) bcb_forward_kernel(
       }
       uint64_t act = __ballot(f != 0);
       while (act) {
-        const int i = __ffsll(static_cast<unsigned long long>(act)) - 1;
-        act &= act - 1;
-        const uint64_t fi = readlane64(f, i);
-        const uint32_t ui = __builtin_amdgcn_readlane(u, i);
-        acc_mask |= fi;
-        if ((fi >> lane) & 1ull) sig += sigma[(goff + ui) * 64 + lane];
+        Rows R;
+        R.take(act, f, u);
+        float x[kRows];
+#pragma unroll
+        for (int k = 0; k < kRows; ++k)
+          x[k] = ((R.mask[k] >> lane) & 1ull) ? sigma[(goff + R.vtx[k]) * 64 + lane] : 0.f;
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+          acc_mask |= R.mask[k];
+          sig += x[k];
+        }
       }
     }
     if (acc_mask == 0) continue;
@@ -488,14 +513,12 @@ __global__ void __launch_bounds__(kBlock) bcb_forward_kernel(
       if ((acc_mask >> lane) & 1ull) atomicAdd(sv, sig);
       if (lane == 0) atomicOr(reinterpret_cast<unsigned long long*>(&Fn[goff + v]), acc_mask);
     }
-    if (lane == 0) found += __popcll(acc_mask);
   }
-  block_add(found, newcount);
 }
 
-// visited |= new frontier.  Counting of new (vertex, source) pairs is done
-// by the forward kernel; multi-chunk vertices may be counted more than once
-// there, so the exact count is recomputed here.
+// visited |= new frontier, and the count of new (vertex, source) pairs.  Its
+// word takes one atomic per workgroup, 12 ns each one after another, so the
+// launch has few workgroups (kVisitGrid); the forward kernel counts nothing.
 __global__ void __launch_bounds__(kBlock) bcb_visit_kernel(uint64_t* const* __restrict__ F, FwdState* S,
                                                            uint64_t* __restrict__ vis, int64_t total) {
   if (S->done) return;
@@ -513,13 +536,19 @@ __global__ void __launch_bounds__(kBlock) bcb_visit_kernel(uint64_t* const* __re
   block_add(wave_sum(cnt), exact);
 }
 
-// Backward pull for level L (successors at L+1).  Whole-adjacency chunks
-// finalise delta and the per-group bc partial directly; split adjacencies
-// accumulate into delta and are finalised by bcb_multi_finish_kernel.
+// Backward pull for level L (successors at L+1).  What a successor w adds is
+// g(w) = (1 + delta(w)) / sigma(w), the same for each of its predecessors: it
+// is worked out once, when w's own level is finished, and kept in delta's
+// place, so that an edge reads one row of 512 bytes instead of two (512 + 256)
+// and divides nothing.  At the deepest level (`deepest`) delta is 0 and g is 1 /
+// sigma; a vertex without out-edges is never finished and its 0 (g is above 0)
+// says the same.  Whole-adjacency chunks finish their vertex and the per-group
+// bc partial directly; split adjacencies accumulate into delta and are finished
+// by bcb_multi_finish_kernel.
 __global__ void __launch_bounds__(kBlock) bcb_backward_kernel(
     const int32_t* __restrict__ row, const int32_t* __restrict__ col, ChunkTable T, BatchDims D,
     const uint64_t* __restrict__ FL, const uint64_t* __restrict__ FL1, const float* __restrict__ sigma,
-    double* __restrict__ delta, double* __restrict__ bcpart, const GroupRange* __restrict__ R) {
+    double* __restrict__ delta, double* __restrict__ bcpart, const GroupRange* __restrict__ R, bool deepest) {
   const unsigned lane = lane_id();
   const int64_t wave = (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x) / kWave;
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * blockDim.x / kWave;
@@ -546,13 +575,24 @@ __global__ void __launch_bounds__(kBlock) bcb_backward_kernel(
       }
       uint64_t act = __ballot(f != 0);
       while (act) {
-        const int i = __ffsll(static_cast<unsigned long long>(act)) - 1;
-        act &= act - 1;
-        const uint64_t fi = readlane64(f, i);
-        const uint32_t wi = __builtin_amdgcn_readlane(w, i);
-        if ((fi >> lane) & 1ull) {
-          const int64_t idx = (goff + wi) * 64 + lane;
-          acc += (1.0 + delta[idx]) / static_cast<double>(sigma[idx]);
+        Rows S;
+        S.take(act, f, w);
+        double x[kRows];
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+          const int64_t idx = (goff + S.vtx[k]) * 64 + lane;
+          x[k] = 0.0;
+          if ((S.mask[k] >> lane) & 1ull) x[k] = deepest ? static_cast<double>(sigma[idx]) : delta[idx];
+        }
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+          if ((S.mask[k] >> lane) & 1ull) {
+            if (deepest)
+              x[k] = 1.0 / x[k];
+            else if (x[k] == 0.0)
+              x[k] = 1.0 / static_cast<double>(sigma[(goff + S.vtx[k]) * 64 + lane]);
+            acc += x[k];
+          }
         }
       }
     }
@@ -561,8 +601,9 @@ __global__ void __launch_bounds__(kBlock) bcb_backward_kernel(
     if (T.whole[c]) {
       double d = 0.0;
       if (mylane) {
-        d = acc * static_cast<double>(sigma[vidx]);
-        delta[vidx] = d;
+        const double sg = static_cast<double>(sigma[vidx]);
+        d = acc * sg;
+        delta[vidx] = (1.0 + d) / sg;
       }
       d = wave_sum(d);
       if (lane == 0) bcpart[goff + v] += d;
@@ -572,7 +613,8 @@ __global__ void __launch_bounds__(kBlock) bcb_backward_kernel(
   }
 }
 
-// Split adjacencies at level L: delta = sigma * accumulated sum; bc partial.
+// Split adjacencies at level L: delta = sigma * accumulated sum, kept as g; bc
+// partial.
 __global__ void __launch_bounds__(kBlock) bcb_multi_finish_kernel(const uint32_t* __restrict__ multi,
                                                                   int64_t nmulti, BatchDims D,
                                                                   const uint64_t* __restrict__ FL,
@@ -593,8 +635,9 @@ __global__ void __launch_bounds__(kBlock) bcb_multi_finish_kernel(const uint32_t
     double d = 0.0;
     if ((mine >> lane) & 1ull) {
       const int64_t idx = (goff + v) * 64 + lane;
-      d = delta[idx] * static_cast<double>(sigma[idx]);
-      delta[idx] = d;
+      const double sg = static_cast<double>(sigma[idx]);
+      d = delta[idx] * sg;
+      delta[idx] = (1.0 + d) / sg;
     }
     d = wave_sum(d);
     if (lane == 0) bcpart[goff + v] += d;
@@ -958,7 +1001,7 @@ extern "C" gx_status gx_bc_batched(gx_graph* g, const uint32_t* sources, uint32_
             bcb_level_begin_kernel<<<grid_for(gn, kBlock, 8192), kBlock, 0, cs>>>(fst, table, gn);
             bcb_forward_kernel<<<wgrid, kBlock, 0, cs>>>(trow, tcol, tin, D, table, fst, vis, sigma, Rin, comp_lo,
                                                          slab);
-            bcb_visit_kernel<<<grid_for(gn, kBlock, 8192), kBlock, 0, cs>>>(table, fst, vis, gn);
+            bcb_visit_kernel<<<grid_for(gn, kBlock, kVisitGrid), kBlock, 0, cs>>>(table, fst, vis, gn);
             bcb_level_end_kernel<<<1, 64, 0, cs>>>(fst);
           }
           GX_LAUNCHED("bcb forward levels");
@@ -975,33 +1018,22 @@ extern "C" gx_status gx_bc_batched(gx_graph* g, const uint32_t* sources, uint32_
       }
     }
     size_t L = fh.level;
-    // Levels 0..L are non-empty (L = deepest).  Backward sweep L-1 .. 1,
-    // captured once into a HIP graph and replayed.
+    // Levels 0..L are non-empty (L = deepest).  Backward sweep L-1 .. 1, launched
+    // as it is: the level buffers change from call to call, and capturing and
+    // instantiating a graph for one use cost 0.4 ms.
     const size_t deepest = L;
     levels_total += static_cast<uint32_t>(deepest + 1);
     if (deepest >= 2) {
-      hipGraph_t graph;
-      hipGraphExec_t exec;
-      // Capture on the graph's own non-null stream (the null stream cannot be
-      // captured); the forward work on `s` has completed (synchronised above).
-      hipStream_t cs = g->capture();
-      GX_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
       for (int64_t lv = static_cast<int64_t>(deepest) - 1; lv >= 1; --lv) {
         const uint64_t* FL = cache.levels[lv].as<uint64_t>();
         const uint64_t* FL1 = cache.levels[lv + 1].as<uint64_t>();
-        bcb_backward_kernel<<<wgrid, kBlock, 0, cs>>>(g->row, g->col, tout, D, FL, FL1, sigma, delta, bcpart,
-                                                       Rout);
+        bcb_backward_kernel<<<wgrid, kBlock, 0, s>>>(g->row, g->col, tout, D, FL, FL1, sigma, delta, bcpart, Rout,
+                                                     lv + 1 == static_cast<int64_t>(deepest));
         if (tout.nmulti > 0)
-          bcb_multi_finish_kernel<<<grid_for(tout.nmulti * D.groups * 64, kBlock, 8192), kBlock, 0, cs>>>(
+          bcb_multi_finish_kernel<<<grid_for(tout.nmulti * D.groups * 64, kBlock, 8192), kBlock, 0, s>>>(
               tout.multi, tout.nmulti, D, FL, sigma, delta, bcpart, Rout);
       }
-      hipError_t cap_err = hipStreamEndCapture(cs, &graph);
-      GX_HIP(cap_err);
-      GX_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-      GX_HIP(hipGraphLaunch(exec, s));
-      GX_HIP(hipStreamSynchronize(s));
-      (void)hipGraphExecDestroy(exec);
-      (void)hipGraphDestroy(graph);
+      GX_LAUNCHED("bcb_backward_kernel");
       launches += static_cast<uint32_t>((deepest - 1) * (tout.nmulti > 0 ? 2 : 1));
     }
     ktimer.end();

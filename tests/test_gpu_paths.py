@@ -183,3 +183,17 @@ def test_frontier_shapes(gx, oracle, n, degrees):
         exp = oracle.kcore(row, col, k)
         assert np.array_equal(u32(deg), exp) and count == int((exp >= k).sum())
         assert np.array_equal(alive.cpu().numpy(), (exp >= k).astype(np.uint8))
+
+
+@pytest.mark.parametrize("n,m,hubs,sources", [(3000, 4000, 0, 3), (3000, 30000, 2, 64), (20011, 60000, 1, 65)])
+def test_bc_batched_leaves_and_split_rows(gx, oracle, n, m, hubs, sources):
+    """Directed graphs with vertices without out-edges at every level (they are
+    never finished by a backward level) and rows over several chunks.  FP64
+    sums of at most n positive terms: 1e-10 relative."""
+    row, col, _ = weighted_csr(n, m, n + m, hubs)
+    srcs = np.random.default_rng(2).integers(0, n, sources).astype(np.uint32)
+    print(f"bc n={n} m={len(col)} sources={sources}", flush=True)
+    G = gx.Graph.from_csr(row, col)
+    exp = oracle.bc(row, col, srcs)
+    got = gx.betweenness_centrality_batched(G, srcs)[0].cpu().numpy()
+    assert np.abs(got - exp).max() <= 1e-10 * max(1.0, np.abs(exp).max())
