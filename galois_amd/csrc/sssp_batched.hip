@@ -14,14 +14,25 @@
 //    vertex improved and has not been pushed along its out-edges yet),
 //    double-buffered between rounds.
 //  - A round is a sweep over the out-edge chunks of the CSR (at most
-//    kEdgeChunk edges each; a hub's chunks go to many wavefronts): a
-//    wavefront reads its vertex's pending mask, skips it when empty, and
-//    pushes the pending lanes whose distance lies below the phase's limit
-//    along the chunk's edges, eight edges in flight: per edge the 64 lanes
-//    load the target's distances (one coalesced row), lower them with
-//    atomicMin and set the improved lanes in the target's next pending mask
-//    (one 64-bit atomicOr per edge).  Lanes at or above the limit stay
-//    pending (carried by the vertex's first chunk).
+//    kEdgeChunk edges each): a wavefront reads its chunks' pending masks, 64 at
+//    a time, skips the empty ones, and pushes the pending lanes whose distance
+//    lies below the phase's limit along the chunk's edges, eight edges in
+//    flight: per edge the 64 lanes load the target's distances (one coalesced
+//    row), lower them with atomicMin and set the improved lanes in the target's
+//    next pending mask (one 64-bit atomicOr per edge).  Lanes at or above the
+//    limit stay pending (carried by the vertex's first chunk).
+//  - A wavefront's chunks lie a whole grid apart, so that a hub's chunks, which
+//    are neighbours, spread over the chip (64 adjacent chunks a wavefront left
+//    most of the chip waiting for the hubs' wavefronts: 70 ms against 25 for 64
+//    sources of an RMAT graph of 2^20 vertices).
+//  - No atomic returns a value.  A lane counts as improved when it beats the
+//    distance that was read before; where another wavefront lowers the distance
+//    further in between, that one has set the same pending bit, with a smaller
+//    distance, so masks, limits and stop are those of the exact answer.
+//  - The next chunk's distances and first 64 edges are loaded while the current
+//    one is pushed, and every workgroup leaves its counts in a record of its
+//    own.  Both together with the above: 25 -> 9.2 ms; the largest round
+//    (1.5 ms) then misses L2 at 4.5 TB/s, the rate of a large copy.
 //  - Phases share one bucket range across the 64 sources: the limit is
 //    (first bucket + width) << shift; a phase ends when no pushed lane lands
 //    below it, the next one starts at the smallest pending bucket.  Width is
@@ -40,7 +51,9 @@ using namespace gx;
 
 namespace {
 
-constexpr int kBlock = 256;
+constexpr int kBlock = 1024;  // two workgroups a CU: every wavefront is resident
+constexpr int kGrid = 512;    // records the step reads, one a thread
+constexpr int kTileBlock = 256;
 constexpr uint32_t kInf = GX_DIST_INFINITY;
 constexpr int kRounds = 8;
 constexpr int kUnroll = 8;
@@ -48,10 +61,8 @@ constexpr unsigned long long kMergeLow = 1ull << 14;
 constexpr unsigned long long kMergeHigh = 1ull << 17;
 
 struct BState {
-  unsigned long long near;     // lanes pushed below the limit this round
   unsigned long long pushed;   // (vertex, lane) pushes admitted in the current phase
   unsigned long long edges;    // edge visits (per lane pushed)
-  unsigned far_min;            // smallest pending bucket at or above the limit
   unsigned bucket;             // first bucket of the phase
   unsigned width, max_width;   // buckets of the phase; most allowed
   unsigned adapt;              // width adapts to the pushes of a phase
@@ -60,6 +71,19 @@ struct BState {
   unsigned done;
   unsigned rounds;
   unsigned phases;
+};
+
+// What a workgroup saw in a round.
+struct BTally {
+  unsigned long long pushed;  // (vertex, lane) pushes admitted
+  unsigned long long edges;   // edge visits (per lane pushed)
+  unsigned far_min;           // smallest pending bucket at or above the limit
+  unsigned near;              // a lane landed below the limit
+};
+
+struct BRound {
+  BState state;
+  BTally tally[kGrid];
 };
 
 struct BBufs {
@@ -74,6 +98,7 @@ struct BBufs {
   uint32_t* dist;         // [group][vertex][64]
   uint64_t* pend[2];      // [group][vertex]
   BState* S;
+  BTally* tally;          // [kGrid]
   uint32_t shift;
 };
 
@@ -105,10 +130,8 @@ __global__ void sb_seed_kernel(const uint32_t* __restrict__ src, int count, int6
                                unsigned shift) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
-    S->near = 0;
     S->pushed = 0;
     S->edges = 0;
-    S->far_min = 0xffffffffu;
     S->bucket = 0;
     S->width = width ? width : 1;
     S->max_width = max_width;
@@ -139,133 +162,177 @@ __global__ void sb_clear_kernel(BBufs B) {
 
 // One round over every (group, chunk).
 __global__ void __launch_bounds__(kBlock) sb_relax_kernel(BBufs B) {
-  BState* S = B.S;
+  const BState* S = B.S;
   if (S->done) return;
   const unsigned lane = lane_id();
   const int64_t wave = (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x) / kWave;
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * blockDim.x / kWave;
   const unsigned sel = S->sel, limit = S->limit, shift = B.shift;
   const uint64_t* __restrict__ cur = B.pend[sel];
-  uint64_t* __restrict__ nxt = B.pend[sel ^ 1];
+  unsigned long long* __restrict__ nxt = reinterpret_cast<unsigned long long*>(B.pend[sel ^ 1]);
   uint32_t* __restrict__ dist = B.dist;
   unsigned far_min = 0xffffffffu;
-  unsigned long long near = 0, pushed = 0, edges = 0;
+  unsigned near = 0;
+  unsigned long long pushed = 0, edges = 0;
   const int64_t items = B.nchunks * B.groups;
-  // 64 items per wavefront pass: every lane reads one item's pending mask,
-  // then the wavefront works through the items that have one.
-  for (int64_t base = wave * kWave; base < items; base += nwaves * kWave) {
-    const int64_t my = base + lane;
-    uint32_t mu = 0;
+  for (int64_t base = wave; base < items; base += nwaves * kWave) {
+    const int64_t my = base + lane * nwaves;
     uint64_t mp = 0;
-    int64_t mg = 0, mc = 0;
+    uint32_t mrow = 0, mrow_hi = 0, mg = 0;  // group * n + vertex, group
+    int32_t mb = 0, me = 0;
+    unsigned mfirst = 0;
     if (my < items) {
-      mg = my / B.nchunks;
-      mc = my - mg * B.nchunks;
-      mu = B.cvtx[mc];
-      mp = cur[mg * B.n + mu];
+      mg = static_cast<uint32_t>(my / B.nchunks);
+      const int64_t mc = my - mg * B.nchunks;
+      const uint32_t mu = B.cvtx[mc];
+      const int64_t r = mg * B.n + mu;
+      mp = cur[r];
+      mrow = static_cast<uint32_t>(r);
+      mrow_hi = static_cast<uint32_t>(r >> 32);
+      if (mp) {
+        mb = B.cbegin[mc];
+        me = min(mb + kEdgeChunk, B.row[mu + 1]);
+        mfirst = mb == B.row[mu];
+      }
     }
     uint64_t live = __ballot(mp != 0);
-    while (live) {
-      const int i = __ffsll(static_cast<unsigned long long>(live)) - 1;
+    // The next item's distances and its first 64 edges are loaded while the
+    // current one is pushed.
+    uint32_t du1 = 0, col1 = 0, w1 = 0;
+    int i1 = 0;
+    auto stage = [&]() {
+      i1 = __ffsll(static_cast<unsigned long long>(live)) - 1;
       live &= live - 1;
-      const uint32_t u = __builtin_amdgcn_readlane(mu, i);
+      const int64_t r = (static_cast<int64_t>(__builtin_amdgcn_readlane(mrow_hi, i1)) << 32) |
+                        static_cast<uint32_t>(__builtin_amdgcn_readlane(mrow, i1));
+      const int32_t e = __builtin_amdgcn_readlane(mb, i1) + static_cast<int32_t>(lane);
+      du1 = dist[r * 64 + lane];
+      if (e < static_cast<int32_t>(__builtin_amdgcn_readlane(me, i1))) {
+        col1 = static_cast<uint32_t>(B.col[e]);
+        w1 = B.w[e];
+      }
+    };
+    bool more = live != 0;
+    if (more) stage();
+    while (more) {
+      const int i = i1;
+      const uint32_t du = du1;
+      uint32_t cv = col1, cw = w1;
+      more = live != 0;
+      if (more) stage();
       const uint64_t pend = readlane64(mp, i);
-      // chunk index < 2^32 (m < 2^31 edges), group < 64
-      const int64_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(mc), i));
-      const int64_t g = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(mg), i));
-      const int64_t goff = g * B.n;
-      const int32_t eb = B.cbegin[c];
-      const int32_t ee = min(eb + kEdgeChunk, B.row[u + 1]);
-      const uint32_t du = dist[(goff + u) * 64 + lane];
-      const bool mine = (pend >> lane) & 1ull;
-      const uint64_t act = __ballot(mine && du < limit);
-      if (eb == B.row[u]) {  // the vertex's first chunk carries the lanes left pending
+      const int32_t eb = __builtin_amdgcn_readlane(mb, i), ee = __builtin_amdgcn_readlane(me, i);
+      const int64_t goff = static_cast<uint32_t>(__builtin_amdgcn_readlane(mg, i)) * B.n;
+      const uint64_t act = __ballot(((pend >> lane) & 1ull) && du < limit);
+      const bool on = (act >> lane) & 1ull;
+      if (__builtin_amdgcn_readlane(mfirst, i)) {  // the vertex's first chunk carries the lanes left pending
         const uint64_t keep = pend & ~act;
         if (keep) {
-          if (lane == 0) atomicOr(reinterpret_cast<unsigned long long*>(&nxt[goff + u]), keep);
+          const int64_t r = (static_cast<int64_t>(__builtin_amdgcn_readlane(mrow_hi, i)) << 32) |
+                            static_cast<uint32_t>(__builtin_amdgcn_readlane(mrow, i));
+          if (lane == 0) atomicOr(&nxt[r], keep);
           if ((keep >> lane) & 1ull) far_min = min(far_min, du >> shift);
         }
-        pushed += (act >> lane) & 1ull;
+        pushed += on;
       }
       if (act == 0) continue;
-      const bool on = (act >> lane) & 1ull;
-      for (int32_t e0 = eb; e0 < ee; e0 += kUnroll) {
-        uint32_t v[kUnroll], wt[kUnroll], dv[kUnroll];
-#pragma unroll
-        for (int k = 0; k < kUnroll; ++k) {
-          const int32_t e = e0 + k;
-          v[k] = e < ee ? static_cast<uint32_t>(B.col[e]) : 0u;
-          wt[k] = e < ee ? B.w[e] : 0u;
+      if (on) edges += static_cast<unsigned>(ee - eb);
+      for (int32_t e0 = eb; e0 < ee; e0 += kWave) {
+        if (e0 != eb) {
+          const int32_t e = e0 + static_cast<int32_t>(lane);
+          if (e < ee) {
+            cv = static_cast<uint32_t>(B.col[e]);
+            cw = B.w[e];
+          }
         }
+        const int left = min(static_cast<int>(kWave), ee - e0);
+        for (int k0 = 0; k0 < left; k0 += kUnroll) {
+          uint32_t v[kUnroll], dv[kUnroll];
 #pragma unroll
-        for (int k = 0; k < kUnroll; ++k)
-          dv[k] = (on && e0 + k < ee) ? dist[(goff + v[k]) * 64 + lane] : 0u;
+          for (int k = 0; k < kUnroll; ++k) {
+            v[k] = __builtin_amdgcn_readlane(cv, k0 + k);
+            dv[k] = 0u;
+            if (on && k0 + k < left) dv[k] = dist[(goff + v[k]) * 64 + lane];
+          }
 #pragma unroll
-        for (int k = 0; k < kUnroll; ++k) {
-          if (e0 + k < ee) {  // wavefront-uniform
-            const uint32_t nd = du + wt[k];
-            bool imp = false;
-            if (on && nd < dv[k]) imp = nd < atomicMin(&dist[(goff + v[k]) * 64 + lane], nd);
+          for (int k = 0; k < kUnroll; ++k) {
+            const uint32_t nd = du + static_cast<uint32_t>(__builtin_amdgcn_readlane(cw, k0 + k));
+            const bool imp = nd < dv[k];
             const uint64_t im = __ballot(imp);
             if (im) {
-              if (lane == 0) atomicOr(reinterpret_cast<unsigned long long*>(&nxt[goff + v[k]]), im);
               if (imp) {
-                if (nd < limit) near += 1;
+                atomicMin(&dist[(goff + v[k]) * 64 + lane], nd);
+                if (nd < limit) near = 1;
                 else far_min = min(far_min, nd >> shift);
               }
+              if (lane == 0) atomicOr(&nxt[goff + v[k]], im);
             }
           }
         }
-        edges += on ? static_cast<unsigned long long>(min(kUnroll, ee - e0)) : 0ull;
       }
     }
   }
-  // Reduced over the workgroup first: one atomic per state word per
-  // workgroup rather than per wavefront.
+  // One record per workgroup, read by the step: same-address atomics of all
+  // workgroups would take longer than a small round.
   constexpr int kW = kBlock / kWave;
-  __shared__ unsigned s_min[kW];
-  __shared__ unsigned long long s_sum[3][kW];
+  __shared__ unsigned s_min[kW], s_near[kW];
+  __shared__ unsigned long long s_sum[2][kW];
   far_min = wave_min(far_min);
-  near = wave_sum(near);
   pushed = wave_sum(pushed);
   edges = wave_sum(edges);
+  const uint64_t any = __ballot(near != 0);
   const unsigned w = threadIdx.x / kWave;
   if (lane == 0) {
     s_min[w] = far_min;
-    s_sum[0][w] = near;
-    s_sum[1][w] = pushed;
-    s_sum[2][w] = edges;
+    s_near[w] = any != 0;
+    s_sum[0][w] = pushed;
+    s_sum[1][w] = edges;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned fm = 0xffffffffu;
-    unsigned long long nr = 0, pu = 0, ed = 0;
+    BTally t{0, 0, 0xffffffffu, 0};
     for (int i = 0; i < kW; ++i) {
-      fm = min(fm, s_min[i]);
-      nr += s_sum[0][i];
-      pu += s_sum[1][i];
-      ed += s_sum[2][i];
+      t.far_min = min(t.far_min, s_min[i]);
+      t.near |= s_near[i];
+      t.pushed += s_sum[0][i];
+      t.edges += s_sum[1][i];
     }
-    if (fm != 0xffffffffu) atomicMin(&S->far_min, fm);
-    if (nr) atomicAdd(&S->near, nr);
-    if (pu) atomicAdd(&S->pushed, pu);
-    if (ed) atomicAdd(&S->edges, ed);
+    B.tally[blockIdx.x] = t;
   }
 }
 
 // End of a round: swap the pending masks; stay in the phase while lanes were
 // pushed below the limit, else start the next phase at the smallest pending
 // bucket (adapting the width to the pushes of the phase), or stop.
-__global__ void sb_step_kernel(BState* S, unsigned shift) {
-  if (threadIdx.x != 0 || S->done) return;
+__global__ void __launch_bounds__(kGrid) sb_step_kernel(BState* S, const BTally* __restrict__ tally, unsigned shift) {
+  if (S->done) return;
+  constexpr int kW = kGrid / kWave;
+  __shared__ unsigned s_min[kW], s_near[kW];
+  __shared__ unsigned long long s_sum[2][kW];
+  const BTally t = tally[threadIdx.x];
+  const unsigned fm = wave_min(t.far_min);
+  const unsigned long long pu = wave_sum(t.pushed), ed = wave_sum(t.edges);
+  const uint64_t any = __ballot(t.near != 0);
+  if (lane_id() == 0) {
+    const unsigned w = threadIdx.x / kWave;
+    s_min[w] = fm;
+    s_near[w] = any != 0;
+    s_sum[0][w] = pu;
+    s_sum[1][w] = ed;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  unsigned far_min = 0xffffffffu, near = 0;
+  for (int i = 0; i < kW; ++i) {
+    far_min = min(far_min, s_min[i]);
+    near |= s_near[i];
+    S->pushed += s_sum[0][i];
+    S->edges += s_sum[1][i];
+  }
   S->rounds += 1;
   S->sel ^= 1;
-  if (S->near > 0) {
-    S->near = 0;
-    S->far_min = 0xffffffffu;
-    return;
-  }
-  if (S->far_min == 0xffffffffu) {
+  if (near) return;
+  if (far_min == 0xffffffffu) {
     S->done = 1;
     return;
   }
@@ -274,26 +341,25 @@ __global__ void sb_step_kernel(BState* S, unsigned shift) {
     else if (S->pushed > kMergeHigh && S->width > 1) S->width >>= 1;
   }
   S->pushed = 0;
-  S->bucket = S->far_min;
+  S->bucket = far_min;
   S->limit = sat_limit(S->bucket, S->width, shift);
-  S->far_min = 0xffffffffu;
   S->phases += 1;
 }
 
 // dist[g][v][lane] -> out[(g * 64 + lane) * n + v] for live lanes, through an
 // LDS tile of 64 vertices x 64 lanes.
-__global__ void __launch_bounds__(kBlock) sb_out_kernel(const uint32_t* __restrict__ dist, int64_t n, int groups,
+__global__ void __launch_bounds__(kTileBlock) sb_out_kernel(const uint32_t* __restrict__ dist, int64_t n, int groups,
                                                         int count, uint32_t* __restrict__ out) {
   __shared__ uint32_t tile[64][65];
   const int64_t tiles = (n + 63) / 64;
   for (int64_t t = blockIdx.x; t < tiles * groups; t += gridDim.x) {
     const int64_t g = t / tiles, v0 = (t - g * tiles) * 64;
-    for (int k = threadIdx.x; k < 64 * 64; k += kBlock) {
+    for (int k = threadIdx.x; k < 64 * 64; k += kTileBlock) {
       const int i = k / 64, j = k % 64;  // vertex v0 + i, lane j
       tile[i][j] = v0 + i < n ? dist[((g * n) + v0 + i) * 64 + j] : kInf;
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < 64 * 64; k += kBlock) {
+    for (int k = threadIdx.x; k < 64 * 64; k += kTileBlock) {
       const int j = k / 64, i = k % 64;  // lane j, vertex v0 + i
       const int64_t srci = g * 64 + j;
       if (srci < count && v0 + i < n) out[srci * n + v0 + i] = tile[i][j];
@@ -330,9 +396,9 @@ extern "C" gx_status gx_sssp_batched(gx_graph* g, const uint32_t* sources, uint3
     const unsigned width = static_cast<unsigned>(tune_effective("sssp.batch_width", n, g->m));
     uint32_t* dsrc = g->scratch<uint32_t>(WS_Q3, count);
     GX_HIP(hipMemcpyAsync(dsrc, sources, count * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    BState* S = g->scratch<BState>(WS_COUNTERS, 1);
+    BRound* R = g->scratch<BRound>(WS_COUNTERS, 1);
+    BState* S = &R->state;
     BState* host = static_cast<BState*>(g->host_pinned(sizeof(BState)));
-    const unsigned wgrid = 256 * 16;
     for (uint32_t first = 0; first < count; first += 64u * max_groups) {
       const uint32_t cnt = std::min<uint32_t>(count - first, 64u * max_groups);
       BBufs B;
@@ -349,6 +415,7 @@ extern "C" gx_status gx_sssp_batched(gx_graph* g, const uint32_t* sources, uint3
       B.pend[0] = g->scratch<uint64_t>(WS_BC_MASK0, gn);
       B.pend[1] = g->scratch<uint64_t>(WS_BC_MASK1, gn);
       B.S = S;
+      B.tally = R->tally;
       B.shift = shift;
       sb_init_kernel<<<grid_for(gn * 64, kBlock, 16384), kBlock, 0, s>>>(B.dist, B.pend[0], B.pend[1], gn);
       GX_LAUNCHED("sb_init_kernel");
@@ -367,8 +434,8 @@ extern "C" gx_status gx_sssp_batched(gx_graph* g, const uint32_t* sources, uint3
         g->replay(g->sssp_batched_batch, key, [&](hipStream_t cs) {
           for (int r = 0; r < kRounds; ++r) {
             sb_clear_kernel<<<grid_for(gn, kBlock, 8192), kBlock, 0, cs>>>(B);
-            sb_relax_kernel<<<wgrid, kBlock, 0, cs>>>(B);
-            sb_step_kernel<<<1, 64, 0, cs>>>(S, shift);
+            sb_relax_kernel<<<kGrid, kBlock, 0, cs>>>(B);
+            sb_step_kernel<<<1, kGrid, 0, cs>>>(S, R->tally, shift);
           }
           GX_LAUNCHED("sssp batched rounds");
         });
@@ -380,7 +447,7 @@ extern "C" gx_status gx_sssp_batched(gx_graph* g, const uint32_t* sources, uint3
       ktimer.end();
       rounds += host->rounds;
       edges += host->edges;
-      sb_out_kernel<<<grid_for(((n + 63) / 64) * B.groups, 1, 8192), kBlock, 0, s>>>(
+      sb_out_kernel<<<grid_for(((n + 63) / 64) * B.groups, 1, 8192), kTileBlock, 0, s>>>(
           B.dist, n, B.groups, static_cast<int>(cnt), dist + static_cast<int64_t>(first) * n);
       GX_LAUNCHED("sb_out_kernel");
       ++launches;

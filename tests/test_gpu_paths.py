@@ -197,3 +197,24 @@ def test_bc_batched_leaves_and_split_rows(gx, oracle, n, m, hubs, sources):
     exp = oracle.bc(row, col, srcs)
     got = gx.betweenness_centrality_batched(G, srcs)[0].cpu().numpy()
     assert np.abs(got - exp).max() <= 1e-10 * max(1.0, np.abs(exp).max())
+
+
+@pytest.mark.parametrize("n,degrees,sources", [(2, [], 1), (130, [127, 128], 63), (3000, [255, 256, 257, 2900], 65),
+                                               (70000, [63, 64, 65, 20000, 60000], 3)])
+def test_sssp_batched_chunks(gx, oracle, n, degrees, sources):
+    """Rows around the chunk and the 64-edge block sizes, hubs over many
+    chunks, groups with few and with all lanes, limits that leave lanes
+    pending: every source's row equals the oracle's."""
+    row, col, w = star_csr(degrees, n, n)
+    G = gx.Graph.from_csr(row, col, w, symmetric=True)
+    srcs = np.random.default_rng(n).integers(0, n, sources).astype(np.uint32)
+    exp = {int(s): oracle.sssp(row, col, w, int(s), 4) for s in set(srcs.tolist())}
+    for shift, width in ((4, 0), (0, 1), (31, 64)):
+        print(f"sssp batched n={n} m={len(col)} sources={sources} shift={shift} width={width}", flush=True)
+        gx.tune_set("sssp.batch_width", width)
+        try:
+            got = u32(gx.sssp_batched(G, srcs, shift)[0])
+        finally:
+            gx.tune_set("sssp.batch_width", -1)
+        for i, s in enumerate(srcs):
+            assert np.array_equal(got[i], exp[int(s)]), (i, shift)
