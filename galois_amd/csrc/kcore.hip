@@ -15,11 +15,12 @@
 // workgroup expansion of frontier.hpp (hubs spread over the grid); each
 // decrement is one atomicSub on the degree word, and the `old == k` winner
 // appends the neighbour to the next frontier through the wavefront's LDS
-// queue.  Random atomics run at 27 G/s on this GPU, which is what the first
-// round's decrements take; the passes over all vertices count per workgroup
-// (init 53 -> 17 us, membership 171 -> 12 us on RMAT-22; the call 908 -> 722
-// us).  On the degree-ordered copy the decrements of the hub ids are
-// counted in LDS first (kHot below).
+// queue.  The first round's decrements take most of the call: random atomics
+// run at 27 G/s on this GPU, those that meet on a line or a word much slower,
+// so that the words are permuted and the hottest counted in LDS (kPage, kHotCap
+// below: RMAT-22 at k = 10, peel 473 -> 233 us).  The passes over all vertices
+// count per workgroup (init 53 -> 28 us, membership 171 -> 20 us).  The call:
+// 899 -> 410 us.
 #include <algorithm>
 
 #include "frontier.hpp"
@@ -43,8 +44,8 @@ struct KcoreCounters {
   unsigned long long items;
   unsigned long long alive;
   unsigned long long edges;
+  unsigned hot_count;
 };
-
 __global__ void kcore_reset_kernel(KcoreCounters* c) {
   if (threadIdx.x == 0) {
     c->count[0] = c->count[1] = 0;
@@ -57,21 +58,55 @@ __global__ void kcore_reset_kernel(KcoreCounters* c) {
     c->items = 0;
     c->alive = 0;
     c->edges = 0;
+    c->hot_count = 0;
   }
 }
 
 constexpr int kQCap = 4096;  // kcore_init_kernel
 constexpr int kHubLanes = 256;  // lanes per step of the hub pass
-// On the degree-ordered copy the hubs are the smallest ids (and on graphs
-// whose generator gives small ids the high degrees, such as RMAT without a
-// relabelling, too), and in the first round (every vertex below k dies at
-// once) most decrements land on them: a hub's degree word then takes
-// millions of returning atomics one after another.  Decrements of ids below
-// kHot are counted per workgroup in LDS instead and applied with one
-// atomicSub per counter at the end of the launch; the atomic that takes a
-// word from k or above to below k finds the death, so every vertex still
-// dies exactly once.
-constexpr uint32_t kHot = 4096;
+// In the first round (every vertex below k dies at once) many decrements land
+// on the few vertices of highest degree, and atomics on one word take 12 ns
+// each, one after another; on RMAT graphs the hubs' ids are powers of two
+// apart, so that their words queue up on the same memory channels.  The init
+// pass therefore lists up to kHotCap vertices with at least 1/8192 of the
+// adjacency entries (and kHotDegree), and every workgroup counts their
+// decrements in an LDS table and applies each counter with one atomicSub at
+// the end of the launch; the atomic that takes a word from k or above to below
+// k finds the death, so every vertex still dies exactly once.  Frontiers of
+// fewer than kHotMin vertices do without: no word can take more decrements
+// than that (25 us), and the table costs a few.
+constexpr uint32_t kHotCap = 512;
+constexpr uint32_t kHotDegree = 256;
+constexpr uint32_t kHotMin = 2048;
+constexpr int kHotBits = 11;  // table slots: at most a quarter in use
+constexpr int kHotProbe = 4;  // a vertex that finds no slot among these is not counted
+constexpr uint32_t kNoVertex = 0xffffffffu;
+
+struct HotTable {
+  uint32_t id[1 << kHotBits];
+  uint32_t count[1 << kHotBits];
+};
+__device__ __forceinline__ uint32_t hot_slot(uint32_t v, int probe) {
+  return (((v * 2654435769u) >> (32 - kHotBits)) + probe) & ((1u << kHotBits) - 1);
+}
+
+struct KcoreState {
+  KcoreCounters c;
+  uint32_t hot[kHotCap];
+};
+
+// Atomics on one cache line queue up as those on one word do.  Neighbouring ids
+// are often alike (ids of RMAT graphs with few set bits are hubs, a relabelled
+// graph has its hubs at the front), so with hubs the degree words are
+// permuted within pages of kPage words: 4.4 M decrements of an RMAT
+// distribution over 2^22 words take 499 us in id order, 225 us permuted
+// (uniform ones 168 us).  Pages keep the passes over all vertices sequential.
+// A graph without hubs keeps its order (and the lines its neighbours share).
+constexpr uint32_t kPage = 4096;
+constexpr uint32_t kPageMul = 1597;  // odd: a permutation of the page
+__device__ __forceinline__ uint32_t degree_pos(uint32_t v, uint32_t mul) {
+  return (v & ~(kPage - 1)) | ((v * mul) & (kPage - 1));
+}
 constexpr int kRoundsPerGraph = 4;
 constexpr int kRoundsFirst = 2;  // first replay: many graphs need one round (plus the empty one)
 
@@ -81,21 +116,27 @@ constexpr int kRoundsFirst = 2;  // first replay: many graphs need one round (pl
 // of it (on RMAT graphs they are a large share of the vertices).
 __global__ void __launch_bounds__(kWideBlock) kcore_init_kernel(const int32_t* __restrict__ row,
                                                             uint32_t* __restrict__ degree, int64_t n, uint32_t k,
-                                                            uint32_t* __restrict__ q, KcoreCounters* c,
-                                                            unsigned cap) {
+                                                            uint32_t* __restrict__ q, KcoreState* st,
+                                                            unsigned cap, uint32_t hot_min, uint32_t mul) {
+  KcoreCounters* c = &st->c;
   __shared__ LdsQueue<kQCap> sq;
   lq_init(sq);
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t b = blockIdx.x * static_cast<int64_t>(blockDim.x); b < n; b += stride) {
-    const int64_t v = b + threadIdx.x;
-    bool dead = false;
-    if (v < n) {
-      const uint32_t d = static_cast<uint32_t>(row[v + 1] - row[v]);
-      degree[v] = d;
-      dead = d < k && d > 0;
+  for (int64_t p = blockIdx.x * static_cast<int64_t>(kPage); p < n; p += gridDim.x * static_cast<int64_t>(kPage)) {
+    for (uint32_t i = threadIdx.x; i < kPage; i += kWideBlock) {
+      const int64_t v = p + i;
+      bool dead = false;
+      if (v < n) {
+        const uint32_t d = static_cast<uint32_t>(row[v + 1] - row[v]);
+        degree[degree_pos(static_cast<uint32_t>(v), mul)] = d;
+        dead = d < k && d > 0;
+        if (d >= hot_min && __hip_atomic_load(&c->hot_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kHotCap) {
+          const unsigned at = atomicAdd(&c->hot_count, 1u);
+          if (at < kHotCap) st->hot[at] = static_cast<uint32_t>(v);
+        }
+      }
+      lq_push(sq, dead, static_cast<uint32_t>(v));
+      lq_flush(sq, q, &c->count[0], cap, &c->overflow, false);
     }
-    lq_push(sq, dead, static_cast<uint32_t>(v));
-    lq_flush(sq, q, &c->count[0], cap, &c->overflow, false);
   }
   lq_flush(sq, q, &c->count[0], cap, &c->overflow, true);
 }
@@ -112,8 +153,22 @@ struct PeelOp {
   unsigned out;
   unsigned cap;
   uint32_t hub;   // frontier.hub_degree
-  uint32_t* hot;  // LDS counters of the ids below nhot (nhot = 0: none)
-  uint32_t nhot;
+  uint32_t mul;   // degree_pos
+  HotTable* hot;  // nullptr: every decrement goes to the degree word
+  // Whether v has a counter, which then takes its decrement.
+  __device__ __forceinline__ bool count_hot(uint32_t v) {
+    if (!hot) return false;
+    for (int p = 0; p < kHotProbe; ++p) {
+      const uint32_t slot = hot_slot(v, p);
+      const uint32_t id = hot->id[slot];
+      if (id == v) {
+        atomicAdd(&hot->count[slot], 1u);
+        return true;
+      }
+      if (id == kNoVertex) return false;
+    }
+    return false;
+  }
   template <int U>
   __device__ __forceinline__ void run(const bool (&valid)[U], const uint32_t (&)[U], const int32_t (&e)[U]) {
     bool dies[U];
@@ -124,10 +179,7 @@ struct PeelOp {
     for (int k = 0; k < U; ++k) {
       dies[k] = false;
       if (valid[k]) {
-        if (v[k] < nhot)
-          atomicAdd(&hot[v[k]], 1u);
-        else
-          dies[k] = atomicSub(&degree[v[k]], 1u) == this->k;
+        if (!count_hot(v[k])) dies[k] = atomicSub(&degree[degree_pos(v[k], mul)], 1u) == this->k;
       }
     }
     wq.push(dies, v);
@@ -158,33 +210,49 @@ struct KcoreBufs {
   uint32_t* hubq;
   uint32_t* hub_off;
   KcoreCounters* c;
+  const uint32_t* hot;  // listed vertices (hot_count of them)
   uint32_t k;
   unsigned cap;
   uint32_t hub;
+  uint32_t mul;
 };
 
-__device__ __forceinline__ PeelOp make_peel(const KcoreBufs& B, uint32_t (&stage)[kWideWaves][kWaveQCap], uint32_t* hot,
-                                            uint32_t nhot) {
+__device__ __forceinline__ PeelOp make_peel(const KcoreBufs& B, uint32_t (&stage)[kWideWaves][kWaveQCap],
+                                            HotTable* hot) {
   const unsigned out = B.c->in ^ 1u;
-  return PeelOp{B.col, B.degree, out ? B.q1 : B.q0, B.c, {stage[threadIdx.x / kWave]}, B.k, out, B.cap, B.hub, hot, nhot};
+  return PeelOp{B.col, B.degree, out ? B.q1 : B.q0, B.c, {stage[threadIdx.x / kWave]}, B.k, out, B.cap, B.hub,
+                B.mul, hot};
 }
 
-// Workgroup-uniform.  Clears the LDS counters of the hot ids.
-__device__ __forceinline__ void hot_clear(uint32_t* hot) {
-  for (uint32_t i = threadIdx.x; i < kHot; i += kWideBlock) hot[i] = 0;
+// Workgroup-uniform.  The table of the listed vertices, or nullptr when there
+// are none or the frontier is small.
+__device__ __forceinline__ HotTable* hot_load(HotTable& T, const KcoreBufs& B, unsigned frontier) {
+  const unsigned nhot = min(B.c->hot_count, kHotCap);
+  if (nhot == 0 || frontier < kHotMin) return nullptr;
+  for (uint32_t i = threadIdx.x; i < (1u << kHotBits); i += kWideBlock) {
+    T.id[i] = kNoVertex;
+    T.count[i] = 0;
+  }
   __syncthreads();
+  if (threadIdx.x < nhot) {
+    const uint32_t v = B.hot[threadIdx.x];
+    for (int p = 0; p < kHotProbe; ++p)
+      if (atomicCAS(&T.id[hot_slot(v, p)], kNoVertex, v) == kNoVertex) break;
+  }
+  __syncthreads();
+  return &T;
 }
 
-// Workgroup-uniform.  Applies the workgroup's counted decrements of the hot
-// ids (ids at or above n are never counted).
+// Workgroup-uniform.  Applies the workgroup's counted decrements.
 __device__ __forceinline__ void hot_apply(PeelOp& op) {
+  if (!op.hot) return;
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < kHot; i += kWideBlock) {
-    const uint32_t cnt = op.hot[i];
+  for (uint32_t i = threadIdx.x; i < (1u << kHotBits); i += kWideBlock) {
+    const uint32_t cnt = op.hot->count[i];
     bool dies[1] = {false};
-    const uint32_t id[1] = {i};
+    const uint32_t id[1] = {op.hot->id[i]};
     if (cnt) {
-      const uint32_t old = atomicSub(&op.degree[i], cnt);
+      const uint32_t old = atomicSub(&op.degree[degree_pos(id[0], op.mul)], cnt);
       dies[0] = old >= op.k && old - cnt < op.k;
     }
     op.wq.push(dies, id);
@@ -192,31 +260,27 @@ __device__ __forceinline__ void hot_apply(PeelOp& op) {
   }
 }
 
-template <bool kAgg>
 __global__ void __launch_bounds__(kWideBlock) kcore_peel_kernel(KcoreBufs B) {
   KcoreCounters* c = B.c;
   if (!c->active) return;
   __shared__ uint32_t stage[kWideWaves][kWaveQCap];
-  __shared__ uint32_t hot[kAgg ? kHot : 1];
-  if constexpr (kAgg) hot_clear(hot);
-  PeelOp op = make_peel(B, stage, hot, kAgg ? kHot : 0u);
-  const unsigned in = c->in;
-  expand_queue<kWideBlock, PeelOp, false, kWideEdges>(B.row, in ? B.q1 : B.q0, c->count[in], B.hub, B.hubq, &c->hub_count, B.cap, &c->overflow,
-                       op);
-  if constexpr (kAgg) hot_apply(op);
+  __shared__ HotTable hot;
+  const unsigned in = c->in, count = c->count[in];
+  PeelOp op = make_peel(B, stage, hot_load(hot, B, count));
+  expand_queue<kWideBlock, PeelOp, false, kWideEdges>(B.row, in ? B.q1 : B.q0, count, B.hub, B.hubq, &c->hub_count,
+                                                      B.cap, &c->overflow, op);
+  hot_apply(op);
   op.finish();
 }
 
-template <bool kAgg>
 __global__ void __launch_bounds__(kWideBlock) kcore_hubs_kernel(KcoreBufs B) {
   KcoreCounters* c = B.c;
   if (!c->active || c->hub_count == 0) return;
   __shared__ uint32_t stage[kWideWaves][kWaveQCap];
-  __shared__ uint32_t hot[kAgg ? kHot : 1];
-  if constexpr (kAgg) hot_clear(hot);
-  PeelOp op = make_peel(B, stage, hot, kAgg ? kHot : 0u);
+  __shared__ HotTable hot;
+  PeelOp op = make_peel(B, stage, hot_load(hot, B, c->hub_count));
   expand_hubs<kWideBlock, PeelOp, kHubLanes, kWideEdges>(B.row, B.hubq, c->hub_count, B.cap, B.hub_off, op);
-  if constexpr (kAgg) hot_apply(op);
+  hot_apply(op);
   op.finish();
 }
 
@@ -256,14 +320,20 @@ __global__ void kcore_round_turn_kernel(KcoreCounters* c) {
   round_begin(c);
 }
 
-__global__ void __launch_bounds__(kWideBlock) kcore_finish_kernel(const uint32_t* __restrict__ degree,
-                                                              uint8_t* __restrict__ alive, int64_t n, uint32_t k,
-                                                              KcoreCounters* c) {
+// The degrees in the caller's order (work may be degree itself: then in place),
+// membership and its count.
+__global__ void __launch_bounds__(kWideBlock) kcore_finish_kernel(const uint32_t* work, uint32_t mul,
+                                                                  const uint32_t* __restrict__ new_of_old,
+                                                                  uint32_t* degree, uint8_t* __restrict__ alive,
+                                                                  int64_t n, uint32_t k, KcoreCounters* c) {
+  if (!c->done) return;  // rounds are left: launched again after the next replay
   int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
   int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   unsigned long long cnt = 0;
   for (; v < n; v += stride) {
-    const bool a = degree[v] >= k;
+    const uint32_t d = work[degree_pos(new_of_old ? new_of_old[v] : static_cast<uint32_t>(v), mul)];
+    if (work != degree) degree[v] = d;
+    const bool a = d >= k;
     if (alive) alive[v] = a ? 1 : 0;
     cnt += a ? 1ull : 0ull;
   }
@@ -294,7 +364,8 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
   uint32_t* q[2] = {g->scratch<uint32_t>(WS_Q0, cap), g->scratch<uint32_t>(WS_Q1, cap)};
   uint32_t* hubq = g->scratch<uint32_t>(WS_Q2, cap);
   uint32_t* hub_off = g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(cap));
-  KcoreCounters* c = g->scratch<KcoreCounters>(WS_COUNTERS, 1);
+  KcoreState* state = g->scratch<KcoreState>(WS_COUNTERS, 1);
+  KcoreCounters* c = &state->c;
   KcoreCounters* host = static_cast<KcoreCounters*>(g->host_pinned(sizeof(KcoreCounters)));
   RegionTimer region(s);
   KernelTimer ktimer(s);
@@ -302,40 +373,36 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
   // Rounds are driven on the device: rounds (begin, peel, hub layout, hubs,
   // end) captured in HIP graphs, kRoundsFirst for the first replay and
   // kRoundsPerGraph for the next ones, replayed until the state says done,
-  // so the host synchronises once per replay.
-  KcoreBufs B{g->row, g->col, degree, q[0], q[1], hubq, hub_off, c, k, cap, hub_degree()};
+  // and the membership pass runs after
+  // the replay that ends with it, so the host synchronises once per replay.
+  KcoreBufs B{g->row, g->col, degree, q[0], q[1], hubq, hub_off, c, state->hot, k, cap, hub_degree(), 1u};
   // No vertex above the hub threshold: the hub list stays empty and its two
   // launches are left out of each round.
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
   // Graphs with hubs peel on the degree-ordered copy of the CSR
-  // (frontier.relabel): the decrements mostly land on the hubs, whose
-  // degree words then share a few cached megabytes; the degrees are mapped
-  // back before the membership pass.
+  // (frontier.relabel): the decrements mostly land on the hubs, whose degree
+  // words then share a few cached megabytes; the membership pass maps the
+  // degrees back.
   const bool relabel = hubs && tune_effective("frontier.relabel", n, g->m) != 0;
   if (relabel) {
     build_relabeled(g);
     B.row = g->relab.row.as<int32_t>();
     B.col = g->relab.col.as<int32_t>();
-    B.degree = g->scratch<uint32_t>(WS_V5, cap);
   }
-  // LDS counting of the ids below kHot: on the degree-ordered copy, or when
-  // those ids hold at least 8 times their share of the adjacency entries.
-  bool agg = relabel;
-  if (!agg && hubs && n > static_cast<int64_t>(kHot)) {
-    int32_t low = 0;
-    GX_HIP(hipMemcpyAsync(&low, B.row + kHot, sizeof(low), hipMemcpyDeviceToHost, s));
-    GX_HIP(hipStreamSynchronize(s));
-    agg = static_cast<double>(low) * static_cast<double>(n) >=
-          8.0 * static_cast<double>(kHot) * static_cast<double>(g->m);
+  if (hubs) {
+    B.degree = g->scratch<uint32_t>(WS_V5, (static_cast<size_t>(cap) + kPage - 1) / kPage * kPage);
+    B.mul = kPageMul;
   }
+  const uint32_t hot_min = static_cast<uint32_t>(std::max<int64_t>(kHotDegree, g->m >> 13));
   kcore_reset_kernel<<<1, 64, 0, s>>>(c);
-  kcore_init_kernel<<<grid_for(n, kWideBlock, kWideGrid), kWideBlock, 0, s>>>(B.row, B.degree, n, k, q[0], c, cap);
+  kcore_init_kernel<<<grid_for(n, kPage, kWideGrid), kWideBlock, 0, s>>>(B.row, B.degree, n, k, q[0], state, cap,
+                                                                            hot_min, B.mul);
   GX_LAUNCHED("kcore_init_kernel");
   uint64_t key = 0;
   for (const void* p : {(const void*)B.row, (const void*)B.col, (const void*)B.degree, (const void*)B.q0,
                         (const void*)B.q1, (const void*)B.hubq, (const void*)B.hub_off, (const void*)B.c})
     key = mix_key(key, reinterpret_cast<uintptr_t>(p));
-  key = mix_key(mix_key(mix_key(mix_key(mix_key(key, k), cap), B.hub), hubs ? 1u : 0u), agg ? 1u : 0u);
+  key = mix_key(mix_key(mix_key(mix_key(key, k), cap), B.hub), hubs ? 1u : 0u);
   uint32_t replays = 0, slots = 0;
   for (;;) {
     const int nr = replays == 0 ? kRoundsFirst : kRoundsPerGraph;
@@ -343,16 +410,10 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
     g->replay(replays == 0 ? g->kcore_head : g->kcore_batch, key, [&](hipStream_t cs) {
       kcore_round_begin_kernel<<<1, 64, 0, cs>>>(c);
       for (int i = 0; i < nr; ++i) {
-        if (agg)
-          kcore_peel_kernel<true><<<kWideGrid, kWideBlock, 0, cs>>>(B);
-        else
-          kcore_peel_kernel<false><<<kWideGrid, kWideBlock, 0, cs>>>(B);
+        kcore_peel_kernel<<<kWideGrid, kWideBlock, 0, cs>>>(B);
         if (hubs) {
           launch_hub_offsets<kHubLanes * kWideEdges>(B.row, B.hubq, &c->hub_count, cap, B.hub_off, cs);
-          if (agg)
-            kcore_hubs_kernel<true><<<kWideGrid, kWideBlock, 0, cs>>>(B);
-          else
-            kcore_hubs_kernel<false><<<kWideGrid, kWideBlock, 0, cs>>>(B);
+          kcore_hubs_kernel<<<kWideGrid, kWideBlock, 0, cs>>>(B);
         }
         if (i + 1 < nr)
           kcore_round_turn_kernel<<<1, 64, 0, cs>>>(c);
@@ -364,25 +425,19 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
     ktimer.end();
     ++replays;
     slots += static_cast<uint32_t>(nr);
+    kcore_finish_kernel<<<grid_for(n, kWideBlock, kWideGrid), kWideBlock, 0, s>>>(
+        B.degree, B.mul, relabel ? g->relab.new_of_old.as<uint32_t>() : nullptr, degree, alive, n, k, c);
+    GX_LAUNCHED("kcore_finish_kernel");
     GX_HIP(hipMemcpyAsync(host, c, sizeof(KcoreCounters), hipMemcpyDeviceToHost, s));
     GX_HIP(hipStreamSynchronize(s));
     if (host->overflow) fail(GX_ERR_CAPACITY, "k-core worklist overflow");
     if (host->done) break;
   }
-  launches += slots * (hubs ? 4 : 2) + replays;
+  launches += slots * (hubs ? 4 : 2) + 2 * replays;
   const uint32_t rounds = host->rounds;
   const uint64_t items = host->items;
   uint64_t edges = 0;
-  if (relabel) {
-    unpermute_u32(B.degree, g->relab.new_of_old.as<uint32_t>(), degree, n, s);
-    launches += 1;
-  }
-  kcore_finish_kernel<<<grid_for(n, kWideBlock, kWideGrid), kWideBlock, 0, s>>>(degree, alive, n, k, c);
-  GX_LAUNCHED("kcore_finish_kernel");
-  launches += 1;
-  GX_HIP(hipMemcpyAsync(host, c, sizeof(KcoreCounters), hipMemcpyDeviceToHost, s));
   double ms = region.stop();
-  GX_HIP(hipStreamSynchronize(s));
   if (alive_count) *alive_count = host->alive;
   (void)edges;
   if (st) {

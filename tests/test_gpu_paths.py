@@ -218,3 +218,19 @@ def test_sssp_batched_chunks(gx, oracle, n, degrees, sources):
             gx.tune_set("sssp.batch_width", -1)
         for i, s in enumerate(srcs):
             assert np.array_equal(got[i], exp[int(s)]), (i, shift)
+
+
+@pytest.mark.parametrize("n,hubs,degree", [(4095, 3, 2500), (4097, 600, 300), (20000, 40, 6000), (70001, 2, 60000)])
+def test_kcore_counted_hubs(gx, oracle, n, hubs, degree):
+    """Degree words around a page, more listed hubs than the table holds, and
+    frontiers above and below the size that counts them in LDS: the hubs
+    themselves die in some of the rounds."""
+    row, col, w = star_csr([degree] * hubs, n, n)
+    G = gx.Graph.from_csr(row, col, w, symmetric=True)
+    for k in (1, 2, 3, hubs + 2, hubs + 3, degree):
+        print(f"kcore n={n} m={len(col)} k={k}", flush=True)
+        exp = oracle.kcore(row, col, k)
+        for _ in range(2):  # scratch of an earlier call
+            deg, alive, count, _ = gx.kcore(G, k)
+            assert np.array_equal(u32(deg), exp) and count == int((exp >= k).sum())
+            assert np.array_equal(alive.cpu().numpy(), (exp >= k).astype(np.uint8))
