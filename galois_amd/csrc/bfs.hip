@@ -24,13 +24,17 @@
 //    them; RMAT-18 375 -> 286 us, direction-optimising RMAT-24 1209 -> 1004
 //    us, 4096 vertices 248 -> 153 us, most of the last from spreading small
 //    frontiers over more workgroups).
-//  - gx_bfs drives its levels on the device: each level is a fixed kernel
-//    sequence (begin, expand, hubs, end) that reads the frontier size from a
-//    device state word; levels are captured in HIP graphs (7 for the first
-//    replay, 8 for the next; the end of a level and the begin of the next in
-//    one launch) and replayed until the frontier is empty.
-//  - Bottom-up steps test a 1-bit-per-vertex frontier bitmap (n/8 bytes, L2
-//    resident for the graphs here) and stop at the first hit.
+//  - gx_bfs drives its levels on the device from a state word: runs of small
+//    levels in one workgroup (narrow_kernel), larger ones as a fixed kernel
+//    sequence (expand, hubs, narrow); four such levels are captured in a HIP
+//    graph and replayed until the frontier is empty.
+//  - On symmetric graphs with hubs the heavy levels of gx_bfs are pulled
+//    instead (level_begin): RMAT-18 240 -> 115 us, 4 M vertices 1272 -> 282 us,
+//    where 130 G neighbour levels a second bound the push.
+//  - Pulls test a 1-bit-per-vertex frontier bitmap (n/8 bytes, L2 resident for
+//    the graphs here), four neighbours at a time, and stop at the first hit
+//    (RMAT-24: the three pulls of the direction-optimising BFS 684 -> 346 us;
+//    the call, with one wait per level instead of up to three, 1177 -> 560).
 #include <algorithm>
 
 #include "frontier.hpp"
@@ -50,8 +54,8 @@ constexpr uint32_t kNoParent = 0xffffffffu;
 // of the workgroups start faster.
 constexpr int kGridNoHubs = 128;
 constexpr int kHubLanes = 256;  // lanes per step of the hub pass
-constexpr int kLevelsPerGraph = 8;
-constexpr int kLevelsFirst = 7;  // first replay: power-law graphs need 5-6 levels plus the empty one
+constexpr int kLevelsPerGraph = 4;
+constexpr int kLevelsFirst = 4;  // wide levels of the first replay: what power-law graphs need
 
 struct BfsState {
   unsigned count[2];      // frontier sizes (double buffered by q)
@@ -60,6 +64,7 @@ struct BfsState {
   unsigned q;             // frontier read this level
   unsigned level;         // level being written
   unsigned active;        // this level has a frontier
+  unsigned pull;          // this level is pulled (gx_bfs)
   unsigned done;
   // Vertices discovered this level (low 32 bits: also the end of the queue a
   // push fills) and their degree sum (high 32 bits; it is at most m < 2^31),
@@ -85,25 +90,30 @@ struct Bufs {
   unsigned cap;
   uint32_t* hub_off;
   uint32_t hub;   // frontier.hub_degree
-  uint32_t* vis;  // visited bitmap (top-down BFS only; null for the DO-BFS)
+  uint32_t* vis;  // visited bitmap (gx_bfs only; null for the DO-BFS)
+  uint64_t* front;    // frontier bitmap of a pulled level (gx_bfs)
+  int64_t n, m;
+  uint64_t pull_min;    // fewest edges out of a frontier that is pulled
+  uint64_t narrow_max;  // most edges out of a frontier that a narrow level takes
 };
 
-__global__ void bfs_init_kernel(uint32_t* __restrict__ level, uint32_t* __restrict__ parent, int64_t n,
-                                uint32_t src) {
-  int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (; v < n; v += stride) {
-    level[v] = (v == src) ? 0u : kInf;
-    if (parent) parent[v] = (v == src) ? src : kNoParent;
+// Levels, parents and the visited bitmap of a search that has found its source,
+// and its state.  src_map (may be null): the source's id in the graph the
+// search runs on.
+__global__ void bfs_init_kernel(Bufs B, int64_t n, uint32_t src, const uint32_t* __restrict__ src_map) {
+  if (src_map) src = src_map[src];
+  const int64_t first = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  for (int64_t v = first; v < n; v += stride) {
+    B.level[v] = (v == src) ? 0u : kInf;
+    if (B.parent) B.parent[v] = (v == src) ? src : kNoParent;
   }
-}
-
-__global__ void bfs_reset_kernel(BfsState* S, uint32_t* q0, uint32_t src, uint32_t* level, uint32_t* parent,
-                                 uint32_t* vis) {
-  if (threadIdx.x == 0) {
-    if (vis) vis[src >> 5] |= 1u << (src & 31);
-    S->level_out = level;
-    S->parent_out = parent;
+  if (B.vis)
+    for (int64_t w = first; w < (n + 31) / 32; w += stride) B.vis[w] = w == src / 32 ? 1u << (src & 31) : 0u;
+  if (first == 0) {
+    BfsState* S = B.S;
+    S->level_out = B.level;
+    S->parent_out = B.parent;
     S->count[0] = 1;
     S->count[1] = 0;
     S->hub_count = 0;
@@ -111,16 +121,25 @@ __global__ void bfs_reset_kernel(BfsState* S, uint32_t* q0, uint32_t src, uint32
     S->q = 0;
     S->level = 0;
     S->active = 0;
+    S->pull = 0;
     S->done = 0;
     S->app = 0;
-    S->scout = 0;
-    S->edges = 0;
+    S->scout = static_cast<unsigned>(B.row[src + 1] - B.row[src]);
+    S->edges = S->scout;
     S->items = 1;
-    q0[0] = src;
+    B.q[0][0] = src;
   }
 }
 
-__device__ __forceinline__ void level_begin(BfsState* S) {
+// A level is pulled when the edges out of its frontier are many (pull_min, a
+// quarter of the vertices: the pull reads every vertex's level and the rows of
+// the unreached) and at least an eighth of those out of the unreached vertices
+// (the most a pull could walk; most scans end at their first neighbours).
+// RMAT-18, symmetric: the two heavy levels took 89 and 92 us pushed.
+constexpr int kPullShare = 8;
+
+__device__ __forceinline__ void level_begin(const Bufs& B) {
+  BfsState* S = B.S;
   if (S->done || S->overflow || S->count[S->q] == 0) {
     S->active = 0;
     S->done = 1;
@@ -130,6 +149,7 @@ __device__ __forceinline__ void level_begin(BfsState* S) {
   S->level += 1;
   S->app = 0;
   S->hub_count = 0;
+  S->pull = S->scout > B.pull_min && S->scout * kPullShare > static_cast<uint64_t>(B.m) - S->edges;
 }
 
 __device__ __forceinline__ void level_end(BfsState* S) {
@@ -140,22 +160,6 @@ __device__ __forceinline__ void level_end(BfsState* S) {
   S->items += S->count[S->q];
   S->edges += S->scout;
   S->active = 0;
-}
-
-__global__ void level_begin_kernel(BfsState* S) {
-  if (threadIdx.x == 0) level_begin(S);
-}
-
-__global__ void level_end_kernel(BfsState* S) {
-  if (threadIdx.x == 0) level_end(S);
-}
-
-// End of one level and begin of the next in one launch (inside a captured
-// batch of levels).
-__global__ void level_turn_kernel(BfsState* S) {
-  if (threadIdx.x != 0) return;
-  level_end(S);
-  level_begin(S);
 }
 
 // Plain pointers only: the output arrays come from the device state and the
@@ -228,21 +232,113 @@ __device__ __forceinline__ TdOp make_td(const Bufs& B, uint32_t (&stage)[kWideWa
               S->level, 0ull, B.vis};
 }
 
+// Per lane: whether one of the in-neighbours col[begin, end) is in the frontier
+// bitmap, and the first found (`who`).  Called by whole wavefronts (lanes
+// without a vertex: begin == end).  A lane tests its first kPullSerial
+// neighbours itself, four in flight; what is left of longer lists is walked by
+// the wavefront together, one list after another, so that an unreached hub does
+// not hold a wavefront for as many steps as it has neighbours.
+constexpr int kPullSerial = 32;
+
+__device__ __forceinline__ bool pull_scan(const int32_t* __restrict__ col, const uint32_t* __restrict__ front,
+                                          int32_t begin, int32_t end, uint32_t& who) {
+  bool hit = false;
+  const int32_t stop = min(end, begin + kPullSerial);
+  for (int32_t e = begin; e < stop && !hit; e += 4) {
+    uint32_t u[4], w[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = static_cast<uint32_t>(col[min(e + k, end - 1)]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = front[u[k] >> 5];
+#pragma unroll
+    for (int k = 3; k >= 0; --k)
+      if ((w[k] >> (u[k] & 31)) & 1u) {
+        hit = true;
+        who = u[k];
+      }
+  }
+  uint64_t rest = __ballot(!hit && stop < end);
+  while (rest) {
+    const int i = __ffsll(static_cast<unsigned long long>(rest)) - 1;
+    rest &= rest - 1;
+    const int32_t b = __builtin_amdgcn_readlane(stop, i), last = __builtin_amdgcn_readlane(end, i);
+    for (int32_t e = b; e < last; e += kWave) {
+      const int32_t mine = e + static_cast<int32_t>(lane_id());
+      const uint32_t u = static_cast<uint32_t>(col[min(mine, last - 1)]);
+      const uint64_t in = __ballot((front[u >> 5] >> (u & 31)) & 1u);
+      if (in) {
+        const uint32_t first = __builtin_amdgcn_readlane(u, __ffsll(static_cast<unsigned long long>(in)) - 1);
+        if (static_cast<int>(lane_id()) == i) {
+          hit = true;
+          who = first;
+        }
+        break;
+      }
+    }
+  }
+  return hit;
+}
+
+// The frontier of a pulled level as a bitmap, from the levels.
+__device__ __forceinline__ void front_bitmap(const Bufs& B) {
+  const uint32_t* __restrict__ level = B.S->level_out;
+  const uint32_t last = B.S->level - 1;
+  for (int64_t b = (blockIdx.x * static_cast<int64_t>(kWideBlock) + threadIdx.x) & ~int64_t(kWave - 1); b < B.n;
+       b += static_cast<int64_t>(gridDim.x) * kWideBlock) {
+    const int64_t v = b + lane_id();
+    const uint64_t in = __ballot(v < B.n && level[v] == last);
+    if (lane_id() == 0) B.front[b / kWave] = in;
+  }
+}
+
+// A pulled level: every unreached vertex looks for a neighbour in the frontier.
+__device__ __forceinline__ void pull_level(const Bufs& B, TdOp& op) {
+  const uint32_t* front = reinterpret_cast<const uint32_t*>(B.front);
+  for (int64_t b = (blockIdx.x * static_cast<int64_t>(kWideBlock) + threadIdx.x) & ~int64_t(kWave - 1); b < B.n;
+       b += static_cast<int64_t>(gridDim.x) * kWideBlock) {
+    const int64_t v = b + lane_id();
+    int32_t rb = 0, re = 0;
+    if (v < B.n && op.level[v] == kInf) {
+      rb = B.row[v];
+      re = B.row[v + 1];
+    }
+    uint32_t who;
+    const bool won[1] = {pull_scan(B.col, front, rb, re, who)};
+    const uint32_t id[1] = {static_cast<uint32_t>(v)};
+    if (won[0]) {
+      op.level[v] = op.nl;
+      if (op.vis) atomicOr(&op.vis[v >> 5], 1u << (v & 31));
+      op.scout += static_cast<unsigned long long>(re - rb);
+    }
+    op.wq.push(won, id);
+    op.after_step();
+  }
+}
+
 __global__ void __launch_bounds__(kWideBlock) td_expand_kernel(Bufs B) {
   BfsState* S = B.S;
   if (!S->active) return;
+  if (S->pull) {
+    front_bitmap(B);
+    return;
+  }
   __shared__ uint32_t stage[kWideWaves][kWaveQCap];
   TdOp op = make_td(B, stage);
   expand_queue<kWideBlock, TdOp, false, kWideEdges>(B.row, B.q[S->q], S->count[S->q], B.hub, B.hubq, &S->hub_count, B.cap, &S->overflow, op);
   op.finish();
 }
 
+// The second half of a level: the hubs' edges, or the pull.
 __global__ void __launch_bounds__(kWideBlock) td_hubs_kernel(Bufs B) {
   BfsState* S = B.S;
-  if (!S->active || S->hub_count == 0) return;
+  const bool pull = S->pull;
+  if (!S->active || (S->hub_count == 0 && !pull)) return;
   __shared__ uint32_t stage[kWideWaves][kWaveQCap];
   TdOp op = make_td(B, stage);
-  expand_hubs<kWideBlock, TdOp, kHubLanes, kWideEdges>(B.row, B.hubq, S->hub_count, B.cap, B.hub_off, op);
+  if (pull)
+    pull_level(B, op);
+  else
+    expand_hubs<kWideBlock, TdOp, kHubLanes, kWideEdges>(B.row, B.hubq, S->hub_count, B.cap, B.hub_off, op);
   op.finish();
 }
 
@@ -256,24 +352,160 @@ void enqueue_expand(const Bufs& B, bool hubs, hipStream_t s) {
   }
 }
 
-// One level with its begin and end (a level launched on its own).
-void enqueue_level(const Bufs& B, bool hubs, hipStream_t s) {
-  level_begin_kernel<<<1, 64, 0, s>>>(B.S);
-  enqueue_expand(B, hubs, s);
-  level_end_kernel<<<1, 64, 0, s>>>(B.S);
-  GX_LAUNCHED("bfs level");
+// Between two wide levels (inside a captured batch): ends the one before, and
+// as long as the frontier is small takes the next levels itself, in one
+// workgroup, then begins a wide level.  A wide level costs its launches and
+// five dependent trips to memory, about 18 us (10 without hubs) however little
+// there is to do; here the frontier's rows stay in LDS and a level of a few
+// thousand edges is three trips (the neighbours, their levels, the exchange
+// and the rows of what was found) and two barriers.  It takes frontiers of up
+// to 8192 edges, 4096 without hubs, where the workgroup's own rate (a step of
+// 4096 edges in 3-4 us) meets the cost of a wide level: RMAT-18 240 us (16384:
+// 240, 4096: 316, all levels wide: 286), a lattice of 100,000 vertices 365
+// (8192: 384, 16384: 432, all wide 400), 4096 RMAT vertices 111 (153).
+constexpr unsigned kNarrowV = 4096;
+constexpr unsigned kNarrowEdges = 1u << 13, kNarrowEdgesNoHubs = 1u << 12;
+
+__global__ void __launch_bounds__(kWideBlock) narrow_kernel(Bufs B) {
+  BfsState* S = B.S;
+  if (S->done) return;
+  __shared__ int32_t s_start[2][kNarrowV];
+  __shared__ uint32_t s_deg[2][kNarrowV];
+  __shared__ uint32_t s_vtx[2][kNarrowV];  // only with parents
+  __shared__ uint32_t s_off[kNarrowV];
+  __shared__ uint32_t s_scan[kWideWaves + 1];
+  __shared__ unsigned s_count;
+  __shared__ unsigned long long s_scout;
+  const unsigned tid = threadIdx.x;
+  if (tid == 0) level_end(S);
+  __syncthreads();
+  uint32_t* __restrict__ level = S->level_out;
+  uint32_t* __restrict__ parent = S->parent_out;
+  unsigned q = S->q, count = S->count[q], nl = S->level;
+  const unsigned overflow = S->overflow;
+  unsigned long long scout = S->scout, items = S->items, edges = S->edges;
+  bool loaded = false;
+  int cur = 0;
+  while (count > 0 && count <= kNarrowV && scout <= B.narrow_max && !overflow) {  // workgroup-uniform
+    if (!loaded) {
+      const uint32_t* __restrict__ fq = B.q[q];
+      for (unsigned i = tid; i < count; i += kWideBlock) {
+        const uint32_t v = fq[i];
+        s_start[cur][i] = B.row[v];
+        s_deg[cur][i] = static_cast<uint32_t>(B.row[v + 1] - B.row[v]);
+        if (parent) s_vtx[cur][i] = v;
+      }
+      loaded = true;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      s_count = 0;
+      s_scout = 0;
+    }
+    constexpr unsigned kPer = kNarrowV / kWideBlock;
+    uint32_t deg[kPer], sum = 0, total;
+#pragma unroll
+    for (unsigned j = 0; j < kPer; ++j) {
+      deg[j] = tid * kPer + j < count ? s_deg[cur][tid * kPer + j] : 0u;
+      sum += deg[j];
+    }
+    uint32_t off = block_exclusive_scan<kWideBlock>(sum, s_scan, &total);
+#pragma unroll
+    for (unsigned j = 0; j < kPer; ++j) {
+      s_off[tid * kPer + j] = off;
+      off += deg[j];
+    }
+    __syncthreads();
+    ++nl;
+    uint32_t* __restrict__ qout = B.q[q ^ 1];
+    unsigned long long found = 0;
+    for (uint32_t e0 = 0; e0 < total; e0 += kWideBlock * kWideEdges) {
+      bool won[kWideEdges];
+      uint32_t v[kWideEdges], at_f[kWideEdges];
+      int32_t rb[kWideEdges], re[kWideEdges];
+#pragma unroll
+      for (int k = 0; k < kWideEdges; ++k) {
+        const uint32_t e = e0 + k * kWideBlock + tid;
+        won[k] = e < total;
+        v[k] = at_f[k] = 0;
+        if (won[k]) {
+          int lo = 0, hi = static_cast<int>(count) - 1;
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (s_off[mid] <= e) lo = mid; else hi = mid - 1;
+          }
+          at_f[k] = static_cast<uint32_t>(lo);
+          v[k] = static_cast<uint32_t>(B.col[s_start[cur][lo] + static_cast<int32_t>(e - s_off[lo])]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kWideEdges; ++k) won[k] = won[k] && level[v[k]] == kInf;
+#pragma unroll
+      for (int k = 0; k < kWideEdges; ++k) {
+        rb[k] = re[k] = 0;
+        if (won[k]) {
+          rb[k] = B.row[v[k]];
+          re[k] = B.row[v[k] + 1];
+        }
+      }
+      unsigned mine = 0;  // found by the wavefront in this step
+#pragma unroll
+      for (int k = 0; k < kWideEdges; ++k) {
+        won[k] = won[k] && atomicCAS(&level[v[k]], kInf, nl) == kInf;
+        if (won[k] && B.vis) atomicOr(&B.vis[v[k] >> 5], 1u << (v[k] & 31));
+        mine += static_cast<unsigned>(__popcll(__ballot(won[k])));
+      }
+      if (mine == 0) continue;  // wavefront-uniform
+      unsigned at = 0;
+      if (lane_id() == 0) at = atomicAdd(&s_count, mine);
+      at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+      for (int k = 0; k < kWideEdges; ++k) {
+        const uint64_t mask = __ballot(won[k]);
+        if (won[k]) {
+          const unsigned p = at + lanes_below(mask);
+          const uint32_t d = static_cast<uint32_t>(re[k] - rb[k]);
+          if (p < B.cap) qout[p] = v[k];
+          if (p < kNarrowV) {
+            s_start[cur ^ 1][p] = rb[k];
+            s_deg[cur ^ 1][p] = d;
+            if (parent) s_vtx[cur ^ 1][p] = v[k];
+          }
+          if (parent) parent[v[k]] = s_vtx[cur][at_f[k]];
+          found += d;
+        }
+        at += static_cast<unsigned>(__popcll(mask));
+      }
+    }
+    found = wave_sum(found);
+    if (lane_id() == 0 && found) atomicAdd(&s_scout, found);
+    __syncthreads();
+    count = s_count;
+    scout = s_scout;
+    items += count;
+    edges += scout;
+    q ^= 1;
+    cur ^= 1;
+  }
+  if (tid == 0) {
+    S->q = q;
+    S->count[q] = count;
+    S->level = nl;
+    S->scout = scout;
+    S->items = items;
+    S->edges = edges;
+    level_begin(B);
+  }
 }
 
-// `levels` consecutive levels with the end of each and the begin of the
-// next in one launch.
-void enqueue_levels(const Bufs& B, bool hubs, int levels, hipStream_t s) {
-  level_begin_kernel<<<1, 64, 0, s>>>(B.S);
+// `levels` wide levels, with the narrow ones between and after them, and
+// before them at the start of a search (the last narrow kernel of a batch has
+// begun the first wide level of the next).
+void enqueue_levels(const Bufs& B, bool hubs, bool start, int levels, hipStream_t s) {
+  if (start) narrow_kernel<<<1, kWideBlock, 0, s>>>(B);
   for (int i = 0; i < levels; ++i) {
     enqueue_expand(B, hubs, s);
-    if (i + 1 < levels)
-      level_turn_kernel<<<1, 64, 0, s>>>(B.S);
-    else
-      level_end_kernel<<<1, 64, 0, s>>>(B.S);
+    narrow_kernel<<<1, kWideBlock, 0, s>>>(B);
   }
   GX_LAUNCHED("bfs levels");
 }
@@ -299,19 +531,24 @@ __global__ void __launch_bounds__(kWideBlock) bu_step_kernel(const int32_t* __re
   __shared__ unsigned long long red[kWideWaves];
   unsigned long long deg = 0;
   unsigned found = 0;
-  for (int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; v < n;
-       v += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    if (level[v] != kInf) continue;
-    for (int32_t e = trow[v], end = trow[v + 1]; e < end; ++e) {
-      const uint32_t u = static_cast<uint32_t>(tcol[e]);
-      if (front[u >> 5] & (1u << (u & 31))) {
-        level[v] = nl;
-        if (parent) parent[v] = u;
-        atomicOr(&next[v >> 5], 1u << (v & 31));
-        deg += static_cast<unsigned long long>(row[v + 1] - row[v]);
-        ++found;
-        break;
-      }
+  for (int64_t b = (blockIdx.x * static_cast<int64_t>(kWideBlock) + threadIdx.x) & ~int64_t(kWave - 1); b < n;
+       b += static_cast<int64_t>(gridDim.x) * kWideBlock) {
+    const int64_t v = b + lane_id();
+    int32_t rb = 0, re = 0;
+    if (v < n && level[v] == kInf) {
+      rb = trow[v];
+      re = trow[v + 1];
+    }
+    uint32_t u;
+    const bool hit = pull_scan(tcol, front, rb, re, u);
+    // The wavefront owns the two words of its vertices.
+    const uint64_t in = __ballot(hit);
+    if (lane_id() < 2 && b + 32 * lane_id() < n) next[b / 32 + lane_id()] = static_cast<uint32_t>(in >> (32 * lane_id()));
+    if (hit) {
+      level[v] = nl;
+      if (parent) parent[v] = u;
+      deg += static_cast<unsigned long long>(row == trow ? re - rb : row[v + 1] - row[v]);
+      ++found;
     }
   }
   // Degree sum and count in one word, as the pushes add them.
@@ -341,8 +578,13 @@ __global__ void do_pull_begin_kernel(BfsState* S) {
   }
 }
 
-__global__ void set_level_kernel(BfsState* S, uint32_t lvl) {
-  if (threadIdx.x == 0) S->level = lvl;
+// The queue made from the last pulled frontier becomes the frontier of a push.
+__global__ void do_pull_end_kernel(BfsState* S, uint32_t lvl) {
+  if (threadIdx.x == 0) {
+    S->level = lvl;
+    S->scout = S->app >> 32;
+    S->active = 0;
+  }
 }
 
 __global__ void do_to_queue_begin_kernel(BfsState* S) {
@@ -374,31 +616,35 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
   uint32_t* vis = use_vis ? g->scratch<uint32_t>(WS_BITMAP0, words) : nullptr;
   Bufs B{g->row, g->col, level, nullptr, {g->scratch<uint32_t>(WS_Q0, n), g->scratch<uint32_t>(WS_Q1, n)},
          g->scratch<uint32_t>(WS_Q2, n), g->scratch<BfsState>(WS_COUNTERS, 1), cap,
-         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), vis};
+         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), vis, nullptr, n, g->m, ~uint64_t(0), kNarrowEdgesNoHubs};
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
+  if (hubs) B.narrow_max = kNarrowEdges;
+  // Symmetric graphs with hubs pull their heavy levels (level_begin).
+  if (hubs && (g->flags & GX_GRAPH_SYMMETRIC)) {
+    B.front = g->scratch<uint64_t>(WS_BITMAP1, (n + 63) / 64);
+    B.pull_min = static_cast<uint64_t>(n) / 4;
+  }
   // Graphs with hubs run on the degree-ordered copy of the CSR
   // (frontier.relabel): the levels of the most often reached vertices then
   // share a few cached megabytes; the source is mapped in, the levels back.
   const bool relabel = hubs && tune_effective("frontier.relabel", n, g->m) != 0;
-  uint32_t run_src = src;
+  const uint32_t* src_map = nullptr;
   if (relabel) {
     build_relabeled(g);
     B.row = g->relab.row.as<int32_t>();
     B.col = g->relab.col.as<int32_t>();
     B.level = g->scratch<uint32_t>(WS_V5, cap);
-    run_src = read_scalar(g, g->relab.new_of_old.as<uint32_t>() + src);
+    src_map = g->relab.new_of_old.as<uint32_t>();
   }
   BfsState* host = static_cast<BfsState*>(g->host_pinned(sizeof(BfsState)));
   RegionTimer region(s);
   KernelTimer ktimer(s);
-  bfs_init_kernel<<<sweep_grid(n), kBlock, 0, s>>>(B.level, nullptr, n, run_src);
-  if (vis) fill_kernel<uint32_t><<<sweep_grid(words), kBlock, 0, s>>>(vis, 0u, words);
-  bfs_reset_kernel<<<1, 64, 0, s>>>(B.S, B.q[0], run_src, B.level, nullptr, B.vis);
-  GX_LAUNCHED("bfs init");
+  bfs_init_kernel<<<sweep_grid(n), kBlock, 0, s>>>(B, n, src, src_map);
+  GX_LAUNCHED("bfs_init_kernel");
   uint64_t key = 0;
   for (const void* p : {(const void*)B.row, (const void*)B.col, (const void*)B.q[0],
                         (const void*)B.q[1], (const void*)B.hubq, (const void*)B.S, (const void*)B.hub_off,
-                        (const void*)B.vis})
+                        (const void*)B.vis, (const void*)B.front})
     key = mix_key(key, reinterpret_cast<uintptr_t>(p));
   key = mix_key(mix_key(mix_key(key, cap), B.hub), hubs ? 1u : 0u);
   uint32_t replays = 0, slots = 0;
@@ -406,7 +652,7 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
     const int nl = replays == 0 ? kLevelsFirst : kLevelsPerGraph;
     ktimer.begin();
     g->replay(replays == 0 ? g->bfs_head : g->bfs_batch, key, [&](hipStream_t cs) {
-      enqueue_levels(B, hubs, nl, cs);
+      enqueue_levels(B, hubs, replays == 0, nl, cs);
     });
     ktimer.end();
     ++replays;
@@ -421,18 +667,12 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
   if (st) {
     std::memset(st, 0, sizeof(*st));
     st->iterations = host->level - 1;  // levels with a non-empty frontier beyond the source
-    st->launches = (vis ? 3 : 2) + slots * (hubs ? 4 : 2) + replays + (relabel ? 1 : 0);
-    st->edges_visited = host->edges + static_cast<uint64_t>(0);
+    st->launches = 2 + slots * (hubs ? 4 : 2) + (relabel ? 1 : 0);
+    st->edges_visited = host->edges;
     st->items = host->items;
     st->elapsed_ms = ms;
     st->main_kernel_ms = ktimer.total_ms();
     st->main_kernel_launches = ktimer.count();
-  }
-  // Count the source's own adjacency in the visited edges.
-  if (st) {
-    int32_t r[2];
-    read_bytes(g, r, g->row + src, sizeof(r));
-    st->edges_visited += static_cast<uint64_t>(r[1] - r[0]);
   }
   GX_API_END
 }
@@ -469,28 +709,25 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
   const unsigned cap = static_cast<unsigned>(n);
   Bufs B{g->row, g->col, level, parent, {g->scratch<uint32_t>(WS_Q0, n), g->scratch<uint32_t>(WS_Q1, n)},
          g->scratch<uint32_t>(WS_Q2, n), g->scratch<BfsState>(WS_COUNTERS, 1), cap,
-         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), nullptr};
+         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), nullptr, nullptr, n, g->m, ~uint64_t(0), kNarrowEdgesNoHubs};
   const int64_t words = (n + 31) / 32;
   uint32_t* bm[2] = {g->scratch<uint32_t>(WS_BITMAP0, words), g->scratch<uint32_t>(WS_BITMAP1, words)};
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
+  if (hubs) B.narrow_max = kNarrowEdges;
   // Symmetric graphs with hubs run on the degree-ordered copy of the CSR
   // (frontier.relabel): a bottom-up step scans each unvisited vertex's
   // neighbours hubs first, and the hubs are the first vertices reached, so
   // most scans stop at their first neighbour; levels and parents are mapped
   // back at the end.
   const bool relabel = (g->flags & GX_GRAPH_SYMMETRIC) && hubs && tune_effective("frontier.relabel", n, g->m) != 0;
-  const int32_t* row = g->row;
-  uint32_t run_src = src;
+  const uint32_t* src_map = nullptr;
   if (relabel) {
     build_relabeled(g);
-    row = g->relab.row.as<int32_t>();
-    trow = row;
-    tcol = g->relab.col.as<int32_t>();
-    B.row = row;
-    B.col = tcol;
+    trow = B.row = g->relab.row.as<int32_t>();
+    tcol = B.col = g->relab.col.as<int32_t>();
     B.level = g->scratch<uint32_t>(WS_V5, cap);
     B.parent = parent ? g->scratch<uint32_t>(WS_V4, cap) : nullptr;
-    run_src = read_scalar(g, g->relab.new_of_old.as<uint32_t>() + src);
+    src_map = g->relab.new_of_old.as<uint32_t>();
   }
   BfsState* host = static_cast<BfsState*>(g->host_pinned(sizeof(BfsState)));
   auto read_state = [&]() {
@@ -501,69 +738,61 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
   RegionTimer region(s);
   KernelTimer ktimer(s);
   uint32_t launches = 2;
-  bfs_init_kernel<<<sweep_grid(n), kBlock, 0, s>>>(B.level, B.parent, n, run_src);
-  bfs_reset_kernel<<<1, 64, 0, s>>>(B.S, B.q[0], run_src, B.level, B.parent, nullptr);
+  bfs_init_kernel<<<sweep_grid(n), kBlock, 0, s>>>(B, n, src, src_map);
+  narrow_kernel<<<1, kWideBlock, 0, s>>>(B);
   GX_LAUNCHED("bfs init");
-  int32_t rsrc[2];
-  read_bytes(g, rsrc, row + run_src, sizeof(rsrc));
-  int64_t scout = rsrc[1] - rsrc[0];
-  int64_t edges_to_check = g->m;
-  uint64_t edges_visited = static_cast<uint64_t>(scout), items = 1;
-  uint32_t lvl = 0;
+  uint64_t pull_edges = 0, pull_items = 0;
+  bool pulled = false;  // the frontier is what a pull phase left: push it
   read_state();
-  unsigned frontier = 1;
-  while (frontier > 0) {
-    if (scout > edges_to_check / static_cast<int64_t>(alpha)) {
+  while (!host->done) {
+    // Edges out of the frontier against those that pushes have not walked.
+    const int64_t scout = static_cast<int64_t>(host->scout);
+    const int64_t edges_to_check = g->m - (static_cast<int64_t>(host->edges) - scout);
+    if (!pulled && scout > edges_to_check / static_cast<int64_t>(alpha)) {
       // Pull phase: queue -> bitmap; pull while the frontier grows or stays
       // above n/beta.
       const unsigned q = host->q;
+      uint32_t lvl = host->level - 1;  // the state has begun the level
       fill_kernel<uint32_t><<<sweep_grid(words), kBlock, 0, s>>>(bm[0], 0u, words);
-      queue_to_bitmap_kernel<<<grid_for(frontier, kBlock, 4096), kBlock, 0, s>>>(B.q[q], &B.S->count[q], bm[0]);
+      queue_to_bitmap_kernel<<<grid_for(host->count[q], kBlock, 4096), kBlock, 0, s>>>(B.q[q], &B.S->count[q], bm[0]);
       launches += 2;
       int b = 0;
       uint64_t work = static_cast<uint64_t>(scout), old_work;
       do {
         old_work = work;
         ++lvl;
-        fill_kernel<uint32_t><<<sweep_grid(words), kBlock, 0, s>>>(bm[b ^ 1], 0u, words);
         do_pull_begin_kernel<<<1, 64, 0, s>>>(B.S);
         ktimer.begin();
-        bu_step_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(trow, tcol, row, B.level, B.parent, bm[b], bm[b ^ 1], B.S,
+        bu_step_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(trow, tcol, B.row, B.level, B.parent, bm[b], bm[b ^ 1], B.S,
                                                         n, lvl);
         ktimer.end();
         GX_LAUNCHED("bu_step_kernel");
-        launches += 3;
+        launches += 2;
         read_state();
         work = static_cast<uint32_t>(host->app);
-        items += work;
-        edges_visited += host->app >> 32;
+        pull_items += work;
+        pull_edges += host->app >> 32;
         b ^= 1;
       } while (work > 0 && (work >= old_work || work > static_cast<uint64_t>(n) / beta));
       // Bitmap -> queue for the next push level.
       do_to_queue_begin_kernel<<<1, 64, 0, s>>>(B.S);
       bitmap_to_queue_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(bm[b], n, B.q[0], &B.S->count[0], cap,
                                                               &B.S->overflow);
+      do_pull_end_kernel<<<1, 64, 0, s>>>(B.S, lvl);
       GX_LAUNCHED("bitmap_to_queue_kernel");
-      launches += 2;
-      read_state();
-      frontier = host->count[0];
-      scout = 1;
-      // The push kernels take the level number from the state.
-      set_level_kernel<<<1, 64, 0, s>>>(B.S, lvl);
-      GX_LAUNCHED("set_level_kernel");
-      continue;
+      launches += 3;
+      pulled = true;
+    } else {
+      ktimer.begin();
+      enqueue_expand(B, hubs, s);
+      ktimer.end();
+      launches += hubs ? 3 : 1;
+      pulled = false;
     }
-    edges_to_check -= scout;
-    ktimer.begin();
-    enqueue_level(B, hubs, s);
-    ktimer.end();
-    launches += hubs ? 5 : 3;
+    narrow_kernel<<<1, kWideBlock, 0, s>>>(B);
+    GX_LAUNCHED("narrow_kernel");
+    ++launches;
     read_state();
-    ++lvl;
-    frontier = host->count[host->q];
-    items += frontier;
-    scout = static_cast<int64_t>(host->scout);
-    edges_visited += host->scout;
   }
   if (relabel) {
     unpermute_u32(B.level, g->relab.new_of_old.as<uint32_t>(), level, n, s);
@@ -577,10 +806,10 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
   double ms = region.stop();
   if (st) {
     std::memset(st, 0, sizeof(*st));
-    st->iterations = lvl;
+    st->iterations = host->level;
     st->launches = launches;
-    st->edges_visited = edges_visited;
-    st->items = items;
+    st->edges_visited = host->edges + pull_edges;
+    st->items = host->items + pull_items;
     st->elapsed_ms = ms;
     st->main_kernel_ms = ktimer.total_ms();
     st->main_kernel_launches = ktimer.count();

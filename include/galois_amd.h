@@ -255,7 +255,8 @@ gx_status gx_degree_power_law(int64_t n, int64_t m, const int32_t* row,
 /* ------------------------------------------------------------ algorithms
  * Outputs are DEVICE pointers owned by the caller. */
 
-/* Level-synchronous BFS (top-down, degree-binned expansion).
+/* Level-synchronous BFS (top-down, degree-binned expansion; the heavy levels
+ * of symmetric graphs with hubs bottom-up).
  * level[v] = hops from src, GX_DIST_INFINITY if unreached.
  * Replaces bfs gg_main (lonestar/analytics/gpu/bfs/bfs.cu:349-362) and
  * bfs-cpu syncAlgo (lonestar/analytics/cpu/bfs/bfs.cpp:245-293). */

@@ -234,3 +234,52 @@ def test_kcore_counted_hubs(gx, oracle, n, hubs, degree):
             deg, alive, count, _ = gx.kcore(G, k)
             assert np.array_equal(u32(deg), exp) and count == int((exp >= k).sum())
             assert np.array_equal(alive.cpu().numpy(), (exp >= k).astype(np.uint8))
+
+
+def two_communities(n, hub_degree, seed):
+    """Symmetric CSR: a random community around a hub, a path of a few vertices
+    out of it, and a star at the far end, whose centre is unreached while the
+    first community's heavy levels run."""
+    rng = np.random.default_rng(seed)
+    a = n // 2
+    u = [rng.integers(0, a, 4 * a), np.full(hub_degree, a // 3), np.arange(a - 1, a + 5), np.full(n - a - 6, a + 5)]
+    v = [rng.integers(0, a, 4 * a), rng.integers(0, a, hub_degree), np.arange(a, a + 6), np.arange(a + 6, n)]
+    u, v = np.concatenate(u), np.concatenate(v)
+    u, v = np.concatenate([u, v]), np.concatenate([v, u])
+    key = np.unique(u[u != v].astype(np.int64) * n + v[u != v])
+    u, v = key // n, key % n
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=n), out=row[1:])
+    return row, v.astype(np.int32)
+
+
+@pytest.mark.parametrize("n,hub_degree,symmetric", [(400, 150, True), (2011, 160, True), (20001, 5000, True),
+                                                    (20001, 5000, False), (300007, 60000, True)])
+@pytest.mark.parametrize("knob", [None, "bfs.visited_bitmap", "frontier.relabel"])
+def test_bfs_narrow_wide_and_pulled_levels(gx, oracle, n, hub_degree, symmetric, knob):
+    """Runs of small levels, wide ones and pulled ones in turn, vertex counts
+    that end inside a bitmap word, unreached hubs during a pull, sources at
+    either end; levels equal the oracle's, parents are one level up."""
+    row, col = two_communities(n, hub_degree, n)
+    G = gx.Graph.from_csr(row, col, symmetric=symmetric)
+    owner = np.repeat(np.arange(n), np.diff(row))
+    edges = owner.astype(np.int64) * n + col
+    if knob:
+        gx.tune_set(knob, 1)
+    try:
+        for src in (n // 6, 0, n // 2 + 2, n - 1):
+            print(f"bfs n={n} m={len(col)} symmetric={symmetric} {knob} src={src}", flush=True)
+            exp = oracle.bfs(row, col, src)
+            for _ in range(2):
+                assert np.array_equal(u32(gx.bfs(G, src)[0]), exp)
+            out = gx.bfs_do(G, src, parents=True)
+            lv, parent = u32(out[0]), u32(out[1])
+            assert np.array_equal(lv, exp)
+            reached = np.flatnonzero((exp != 0) & (exp < 1 << 30))
+            p = parent[reached].astype(np.int64)
+            assert np.array_equal(exp[p] + 1, exp[reached])
+            assert np.isin(p * n + reached, edges).all()
+            assert parent[src] == src and np.all(parent[exp > 1 << 30] == 0xffffffff)
+    finally:
+        if knob:
+            gx.tune_set(knob, -1)
