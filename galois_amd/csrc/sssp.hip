@@ -26,6 +26,9 @@
 //    and keeps the rest.  The running minimum can name a bucket whose items
 //    have meanwhile moved nearer; that split then moves nothing and the next
 //    one uses the exact minimum of the items it kept.
+//  - A relax step of few items (relax_local) goes on with what its workgroups
+//    improved into the near range for a few rounds before it ends: 153 steps
+//    of 17 us become about 50 on a lattice of 2048 x 2048 (3.67 -> 2.17 ms).
 //  - Merged buckets: a step covers the buckets [bucket, bucket + width).
 //    width starts at 1 and doubles at an advance when the phase just ended
 //    admitted fewer than kMergeLow items (up to the knob sssp.max_merge),
@@ -87,15 +90,18 @@ namespace {
 constexpr int kBlock = 256;
 constexpr uint32_t kInf = GX_DIST_INFINITY;
 // Graphs without hubs (maximum degree at or below the hub threshold, such as
-// road-like grids) have small frontiers per step and many steps: a quarter of
-// the workgroups start faster and meet less at the step's counters.
-constexpr int kGridNoHubs = 128;
+// road-like grids) have small frontiers per step and many steps: half of the
+// workgroups start faster and meet less at the step's counters (128: 2.88 ms on
+// a lattice of 2048 x 2048, 256: 2.57, 512: 2.72).
+constexpr int kGridNoHubs = 256;
 constexpr int kHubLanes = 256;  // lanes per step of the hub pass
 constexpr int kStepsPerGraph = 16;
 constexpr int kHubSelectGrid = 128;
-// Bucket merging thresholds (items admitted per phase).
-constexpr unsigned long long kMergeLow = 1ull << 14;
-constexpr unsigned long long kMergeHigh = 1ull << 17;
+// Bucket merging thresholds (items per phase).  2^14 and 2^17: lattice of 2048 x
+// 2048 with weights to 1000 the same, to 60000 5.4 ms against 4.2; 2^16 and
+// 2^19: 2.64 ms against 2.17 and 3.8 against 4.2.
+constexpr unsigned long long kMergeLow = 1ull << 15;
+constexpr unsigned long long kMergeHigh = 1ull << 18;
 
 enum Mode : unsigned { kIdle = 0, kRelax = 1, kAdvance = 2, kHubs = 3 };
 
@@ -125,7 +131,8 @@ struct SsspState {
   unsigned hub_step;       // this step selects and expands pending hubs
   uint32_t near_min;       // smallest distance in the near queue the step reads
   uint32_t near_min_next;  // the same for the near queue the step fills
-  unsigned long long phase_items;  // items queued in the current phase
+  unsigned long long phase_start;  // items before the current phase
+  unsigned long long queued;       // items of the near queues read so far
   unsigned round;
   unsigned phase;
   unsigned steps;
@@ -159,6 +166,7 @@ struct Bufs {
   // sssp.hub_refine r: a hub step expands the pending hubs within
   // hub_span = 2^(r - 1) of the smallest pending hub distance; 0 = all.
   uint32_t hub_span;
+  int local_rounds;  // kLocalRounds or kLocalRoundsNoHubs
 };
 
 __global__ void sssp_init_kernel(uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp,
@@ -201,7 +209,8 @@ __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint3
     S->hub_step = 0;
     S->near_min = 0;  // the source
     S->near_min_next = 0xffffffffu;
-    S->phase_items = 0;
+    S->phase_start = 0;
+    S->queued = 0;
     S->round = 0;
     S->phase = 0;
     S->steps = 0;
@@ -252,12 +261,23 @@ __device__ __forceinline__ void begin_hub_step(SsspState* S, uint32_t limit) {
 // counters it appends to: relax while the near frontier has items, then
 // expand the pending hubs, then advance.  An advance takes the running far
 // minimum as the new first bucket and sets the phase's width from the items
-// the last phase admitted; with far items left but no live far bucket
-// (minimum unset) every far item is settled and the run is done.
-__global__ void step_kernel(SsspState* S, uint32_t defer, uint32_t hub_span) {
+// of the last phase; with far items left but no live far bucket (minimum
+// unset) every far item is settled and the run is done.  A phase's items are
+// those expanded (the workgroups' counts: local rounds expand many that no
+// queue has seen), with hubs those queued (tally null), which saves a step the
+// read of the counts.
+__global__ void __launch_bounds__(kWave) step_kernel(SsspState* S, const unsigned long long* __restrict__ tally,
+                                                     uint32_t defer, uint32_t hub_span) {
+  if (S->done) return;
+  unsigned long long items = 0;
+  if (tally) {  // kernel argument: the same for every lane
+    for (int i = threadIdx.x; i < kWideGrid; i += kWave) items += tally[2 * i + 1];
+    items = wave_sum(items);
+  }
   if (threadIdx.x != 0) return;
   close_step(S);
-  if (S->done || S->overflow) return;
+  if (S->overflow) return;
+  if (!tally) items = S->queued += S->near_count[S->q];
   S->round += 1;
   S->app = static_cast<unsigned long long>(S->far_count[S->far_sel]) << 32;
   if (!defer) S->hub_count = 0;  // hubs of a relax step are expanded in that step
@@ -265,7 +285,6 @@ __global__ void step_kernel(SsspState* S, uint32_t defer, uint32_t hub_span) {
       (hub_span == 0 || S->hub_min >= 0xffffffffu - hub_span) ? 0xffffffffu : S->hub_min + (hub_span - 1u);
   if (S->near_count[S->q] > 0) {
     S->mode = kRelax;
-    S->phase_items += S->near_count[S->q];
     // With hub slices, the pending hubs at or below every near distance are
     // expanded in the same step as the near frontier: nothing left to
     // expand can still lower them (weights are positive).
@@ -276,11 +295,12 @@ __global__ void step_kernel(SsspState* S, uint32_t defer, uint32_t hub_span) {
     begin_hub_step(S, span_limit);
   } else if (S->far_count[S->far_sel] > 0 && S->far_min != 0xffffffffu) {
     S->mode = kAdvance;
-    if (S->phase_items < kMergeLow && S->width < S->max_width)
+    const unsigned long long in_phase = items - S->phase_start;
+    if (in_phase < kMergeLow && S->width < S->max_width)
       S->width = min(2 * S->width, S->max_width);
-    else if (S->phase_items > kMergeHigh && S->width > 1)
+    else if (in_phase > kMergeHigh && S->width > 1)
       S->width >>= 1;
-    S->phase_items = 0;
+    S->phase_start = items;
     S->phase += 1;
     S->bucket = S->far_min;
     S->far_min = 0xffffffffu;
@@ -493,6 +513,171 @@ __device__ __forceinline__ void relax_step(const Bufs& B, Stage& sn, Stage& sf) 
   op.finish();
 }
 
+// Relax step of a small near frontier: a workgroup takes one batch of it and
+// goes on with what it improved into the near range itself, for up to
+// kLocalRounds rounds, before the rest goes to the global queue.  Such a step
+// is bound by its dependent trips to memory (about ten, 17 us, and 4 us to the
+// next one) and not by its edges; a local round takes four: the rows of the
+// listed vertices with their distances, the edges, the targets' distances, the
+// atomic.  The list holds the distance a vertex was listed with, so that one
+// listed twice is expanded once, at the smaller.  Rounds run ahead of what
+// other workgroups find, which costs some expansions at distances that are not
+// final yet.
+constexpr unsigned kLocalMax = 1u << 16;  // near items: at most one batch per workgroup
+// Rounds: a lattice of 2048 x 2048 takes 3.54 ms with one, 2.84 with 2, 2.87
+// with 8, 3.10 with 16, one of 300,000 vertices 1.52, 0.96, 0.59 and 0.56; RMAT
+// graphs run ahead for less (4096 vertices 640 us with one, 416 with 2, 464
+// with 8).
+constexpr int kLocalRounds = 3, kLocalRoundsNoHubs = 8;
+constexpr int kLocalEdges = 2;
+
+// Lists of the workgroup, in the space of the near stage (used by then).
+struct LocalLists {
+  uint32_t v[2][kWideBlock], d[2][kWideBlock];
+  int32_t start[kWideBlock];
+  uint32_t off[kWideBlock];
+};
+static_assert(sizeof(LocalLists) <= sizeof(Stage), "fits the stage");
+
+__device__ __forceinline__ void relax_local(const Bufs& B, Stage& sn, Stage& sf) {
+  __shared__ uint32_t s_scan[kWideWaves + 1];
+  __shared__ unsigned s_count;
+  SsspState* S = B.S;
+  RelaxOp op = make_relax(B, sn, sf);
+  LocalLists& L = *reinterpret_cast<LocalLists*>(&sn[0][0]);
+  const unsigned tid = threadIdx.x, qcount = S->near_count[S->q];
+  const uint32_t* __restrict__ near = B.nearq[S->q];
+  uint32_t* __restrict__ nout = op.q.nq;
+  uint32_t* __restrict__ hubq = B.hubq[S->hq];
+  // Wavefront-collective: v to the global near queue, once a step.
+  auto to_queue = [&](bool pred, uint32_t v) {
+    if (__ballot(pred) == 0) return;
+    const bool won = pred && atomicExch(&B.stamp[v], op.round) != op.round;
+    const uint64_t mask = __ballot(won);
+    if (mask == 0) return;
+    unsigned base = 0;
+    if (lane_id() == 0)
+      base = static_cast<unsigned>(atomicAdd(&S->app, static_cast<unsigned long long>(__popcll(mask))));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (won) {
+      const unsigned p = base + lanes_below(mask);
+      if (p < B.cap) nout[p] = v; else atomicOr(&S->overflow, 1u);
+    }
+  };
+  const unsigned per = batch_vertices<kWideBlock>(qcount);
+  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * per;
+  unsigned count = base < qcount ? min(per, static_cast<unsigned>(qcount - base)) : 0u;
+  int cur = 0;
+  for (int r = 0; count > 0 && r < B.local_rounds; ++r) {  // workgroup-uniform
+    uint32_t v = 0, d = 0, deg = 0;
+    int32_t start = 0;
+    bool in = tid < count, hub = false;
+    if (in) {
+      v = r == 0 ? near[base + tid] : L.v[cur][tid];
+      start = B.row[v];
+      deg = static_cast<uint32_t>(B.row[v + 1] - start);
+      if (r == 0) {
+        d = op.dist[v];
+        in = B.done[v] != d;
+      } else {
+        d = L.d[cur][tid];
+        in = __hip_atomic_load(&op.dist[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == d;
+      }
+      hub = in && deg > B.hub;
+      if (in && (r == 0 || !hub)) B.done[v] = d;
+      if (in && !hub) {
+        op.edges += deg;
+        op.items += 1;
+      } else {
+        deg = 0;
+      }
+    }
+    if (r == 0) {  // hubs go to the hub list, expanded in this step
+      const uint64_t mask = __ballot(hub);
+      if (mask) {
+        unsigned at = 0;
+        if (lane_id() == 0) at = atomicAdd(&S->hub_count, static_cast<unsigned>(__popcll(mask)));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (hub) {
+          const unsigned p = at + lanes_below(mask);
+          if (p < B.cap) hubq[p] = v; else atomicOr(&S->overflow, 1u);
+        }
+      }
+    } else {
+      to_queue(hub, v);
+    }
+    uint32_t total;
+    const uint32_t off = block_exclusive_scan<kWideBlock>(deg, s_scan, &total);
+    L.start[tid] = start;
+    L.off[tid] = off;
+    L.d[cur][tid] = d;
+    if (tid == 0) s_count = 0;
+    __syncthreads();
+    for (uint32_t e0 = 0; e0 < total; e0 += kWideBlock * kLocalEdges) {
+      bool valid[kLocalEdges], to_near[kLocalEdges], to_far[kLocalEdges];
+      uint32_t t[kLocalEdges], nd[kLocalEdges], dv[kLocalEdges];
+#pragma unroll
+      for (int k = 0; k < kLocalEdges; ++k) {
+        const uint32_t e = e0 + k * kWideBlock + tid;
+        valid[k] = e < total;
+        t[k] = nd[k] = 0;
+        if (valid[k]) {
+          int lo = 0, hi = static_cast<int>(count) - 1;
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (L.off[mid] <= e) lo = mid; else hi = mid - 1;
+          }
+          const int32_t edge = L.start[lo] + static_cast<int32_t>(e - L.off[lo]);
+          t[k] = static_cast<uint32_t>(B.col[edge]);
+          nd[k] = L.d[cur][lo] + B.w[edge];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kLocalEdges; ++k) dv[k] = valid[k] ? op.dist[t[k]] : 0u;
+      uint32_t old[kLocalEdges];
+#pragma unroll
+      for (int k = 0; k < kLocalEdges; ++k) old[k] = nd[k] < dv[k] ? atomicMin(&op.dist[t[k]], nd[k]) : 0u;
+      unsigned mine = 0;  // near improvements of the wavefront in this step
+#pragma unroll
+      for (int k = 0; k < kLocalEdges; ++k) {
+        const bool better = nd[k] < old[k];
+        const uint32_t nb = nd[k] >> B.shift;
+        to_near[k] = better && nb <= op.bucket_end;
+        to_far[k] = better && nb > op.bucket_end;
+        if (to_far[k]) op.far_min = min(op.far_min, nb);
+        to_far[k] = to_far[k] && old[k] == kInf;  // reached before: it is in the far pile
+        mine += static_cast<unsigned>(__popcll(__ballot(to_near[k])));
+      }
+      op.q.far.push(to_far, t);
+      op.q.after_step(kWave * kLocalEdges);
+      if (mine == 0) continue;  // wavefront-uniform
+      unsigned at = 0;
+      if (lane_id() == 0) at = atomicAdd(&s_count, mine);
+      at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+      for (int k = 0; k < kLocalEdges; ++k) {
+        const uint64_t mask = __ballot(to_near[k]);
+        const unsigned p = at + lanes_below(mask);
+        if (to_near[k] && p < kWideBlock) {
+          L.v[cur ^ 1][p] = t[k];
+          L.d[cur ^ 1][p] = nd[k];
+        }
+        to_queue(to_near[k] && p >= kWideBlock, t[k]);  // no room in the list
+        at += static_cast<unsigned>(__popcll(mask));
+      }
+    }
+    __syncthreads();
+    count = min(s_count, static_cast<unsigned>(kWideBlock));
+    cur ^= 1;
+  }
+  // What is left goes to the next step; the lists' space is the near stage's again.
+  const uint32_t rest[1] = {tid < count ? L.v[cur][tid] : 0u};
+  const bool won[1] = {tid < count && atomicExch(&B.stamp[rest[0]], op.round) != op.round};
+  __syncthreads();
+  op.q.near.push(won, rest);
+  op.finish();
+}
+
 // The hubs of a relax step (hub_count), or with deferral the pending hubs
 // of a hub step (hub_expand, 0 outside hub steps), spread over the grid;
 // hub_offsets ran over the same count.
@@ -614,7 +799,9 @@ __global__ void __launch_bounds__(kWideBlock) work_kernel(Bufs B) {
   const unsigned mode = B.S->mode;
   if (mode != kRelax && mode != kAdvance) return;
   __shared__ Stage s0, s1;
-  if (mode == kRelax)
+  if (mode == kRelax && !B.defer && B.S->near_count[B.S->q] <= kLocalMax)
+    relax_local(B, s0, s1);
+  else if (mode == kRelax)
     relax_step(B, s0, s1);
   else
     far_split_step(B, s0, s1);
@@ -623,7 +810,7 @@ __global__ void __launch_bounds__(kWideBlock) work_kernel(Bufs B) {
 // `hubs` false: no vertex exceeds the hub threshold, so the hub list stays
 // empty and its two launches are left out of the step.
 void enqueue_step(const Bufs& B, bool hubs, hipStream_t s) {
-  step_kernel<<<1, 64, 0, s>>>(B.S, B.defer, B.hub_span);
+  step_kernel<<<1, kWave, 0, s>>>(B.S, hubs ? nullptr : B.tally, B.defer, B.hub_span);
   work_kernel<<<hubs ? kWideGrid : kGridNoHubs, kWideBlock, 0, s>>>(B);
   if (hubs) {
     if (B.defer) hub_select_kernel<<<kHubSelectGrid, kWideBlock, 0, s>>>(B);
@@ -671,6 +858,7 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   B.defer = static_cast<uint32_t>(tune_effective("sssp.defer_hubs", n, g->m)) | (refine > 0 ? 1u : 0u);
   B.hub_span = refine > 0 ? 1u << std::min<int64_t>(refine - 1, 31) : 0u;
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
+  B.local_rounds = hubs ? kLocalRounds : kLocalRoundsNoHubs;
   // Graphs with hubs run on the degree-ordered copy (frontier.relabel).
   const bool relabel = hubs && tune_effective("frontier.relabel", n, g->m) != 0;
   uint32_t run_src = src;

@@ -283,3 +283,52 @@ def test_bfs_narrow_wide_and_pulled_levels(gx, oracle, n, hub_degree, symmetric,
     finally:
         if knob:
             gx.tune_set(knob, -1)
+
+
+def lattice_csr(rows, cols, whi, seed):
+    """Symmetric weighted CSR of a rows x cols lattice with a few long edges."""
+    rng = np.random.default_rng(seed)
+    i = np.arange(rows * cols).reshape(rows, cols)
+    extra = rng.integers(0, rows * cols, (2, max(1, rows * cols // 500)))
+    u = np.concatenate([i[:, :-1].ravel(), i[:-1].ravel(), extra[0]])
+    v = np.concatenate([i[:, 1:].ravel(), i[1:].ravel(), extra[1]])
+    n = rows * cols
+    lo, hi = np.minimum(u, v), np.maximum(u, v)
+    key = np.unique(lo[lo != hi].astype(np.int64) * n + hi[lo != hi])
+    lo, hi = key // n, key % n
+    w = rng.integers(1, whi + 1, len(lo)).astype(np.uint32)
+    u, v, w = np.concatenate([lo, hi]), np.concatenate([hi, lo]), np.concatenate([w, w])
+    o = np.lexsort((v, u))
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=n), out=row[1:])
+    return row, v[o].astype(np.int32), w[o]
+
+
+@pytest.mark.parametrize("rows,cols,whi,shift", [(1, 2, 1, 0), (3, 5, 7, 4), (64, 1000, 1000, 6), (700, 701, 60000, 6),
+                                                 (300, 1000, 1, 13)])
+def test_sssp_local_rounds(gx, oracle, rows, cols, whi, shift):
+    """Steps with local rounds: one item to more than a batch per workgroup
+    lists, phases of one bucket to all of them, near lists that overflow (unit
+    weights in one bucket)."""
+    row, col, w = lattice_csr(rows, cols, whi, rows)
+    G = gx.Graph.from_csr(row, col, w, symmetric=True)
+    for src in {0, rows * cols // 2, rows * cols - 1}:
+        print(f"sssp {rows}x{cols} whi={whi} shift={shift} src={src}", flush=True)
+        exp = oracle.sssp(row, col, w, src, shift)
+        for merge in (1, 1024, -1):
+            gx.tune_set("sssp.max_merge", merge)
+            try:
+                assert np.array_equal(u32(gx.sssp(G, src, shift)[0]), exp), merge
+            finally:
+                gx.tune_set("sssp.max_merge", -1)
+
+
+@pytest.mark.parametrize("n,degrees", [(3000, [129, 1000, 2500]), (40000, [200] * 300), (40000, [30000, 128, 129])])
+def test_sssp_local_rounds_with_hubs(gx, oracle, n, degrees):
+    """Hubs met in local rounds wait for the next step."""
+    row, col, w = star_csr(degrees, n, n + 1)
+    G = gx.Graph.from_csr(row, col, w, symmetric=True)
+    for src in (0, n - 1):
+        for shift in (0, 4, 31):
+            print(f"sssp n={n} m={len(col)} shift={shift} src={src}", flush=True)
+            assert np.array_equal(u32(gx.sssp(G, src, shift)[0]), oracle.sssp(row, col, w, src, 4))
