@@ -450,7 +450,7 @@ __global__ void relabel_out_keys_kernel(const int32_t* __restrict__ col, const u
   int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (; e < m; e += stride) {
     keys[e] = (static_cast<uint64_t>(new_of_old[src[e]]) << bits) | new_of_old[col[e]];
-    ids[e] = static_cast<uint32_t>(e);
+    if (ids) ids[e] = static_cast<uint32_t>(e);
   }
 }
 
@@ -493,7 +493,7 @@ void build_relabeled(gx_graph* g) {
     DevBuf src, k0, k1, i0, perm;
     src.ensure(m * 4);
     k0.ensure(m * 8);
-    i0.ensure(m * 4);
+    if (weighted) i0.ensure(m * 4);  // the edge ids order the weights
     edge_sources(g->row, n, m, src.as<uint32_t>(), s);
     relabel_out_keys_kernel<<<grid_for(m, 256, 1 << 16), 256, 0, s>>>(
         g->col, src.as<uint32_t>(), R.new_of_old.as<uint32_t>(), k0.as<uint64_t>(), i0.as<uint32_t>(), m, bits);
@@ -501,7 +501,7 @@ void build_relabeled(gx_graph* g) {
     GX_HIP(hipStreamSynchronize(s));
     src.release();
     k1.ensure(m * 8);
-    perm.ensure(m * 4);
+    if (weighted) perm.ensure(m * 4);
     radix_sort_u64(k0.as<uint64_t>(), k1.as<uint64_t>(), i0.as<uint32_t>(), perm.as<uint32_t>(), m, 2 * bits, s);
     k0.release();
     i0.release();

@@ -14,10 +14,14 @@
 //     stretch, long runs first, then mid, then short: each of phase 2's
 //     three passes over a bin reads one contiguous part); group_kernel
 //     writes gsrc16 (groups stay in run-major order, as phase 1 writes them).
-//  4. host: phase-1 pieces per chunk (in groups), phase-2 jobs per bin in
-//     three length classes (start in bin-major dst16), tasks (bins, heavy
-//     bins sliced), sorted longest first; job_base_kernel then fills every
-//     job's group base from its run-major first edge.
+//  4. run_classes_kernel and two scans over (bin, class, chunk) and (class,
+//     bin, chunk): where every run's edges and jobs start; jobs_kernel writes
+//     the phase-2 jobs (start in bin-major dst16, length, group base).
+//  5. host: phase-1 pieces per chunk (in groups) and tasks (bins, heavy bins
+//     sliced), sorted longest first.
+// The tables have bins^2 entries (16.7 M for 2^26 vertices); made on the host,
+// with the job lists in a vector per bin, they took 150 ms of the 470 ms of a
+// first solve of RMAT-26 (322 now).
 //
 // Edges within a run are in (source, destination) order: neighbouring edges
 // of a group have distinct, ascending destinations, so a wavefront's adds
@@ -98,27 +102,126 @@ __global__ void __launch_bounds__(kBuildBlock) group_kernel(const uint64_t* __re
     if (flag[e]) gsrc16[gpos[e]] = static_cast<uint16_t>((keys[e] >> kShift) & (kSpan - 1));
 }
 
-// dst16 from run-major (chunk, bin) order into bin-major (bin, chunk)
-// order: edge e of run r moves from cstart[r] + i to bstart[r] + i.
+// Job class of the first job of a run of len edges: long, mid or short.
+__device__ __forceinline__ int run_class(uint32_t len) { return len > kMid ? 0 : (len > kShort ? 1 : 2); }
+
+// Per run (chunk, bin): its edges at (bin, class of its first job, chunk), and
+// its jobs at (class, bin, chunk); 0 in the other classes.
+__global__ void __launch_bounds__(kBuildBlock) run_classes_kernel(const uint32_t* __restrict__ cstart, int64_t nb,
+                                                                  uint32_t* __restrict__ edges,
+                                                                  uint32_t* __restrict__ jobs) {
+  const int64_t nkeys = nb * nb, stride = static_cast<int64_t>(gridDim.x) * kBuildBlock;
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(kBuildBlock) + threadIdx.x; i < nkeys; i += stride) {
+    const int64_t b = i / nb, c = i - b * nb;  // chunks vary fastest: the writes are sequential
+    const uint32_t len = cstart[c * nb + b + 1] - cstart[c * nb + b];
+    const uint32_t tail = len % kJob;
+    const int first = run_class(len), last = run_class(tail);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      edges[(b * 3 + k) * nb + c] = k == first ? len : 0u;
+      jobs[(k * nb + b) * nb + c] = (k == 0 ? len / kJob : 0u) + (tail > 0 && k == last ? 1u : 0u);
+    }
+  }
+}
+
+// Where run r of len edges starts in bin-major order.
+__device__ __forceinline__ uint32_t run_start(const uint32_t* __restrict__ estart, int64_t nb, uint32_t r,
+                                              uint32_t len) {
+  const int64_t c = r / nb, b = r - c * nb;
+  return estart[(b * 3 + run_class(len)) * nb + c];
+}
+
+// dst16 from run-major (chunk, bin) order into bin-major order: phase 2 reads
+// the runs of one bin, from every chunk, as one stretch of dst16, and inside
+// it the runs whose first job is long, then mid, then short, so that each of
+// its three passes over the bin (one per job class) reads a contiguous part.
+// Edge e of run r moves from cstart[r] + i to the run's start + i.
 __global__ void __launch_bounds__(kBuildBlock) bin_major_kernel(const uint64_t* __restrict__ keys, int64_t m,
-                                                                const uint32_t* __restrict__ cstart,
-                                                                const uint32_t* __restrict__ bstart,
+                                                                int64_t nb, const uint32_t* __restrict__ cstart,
+                                                                const uint32_t* __restrict__ estart,
                                                                 const uint16_t* __restrict__ in,
                                                                 uint16_t* __restrict__ out) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kBuildBlock;
   for (int64_t e = blockIdx.x * static_cast<int64_t>(kBuildBlock) + threadIdx.x; e < m; e += stride) {
     const uint32_t r = static_cast<uint32_t>(keys[e] >> (2 * kShift));
-    out[bstart[r] + (static_cast<uint32_t>(e) - cstart[r])] = in[e];
+    const uint32_t c0 = cstart[r];
+    out[run_start(estart, nb, r, cstart[r + 1] - c0) + (static_cast<uint32_t>(e) - c0)] = in[e];
   }
 }
 
-// gbase of every job: groups opened before its first edge, minus one.  The
-// gbase field holds the job's first edge in run-major order on entry.
-__global__ void __launch_bounds__(kBuildBlock) job_base_kernel(Job* __restrict__ jobs, int64_t njobs,
-                                                               const uint32_t* __restrict__ gpos) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kBuildBlock;
-  for (int64_t j = blockIdx.x * static_cast<int64_t>(kBuildBlock) + threadIdx.x; j < njobs; j += stride)
-    jobs[j].gbase = gpos[jobs[j].gbase] - 1u;
+// The jobs of every run: full ones, then the tail, at the run's place in the
+// list of their class.  A lane takes a run; the full jobs of long runs are
+// written by the wavefront together.
+__global__ void __launch_bounds__(kBuildBlock) jobs_kernel(const uint32_t* __restrict__ cstart, int64_t nb,
+                                                           const uint32_t* __restrict__ estart,
+                                                           const uint32_t* __restrict__ jstart,
+                                                           const uint32_t* __restrict__ gpos, Job* __restrict__ jobs) {
+  const int64_t nkeys = nb * nb, stride = static_cast<int64_t>(gridDim.x) * kBuildBlock;
+  const unsigned lane = lane_id();
+  for (int64_t i0 = blockIdx.x * static_cast<int64_t>(kBuildBlock) + (threadIdx.x & ~(kWave - 1)); i0 < nkeys;
+       i0 += stride) {
+    const int64_t i = i0 + lane;
+    uint32_t from = 0, to = 0, len = 0, at = 0;  // run-major start, bin-major start, edges, first full job
+    if (i < nkeys) {
+      const int64_t b = i / nb, c = i - b * nb;
+      from = cstart[c * nb + b];
+      len = cstart[c * nb + b + 1] - from;
+      if (len > 0) {
+        to = estart[(b * 3 + run_class(len)) * nb + c];
+        at = jstart[b * nb + c];
+        const uint32_t full = len / kJob, tail = len % kJob;
+        if (tail > 0) {
+          const int k = run_class(tail);
+          const uint32_t p = k == 0 ? at + full : jstart[(k * nb + b) * nb + c];
+          jobs[p] = Job{to + full * kJob, tail, gpos[from + full * kJob] - 1u};
+        }
+      }
+    }
+    uint64_t runs = __ballot(len >= kJob);
+    while (runs) {
+      const int r = __ffsll(static_cast<unsigned long long>(runs)) - 1;
+      runs &= runs - 1;
+      const uint32_t full = static_cast<uint32_t>(__builtin_amdgcn_readlane(len, r)) / kJob;
+      const uint32_t f0 = __builtin_amdgcn_readlane(from, r), t0 = __builtin_amdgcn_readlane(to, r);
+      const uint32_t a0 = __builtin_amdgcn_readlane(at, r);
+      for (uint32_t j = lane; j < full; j += kWave) jobs[a0 + j] = Job{t0 + j * kJob, kJob, gpos[f0 + j * kJob] - 1u};
+    }
+  }
+}
+
+// out[i] = in[i * step] for i in [0, count).
+__global__ void strided_kernel(const uint32_t* __restrict__ in, int64_t step, int64_t count,
+                               uint32_t* __restrict__ out) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < count;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    out[i] = in[i * step];
+}
+
+// One workgroup per bin: its jobs lie in its stretch of dst16 and hold as many
+// edges as it has; raises *bad otherwise.
+__global__ void __launch_bounds__(kBuildBlock) check_jobs_kernel(const Job* __restrict__ jobs, int64_t nb,
+                                                                 const uint32_t* __restrict__ first,
+                                                                 const uint32_t* __restrict__ bin_edge,
+                                                                 uint32_t* __restrict__ bad) {
+  __shared__ unsigned long long s_sum[kBuildBlock / kWave];
+  for (int64_t b = blockIdx.x; b < nb; b += gridDim.x) {
+    const uint32_t e0 = bin_edge[b], e1 = bin_edge[b + 1];
+    unsigned long long sum = 0;
+    bool ok = true;
+    for (int k = 0; k < 3; ++k)
+      for (uint32_t j = first[k * nb + b] + threadIdx.x; j < first[k * nb + b + 1]; j += kBuildBlock) {
+        const Job J = jobs[j];
+        ok = ok && J.len > 0 && J.len <= kJob && J.start >= e0 && J.start < e1 && J.len <= e1 - J.start;
+        sum += J.len;
+      }
+    sum = wave_sum(sum);
+    if (lane_id() == 0) s_sum[threadIdx.x / kWave] = sum;
+    __syncthreads();
+    unsigned long long all = 0;
+    for (int w = 0; w < kBuildBlock / kWave; ++w) all += s_sum[w];
+    if (!ok || all != e1 - e0) *bad = 1u;
+    __syncthreads();
+  }
 }
 
 // Number of vertices with out-edges: out-degrees are non-increasing in
@@ -146,10 +249,17 @@ void build_layout(gx_graph* g) {
   hipStream_t s = g->stream;
   const int64_t nb = (n + kSpan - 1) / kSpan;
   const int64_t nkeys = nb * nb;
+  auto scalar = [s](const uint32_t* d) {
+    uint32_t v = 0;
+    GX_HIP(hipMemcpyAsync(&v, d, 4, hipMemcpyDeviceToHost, s));
+    GX_HIP(hipStreamSynchronize(s));
+    return v;
+  };
 
-  std::vector<uint32_t> start(nkeys + 1), gstart(nkeys + 1), bstart;
-  DevBuf gpos;  // exclusive scan of the group flags, m + 1 entries
   int64_t ngroups = 0;
+  // First job of every (class, bin), and one past the last; first edge of
+  // every bin in bin-major order; first group of every chunk.
+  std::vector<uint32_t> first(3 * nb + 1), bin_edge(nb + 1), chunk_group(nb + 1);
   {
     DevBuf keys, sorted;
     keys.ensure(m * 8);
@@ -167,7 +277,7 @@ void build_layout(gx_graph* g) {
     sorted.ensure(m * 8);
     sort_keys_u64(keys.as<uint64_t>(), sorted.as<uint64_t>(), m, 2 * kShift + run_bits, s);
     keys.release();
-    DevBuf flag, cnt, gcnt, cur, gcur;
+    DevBuf flag, cnt, gcnt, cur, gcur, gpos;  // gpos: exclusive scan of the group flags
     flag.ensure((m + 1) * 4);
     cnt.ensure((nkeys + 1) * 4);
     gcnt.ensure((nkeys + 1) * 4);
@@ -186,103 +296,72 @@ void build_layout(gx_graph* g) {
     exclusive_scan_u32(cnt.as<uint32_t>(), cur.as<uint32_t>(), nkeys + 1, s);
     exclusive_scan_u32(gcnt.as<uint32_t>(), gcur.as<uint32_t>(), nkeys + 1, s);
     exclusive_scan_u32(flag.as<uint32_t>(), gpos.as<uint32_t>(), m + 1, s);
-    GX_HIP(hipStreamSynchronize(s));
-    GX_HIP(hipMemcpy(start.data(), cur.p, (nkeys + 1) * 4, hipMemcpyDeviceToHost));
-    GX_HIP(hipMemcpy(gstart.data(), gcur.p, (nkeys + 1) * 4, hipMemcpyDeviceToHost));
-    uint32_t total = 0;
-    GX_HIP(hipMemcpy(&total, gpos.as<uint32_t>() + m, 4, hipMemcpyDeviceToHost));
+    const uint32_t edges = scalar(cur.as<uint32_t>() + nkeys), groups = scalar(gcur.as<uint32_t>() + nkeys),
+                   total = scalar(gpos.as<uint32_t>() + m);
     ngroups = total;
-    GX_REQUIRE(start[nkeys] == static_cast<uint32_t>(m), "propagation-blocking layout: edge count mismatch");
-    GX_REQUIRE(gstart[nkeys] == total && ngroups >= 1 && ngroups <= m,
+    GX_REQUIRE(edges == static_cast<uint32_t>(m), "propagation-blocking layout: edge count mismatch");
+    GX_REQUIRE(groups == total && ngroups >= 1 && ngroups <= m,
                "propagation-blocking layout: group count mismatch");
-    // Bin-major run offsets: phase 2 reads the runs of one bin, from every
-    // chunk, as one stretch of dst16, and inside it the runs whose first job
-    // is long, then mid, then short, so that each of its three passes over
-    // the bin (one per job class) reads a contiguous part.
-    // Two passes in run order (the table is 4 bytes x bins^2): edges per
-    // (bin, class), their exclusive scan, then a cursor per (bin, class) that
-    // the chunks, in ascending order, advance.
-    bstart.resize(nkeys + 1);
-    {
-      auto cls_of = [](uint32_t len) {
-        const uint32_t l = std::min<uint32_t>(len, kJob);
-        return l > kMid ? 0 : (l > kShort ? 1 : 2);
-      };
-      std::vector<uint32_t> cursor(nb * 3, 0);
-      for (int64_t key = 0; key < nkeys; ++key) {
-        const uint32_t len = start[key + 1] - start[key];
-        cursor[(key % nb) * 3 + cls_of(len)] += len;
-      }
-      uint32_t at = 0;
-      for (uint32_t& v : cursor) {
-        const uint32_t t = v;
-        v = at;
-        at += t;
-      }
-      GX_REQUIRE(at == static_cast<uint32_t>(m), "propagation-blocking layout: bin-major offsets");
-      for (int64_t key = 0; key < nkeys; ++key) {
-        const uint32_t len = start[key + 1] - start[key];
-        uint32_t& p = cursor[(key % nb) * 3 + cls_of(len)];
-        bstart[key] = p;
-        p += len;
-      }
-      bstart[nkeys] = at;
-    }
-    {
-      DevBuf bst;
-      bst.ensure(nkeys * 4);
-      GX_HIP(hipMemcpy(bst.p, bstart.data(), nkeys * 4, hipMemcpyHostToDevice));
-      L.dst16.ensure(m * 2);
-      bin_major_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
-          sorted.as<uint64_t>(), m, cur.as<uint32_t>(), bst.as<uint32_t>(), d16.as<uint16_t>(),
-          L.dst16.as<uint16_t>());
-      GX_LAUNCHED("pb bin_major_kernel");
-      GX_HIP(hipStreamSynchronize(s));
-    }
+    cnt.release();
+    gcnt.release();
+    DevBuf ecount, estart, jcount, jstart;
+    const unsigned kgrid = grid_for(nkeys, kBuildBlock, 1 << 16);
+    ecount.ensure((3 * nkeys + 1) * 4);
+    jcount.ensure((3 * nkeys + 1) * 4);
+    estart.ensure((3 * nkeys + 1) * 4);
+    jstart.ensure((3 * nkeys + 1) * 4);
+    GX_HIP(hipMemsetAsync(ecount.as<uint32_t>() + 3 * nkeys, 0, 4, s));
+    GX_HIP(hipMemsetAsync(jcount.as<uint32_t>() + 3 * nkeys, 0, 4, s));
+    run_classes_kernel<<<kgrid, kBuildBlock, 0, s>>>(cur.as<uint32_t>(), nb, ecount.as<uint32_t>(),
+                                                     jcount.as<uint32_t>());
+    GX_LAUNCHED("pb run_classes_kernel");
+    exclusive_scan_u32(ecount.as<uint32_t>(), estart.as<uint32_t>(), 3 * nkeys + 1, s);
+    exclusive_scan_u32(jcount.as<uint32_t>(), jstart.as<uint32_t>(), 3 * nkeys + 1, s);
+    DevBuf small;  // the three small tables, then the check's flag
+    small.ensure((5 * nb + 4) * 4);
+    uint32_t* d_first = small.as<uint32_t>();
+    uint32_t* d_bin = d_first + 3 * nb + 1;
+    uint32_t* d_chunk = d_bin + nb + 1;
+    uint32_t* d_bad = d_chunk + nb + 1;
+    const unsigned sgrid = grid_for(3 * nb + 1, kBuildBlock, 256);
+    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(jstart.as<uint32_t>(), nb, 3 * nb + 1, d_first);
+    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(estart.as<uint32_t>(), 3 * nb, nb + 1, d_bin);
+    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(gcur.as<uint32_t>(), nb, nb + 1, d_chunk);
+    GX_LAUNCHED("pb strided_kernel");
+    GX_HIP(hipMemsetAsync(d_bad, 0, 4, s));
+    GX_HIP(hipStreamSynchronize(s));
+    GX_HIP(hipMemcpy(first.data(), d_first, first.size() * 4, hipMemcpyDeviceToHost));
+    GX_HIP(hipMemcpy(bin_edge.data(), d_bin, bin_edge.size() * 4, hipMemcpyDeviceToHost));
+    GX_HIP(hipMemcpy(chunk_group.data(), d_chunk, chunk_group.size() * 4, hipMemcpyDeviceToHost));
+    GX_REQUIRE(bin_edge[nb] == static_cast<uint32_t>(m), "propagation-blocking layout: bin-major offsets");
+    L.dst16.ensure(m * 2);
+    bin_major_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
+        sorted.as<uint64_t>(), m, nb, cur.as<uint32_t>(), estart.as<uint32_t>(), d16.as<uint16_t>(),
+        L.dst16.as<uint16_t>());
+    GX_LAUNCHED("pb bin_major_kernel");
+    L.jobs.ensure(std::max<size_t>(first[3 * nb], 1) * sizeof(Job));
+    jobs_kernel<<<kgrid, kBuildBlock, 0, s>>>(cur.as<uint32_t>(), nb, estart.as<uint32_t>(), jstart.as<uint32_t>(),
+                                              gpos.as<uint32_t>(), L.jobs.as<Job>());
+    GX_LAUNCHED("pb jobs_kernel");
+    check_jobs_kernel<<<static_cast<unsigned>(std::min<int64_t>(nb, 4096)), kBuildBlock, 0, s>>>(
+        L.jobs.as<Job>(), nb, d_first, d_bin, d_bad);
+    GX_LAUNCHED("pb check_jobs_kernel");
     L.gsrc16.ensure(ngroups * 2);
     group_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
         sorted.as<uint64_t>(), flag.as<uint32_t>(), gpos.as<uint32_t>(), m, L.gsrc16.as<uint16_t>());
     GX_LAUNCHED("pb group_kernel");
     GX_HIP(hipStreamSynchronize(s));
+    GX_REQUIRE(scalar(d_bad) == 0, "propagation-blocking layout: jobs do not cover their bin");
   }
 
   // Phase-1 pieces: the groups of every nonempty chunk in slices of
   // kPieceEntries.
   std::vector<Piece> pieces;
   for (int64_t c = 0; c < nb; ++c) {
-    const uint32_t a = gstart[c * nb], b = gstart[(c + 1) * nb];
+    const uint32_t a = chunk_group[c], b = chunk_group[c + 1];
     for (uint64_t p = a; p < b; p += kPieceEntries)
       pieces.push_back(Piece{static_cast<uint32_t>(c), static_cast<uint32_t>(p),
                              static_cast<uint32_t>(std::min<uint64_t>(b, p + kPieceEntries)), 0u});
-  }
-
-  // Phase-2 jobs per bin and class (chunk-major scan, appended per bin).
-  std::vector<std::vector<Job>> per[3];
-  for (auto& v : per) v.resize(nb);
-  for (int64_t c = 0; c < nb; ++c) {
-    for (int64_t b = 0; b < nb; ++b) {
-      const int64_t key = c * nb + b;
-      uint32_t p = start[key];
-      uint32_t len = start[key + 1] - p;
-      while (len > 0) {
-        const uint32_t l = std::min<uint32_t>(len, kJob);
-        const int cls = l > kMid ? 0 : (l > kShort ? 1 : 2);
-        per[cls][b].push_back(Job{bstart[key] + (p - start[key]), l, p});  // gbase: set on the device
-        p += l;
-        len -= l;
-      }
-    }
-  }
-  std::vector<Job> jobs[3];
-  std::vector<uint32_t> first[3];  // first job of every bin in each class list
-  for (int cls = 0; cls < 3; ++cls) {
-    first[cls].resize(nb + 1);
-    for (int64_t b = 0; b < nb; ++b) {
-      first[cls][b] = static_cast<uint32_t>(jobs[cls].size());
-      jobs[cls].insert(jobs[cls].end(), per[cls][b].begin(), per[cls][b].end());
-      std::vector<Job>().swap(per[cls][b]);
-    }
-    first[cls][nb] = static_cast<uint32_t>(jobs[cls].size());
   }
 
   // Tasks: a bin with at most `task_entries` edges (knob "pr.task_edges")
@@ -295,17 +374,19 @@ void build_layout(gx_graph* g) {
   const uint64_t task_entries = static_cast<uint64_t>(tune_effective("pr.task_edges", n, m));
   std::vector<std::pair<uint64_t, Task>> tasks;
   std::vector<Multi> multi;
+  // Jobs of class cls and bin b: [first_of(cls, b), first_of(cls, b + 1)) of
+  // the class's list.
+  auto first_of = [&](int cls, int64_t b) { return first[cls * nb + b] - first[cls * nb]; };
+  std::vector<Job> heavy;  // the jobs of one class of a bin that is cut
   for (int64_t b = 0; b < nb; ++b) {
-    uint64_t entries = 0;
-    for (int cls = 0; cls < 3; ++cls)
-      for (uint32_t j = first[cls][b]; j < first[cls][b + 1]; ++j) entries += jobs[cls][j].len;
+    const uint64_t entries = bin_edge[b + 1] - bin_edge[b];
     Task t{};
     t.bin = static_cast<uint32_t>(b);
     if (entries <= task_entries) {
       t.slot = kSingle;
       for (int cls = 0; cls < 3; ++cls) {
-        t.job0[cls] = first[cls][b];
-        t.job1[cls] = first[cls][b + 1];
+        t.job0[cls] = first_of(cls, b);
+        t.job1[cls] = first_of(cls, b + 1);
       }
       tasks.push_back({entries, t});
       continue;
@@ -316,14 +397,20 @@ void build_layout(gx_graph* g) {
     // ones start at the bin's first job; every range is empty until filled.
     auto reset = [&](int cls, uint32_t j) {
       for (int k = 0; k < 3; ++k)
-        t.job0[k] = t.job1[k] = k < cls ? first[k][b + 1] : (k == cls ? j : first[k][b]);
+        t.job0[k] = t.job1[k] = k < cls ? first_of(k, b + 1) : (k == cls ? j : first_of(k, b));
     };
-    reset(0, first[0][b]);
-    uint64_t acc = 0;
+    reset(0, first_of(0, b));
+    uint64_t acc = 0, sum = 0;
     for (int cls = 0; cls < 3; ++cls) {
-      for (uint32_t j = first[cls][b]; j < first[cls][b + 1]; ++j) {
+      const uint32_t j0 = first_of(cls, b), j1 = first_of(cls, b + 1);
+      heavy.resize(j1 - j0);
+      if (j1 > j0)
+        GX_HIP(hipMemcpy(heavy.data(), L.jobs.as<Job>() + first[cls * nb + b], heavy.size() * sizeof(Job),
+                         hipMemcpyDeviceToHost));
+      for (uint32_t j = j0; j < j1; ++j) {
         t.job1[cls] = j + 1;
-        acc += jobs[cls][j].len;
+        acc += heavy[j - j0].len;
+        sum += heavy[j - j0].len;
         if (acc >= task_entries) {
           tasks.push_back({acc, t});
           acc = 0;
@@ -332,6 +419,7 @@ void build_layout(gx_graph* g) {
       }
     }
     if (acc > 0) tasks.push_back({acc, t});
+    GX_REQUIRE(sum == entries, "propagation-blocking layout: task size mismatch");
   }
   std::stable_sort(tasks.begin(), tasks.end(),
                    [](const std::pair<uint64_t, Task>& a, const std::pair<uint64_t, Task>& b) {
@@ -339,21 +427,17 @@ void build_layout(gx_graph* g) {
                    });
 
   // The tables must cover every edge exactly once, every job range must lie
-  // in its list and every bin must be finalised once, before any launch.
+  // in its bin's and every bin must be finalised once, before any launch.
   {
     uint64_t covered = 0, pieced = 0;
     std::vector<uint8_t> fin(nb, 0);
     for (const auto& pt : tasks) {
       const Task& t = pt.second;
-      uint64_t e = 0;
-      for (int cls = 0; cls < 3; ++cls) {
-        GX_REQUIRE(t.job0[cls] <= t.job1[cls] && t.job1[cls] <= jobs[cls].size() &&
-                       t.job0[cls] >= first[cls][t.bin] && t.job1[cls] <= first[cls][t.bin + 1],
+      for (int cls = 0; cls < 3; ++cls)
+        GX_REQUIRE(t.job0[cls] <= t.job1[cls] && t.job0[cls] >= first_of(cls, t.bin) &&
+                       t.job1[cls] <= first_of(cls, t.bin + 1),
                    "propagation-blocking layout: bad job range");
-        for (uint32_t j = t.job0[cls]; j < t.job1[cls]; ++j) e += jobs[cls][j].len;
-      }
-      GX_REQUIRE(e == pt.first, "propagation-blocking layout: task size mismatch");
-      covered += e;
+      covered += pt.first;
       if (t.slot == kSingle) fin[t.bin] += 1;
       else GX_REQUIRE(t.slot < multi.size() && multi[t.slot].bin == t.bin, "propagation-blocking layout: bad slot");
     }
@@ -374,25 +458,11 @@ void build_layout(gx_graph* g) {
   L.pieces.ensure(std::max<size_t>(pieces.size(), 1) * sizeof(Piece));
   L.tasks.ensure(tv.size() * sizeof(Task));
   L.multi.ensure(std::max<size_t>(multi.size(), 1) * sizeof(Multi));
-  const size_t nj = jobs[0].size() + jobs[1].size() + jobs[2].size();
-  L.jobs.ensure(std::max<size_t>(nj, 1) * sizeof(Job));
   GX_HIP(hipMemcpy(L.pieces.p, pieces.data(), pieces.size() * sizeof(Piece), hipMemcpyHostToDevice));
   GX_HIP(hipMemcpy(L.tasks.p, tv.data(), tv.size() * sizeof(Task), hipMemcpyHostToDevice));
   if (!multi.empty())
     GX_HIP(hipMemcpy(L.multi.p, multi.data(), multi.size() * sizeof(Multi), hipMemcpyHostToDevice));
-  size_t off = 0;
-  for (int cls = 0; cls < 3; ++cls) {
-    if (!jobs[cls].empty())
-      GX_HIP(hipMemcpy(L.jobs.as<Job>() + off, jobs[cls].data(), jobs[cls].size() * sizeof(Job),
-                       hipMemcpyHostToDevice));
-    L.njobs[cls] = static_cast<int64_t>(jobs[cls].size());
-    off += jobs[cls].size();
-  }
-  if (nj > 0) {
-    job_base_kernel<<<grid_for(static_cast<int64_t>(nj), kBuildBlock, 1 << 14), kBuildBlock, 0, s>>>(
-        L.jobs.as<Job>(), static_cast<int64_t>(nj), gpos.as<uint32_t>());
-    GX_LAUNCHED("pb job_base_kernel");
-  }
+  for (int cls = 0; cls < 3; ++cls) L.njobs[cls] = first[(cls + 1) * nb] - first[cls * nb];
   L.gacc.ensure(std::max<size_t>(multi.size(), 1) * kSpan * sizeof(unsigned long long));
   GX_HIP(hipMemsetAsync(L.gacc.p, 0, std::max<size_t>(multi.size(), 1) * kSpan * sizeof(unsigned long long), s));
   L.vals.ensure(ngroups * sizeof(float));
