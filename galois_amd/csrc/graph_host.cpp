@@ -100,6 +100,11 @@ int64_t tune_effective(const char* key, int64_t n, int64_t m) {
   const int64_t v = k->value.load();
   return v < 0 ? k->dflt(n, m) : v;
 }
+
+bool tune_is_set(const char* key) {
+  const Knob* k = find_knob(key);
+  return k && k->value.load() >= 0;
+}
 }  // namespace gx
 
 extern "C" gx_status gx_tune_set(const char* key, int64_t value) {

@@ -262,6 +262,7 @@ unsigned char* noalloc_scratch();
 // Value of a tuning knob (gx_tune_set) for a graph of n vertices and m
 // edges: the value set, or the built-in default for that size when unset.
 int64_t tune_effective(const char* key, int64_t n, int64_t m);
+bool tune_is_set(const char* key);  // a value has been chosen for the knob
 // Default of "pr.task_edges": m / 1024 within [2^19, 2^20].
 int64_t pr_task_edges_default(int64_t n, int64_t m);
 // Degree above which a frontier vertex is expanded by the whole grid.

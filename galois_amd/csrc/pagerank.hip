@@ -361,10 +361,17 @@ static int64_t hot_sources(int64_t n, size_t real_bytes) {
 
 // Knob "pr.blocking": 1 (default) = propagation-blocked sweep for FP32,
 // 2 = also for FP64 (its sums then depend on the addition order in the last
-// bit), 0 = merge-path pull for both.  Graphs outside the layout's table
-// limits always use the pull.
+// bit), 0 = row-sweep pull for both.  Graphs outside the layout's table limits
+// always use the pull, and so do, unless the knob is set, those of fewer than
+// kBlockedMin edges: an iteration of the blocked sweep zeroes and finalises
+// whole bins of 16384 rows in a handful of workgroups (30,000 vertices, 0.48 M
+// edges: 0.93 ms a solve against 0.52; 100,000, 1.6 M: 1.6 against 0.78).
+// Sums are 64-bit in both, and both finalise a row alike.
+constexpr int64_t kBlockedMin = int64_t(1) << 21;
+
 static bool use_blocking(const gx_graph* g, size_t real_bytes) {
   const int64_t k = tune_effective("pr.blocking", g->n, g->m);
+  if (real_bytes == sizeof(float) && g->m < kBlockedMin && !tune_is_set("pr.blocking")) return false;
   const bool on = real_bytes == sizeof(float) ? k != 0 : k == 2;
   return on && pb::supported(g->n, g->m);
 }

@@ -114,14 +114,18 @@ void gx_set_profiling(int on);
  *                          blocked sweep for FP32 (streamed per-group
  *                          contributions, exact fixed-point row sums), 2 =
  *                          also for FP64 (FP64 atomic row sums, order
- *                          dependent in the last bit), 0 = merge-path pull
- *                          sweep for both (Kahan row sums in FP32)
+ *                          dependent in the last bit), 0 = pull sweep for
+ *                          both (FP64 row sums; FP64 solves of 2^23 edges or
+ *                          more sum in blocks); while not set, FP32 solves of
+ *                          fewer than 2^21 edges pull as well
  *   "pr.task_edges"        propagation-blocked sweep: a destination bin
  *                          with more in-edges than this is summed by
  *                          several workgroups (slices) that meet in a
  *                          global accumulator; read when a graph's layout
  *                          is built; default m/1024 within [2^19, 2^20],
- *                          range [2^12, 2^30]
+ *                          range [2^12, 2^30]; while not set, smaller graphs
+ *                          are cut finer (m/160, at least 2^13), so that every
+ *                          CU has a task
  *   "bfs.visited_bitmap"   gx_bfs: 1 = test a visited bitmap before the
  *                          level word of every edge's target, 0 = not; the
  *                          default uses it from 2^25 vertices on

@@ -332,3 +332,31 @@ def test_sssp_local_rounds_with_hubs(gx, oracle, n, degrees):
         for shift in (0, 4, 31):
             print(f"sssp n={n} m={len(col)} shift={shift} src={src}", flush=True)
             assert np.array_equal(u32(gx.sssp(G, src, shift)[0]), oracle.sssp(row, col, w, src, 4))
+
+
+@pytest.mark.parametrize("n,m,hubs", [(900, 5000, 0), (40000, 300000, 3), (16384, 2200000, 0), (120011, 2600000, 2)])
+def test_pagerank_fp32_sweep_choice(gx, n, m, hubs):
+    """Below 2^21 edges the default FP32 solve is the pull, from there on the
+    blocked sweep in fine slices; a set knob is obeyed.  Both sum in 64 bits and
+    round a row once per iteration: 2e-6 relative to the FP64 solve."""
+    row, col, _ = weighted_csr(n, m, n, hubs)
+    print(f"pagerank fp32 n={n} m={len(col)} hubs={hubs}", flush=True)
+    exp = gx.pagerank(gx.Graph.from_csr(row, col), tol=1e-12, max_iter=60, precision="fp64")[0].cpu().numpy()
+    got, tasks = {}, {}
+    for blocking, edges in ((-1, -1), (0, -1), (1, -1), (1, 1 << 30)):
+        gx.tune_set("pr.blocking", blocking)
+        gx.tune_set("pr.task_edges", edges)
+        try:
+            G = gx.Graph.from_csr(row, col)
+            x = gx.pagerank(G, tol=0.0, max_iter=60, precision="fp32")[0].cpu().numpy()
+        finally:
+            gx.tune_set("pr.blocking", -1)
+            gx.tune_set("pr.task_edges", -1)
+        np.testing.assert_allclose(x, exp, rtol=2e-6)
+        got[blocking, edges] = x
+        tasks[blocking, edges] = gx.pagerank_layout_info(G).get("tasks", 0)
+    blocked = len(col) >= 1 << 21
+    assert tasks[-1, -1] == (tasks[1, -1] if blocked else 0) and tasks[0, -1] == 0
+    assert np.array_equal(got[-1, -1], got[1 if blocked else 0, -1])
+    assert np.array_equal(got[1, -1], got[1, 1 << 30])  # exact sums: slices do not matter
+    assert tasks[1, 1 << 30] == -(-n // 16384) and tasks[1, -1] >= min(len(col) // (2 << 13), 64)
