@@ -367,6 +367,9 @@ void inclusive_max_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hi
 void radix_sort_u64(const uint64_t* kin, uint64_t* kout, const uint32_t* vin, uint32_t* vout, int64_t count,
                     int end_bit, hipStream_t s);
 // Ascending radix sort of count keys over bits [0, end_bit) (in is not changed).
+// The same sort of a's keys with b (as long) as the other buffer: returns the
+// one that holds the result, the other's contents are lost.
+uint64_t* radix_sort_pair_u64(uint64_t* a, uint64_t* b, int64_t count, int end_bit, hipStream_t s);
 void sort_keys_u64(const uint64_t* in, uint64_t* out, int64_t count, int end_bit, hipStream_t s);
 // Out-edge chunks of the CSR: every vertex's adjacency cut into pieces of at
 // most kEdgeChunk edges, (vertex, first edge) per chunk in vertex order;

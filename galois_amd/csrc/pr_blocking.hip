@@ -21,7 +21,7 @@
 //     sliced), sorted longest first.
 // The tables have bins^2 entries (16.7 M for 2^26 vertices); made on the host,
 // with the job lists in a vector per bin, they took 150 ms of the 470 ms of a
-// first solve of RMAT-26 (322 now).
+// first solve of RMAT-26.
 //
 // Edges within a run are in (source, destination) order: neighbouring edges
 // of a group have distinct, ascending destinations, so a wavefront's adds
@@ -261,72 +261,73 @@ void build_layout(gx_graph* g) {
   // every bin in bin-major order; first group of every chunk.
   std::vector<uint32_t> first(3 * nb + 1), bin_edge(nb + 1), chunk_group(nb + 1);
   {
-    DevBuf keys, sorted;
-    keys.ensure(m * 8);
-    {
-      DevBuf esrc;
-      esrc.ensure(m * 4);
-      edge_sources(g->row, n, m, esrc.as<uint32_t>(), s);
-      const uint32_t* rank = D.new_of_old.as<uint32_t>();
-      key_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
-          esrc.as<uint32_t>(), g->col, rank, m, static_cast<uint32_t>(nb), keys.as<uint64_t>());
-      GX_LAUNCHED("pb key_kernel");
-    }
+    // One working allocation of 18 bytes an edge and 64 a run: the keys' two
+    // buffers, of which the one that the sort leaves free takes the flags and
+    // their scan, the run-major dst16, the tables.  Large allocations are what a
+    // first solve waits for: some ten of them, 40 bytes an edge, could take a
+    // second or more where the device's memory had been in use (first solve of
+    // RMAT-26 on an idle device 322 -> 311 ms).
+    DevBuf arena;
+    size_t used = 0;
+    auto carve = [&used](size_t bytes) {
+      const size_t at = used;
+      used += (bytes + 255) & ~size_t(255);
+      return at;
+    };
+    const size_t o_a = carve(m * 8 + 64), o_b = carve(m * 8 + 64), o_d16 = carve(m * 2);
+    const size_t o_cnt = carve((nkeys + 1) * 4), o_gcnt = carve((nkeys + 1) * 4), o_cur = carve((nkeys + 1) * 4),
+                 o_gcur = carve((nkeys + 1) * 4);
+    const size_t o_ecount = carve((3 * nkeys + 1) * 4), o_jcount = carve((3 * nkeys + 1) * 4),
+                 o_estart = carve((3 * nkeys + 1) * 4), o_jstart = carve((3 * nkeys + 1) * 4);
+    const size_t o_small = carve((5 * nb + 4) * 4);
+    arena.ensure(used);
+    char* base = arena.as<char>();
+    auto words = [base](size_t o) { return reinterpret_cast<uint32_t*>(base + o); };
+    uint64_t* keys = reinterpret_cast<uint64_t*>(base + o_a);
+    uint64_t* other = reinterpret_cast<uint64_t*>(base + o_b);
+    uint32_t* esrc = words(o_b);  // done with before the sort
+    edge_sources(g->row, n, m, esrc, s);
+    key_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(esrc, g->col, D.new_of_old.as<uint32_t>(), m,
+                                                                         static_cast<uint32_t>(nb), keys);
+    GX_LAUNCHED("pb key_kernel");
     int run_bits = 0;
     while ((int64_t(1) << run_bits) < nkeys) ++run_bits;
-    sorted.ensure(m * 8);
-    sort_keys_u64(keys.as<uint64_t>(), sorted.as<uint64_t>(), m, 2 * kShift + run_bits, s);
-    keys.release();
-    DevBuf flag, cnt, gcnt, cur, gcur, gpos;  // gpos: exclusive scan of the group flags
-    flag.ensure((m + 1) * 4);
-    cnt.ensure((nkeys + 1) * 4);
-    gcnt.ensure((nkeys + 1) * 4);
-    cur.ensure((nkeys + 1) * 4);
-    gcur.ensure((nkeys + 1) * 4);
-    gpos.ensure((m + 1) * 4);
-    DevBuf d16;  // run-major dst16; L.dst16 gets it bin-major below
-    d16.ensure(m * 2);
-    GX_HIP(hipMemsetAsync(cnt.p, 0, (nkeys + 1) * 4, s));
-    GX_HIP(hipMemsetAsync(gcnt.p, 0, (nkeys + 1) * 4, s));
-    GX_HIP(hipMemsetAsync(flag.as<uint32_t>() + m, 0, 4, s));
+    const uint64_t* sorted = radix_sort_pair_u64(keys, other, m, 2 * kShift + run_bits, s);
+    uint32_t* flag = sorted == keys ? words(o_b) : words(o_a);
+    uint32_t* gpos = flag + m + 1;  // exclusive scan of the group flags
+    uint32_t *cnt = words(o_cnt), *gcnt = words(o_gcnt), *cur = words(o_cur), *gcur = words(o_gcur);
+    uint32_t *ecount = words(o_ecount), *jcount = words(o_jcount), *estart = words(o_estart),
+             *jstart = words(o_jstart);
+    uint16_t* d16 = reinterpret_cast<uint16_t*>(base + o_d16);  // run-major; L.dst16 gets it bin-major below
+    GX_HIP(hipMemsetAsync(cnt, 0, (nkeys + 1) * 4, s));
+    GX_HIP(hipMemsetAsync(gcnt, 0, (nkeys + 1) * 4, s));
+    GX_HIP(hipMemsetAsync(flag + m, 0, 4, s));
     mark_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
-        sorted.as<uint64_t>(), m, d16.as<uint16_t>(), flag.as<uint32_t>(), cnt.as<uint32_t>(),
-        gcnt.as<uint32_t>());
+        sorted, m, d16, flag, cnt, gcnt);
     GX_LAUNCHED("pb mark_kernel");
-    exclusive_scan_u32(cnt.as<uint32_t>(), cur.as<uint32_t>(), nkeys + 1, s);
-    exclusive_scan_u32(gcnt.as<uint32_t>(), gcur.as<uint32_t>(), nkeys + 1, s);
-    exclusive_scan_u32(flag.as<uint32_t>(), gpos.as<uint32_t>(), m + 1, s);
-    const uint32_t edges = scalar(cur.as<uint32_t>() + nkeys), groups = scalar(gcur.as<uint32_t>() + nkeys),
-                   total = scalar(gpos.as<uint32_t>() + m);
+    exclusive_scan_u32(cnt, cur, nkeys + 1, s);
+    exclusive_scan_u32(gcnt, gcur, nkeys + 1, s);
+    exclusive_scan_u32(flag, gpos, m + 1, s);
+    const uint32_t edges = scalar(cur + nkeys), groups = scalar(gcur + nkeys), total = scalar(gpos + m);
     ngroups = total;
     GX_REQUIRE(edges == static_cast<uint32_t>(m), "propagation-blocking layout: edge count mismatch");
     GX_REQUIRE(groups == total && ngroups >= 1 && ngroups <= m,
                "propagation-blocking layout: group count mismatch");
-    cnt.release();
-    gcnt.release();
-    DevBuf ecount, estart, jcount, jstart;
     const unsigned kgrid = grid_for(nkeys, kBuildBlock, 1 << 16);
-    ecount.ensure((3 * nkeys + 1) * 4);
-    jcount.ensure((3 * nkeys + 1) * 4);
-    estart.ensure((3 * nkeys + 1) * 4);
-    jstart.ensure((3 * nkeys + 1) * 4);
-    GX_HIP(hipMemsetAsync(ecount.as<uint32_t>() + 3 * nkeys, 0, 4, s));
-    GX_HIP(hipMemsetAsync(jcount.as<uint32_t>() + 3 * nkeys, 0, 4, s));
-    run_classes_kernel<<<kgrid, kBuildBlock, 0, s>>>(cur.as<uint32_t>(), nb, ecount.as<uint32_t>(),
-                                                     jcount.as<uint32_t>());
+    GX_HIP(hipMemsetAsync(ecount + 3 * nkeys, 0, 4, s));
+    GX_HIP(hipMemsetAsync(jcount + 3 * nkeys, 0, 4, s));
+    run_classes_kernel<<<kgrid, kBuildBlock, 0, s>>>(cur, nb, ecount, jcount);
     GX_LAUNCHED("pb run_classes_kernel");
-    exclusive_scan_u32(ecount.as<uint32_t>(), estart.as<uint32_t>(), 3 * nkeys + 1, s);
-    exclusive_scan_u32(jcount.as<uint32_t>(), jstart.as<uint32_t>(), 3 * nkeys + 1, s);
-    DevBuf small;  // the three small tables, then the check's flag
-    small.ensure((5 * nb + 4) * 4);
-    uint32_t* d_first = small.as<uint32_t>();
+    exclusive_scan_u32(ecount, estart, 3 * nkeys + 1, s);
+    exclusive_scan_u32(jcount, jstart, 3 * nkeys + 1, s);
+    uint32_t* d_first = words(o_small);  // the three small tables, then the check's flag
     uint32_t* d_bin = d_first + 3 * nb + 1;
     uint32_t* d_chunk = d_bin + nb + 1;
     uint32_t* d_bad = d_chunk + nb + 1;
     const unsigned sgrid = grid_for(3 * nb + 1, kBuildBlock, 256);
-    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(jstart.as<uint32_t>(), nb, 3 * nb + 1, d_first);
-    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(estart.as<uint32_t>(), 3 * nb, nb + 1, d_bin);
-    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(gcur.as<uint32_t>(), nb, nb + 1, d_chunk);
+    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(jstart, nb, 3 * nb + 1, d_first);
+    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(estart, 3 * nb, nb + 1, d_bin);
+    strided_kernel<<<sgrid, kBuildBlock, 0, s>>>(gcur, nb, nb + 1, d_chunk);
     GX_LAUNCHED("pb strided_kernel");
     GX_HIP(hipMemsetAsync(d_bad, 0, 4, s));
     GX_HIP(hipStreamSynchronize(s));
@@ -336,19 +337,18 @@ void build_layout(gx_graph* g) {
     GX_REQUIRE(bin_edge[nb] == static_cast<uint32_t>(m), "propagation-blocking layout: bin-major offsets");
     L.dst16.ensure(m * 2);
     bin_major_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
-        sorted.as<uint64_t>(), m, nb, cur.as<uint32_t>(), estart.as<uint32_t>(), d16.as<uint16_t>(),
-        L.dst16.as<uint16_t>());
+        sorted, m, nb, cur, estart, d16, L.dst16.as<uint16_t>());
     GX_LAUNCHED("pb bin_major_kernel");
     L.jobs.ensure(std::max<size_t>(first[3 * nb], 1) * sizeof(Job));
-    jobs_kernel<<<kgrid, kBuildBlock, 0, s>>>(cur.as<uint32_t>(), nb, estart.as<uint32_t>(), jstart.as<uint32_t>(),
-                                              gpos.as<uint32_t>(), L.jobs.as<Job>());
+    jobs_kernel<<<kgrid, kBuildBlock, 0, s>>>(cur, nb, estart, jstart,
+                                              gpos, L.jobs.as<Job>());
     GX_LAUNCHED("pb jobs_kernel");
     check_jobs_kernel<<<static_cast<unsigned>(std::min<int64_t>(nb, 4096)), kBuildBlock, 0, s>>>(
         L.jobs.as<Job>(), nb, d_first, d_bin, d_bad);
     GX_LAUNCHED("pb check_jobs_kernel");
     L.gsrc16.ensure(ngroups * 2);
     group_kernel<<<grid_for(m, kBuildBlock, 1 << 16), kBuildBlock, 0, s>>>(
-        sorted.as<uint64_t>(), flag.as<uint32_t>(), gpos.as<uint32_t>(), m, L.gsrc16.as<uint16_t>());
+        sorted, flag, gpos, m, L.gsrc16.as<uint16_t>());
     GX_LAUNCHED("pb group_kernel");
     GX_HIP(hipStreamSynchronize(s));
     GX_REQUIRE(scalar(d_bad) == 0, "propagation-blocking layout: jobs do not cover their bin");

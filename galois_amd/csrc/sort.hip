@@ -21,6 +21,7 @@
 // slots of one digit's run.  Passes alternate between the output and a
 // scratch buffer so that the last one writes the output.
 #include <algorithm>
+#include <utility>
 
 #include "gx_device.hpp"
 #include "gx_internal.hpp"
@@ -320,6 +321,29 @@ void radix_sort_u64(const uint64_t* kin, uint64_t* kout, const uint32_t* vin, ui
     sv = dv;
   }
   GX_HIP(hipStreamSynchronize(s));  // scratch buffers are freed on return
+}
+
+uint64_t* radix_sort_pair_u64(uint64_t* a, uint64_t* b, int64_t count, int end_bit, hipStream_t s) {
+  GX_REQUIRE(count >= 0 && count < (int64_t(1) << 32), "sort: too many keys");
+  GX_REQUIRE(end_bit >= 0 && end_bit <= 64, "sort: bad bit range");
+  if (count == 0) return a;
+  const int64_t tiles = (count + kSortTile - 1) / kSortTile;
+  GX_REQUIRE(tiles * kDigits < (int64_t(1) << 32), "sort: too many tiles");
+  DevBuf counts;
+  counts.ensure(tiles * kDigits * 4);
+  for (int shift = 0; shift < end_bit; shift += 8) {
+    const uint32_t mask = (1u << std::min(8, end_bit - shift)) - 1u;
+    radix_hist_kernel<<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(a, count, shift, mask,
+                                                                          counts.as<uint32_t>(), tiles);
+    GX_LAUNCHED("radix_hist_kernel");
+    scan_u32(counts.as<uint32_t>(), counts.as<uint32_t>(), tiles * kDigits, true, SumOp{}, s);
+    radix_scatter_kernel<false><<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(
+        a, nullptr, count, shift, mask, counts.as<uint32_t>(), tiles, b, nullptr);
+    GX_LAUNCHED("radix_scatter_kernel");
+    std::swap(a, b);
+  }
+  GX_HIP(hipStreamSynchronize(s));  // the counts are freed on return
+  return a;
 }
 
 }  // namespace gx
