@@ -34,7 +34,8 @@
 //  - Pulls test a 1-bit-per-vertex frontier bitmap (n/8 bytes, L2 resident for
 //    the graphs here), four neighbours at a time, and stop at the first hit
 //    (RMAT-24: the three pulls of the direction-optimising BFS 684 -> 346 us;
-//    the call, with one wait per level instead of up to three, 1177 -> 560).
+//    the call, with one wait per level instead of up to three, 1177 -> 560;
+//    with pull_vertex 432).
 #include <algorithm>
 
 #include "frontier.hpp"
@@ -46,7 +47,6 @@ using namespace gx;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kQCap = 4096;  // bitmap_to_queue_kernel
 constexpr uint32_t kInf = GX_DIST_INFINITY;
 constexpr uint32_t kNoParent = 0xffffffffu;
 // Graphs without hubs (maximum degree at or below the hub threshold, such as
@@ -93,6 +93,10 @@ struct Bufs {
   uint32_t* vis;  // visited bitmap (gx_bfs only; null for the DO-BFS)
   uint64_t* front;    // frontier bitmap of a pulled level (gx_bfs)
   int64_t n, m;
+  // On the degree-ordered copy: every vertex's first neighbour, and the number
+  // of vertices with edges (the first ones); otherwise null and n.
+  const uint32_t* first;
+  int64_t nonzero;
   uint64_t pull_min;    // fewest edges out of a frontier that is pulled
   uint64_t narrow_max;  // most edges out of a frontier that a narrow level takes
 };
@@ -291,24 +295,47 @@ __device__ __forceinline__ void front_bitmap(const Bufs& B) {
   }
 }
 
+// Per lane: whether unreached vertex v (or none: live false) has a neighbour in
+// the frontier, and which.  On the degree-ordered copy most vertices are found
+// by their first neighbour, a hub, which is read in sequence from a list of its
+// own: the row and, a cache line each, the neighbours are left to the others
+// (RMAT-24: the three pulls 346 -> 240 us).
+__device__ __forceinline__ bool pull_vertex(const int32_t* __restrict__ row, const int32_t* __restrict__ col,
+                                            const uint32_t* __restrict__ first, const uint32_t* __restrict__ front,
+                                            bool live, int64_t v, uint32_t& who) {
+  bool hit = false;
+  int32_t rb = 0, re = 0;
+  if (live) {
+    if (first) {
+      who = first[v];  // v < nonzero: it has one
+      hit = (front[who >> 5] >> (who & 31)) & 1u;
+    }
+    if (!hit) {
+      rb = row[v];
+      re = row[v + 1];
+    }
+  }
+  uint32_t u;
+  if (pull_scan(col, front, rb, re, u)) {
+    who = u;
+    hit = true;
+  }
+  return hit;
+}
+
 // A pulled level: every unreached vertex looks for a neighbour in the frontier.
 __device__ __forceinline__ void pull_level(const Bufs& B, TdOp& op) {
   const uint32_t* front = reinterpret_cast<const uint32_t*>(B.front);
-  for (int64_t b = (blockIdx.x * static_cast<int64_t>(kWideBlock) + threadIdx.x) & ~int64_t(kWave - 1); b < B.n;
+  for (int64_t b = (blockIdx.x * static_cast<int64_t>(kWideBlock) + threadIdx.x) & ~int64_t(kWave - 1); b < B.nonzero;
        b += static_cast<int64_t>(gridDim.x) * kWideBlock) {
     const int64_t v = b + lane_id();
-    int32_t rb = 0, re = 0;
-    if (v < B.n && op.level[v] == kInf) {
-      rb = B.row[v];
-      re = B.row[v + 1];
-    }
     uint32_t who;
-    const bool won[1] = {pull_scan(B.col, front, rb, re, who)};
+    const bool won[1] = {pull_vertex(B.row, B.col, B.first, front, v < B.nonzero && op.level[v] == kInf, v, who)};
     const uint32_t id[1] = {static_cast<uint32_t>(v)};
     if (won[0]) {
       op.level[v] = op.nl;
       if (op.vis) atomicOr(&op.vis[v >> 5], 1u << (v & 31));
-      op.scout += static_cast<unsigned long long>(re - rb);
+      op.scout += static_cast<unsigned long long>(B.row[v + 1] - B.row[v]);
     }
     op.wq.push(won, id);
     op.after_step();
@@ -520,34 +547,31 @@ __global__ void queue_to_bitmap_kernel(const uint32_t* __restrict__ q, const uns
   }
 }
 
-// Every unreached vertex looks for a frontier in-neighbour.
+// Every unreached vertex below `last` looks for a frontier in-neighbour; the
+// words of `next` behind it are cleared.
 __global__ void __launch_bounds__(kWideBlock) bu_step_kernel(const int32_t* __restrict__ trow,
                                                          const int32_t* __restrict__ tcol,
+                                                         const uint32_t* __restrict__ first,
                                                          const int32_t* __restrict__ row,
                                                          uint32_t* __restrict__ level, uint32_t* __restrict__ parent,
                                                          const uint32_t* __restrict__ front,
                                                          uint32_t* __restrict__ next, BfsState* S, int64_t n,
-                                                         uint32_t nl) {
+                                                         int64_t last, uint32_t nl) {
   __shared__ unsigned long long red[kWideWaves];
   unsigned long long deg = 0;
   unsigned found = 0;
   for (int64_t b = (blockIdx.x * static_cast<int64_t>(kWideBlock) + threadIdx.x) & ~int64_t(kWave - 1); b < n;
        b += static_cast<int64_t>(gridDim.x) * kWideBlock) {
     const int64_t v = b + lane_id();
-    int32_t rb = 0, re = 0;
-    if (v < n && level[v] == kInf) {
-      rb = trow[v];
-      re = trow[v + 1];
-    }
     uint32_t u;
-    const bool hit = pull_scan(tcol, front, rb, re, u);
+    const bool hit = b < last && pull_vertex(trow, tcol, first, front, v < last && level[v] == kInf, v, u);
     // The wavefront owns the two words of its vertices.
     const uint64_t in = __ballot(hit);
     if (lane_id() < 2 && b + 32 * lane_id() < n) next[b / 32 + lane_id()] = static_cast<uint32_t>(in >> (32 * lane_id()));
     if (hit) {
       level[v] = nl;
       if (parent) parent[v] = u;
-      deg += static_cast<unsigned long long>(row == trow ? re - rb : row[v + 1] - row[v]);
+      deg += static_cast<unsigned long long>(row[v + 1] - row[v]);
       ++found;
     }
   }
@@ -557,19 +581,27 @@ __global__ void __launch_bounds__(kWideBlock) bu_step_kernel(const int32_t* __re
   if (threadIdx.x == 0 && both) atomicAdd(&S->app, both);
 }
 
-__global__ void __launch_bounds__(kWideBlock) bitmap_to_queue_kernel(const uint32_t* __restrict__ bm, int64_t n,
+// A lane per bitmap word: one scan and one atomic per 32768 vertices.
+__global__ void __launch_bounds__(kWideBlock) bitmap_to_queue_kernel(const uint32_t* __restrict__ bm, int64_t words,
                                                                  uint32_t* __restrict__ q, unsigned* count,
                                                                  unsigned cap, unsigned* overflow) {
-  __shared__ LdsQueue<kQCap> sq;
-  lq_init(sq);
-  for (int64_t b = blockIdx.x * static_cast<int64_t>(blockDim.x); b < n;
-       b += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t v = b + threadIdx.x;
-    const bool set = v < n && (bm[v >> 5] & (1u << (v & 31)));
-    lq_push(sq, set, static_cast<uint32_t>(v));
-    lq_flush(sq, q, count, cap, overflow, false);
+  __shared__ uint32_t s_scan[kWideWaves + 1];
+  __shared__ unsigned s_base;
+  for (int64_t b = blockIdx.x * static_cast<int64_t>(kWideBlock); b < words;
+       b += static_cast<int64_t>(gridDim.x) * kWideBlock) {
+    const int64_t i = b + threadIdx.x;
+    uint32_t bits = i < words ? bm[i] : 0u, total;
+    const uint32_t before = block_exclusive_scan<kWideBlock>(static_cast<uint32_t>(__popc(bits)), s_scan, &total);
+    if (total == 0) continue;  // workgroup-uniform
+    if (threadIdx.x == 0) s_base = atomicAdd(count, total);
+    __syncthreads();
+    unsigned p = s_base + before;
+    for (; bits; bits &= bits - 1, ++p) {
+      const uint32_t v = static_cast<uint32_t>(i) * 32 + static_cast<uint32_t>(__ffs(static_cast<int>(bits)) - 1);
+      if (p < cap) q[p] = v; else atomicOr(overflow, 1u);
+    }
+    __syncthreads();
   }
-  lq_flush(sq, q, count, cap, overflow, true);
 }
 
 __global__ void do_pull_begin_kernel(BfsState* S) {
@@ -616,7 +648,7 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
   uint32_t* vis = use_vis ? g->scratch<uint32_t>(WS_BITMAP0, words) : nullptr;
   Bufs B{g->row, g->col, level, nullptr, {g->scratch<uint32_t>(WS_Q0, n), g->scratch<uint32_t>(WS_Q1, n)},
          g->scratch<uint32_t>(WS_Q2, n), g->scratch<BfsState>(WS_COUNTERS, 1), cap,
-         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), vis, nullptr, n, g->m, ~uint64_t(0), kNarrowEdgesNoHubs};
+         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), vis, nullptr, n, g->m, nullptr, n, ~uint64_t(0), kNarrowEdgesNoHubs};
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
   if (hubs) B.narrow_max = kNarrowEdges;
   // Symmetric graphs with hubs pull their heavy levels (level_begin).
@@ -635,6 +667,8 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
     B.col = g->relab.col.as<int32_t>();
     B.level = g->scratch<uint32_t>(WS_V5, cap);
     src_map = g->relab.new_of_old.as<uint32_t>();
+    B.first = g->relab.first.as<uint32_t>();
+    B.nonzero = g->relab.nonzero;
   }
   BfsState* host = static_cast<BfsState*>(g->host_pinned(sizeof(BfsState)));
   RegionTimer region(s);
@@ -709,7 +743,7 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
   const unsigned cap = static_cast<unsigned>(n);
   Bufs B{g->row, g->col, level, parent, {g->scratch<uint32_t>(WS_Q0, n), g->scratch<uint32_t>(WS_Q1, n)},
          g->scratch<uint32_t>(WS_Q2, n), g->scratch<BfsState>(WS_COUNTERS, 1), cap,
-         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), nullptr, nullptr, n, g->m, ~uint64_t(0), kNarrowEdgesNoHubs};
+         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), nullptr, nullptr, n, g->m, nullptr, n, ~uint64_t(0), kNarrowEdgesNoHubs};
   const int64_t words = (n + 31) / 32;
   uint32_t* bm[2] = {g->scratch<uint32_t>(WS_BITMAP0, words), g->scratch<uint32_t>(WS_BITMAP1, words)};
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
@@ -728,6 +762,8 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
     B.level = g->scratch<uint32_t>(WS_V5, cap);
     B.parent = parent ? g->scratch<uint32_t>(WS_V4, cap) : nullptr;
     src_map = g->relab.new_of_old.as<uint32_t>();
+    B.first = g->relab.first.as<uint32_t>();
+    B.nonzero = g->relab.nonzero;
   }
   BfsState* host = static_cast<BfsState*>(g->host_pinned(sizeof(BfsState)));
   auto read_state = [&]() {
@@ -763,8 +799,8 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
         ++lvl;
         do_pull_begin_kernel<<<1, 64, 0, s>>>(B.S);
         ktimer.begin();
-        bu_step_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(trow, tcol, B.row, B.level, B.parent, bm[b], bm[b ^ 1], B.S,
-                                                        n, lvl);
+        bu_step_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(trow, tcol, B.first, B.row, B.level, B.parent, bm[b],
+                                                           bm[b ^ 1], B.S, n, B.nonzero, lvl);
         ktimer.end();
         GX_LAUNCHED("bu_step_kernel");
         launches += 2;
@@ -776,7 +812,7 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
       } while (work > 0 && (work >= old_work || work > static_cast<uint64_t>(n) / beta));
       // Bitmap -> queue for the next push level.
       do_to_queue_begin_kernel<<<1, 64, 0, s>>>(B.S);
-      bitmap_to_queue_kernel<<<wide_grid(n), kWideBlock, 0, s>>>(bm[b], n, B.q[0], &B.S->count[0], cap,
+      bitmap_to_queue_kernel<<<wide_grid(words), kWideBlock, 0, s>>>(bm[b], words, B.q[0], &B.S->count[0], cap,
                                                               &B.S->overflow);
       do_pull_end_kernel<<<1, 64, 0, s>>>(B.S, lvl);
       GX_LAUNCHED("bitmap_to_queue_kernel");

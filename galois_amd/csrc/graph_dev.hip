@@ -461,6 +461,18 @@ __global__ void gather_u32_kernel(const uint32_t* __restrict__ in, const uint32_
   for (; i < m; i += stride) out[i] = in[idx[i]];
 }
 
+// First out-neighbour per vertex (0 without out-edges), and the number of
+// vertices with out-edges: degrees are non-increasing, so they come first.
+__global__ void first_neighbour_kernel(const int32_t* __restrict__ row, const int32_t* __restrict__ col, int64_t n,
+                                       uint32_t* __restrict__ first, unsigned long long* __restrict__ nonzero) {
+  for (int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; v < n;
+       v += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int32_t b = row[v], e = row[v + 1];
+    first[v] = b < e ? static_cast<uint32_t>(col[b]) : 0u;
+    if (b < e && (v + 1 == n || row[v + 2] == e)) *nonzero = static_cast<unsigned long long>(v) + 1;
+  }
+}
+
 void build_relabeled(gx_graph* g) {
   Relabeled& R = g->relab;
   if (R.ready) return;
@@ -516,7 +528,18 @@ void build_relabeled(gx_graph* g) {
       GX_LAUNCHED("gather_u32_kernel");
     }
   }
+  R.first.ensure(std::max<int64_t>(n, 1) * 4);
+  DevBuf nz;
+  nz.ensure(8);
+  fill<uint32_t>(nz.as<uint32_t>(), 0u, 2, s);
+  first_neighbour_kernel<<<grid_for(n, 256, 1 << 14), 256, 0, s>>>(R.row.as<int32_t>(), R.col.as<int32_t>(), n,
+                                                                   R.first.as<uint32_t>(),
+                                                                   nz.as<unsigned long long>());
+  GX_LAUNCHED("first_neighbour_kernel");
+  unsigned long long nonzero = 0;
+  GX_HIP(hipMemcpyAsync(&nonzero, nz.p, 8, hipMemcpyDeviceToHost, s));
   GX_HIP(hipStreamSynchronize(s));
+  R.nonzero = static_cast<int64_t>(nonzero);
   R.ready = true;
 }
 

@@ -165,6 +165,10 @@ struct DegreeOrder {
 struct Relabeled {
   bool ready = false;
   DevBuf new_of_old, old_of_new, row, col, w;
+  // First (smallest) out-neighbour of every vertex; the vertices with
+  // out-edges are [0, nonzero).
+  DevBuf first;
+  int64_t nonzero = 0;
 };
 
 // A fixed kernel sequence captured once into an executable HIP graph and
