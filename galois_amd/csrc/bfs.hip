@@ -53,7 +53,7 @@ constexpr uint32_t kNoParent = 0xffffffffu;
 // road-like grids) have small frontiers per level and many levels: a quarter
 // of the workgroups start faster.
 constexpr int kGridNoHubs = 128;
-constexpr int kHubLanes = 256;  // lanes per step of the hub pass
+constexpr int kHubLanes = 64;  // lanes per step of the hub pass
 constexpr int kLevelsPerGraph = 4;
 constexpr int kLevelsFirst = 4;  // wide levels of the first replay: what power-law graphs need
 

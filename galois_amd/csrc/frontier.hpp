@@ -1,7 +1,7 @@
 // Load-balanced neighbour expansion shared by the frontier-driven kernels
 // (BFS, SSSP, k-core, CC hooking, BC forward).
 //
-// A workgroup of BLOCK lanes takes up to BLOCK frontier vertices (fewer when the
+// A workgroup of BLOCK lanes takes up to kBatchMax frontier vertices (fewer when the
 // frontier has fewer than that for every workgroup of the launch, see
 // batch_vertices), exclusive-scans their degrees in LDS and walks the
 // concatenated edge list with all lanes; the owning vertex of edge slot e is
@@ -39,14 +39,17 @@ constexpr int kWideStep = kWave * kWideEdges;       // most items a wavefront pu
 constexpr int kWaveQCap = 2 * kWideStep;            // items a wavefront stages
 
 // Frontier vertices a workgroup takes at a time: an equal share of the frontier
-// between kBatchMin and BLOCK.  With whole blocks a frontier of a few thousand
+// between kBatchMin and kBatchMax.  With whole blocks a frontier of a few thousand
 // vertices kept a dozen workgroups busy, each walking up to 32K edges alone
-// (BFS on 4096 vertices, 97K edges: one level 77 us).
-constexpr unsigned kBatchMin = 4;
+// (BFS on 4096 vertices, 97K edges: one level 77 us).  More than kBatchMax at a
+// time leave the last workgroups of a launch with uneven shares (directed BFS of
+// 3 M vertices 628 us with 1024, 613 with 256).
+constexpr unsigned kBatchMin = 4, kBatchMax = 256;
 template <int BLOCK>
 __device__ __forceinline__ unsigned batch_vertices(unsigned qcount) {
   const unsigned share = (qcount + gridDim.x - 1) / gridDim.x;
-  return share < kBatchMin ? kBatchMin : (share < BLOCK ? share : BLOCK);
+  constexpr unsigned most = BLOCK < kBatchMax ? BLOCK : kBatchMax;
+  return share < kBatchMin ? kBatchMin : (share < most ? share : most);
 }
 
 // Identity frontier (q null): vertex first + i for i in [0, count).
@@ -359,14 +362,12 @@ __device__ __forceinline__ unsigned long long waves_exclusive_sum(unsigned long 
   const unsigned w = threadIdx.x / kWave;
   if (lane_id() == 0) lds[w] = v;
   __syncthreads();
-  unsigned long long before = 0, all = 0;
-#pragma unroll
-  for (int i = 0; i < kW; ++i) {
-    const unsigned long long x = lds[i];
-    before += static_cast<unsigned>(i) < w ? x : 0ull;
-    all += x;
-  }
-  *total = all;
+  // A lane per wavefront: an unrolled loop over 16 words would hold them all in
+  // registers and halve the wavefronts that fit a CU.
+  const unsigned lane = lane_id();
+  const unsigned long long x = lane < kW ? lds[lane] : 0ull;
+  *total = wave_sum(x);
+  const unsigned long long before = wave_sum(lane < w ? x : 0ull);
   return before;
 }
 

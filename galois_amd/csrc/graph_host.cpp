@@ -53,11 +53,12 @@ int64_t default_relabel(int64_t n, int64_t) { return n >= (int64_t(1) << 24) ? 1
 // Hubs expanded in distance order, one distance at a time (r = 1), in the
 // relax steps whenever no near item is closer: RMAT-26 SSSP 49.7 -> 39.0 ms
 // (1.84 -> 1.10 relaxations per edge; two distances 39.8 ms).  Each extra step
-// costs about 20 us whatever the graph, a relaxation saved 1/60 ns, so on
-// smaller graphs the number of edges decides: RMAT-22 (128M edges, 2.3 -> 1.2
-// relaxations per edge) 4.87 -> 4.04 ms; RMAT-15 (0.9M edges) 0.83 -> 1.50 ms.
+// costs about 20 us whatever the graph, so on smaller graphs the number of edges
+// decides.  RMAT graphs, weights to 255: 94M edges 3.19 ms without and 3.85 with
+// it, 130M edges 4.31 and 3.77 (weights to 20: 2.58 and 2.42, to 1000: 5.9 and
+// 6.1).  The line is drawn between the two, at 7 * 2^24 edges.
 int64_t default_hub_refine(int64_t n, int64_t m) {
-  return n >= (int64_t(1) << 24) || m >= (int64_t(1) << 26) ? 1 : 0;
+  return n >= (int64_t(1) << 24) || m >= (int64_t(7) << 24) ? 1 : 0;
 }
 int64_t default_batch_width(int64_t, int64_t) { return 64; }
 int64_t default_bc_grid(int64_t, int64_t) { return 256 * 32; }

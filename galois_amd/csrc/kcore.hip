@@ -63,7 +63,7 @@ __global__ void kcore_reset_kernel(KcoreCounters* c) {
 }
 
 constexpr int kQCap = 4096;  // kcore_init_kernel
-constexpr int kHubLanes = 256;  // lanes per step of the hub pass
+constexpr int kHubLanes = 64;  // lanes per step of the hub pass
 // In the first round (every vertex below k dies at once) many decrements land
 // on the few vertices of highest degree, and atomics on one word take 12 ns
 // each, one after another; on RMAT graphs the hubs' ids are powers of two

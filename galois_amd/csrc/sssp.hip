@@ -61,6 +61,11 @@
 //    one packed word, lowers a minimum only when a read shows it would, and
 //    counts edges and items in a pair of its own (RMAT-22 5.16 -> 4.20 ms
 //    with these, the wavefronts' own queues and the hub order by edges).
+//  - Wide steps are bound by the gathers in flight: the kernels keep to 64
+//    registers, so that two workgroups share a CU, and the hub pass cuts hubs
+//    into steps of a wavefront (256 edges; most hubs of an RMAT graph have
+//    fewer than 1000), RMAT-22 4.07 -> 3.81 ms, one with 2 M vertices and all
+//    weights in one bucket 1.60 -> 1.34.
 //  - Locality: on graphs with hubs (knob frontier.relabel) the kernels run
 //    on the degree-ordered copy of the CSR (gx_graph::relab): the hubs and
 //    the vertices most often relaxed get the smallest ids, so their
@@ -94,7 +99,7 @@ constexpr uint32_t kInf = GX_DIST_INFINITY;
 // workgroups start faster and meet less at the step's counters (128: 2.88 ms on
 // a lattice of 2048 x 2048, 256: 2.57, 512: 2.72).
 constexpr int kGridNoHubs = 256;
-constexpr int kHubLanes = 256;  // lanes per step of the hub pass
+constexpr int kHubLanes = 64;  // lanes per step of the hub pass
 constexpr int kStepsPerGraph = 16;
 constexpr int kHubSelectGrid = 128;
 // Bucket merging thresholds (items per phase).  2^14 and 2^17: lattice of 2048 x
@@ -102,6 +107,12 @@ constexpr int kHubSelectGrid = 128;
 // 2^19: 2.64 ms against 2.17 and 3.8 against 4.2.
 constexpr unsigned long long kMergeLow = 1ull << 15;
 constexpr unsigned long long kMergeHigh = 1ull << 18;
+
+// A hub step's slice of distances (sssp.hub_refine) doubles when the step
+// expanded few hubs and halves when it expanded many: a step costs 20 us however
+// few hubs it has.  With weights to 60000 fixed slices of one distance took 90 ms
+// on RMAT-22, these 8 (2^8 and 2^12 to 2^14 and 2^18 within 1% of each other).
+constexpr unsigned kHubsFew = 1u << 10, kHubsMany = 1u << 14;
 
 enum Mode : unsigned { kIdle = 0, kRelax = 1, kAdvance = 2, kHubs = 3 };
 
@@ -128,6 +139,7 @@ struct SsspState {
   uint32_t hub_min;        // smallest distance a pending hub had when it was listed
   uint32_t hub_min_next;   // the same over the hubs a hub step keeps
   uint32_t hub_limit;      // a hub step expands the pending hubs at or below this distance
+  uint32_t hub_span;       // a hub step's slice of distances
   unsigned hub_step;       // this step selects and expands pending hubs
   uint32_t near_min;       // smallest distance in the near queue the step reads
   uint32_t near_min_next;  // the same for the near queue the step fills
@@ -166,7 +178,8 @@ struct Bufs {
   // sssp.hub_refine r: a hub step expands the pending hubs within
   // hub_span = 2^(r - 1) of the smallest pending hub distance; 0 = all.
   uint32_t hub_span;
-  int local_rounds;  // kLocalRounds or kLocalRoundsNoHubs
+  int local_rounds;    // kLocalRounds or kLocalRoundsNoHubs
+  unsigned local_max;  // most near items of a step with local rounds
 };
 
 __global__ void sssp_init_kernel(uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp,
@@ -183,7 +196,8 @@ __global__ void sssp_init_kernel(uint32_t* __restrict__ dist, uint32_t* __restri
 }
 
 __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint32_t* nearq0, uint32_t src,
-                                  uint32_t* dist, unsigned max_width) {
+                                  uint32_t* dist, unsigned max_width,
+                                  uint32_t hub_span) {
   for (int i = threadIdx.x; i < 2 * kWideGrid; i += blockDim.x) tally[i] = 0;
   if (threadIdx.x == 0) {
     S->dist_out = dist;
@@ -206,6 +220,7 @@ __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint3
     S->hq = 0;
     S->hub_kept = 0;
     S->hub_min = S->hub_min_next = S->hub_limit = 0xffffffffu;
+    S->hub_span = hub_span;
     S->hub_step = 0;
     S->near_min = 0;  // the source
     S->near_min_next = 0xffffffffu;
@@ -226,6 +241,10 @@ __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint3
 __device__ __forceinline__ void close_step(SsspState* S) {
   if (S->hub_step) {
     S->hq ^= 1;
+    if (S->hub_span != 0) {
+      if (S->hub_expand < kHubsFew && S->hub_span < (1u << 30)) S->hub_span *= 2;
+      else if (S->hub_expand > kHubsMany && S->hub_span > 1) S->hub_span /= 2;
+    }
     S->hub_count = S->hub_kept;  // kept hubs carry the new generation's mark
     S->hub_kept = 0;
     S->hub_expand = 0;
@@ -281,6 +300,7 @@ __global__ void __launch_bounds__(kWave) step_kernel(SsspState* S, const unsigne
   S->round += 1;
   S->app = static_cast<unsigned long long>(S->far_count[S->far_sel]) << 32;
   if (!defer) S->hub_count = 0;  // hubs of a relax step are expanded in that step
+  if (hub_span) hub_span = S->hub_span;
   const uint32_t span_limit =
       (hub_span == 0 || S->hub_min >= 0xffffffffu - hub_span) ? 0xffffffffu : S->hub_min + (hub_span - 1u);
   if (S->near_count[S->q] > 0) {
@@ -462,16 +482,12 @@ struct RelaxOp {
       s_sum[1][w] = it;
     }
     __syncthreads();
+    if (w != 0) return;
+    const unsigned i = lane_id() < kW ? lane_id() : 0u;  // a lane per wavefront
+    const uint32_t f = wave_min(s_min[0][i]), h = wave_min(s_min[1][i]), nn = wave_min(s_min[2][i]);
+    const unsigned long long e = wave_sum(lane_id() < kW ? s_sum[0][i] : 0ull),
+                             t = wave_sum(lane_id() < kW ? s_sum[1][i] : 0ull);
     if (threadIdx.x == 0) {
-      uint32_t f = 0xffffffffu, h = 0xffffffffu, nn = 0xffffffffu;
-      unsigned long long e = 0, t = 0;
-      for (int i = 0; i < kW; ++i) {
-        f = min(f, s_min[0][i]);
-        h = min(h, s_min[1][i]);
-        nn = min(nn, s_min[2][i]);
-        e += s_sum[0][i];
-        t += s_sum[1][i];
-      }
       if (f != 0xffffffffu) lower(&B.S->far_min, f);
       if (h != 0xffffffffu) lower(&B.S->hub_min, h);
       if (nn != 0xffffffffu && B.hub_span) lower(&B.S->near_min_next, nn);  // read only with hub slices
@@ -523,13 +539,20 @@ __device__ __forceinline__ void relax_step(const Bufs& B, Stage& sn, Stage& sf) 
 // listed twice is expanded once, at the smaller.  Rounds run ahead of what
 // other workgroups find, which costs some expansions at distances that are not
 // final yet.
+// On graphs with hubs, whose shorter paths local rounds run ahead of, only the
+// smallest steps of small graphs have them: unit weights in wide buckets,
+// 4096 vertices 258 -> 245 us with up to 2048 items (328 with three rounds),
+// 1 M vertices 699 -> 729; weights to 255, 4096 vertices 652 -> 414 us, 100,000
+// 1012 -> 974.
+constexpr unsigned kLocalMaxHubs = 1u << 11;
+constexpr int64_t kLocalHubEdges = int64_t(1) << 22;
 constexpr unsigned kLocalMax = 1u << 16;  // near items: at most one batch per workgroup
 // Rounds: a lattice of 2048 x 2048 takes 3.54 ms with one, 2.84 with 2, 2.87
-// with 8, 3.10 with 16, one of 300,000 vertices 1.52, 0.96, 0.59 and 0.56; RMAT
-// graphs run ahead for less (4096 vertices 640 us with one, 416 with 2, 464
-// with 8).
-constexpr int kLocalRounds = 3, kLocalRoundsNoHubs = 8;
+// with 8, 3.10 with 16, one of 300,000 vertices 1.52, 0.96, 0.59 and 0.56.
+constexpr int kLocalRounds = 2, kLocalRoundsNoHubs = 8;
 constexpr int kLocalEdges = 2;
+
+static_assert(kLocalMax <= kGridNoHubs * kWideBlock && kLocalMaxHubs <= kWideGrid * kWideBlock, "one batch each");
 
 // Lists of the workgroup, in the space of the near stage (used by then).
 struct LocalLists {
@@ -564,7 +587,7 @@ __device__ __forceinline__ void relax_local(const Bufs& B, Stage& sn, Stage& sf)
       if (p < B.cap) nout[p] = v; else atomicOr(&S->overflow, 1u);
     }
   };
-  const unsigned per = batch_vertices<kWideBlock>(qcount);
+  const unsigned per = max(kBatchMin, (qcount + gridDim.x - 1) / gridDim.x);  // at most a vertex a lane (kLocalMax)
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * per;
   unsigned count = base < qcount ? min(per, static_cast<unsigned>(qcount - base)) : 0u;
   int cur = 0;
@@ -737,11 +760,12 @@ __device__ __forceinline__ void far_split_step(const Bufs& B, Stage& sn, Stage& 
     s_min[1][threadIdx.x / kWave] = near_min;
   }
   __syncthreads();
+  if (threadIdx.x < kWave) {
+    const unsigned i = lane_id() < kW ? lane_id() : 0u;
+    kept_min = wave_min(s_min[0][i]);
+    near_min = wave_min(s_min[1][i]);
+  }
   if (threadIdx.x == 0) {
-    for (int i = 1; i < kW; ++i) {
-      kept_min = min(kept_min, s_min[0][i]);
-      near_min = min(near_min, s_min[1][i]);
-    }
     if (kept_min != 0xffffffffu) lower(&S->far_min, kept_min);
     if (near_min != 0xffffffffu && B.hub_span) lower(&S->near_min_next, near_min);
   }
@@ -794,24 +818,35 @@ __global__ void __launch_bounds__(kWideBlock) hub_select_kernel(Bufs B) {
 }
 
 // The work of a step: a relax or an advance (the step's mode picks one; the
-// two never share a step, so one launch serves both).
-__global__ void __launch_bounds__(kWideBlock) work_kernel(Bufs B) {
+// two never share a step, so one launch serves both).  LOCAL: with local rounds
+// (see local_max); left out elsewhere, where they would cost the wide steps
+// half of the wavefronts a CU holds (78 registers against 64).
+template <bool LOCAL>
+__global__ void __launch_bounds__(kWideBlock, LOCAL ? 4 : 8) work_kernel(Bufs B) {
   const unsigned mode = B.S->mode;
   if (mode != kRelax && mode != kAdvance) return;
   __shared__ Stage s0, s1;
-  if (mode == kRelax && !B.defer && B.S->near_count[B.S->q] <= kLocalMax)
-    relax_local(B, s0, s1);
-  else if (mode == kRelax)
-    relax_step(B, s0, s1);
-  else
+  if (mode == kAdvance) {
     far_split_step(B, s0, s1);
+    return;
+  }
+  if constexpr (LOCAL) {
+    if (B.S->near_count[B.S->q] <= B.local_max) {
+      relax_local(B, s0, s1);
+      return;
+    }
+  }
+  relax_step(B, s0, s1);
 }
 
 // `hubs` false: no vertex exceeds the hub threshold, so the hub list stays
 // empty and its two launches are left out of the step.
 void enqueue_step(const Bufs& B, bool hubs, hipStream_t s) {
   step_kernel<<<1, kWave, 0, s>>>(B.S, hubs ? nullptr : B.tally, B.defer, B.hub_span);
-  work_kernel<<<hubs ? kWideGrid : kGridNoHubs, kWideBlock, 0, s>>>(B);
+  if (B.local_max > 0)
+    work_kernel<true><<<hubs ? kWideGrid : kGridNoHubs, kWideBlock, 0, s>>>(B);
+  else
+    work_kernel<false><<<hubs ? kWideGrid : kGridNoHubs, kWideBlock, 0, s>>>(B);
   if (hubs) {
     if (B.defer) hub_select_kernel<<<kHubSelectGrid, kWideBlock, 0, s>>>(B);
     launch_hub_offsets<kHubLanes * kWideEdges>(B.row, B.defer ? B.hubx : B.hubq[0], B.defer ? &B.S->hub_expand : &B.S->hub_count,
@@ -854,10 +889,17 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   B.cap = cap;
   B.hub_off = g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(cap));
   B.hub = hub_degree();
-  const int64_t refine = tune_effective("sssp.hub_refine", n, g->m);
+  int64_t refine = tune_effective("sssp.hub_refine", n, g->m);
+  // Wide buckets hold many slices of a weight range, and each slice is a step:
+  // RMAT-22 with 2^13 and weights to 1000 5.8 ms without slices and 8.1 with
+  // them, to 255 4.2 and 4.2, to 20 2.6 and 2.4 (2^6 and 2^8, to 255: 4.3 and
+  // 3.8).  The default leaves them out there; on the largest graphs they pay
+  // whatever the buckets.
+  if (!tune_is_set("sssp.hub_refine") && n < (int64_t(1) << 24) && shift > 8) refine = 0;
   B.defer = static_cast<uint32_t>(tune_effective("sssp.defer_hubs", n, g->m)) | (refine > 0 ? 1u : 0u);
   B.hub_span = refine > 0 ? 1u << std::min<int64_t>(refine - 1, 31) : 0u;
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
+  B.local_max = !hubs ? kLocalMax : g->m < kLocalHubEdges && !B.defer ? kLocalMaxHubs : 0u;
   B.local_rounds = hubs ? kLocalRounds : kLocalRoundsNoHubs;
   // Graphs with hubs run on the degree-ordered copy (frontier.relabel).
   const bool relabel = hubs && tune_effective("frontier.relabel", n, g->m) != 0;
@@ -878,7 +920,7 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   sssp_init_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(B.dist, B.stamp, B.done, B.hubmark, n,
                                                                  run_src);
   GX_LAUNCHED("sssp_init_kernel");
-  sssp_reset_kernel<<<1, kBlock, 0, s>>>(B.S, B.tally, B.nearq[0], run_src, B.dist, max_width);
+  sssp_reset_kernel<<<1, kBlock, 0, s>>>(B.S, B.tally, B.nearq[0], run_src, B.dist, max_width, B.hub_span);
   GX_LAUNCHED("sssp_reset_kernel");
   uint64_t key = 0;
   for (const void* p : {(const void*)B.row, (const void*)B.col, (const void*)B.w,
