@@ -240,8 +240,22 @@ __global__ void __launch_bounds__(kBlock) split_copy_kernel(const int32_t* __res
   }
 }
 
-// Fixed-order reduction of the per-workgroup partials; sets the next base,
-// the convergence flag and the buffer index of the newest iterate.
+// End of an iteration, given its sums: the next base, the convergence flag and
+// the buffer index of the newest iterate.
+struct PrClose {
+  PrState* state;
+  unsigned newest_buf;
+  __device__ __forceinline__ void operator()(double r, double d) const {
+    state->resid = r;
+    state->dang = d;
+    state->base = (1.0 - state->alpha) * state->inv_n + state->alpha * d * state->inv_n;
+    state->iters += 1;
+    state->final_buf = newest_buf;
+    if (r < state->tol || state->iters >= state->max_iter) state->converged = 1;
+  }
+};
+
+// Fixed-order reduction of the per-workgroup partials.
 __global__ void __launch_bounds__(kBlock) pr_reduce_kernel(PrState* state, const double* __restrict__ part_resid,
                                                            const double* __restrict__ part_dang, int nparts,
                                                            unsigned newest_buf) {
@@ -254,14 +268,7 @@ __global__ void __launch_bounds__(kBlock) pr_reduce_kernel(PrState* state, const
   }
   r = block_sum(r, red);
   d = block_sum(d, red);
-  if (threadIdx.x == 0) {
-    state->resid = r;
-    state->dang = d;
-    state->base = (1.0 - state->alpha) * state->inv_n + state->alpha * d * state->inv_n;
-    state->iters += 1;
-    state->final_buf = newest_buf;
-    if (r < state->tol || state->iters >= state->max_iter) state->converged = 1;
-  }
+  if (threadIdx.x == 0) PrClose{state, newest_buf}(r, d);
 }
 
 // x0 = 1/n, y0 = x0/outdeg; dangling partials.
@@ -499,11 +506,14 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
                                nullptr);
         launches += 2;
       }
-      const int np = rs::launch_sweep<Real>(P, src, fin, &state->converged, part_resid, part_dang, carry, s, nullptr);
+      const int np = rs::launch_sweep<Real>(P, src, fin, &state->converged, part_resid, part_dang, carry, s, nullptr,
+                                            PrClose{state, static_cast<unsigned>(nxt)});
       ktimer.end();
-      pr_reduce_kernel<<<1, kBlock, 0, s>>>(state, part_resid, part_dang, np, static_cast<unsigned>(nxt));
-      GX_LAUNCHED("pr_reduce_kernel");
-      launches += 3;
+      if (np > 0) {
+        pr_reduce_kernel<<<1, kBlock, 0, s>>>(state, part_resid, part_dang, np, static_cast<unsigned>(nxt));
+        GX_LAUNCHED("pr_reduce_kernel");
+      }
+      launches += np > 0 ? 3 : 2;
       cur = nxt;
     }
     GX_HIP(hipMemcpyAsync(host, state, sizeof(PrState), hipMemcpyDeviceToHost, s));

@@ -165,7 +165,22 @@ struct AdjFin {
   }
 };
 
-// mode 0 (forward): base = alpha*acc/n.  mode 1 (adjoint): base = acc/n.
+// End of an iteration, given its sums.  mode 0 (forward): base = alpha*acc/n.
+// mode 1 (adjoint): base = acc/n.
+struct AdClose {
+  AdState* state;
+  int mode;
+  unsigned newest_buf;
+  __device__ __forceinline__ void operator()(double r, double a) const {
+    state->resid = r;
+    state->acc = a;
+    state->base = (mode == 0 ? state->alpha : 1.0) * a * state->inv_n;
+    state->iters += 1;
+    state->final_buf = newest_buf;
+    if (r < state->tol || state->iters >= state->max_iter) state->converged = 1;
+  }
+};
+
 __global__ void __launch_bounds__(kBlock) ad_reduce_kernel(AdState* state, const double* __restrict__ p0,
                                                            const double* __restrict__ p1, int nparts, int mode,
                                                            unsigned newest_buf) {
@@ -178,14 +193,7 @@ __global__ void __launch_bounds__(kBlock) ad_reduce_kernel(AdState* state, const
   }
   r = block_sum(r, red);
   a = block_sum(a, red);
-  if (threadIdx.x == 0) {
-    state->resid = r;
-    state->acc = a;
-    state->base = (mode == 0 ? state->alpha : 1.0) * a * state->inv_n;
-    state->iters += 1;
-    state->final_buf = newest_buf;
-    if (r < state->tol || state->iters >= state->max_iter) state->converged = 1;
-  }
+  if (threadIdx.x == 0) AdClose{state, mode, newest_buf}(r, a);
 }
 
 __global__ void ad_state_init_kernel(AdState* s, double alpha, double tol, double inv_n, unsigned max_iter) {
@@ -310,9 +318,11 @@ uint32_t iterate(gx_graph* g, AdState* state, AdState* host, double* p0, double*
     for (; it < end; ++it) {
       const int nxt = cur ^ 1;
       const int np = sweep(cur, nxt);
-      ad_reduce_kernel<<<1, kBlock, 0, s>>>(state, p0, p1, np, mode, static_cast<unsigned>(nxt));
-      GX_LAUNCHED("ad_reduce_kernel");
-      launches += 3;
+      if (np > 0) {  // else the sweep has closed the iteration
+        ad_reduce_kernel<<<1, kBlock, 0, s>>>(state, p0, p1, np, mode, static_cast<unsigned>(nxt));
+        GX_LAUNCHED("ad_reduce_kernel");
+      }
+      launches += np > 0 ? 3 : 2;
       cur = nxt;
     }
     GX_HIP(hipMemcpyAsync(host, state, sizeof(AdState), hipMemcpyDeviceToHost, s));
@@ -370,8 +380,8 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
       return np;
     }
     WSrc<Real> src{ys[cur], wt};
-    return rs::launch_sweep<Real>(P, src, fin, &state->converged, parts, parts + nparts, carry, s,
-                                  &ktimer);
+    return rs::launch_sweep<Real>(P, src, fin, &state->converged, parts, parts + nparts, carry, s, &ktimer,
+                                  AdClose{state, 0, static_cast<unsigned>(nxt)});
   };
   const uint32_t iters = iterate(g, state, host, parts, parts + nparts, 0, max_iter, sweep, launches);
   GX_HIP(hipMemcpyAsync(x, xs[host->final_buf], n * sizeof(Real), hipMemcpyDeviceToDevice, s));
@@ -425,24 +435,25 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   ad_init_reduce_kernel<<<1, kBlock, 0, s>>>(state, parts, kSweepGrid, 1);
   GX_LAUNCHED("adjoint init");
   // One sweep over the vector lv, timed when it iterates.
-  auto sums = [&](const Real* lv, const AdjFin<Real>& fin, const unsigned* skip, KernelTimer* timer) {
+  auto sums = [&](const Real* lv, const AdjFin<Real>& fin, const unsigned* skip, KernelTimer* timer,
+                  const auto& close) {
     if (blocked) {
       if (timer) timer->begin();
       const int np = bs::launch<Real>(L, wl, lv, n, partial, fin, skip, parts, parts + nparts, s);
       if (timer) timer->end();
       return np;
     }
-    return rs::launch_sweep<Real>(P, WSrc<Real>{lv, wr}, fin, skip, parts, parts + nparts, carry, s, timer);
+    return rs::launch_sweep<Real>(P, WSrc<Real>{lv, wr}, fin, skip, parts, parts + nparts, carry, s, timer, close);
   };
   auto sweep = [&](int cur, int nxt) {
     return sums(lam[cur], AdjFin<Real>{state, c, inv_s, lam[cur], lam[nxt], pl, 0, Real(0), Real(0)},
-                &state->converged, &ktimer);
+                &state->converged, &ktimer, AdClose{state, 1, static_cast<unsigned>(nxt)});
   };
   const uint32_t iters = iterate(g, state, host, parts, parts + nparts, 1, max_iter, sweep, launches);
   const Real* lam_f = lam[host->final_buf];
   // (P lambda) at the converged lambda: one more sweep with final_pass set.
   // Its dangling value is sum(lambda)/n, which the last reduce stored in base.
-  sums(lam_f, AdjFin<Real>{state, c, inv_s, lam_f, nullptr, pl, 1, Real(0), Real(0)}, nullptr, nullptr);
+  sums(lam_f, AdjFin<Real>{state, c, inv_s, lam_f, nullptr, pl, 1, Real(0), Real(0)}, nullptr, nullptr, rs::NoClose{});
   launches += 2;
   zero_u32_kernel<<<1, 64, 0, s>>>(hubc, 2);
   GradOp<Real> op{g->col, x, lam_f, pl, inv_s, grad_w, static_cast<Real>(alpha)};

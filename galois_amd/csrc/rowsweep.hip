@@ -63,9 +63,24 @@ __global__ void lane_info_kernel(const int32_t* __restrict__ rowoff, const uint3
   }
 }
 
+// Per chunk: the row that began in an earlier chunk and ends in this one
+// (kNoRow: none), and the chunk it began in.
+__global__ void spans_kernel(RowPlan P, uint32_t* __restrict__ row, uint32_t* __restrict__ first) {
+  const int64_t chunk_edges = static_cast<int64_t>(P.kt) * kTile;
+  for (int64_t c = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; c < P.nchunks;
+       c += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const uint32_t r = P.rid[P.tile_row[c * P.kt]];
+    const int32_t rb = P.rowoff[r], re = P.rowoff[r + 1];
+    const bool spans = rb < c * chunk_edges && re <= (c + 1) * chunk_edges;
+    row[c] = spans ? r : kNoRow;
+    first[c] = static_cast<uint32_t>(rb / chunk_edges);
+  }
+}
+
 }  // namespace
 
-// Layout of cache.buf (words): rid[n] | tile_row[ntiles + 1] | lane_info[64 * ntiles].
+// Layout of cache.buf (words): rid[n] | tile_row[ntiles + 1] |
+// lane_info[64 * ntiles] | span_row[nchunks] | span_first[nchunks].
 RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64_t n, int64_t m, PullPlan& cache) {
   GX_REQUIRE(n > 0, "row sweep over an empty graph");
   const int64_t ntiles = (m + kTile - 1) / kTile;
@@ -82,11 +97,14 @@ RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64
     P.ntiles = ntiles;
     P.kt = tiles_per_chunk(ntiles);
     P.nchunks = (ntiles + P.kt - 1) / P.kt;
+    P.span_row = P.lane_info + ntiles * kWave;
+    P.span_first = P.span_row + P.nchunks;
     return P;
   };
   if (cache.ready) return view();
   hipStream_t s = g->stream;
-  cache.buf.ensure((n + ntiles + 1 + ntiles * kWave) * sizeof(uint32_t));
+  const int64_t nchunks = view().nchunks;
+  cache.buf.ensure((n + ntiles + 1 + ntiles * kWave + 2 * nchunks) * sizeof(uint32_t));
   uint32_t* rid = cache.buf.as<uint32_t>();
   uint32_t* tile_row = rid + n;
   DevBuf pos;
@@ -105,6 +123,9 @@ RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64
     lane_info_kernel<<<grid_for(ntiles * kWave, kBlock, 16384), kBlock, 0, s>>>(rowoff, rid, full, m, ntiles, tile_row,
                                                                                 tile_row + ntiles + 1);
     GX_LAUNCHED("lane_info_kernel");
+    uint32_t* span_row = tile_row + ntiles + 1 + ntiles * kWave;
+    spans_kernel<<<grid_for(nchunks, kBlock, 8192), kBlock, 0, s>>>(view(), span_row, span_row + nchunks);
+    GX_LAUNCHED("spans_kernel");
   }
   GX_HIP(hipStreamSynchronize(s));
   cache.ready = true;
