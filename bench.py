@@ -711,7 +711,7 @@ def main() -> int:
         "data": "synthetic",
         "config": {"workload": f"pagerank_fp32_rmat{args.scale}_directed", "n": n, "m": m,
                    "edge_factor": 16, "alpha": 0.85, "tol": 1e-9, "max_iter": 100, "seed": SEED,
-                   "sweep": "propagation_blocked" if blocked else "merge_path_pull",
+                   "sweep": "propagation_blocked" if blocked else "row_sweep_pull",
                    "knobs": {k: {"set": gx.tune_get(k), "effective": gx.tune_effective(k, n, m)}
                              for k in ("pr.blocking", "pr.hot_sources", "pr.task_edges", "frontier.hub_degree",
                                        "bfs.visited_bitmap", "sssp.max_merge", "sssp.defer_hubs", "sssp.hub_refine", "bc.chunk",

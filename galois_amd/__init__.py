@@ -336,7 +336,8 @@ def kcore(g: Graph, k: int):
 
 def pagerank(g: Graph, alpha: float = 0.85, tol: float = 1e-9, max_iter: int = 100, precision: str = "fp32"):
     """Normalised pull PageRank; precision 'fp32' or 'fp64'.  FP32 row sums are exact 64-bit fixed-point
-    sums in the default propagation-blocked sweep; the merge-path pull (pr.blocking = 0) uses Kahan sums.
+    sums in the default propagation-blocked sweep; the pull (pr.blocking = 0, and by default graphs of
+    fewer than 2^21 edges) sums in FP64.
     Returns (pr, Stats)."""
     torch = _torch()
     fp64 = precision == "fp64"

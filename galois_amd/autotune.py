@@ -14,7 +14,7 @@ knobs respond to (hub count, gathered working set).
 Knobs and candidates:
   frontier.hub_degree  degree above which a frontier vertex is expanded by the
                        whole grid (BFS, SSSP, CC, k-core, BC)
-  pr.blocking          FP32 PageRank: propagation-blocked sweep (1) or merge-path pull (0);
+  pr.blocking          FP32 PageRank: propagation-blocked sweep (1) or pull (0);
                        2 also sends FP64 through the blocked sweep (not a
                        candidate: it changes FP64 results in the last bit)
   pr.hot_sources       sources of the first PageRank pull pass (0 = one pass)
@@ -82,8 +82,8 @@ def signature(gx, G, algo: str, args: dict | None = None) -> str:
 def _applies(knob: str, algo: str, args: dict, choice: dict) -> bool:
     """Whether the kernel that runs responds to `knob`, given the choices made
     so far.  PageRank: pr.blocking candidates (1, 0) differ only for FP32 (FP64
-    takes the merge-path pull under both); pr.hot_sources splits the
-    merge-path pull only, so it is not timed while the blocked sweep runs."""
+    takes the pull under both); pr.hot_sources splits the
+    pull only, so it is not timed while the blocked sweep runs."""
     if algo != "pagerank":
         return True
     fp64 = args.get("precision", "fp32") == "fp64"

@@ -120,25 +120,6 @@ __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e) {
   e = (a - (s - bb)) + (b - bb);
 }
 
-// Compensated (Kahan-Babuska / Neumaier) accumulator in FP32.
-struct KahanF32 {
-  float s = 0.f, c = 0.f;
-  __device__ __forceinline__ void add(float x) {
-    float t = s + x;
-    if (fabsf(s) >= fabsf(x))
-      c += (s - t) + x;
-    else
-      c += (x - t) + s;
-    s = t;
-  }
-  // Merge another accumulator.
-  __device__ __forceinline__ void merge(float os, float oc) {
-    add(os);
-    c += oc;
-  }
-  __device__ __forceinline__ float value() const { return s + c; }
-};
-
 // ---------------------------------------------------------- hashing (PRNG)
 // splitmix64 finaliser; the generators draw every random number as
 // mix64(seed ^ f(counter)) so results depend only on (seed, counter).

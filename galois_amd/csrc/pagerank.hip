@@ -18,7 +18,7 @@
 // default (knob "pr.blocking"): per-edge contributions streamed through a
 // static (source chunk, destination bin) layout and exact fixed-point row
 // sums, instead of a random gather per edge.  FP64 iterations and
-// pr.blocking = 0 use the merge-path pull sweep below.
+// pr.blocking = 0 use the pull sweep below, and so do small FP32 graphs.
 //
 // Design of the pull sweep (gfx950, HBM/latency bound, no MFMA)
 //  - The pull runs over the transpose in degree order (vertices relabelled

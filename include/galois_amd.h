@@ -327,11 +327,10 @@ gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t* alive,
  * precision: 0 = FP32 ranks, 1 = FP64 ranks.  FP32 runs by default
  * through the propagation-blocked sweep, whose row sums are exact (every
  * contribution rounded to 64-bit fixed point with resolution 2^-62 and
- * summed with integer atomics, so the sum is order independent and more
- * accurate than a compensated FP32 sum), and x' = base + alpha*sum is
- * evaluated in FP32 with error-free transformations; with the knob
- * "pr.blocking" = 0 it runs the merge-path pull with Kahan-compensated FP32
- * row sums.  In both, the residual and the dangling mass D are reduced in
+ * summed with integer atomics, so the sum is order independent), and x' =
+ * base + alpha*sum is evaluated in FP32 with error-free transformations; with
+ * the knob "pr.blocking" = 0, and while it is not set on graphs of fewer than
+ * 2^21 edges, it runs the pull with FP64 row sums and the same update.  In both, the residual and the dangling mass D are reduced in
  * FP64 (more accurate than an FP32 reduction and read once per iteration).
  * pr: device float[n] (precision 0) or double[n] (precision 1).
  * Replaces computePRTopological (PageRank-pull.cpp:196-251) with the
