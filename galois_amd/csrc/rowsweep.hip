@@ -84,6 +84,8 @@ __global__ void spans_kernel(RowPlan P, uint32_t* __restrict__ row, uint32_t* __
 RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64_t n, int64_t m, PullPlan& cache) {
   GX_REQUIRE(n > 0, "row sweep over an empty graph");
   const int64_t ntiles = (m + kTile - 1) / kTile;
+  const int kt = tiles_per_chunk(ntiles);
+  const int64_t nchunks = (ntiles + kt - 1) / kt;
   auto view = [&]() {
     RowPlan P{};
     P.rowoff = rowoff;
@@ -95,15 +97,14 @@ RowPlan build_plan(gx_graph* g, const int32_t* rowoff, const int32_t* col, int64
     P.tile_row = P.rid + n;
     P.lane_info = P.tile_row + ntiles + 1;
     P.ntiles = ntiles;
-    P.kt = tiles_per_chunk(ntiles);
-    P.nchunks = (ntiles + P.kt - 1) / P.kt;
+    P.kt = kt;
+    P.nchunks = nchunks;
     P.span_row = P.lane_info + ntiles * kWave;
-    P.span_first = P.span_row + P.nchunks;
+    P.span_first = P.span_row + nchunks;
     return P;
   };
   if (cache.ready) return view();
   hipStream_t s = g->stream;
-  const int64_t nchunks = view().nchunks;
   cache.buf.ensure((n + ntiles + 1 + ntiles * kWave + 2 * nchunks) * sizeof(uint32_t));
   uint32_t* rid = cache.buf.as<uint32_t>();
   uint32_t* tile_row = rid + n;
