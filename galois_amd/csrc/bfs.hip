@@ -99,6 +99,7 @@ struct Bufs {
   int64_t nonzero;
   uint64_t pull_min;    // fewest edges out of a frontier that is pulled
   uint64_t narrow_max;  // most edges out of a frontier that a narrow level takes
+  unsigned batch;       // most vertices a workgroup takes at a time
 };
 
 // Levels, parents and the visited bitmap of a search that has found its source,
@@ -351,7 +352,8 @@ __global__ void __launch_bounds__(kWideBlock) td_expand_kernel(Bufs B) {
   }
   __shared__ uint32_t stage[kWideWaves][kWaveQCap];
   TdOp op = make_td(B, stage);
-  expand_queue<kWideBlock, TdOp, false, kWideEdges>(B.row, B.q[S->q], S->count[S->q], B.hub, B.hubq, &S->hub_count, B.cap, &S->overflow, op);
+  expand_queue<kWideBlock, TdOp, false, kWideEdges>(B.row, B.q[S->q], S->count[S->q], B.hub, B.hubq, &S->hub_count, B.cap, &S->overflow, op, 0,
+                                                    B.batch);
   op.finish();
 }
 
@@ -648,9 +650,12 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
   uint32_t* vis = use_vis ? g->scratch<uint32_t>(WS_BITMAP0, words) : nullptr;
   Bufs B{g->row, g->col, level, nullptr, {g->scratch<uint32_t>(WS_Q0, n), g->scratch<uint32_t>(WS_Q1, n)},
          g->scratch<uint32_t>(WS_Q2, n), g->scratch<BfsState>(WS_COUNTERS, 1), cap,
-         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), vis, nullptr, n, g->m, nullptr, n, ~uint64_t(0), kNarrowEdgesNoHubs};
+         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), vis, nullptr, n, g->m, nullptr, n, ~uint64_t(0), kNarrowEdgesNoHubs, kWideBlock};
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
-  if (hubs) B.narrow_max = kNarrowEdges;
+  if (hubs) {
+    B.narrow_max = kNarrowEdges;
+    B.batch = kBatchMax;
+  }
   // Symmetric graphs with hubs pull their heavy levels (level_begin).
   if (hubs && (g->flags & GX_GRAPH_SYMMETRIC)) {
     B.front = g->scratch<uint64_t>(WS_BITMAP1, (n + 63) / 64);
@@ -743,11 +748,14 @@ extern "C" gx_status gx_bfs_do(gx_graph* g, uint32_t src, uint32_t alpha, uint32
   const unsigned cap = static_cast<unsigned>(n);
   Bufs B{g->row, g->col, level, parent, {g->scratch<uint32_t>(WS_Q0, n), g->scratch<uint32_t>(WS_Q1, n)},
          g->scratch<uint32_t>(WS_Q2, n), g->scratch<BfsState>(WS_COUNTERS, 1), cap,
-         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), nullptr, nullptr, n, g->m, nullptr, n, ~uint64_t(0), kNarrowEdgesNoHubs};
+         g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(n)), hub_degree(), nullptr, nullptr, n, g->m, nullptr, n, ~uint64_t(0), kNarrowEdgesNoHubs, kWideBlock};
   const int64_t words = (n + 31) / 32;
   uint32_t* bm[2] = {g->scratch<uint32_t>(WS_BITMAP0, words), g->scratch<uint32_t>(WS_BITMAP1, words)};
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
-  if (hubs) B.narrow_max = kNarrowEdges;
+  if (hubs) {
+    B.narrow_max = kNarrowEdges;
+    B.batch = kBatchMax;
+  }
   // Symmetric graphs with hubs run on the degree-ordered copy of the CSR
   // (frontier.relabel): a bottom-up step scans each unvisited vertex's
   // neighbours hubs first, and the hubs are the first vertices reached, so

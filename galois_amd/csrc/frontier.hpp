@@ -1,7 +1,7 @@
 // Load-balanced neighbour expansion shared by the frontier-driven kernels
 // (BFS, SSSP, k-core, CC hooking, BC forward).
 //
-// A workgroup of BLOCK lanes takes up to kBatchMax frontier vertices (fewer when the
+// A workgroup of BLOCK lanes takes up to `most` frontier vertices (fewer when the
 // frontier has fewer than that for every workgroup of the launch, see
 // batch_vertices), exclusive-scans their degrees in LDS and walks the
 // concatenated edge list with all lanes; the owning vertex of edge slot e is
@@ -39,16 +39,18 @@ constexpr int kWideStep = kWave * kWideEdges;       // most items a wavefront pu
 constexpr int kWaveQCap = 2 * kWideStep;            // items a wavefront stages
 
 // Frontier vertices a workgroup takes at a time: an equal share of the frontier
-// between kBatchMin and kBatchMax.  With whole blocks a frontier of a few thousand
+// between kBatchMin and `most`.  With whole blocks a frontier of a few thousand
 // vertices kept a dozen workgroups busy, each walking up to 32K edges alone
 // (BFS on 4096 vertices, 97K edges: one level 77 us).  More than kBatchMax at a
 // time leave the last workgroups of a launch with uneven shares (directed BFS of
-// 3 M vertices 628 us with 1024, 613 with 256).
+// 3 M vertices 628 us with 1024, 613 with 256).  Graphs without hubs take up to
+// BLOCK: their edges are few and alike (`most`; k-core of a 2048 x 2048 lattice,
+// all vertices at once, 271 us with 256, 209 with 1024).
 constexpr unsigned kBatchMin = 4, kBatchMax = 256;
 template <int BLOCK>
-__device__ __forceinline__ unsigned batch_vertices(unsigned qcount) {
+__device__ __forceinline__ unsigned batch_vertices(unsigned qcount, unsigned most) {
   const unsigned share = (qcount + gridDim.x - 1) / gridDim.x;
-  constexpr unsigned most = BLOCK < kBatchMax ? BLOCK : kBatchMax;
+  if (most > BLOCK) most = BLOCK;
   return share < kBatchMin ? kBatchMin : (share < most ? share : most);
 }
 
@@ -59,14 +61,14 @@ template <int BLOCK, class Op, bool ADMIT = false, int U = 1>
 __device__ __forceinline__ void expand_queue(const int32_t* __restrict__ row, const uint32_t* __restrict__ q,
                                              unsigned qcount, uint32_t hub_thresh, uint32_t* __restrict__ hubq,
                                              unsigned* hub_count, unsigned cap, unsigned* overflow, Op& op,
-                                             uint32_t first = 0) {
+                                             uint32_t first = 0, unsigned most = kBatchMax) {
   __shared__ int32_t s_start[BLOCK];
   __shared__ uint32_t s_off[BLOCK];
   __shared__ uint32_t s_src[BLOCK];
   __shared__ uint64_t s_scan[BLOCK / kWave + 1];
   __shared__ unsigned s_hub_base;
   const unsigned tid = threadIdx.x;
-  const unsigned per = batch_vertices<BLOCK>(qcount);
+  const unsigned per = batch_vertices<BLOCK>(qcount, most);
   for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * per; base < qcount;
        base += static_cast<uint64_t>(gridDim.x) * per) {
     const unsigned i = static_cast<unsigned>(base) + tid;
@@ -118,10 +120,17 @@ __device__ __forceinline__ void expand_queue(const int32_t* __restrict__ row, co
         u[k] = 0;
         edge[k] = 0;
         if (valid[k]) {
-          int lo = 0, hi = static_cast<int>(per) - 1;
-          while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (s_off[mid] <= e) lo = mid; else hi = mid - 1;
+          int lo = 0;
+          if constexpr (BLOCK <= 256) {  // unrolled; lanes without a vertex hold the total, which is above e
+#pragma unroll
+            for (int step = BLOCK / 2; step > 0; step >>= 1)
+              if (s_off[lo + step] <= e) lo += step;
+          } else {
+            int hi = static_cast<int>(per) - 1;
+            while (lo < hi) {
+              const int mid = (lo + hi + 1) >> 1;
+              if (s_off[mid] <= e) lo = mid; else hi = mid - 1;
+            }
           }
           u[k] = s_src[lo];
           edge[k] = s_start[lo] + static_cast<int32_t>(e - s_off[lo]);

@@ -82,10 +82,14 @@ constexpr int kHotBits = 11;  // table slots: at most a quarter in use
 constexpr int kHotProbe = 4;  // a vertex that finds no slot among these is not counted
 constexpr uint32_t kNoVertex = 0xffffffffu;
 
+// On the degree-ordered copy the hottest vertices are the first ids: every word
+// of the table then is the counter of its own index (RMAT-26, k = 10, with the
+// words in order: 3.2 ms, with the list and permuted words 4.27).
 struct HotTable {
   uint32_t id[1 << kHotBits];
   uint32_t count[1 << kHotBits];
 };
+constexpr uint32_t kFirstHot = 2u << kHotBits;
 __device__ __forceinline__ uint32_t hot_slot(uint32_t v, int probe) {
   return (((v * 2654435769u) >> (32 - kHotBits)) + probe) & ((1u << kHotBits) - 1);
 }
@@ -96,12 +100,14 @@ struct KcoreState {
 };
 
 // Atomics on one cache line queue up as those on one word do.  Neighbouring ids
-// are often alike (ids of RMAT graphs with few set bits are hubs, a relabelled
-// graph has its hubs at the front), so with hubs the degree words are
+// are often alike (ids of RMAT graphs with few set bits are hubs), so with hubs the degree words are
 // permuted within pages of kPage words: 4.4 M decrements of an RMAT
 // distribution over 2^22 words take 499 us in id order, 225 us permuted
 // (uniform ones 168 us).  Pages keep the passes over all vertices sequential.
-// A graph without hubs keeps its order (and the lines its neighbours share).
+// A graph without hubs keeps its order (and the lines its neighbours share), and
+// so does the degree-ordered copy, whose hottest ids are all counted in LDS and
+// whose degrees are read back in runs of neighbouring words (RMAT-26: the last
+// pass 534 us, permuted 1020, the peel 2.47 ms either way).
 constexpr uint32_t kPage = 4096;
 constexpr uint32_t kPageMul = 1597;  // odd: a permutation of the page
 __device__ __forceinline__ uint32_t degree_pos(uint32_t v, uint32_t mul) {
@@ -155,9 +161,14 @@ struct PeelOp {
   uint32_t hub;   // frontier.hub_degree
   uint32_t mul;   // degree_pos
   HotTable* hot;  // nullptr: every decrement goes to the degree word
+  bool first_hot;
   // Whether v has a counter, which then takes its decrement.
   __device__ __forceinline__ bool count_hot(uint32_t v) {
     if (!hot) return false;
+    if (first_hot) {
+      if (v < kFirstHot) atomicAdd(&hot->id[0] + v, 1u);
+      return v < kFirstHot;
+    }
     for (int p = 0; p < kHotProbe; ++p) {
       const uint32_t slot = hot_slot(v, p);
       const uint32_t id = hot->id[slot];
@@ -215,13 +226,15 @@ struct KcoreBufs {
   unsigned cap;
   uint32_t hub;
   uint32_t mul;
+  unsigned batch;  // most vertices a workgroup takes at a time
+  bool first_hot;  // the hottest are the first ids
 };
 
 __device__ __forceinline__ PeelOp make_peel(const KcoreBufs& B, uint32_t (&stage)[kWideWaves][kWaveQCap],
                                             HotTable* hot) {
   const unsigned out = B.c->in ^ 1u;
   return PeelOp{B.col, B.degree, out ? B.q1 : B.q0, B.c, {stage[threadIdx.x / kWave]}, B.k, out, B.cap, B.hub,
-                B.mul, hot};
+                B.mul, hot, B.first_hot};
 }
 
 // Workgroup-uniform.  The table of the listed vertices, or nullptr when there
@@ -229,6 +242,11 @@ __device__ __forceinline__ PeelOp make_peel(const KcoreBufs& B, uint32_t (&stage
 __device__ __forceinline__ HotTable* hot_load(HotTable& T, const KcoreBufs& B, unsigned frontier) {
   const unsigned nhot = min(B.c->hot_count, kHotCap);
   if (nhot == 0 || frontier < kHotMin) return nullptr;
+  if (B.first_hot) {
+    for (uint32_t i = threadIdx.x; i < kFirstHot; i += kWideBlock) (&T.id[0])[i] = 0;
+    __syncthreads();
+    return &T;
+  }
   for (uint32_t i = threadIdx.x; i < (1u << kHotBits); i += kWideBlock) {
     T.id[i] = kNoVertex;
     T.count[i] = 0;
@@ -247,10 +265,11 @@ __device__ __forceinline__ HotTable* hot_load(HotTable& T, const KcoreBufs& B, u
 __device__ __forceinline__ void hot_apply(PeelOp& op) {
   if (!op.hot) return;
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < (1u << kHotBits); i += kWideBlock) {
-    const uint32_t cnt = op.hot->count[i];
+  const uint32_t slots = op.first_hot ? kFirstHot : 1u << kHotBits;
+  for (uint32_t i = threadIdx.x; i < slots; i += kWideBlock) {
+    const uint32_t cnt = op.first_hot ? (&op.hot->id[0])[i] : op.hot->count[i];
     bool dies[1] = {false};
-    const uint32_t id[1] = {op.hot->id[i]};
+    const uint32_t id[1] = {op.first_hot ? i : op.hot->id[i]};
     if (cnt) {
       const uint32_t old = atomicSub(&op.degree[degree_pos(id[0], op.mul)], cnt);
       dies[0] = old >= op.k && old - cnt < op.k;
@@ -268,7 +287,7 @@ __global__ void __launch_bounds__(kWideBlock) kcore_peel_kernel(KcoreBufs B) {
   const unsigned in = c->in, count = c->count[in];
   PeelOp op = make_peel(B, stage, hot_load(hot, B, count));
   expand_queue<kWideBlock, PeelOp, false, kWideEdges>(B.row, in ? B.q1 : B.q0, count, B.hub, B.hubq, &c->hub_count,
-                                                      B.cap, &c->overflow, op);
+                                                      B.cap, &c->overflow, op, 0, B.batch);
   hot_apply(op);
   op.finish();
 }
@@ -375,7 +394,7 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
   // kRoundsPerGraph for the next ones, replayed until the state says done,
   // and the membership pass runs after
   // the replay that ends with it, so the host synchronises once per replay.
-  KcoreBufs B{g->row, g->col, degree, q[0], q[1], hubq, hub_off, c, state->hot, k, cap, hub_degree(), 1u};
+  KcoreBufs B{g->row, g->col, degree, q[0], q[1], hubq, hub_off, c, state->hot, k, cap, hub_degree(), 1u, kWideBlock, false};
   // No vertex above the hub threshold: the hub list stays empty and its two
   // launches are left out of each round.
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
@@ -391,7 +410,9 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
   }
   if (hubs) {
     B.degree = g->scratch<uint32_t>(WS_V5, (static_cast<size_t>(cap) + kPage - 1) / kPage * kPage);
-    B.mul = kPageMul;
+    if (!relabel) B.mul = kPageMul;
+    B.batch = kBatchMax;
+    B.first_hot = relabel;
   }
   const uint32_t hot_min = static_cast<uint32_t>(std::max<int64_t>(kHotDegree, g->m >> 13));
   kcore_reset_kernel<<<1, 64, 0, s>>>(c);

@@ -180,6 +180,7 @@ struct Bufs {
   uint32_t hub_span;
   int local_rounds;    // kLocalRounds or kLocalRoundsNoHubs
   unsigned local_max;  // most near items of a step with local rounds
+  unsigned batch;      // most vertices a workgroup takes at a time
 };
 
 __global__ void sssp_init_kernel(uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp,
@@ -525,7 +526,7 @@ __device__ __forceinline__ void relax_step(const Bufs& B, Stage& sn, Stage& sf) 
   RelaxOp op = make_relax(B, sn, sf);
   const unsigned q = S->q;
   expand_queue<kWideBlock, RelaxOp, true, kWideEdges>(B.row, B.nearq[q], S->near_count[q], B.hub, B.hubq[S->hq], &S->hub_count, B.cap,
-                                      &S->overflow, op);
+                                      &S->overflow, op, 0, B.batch);
   op.finish();
 }
 
@@ -899,6 +900,7 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   B.defer = static_cast<uint32_t>(tune_effective("sssp.defer_hubs", n, g->m)) | (refine > 0 ? 1u : 0u);
   B.hub_span = refine > 0 ? 1u << std::min<int64_t>(refine - 1, 31) : 0u;
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);
+  B.batch = hubs ? kBatchMax : kWideBlock;
   B.local_max = !hubs ? kLocalMax : g->m < kLocalHubEdges && !B.defer ? kLocalMaxHubs : 0u;
   B.local_rounds = hubs ? kLocalRounds : kLocalRoundsNoHubs;
   // Graphs with hubs run on the degree-ordered copy (frontier.relabel).
