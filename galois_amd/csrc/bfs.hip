@@ -26,7 +26,7 @@
 //    frontiers over more workgroups).
 //  - gx_bfs drives its levels on the device from a state word: runs of small
 //    levels in one workgroup (narrow_kernel), larger ones as a fixed kernel
-//    sequence (expand, hubs, narrow); four such levels are captured in a HIP
+//    sequence (expand, hubs, narrow); a few such levels are captured in a HIP
 //    graph and replayed until the frontier is empty.
 //  - On symmetric graphs with hubs the heavy levels of gx_bfs are pulled
 //    instead (level_begin): RMAT-18 240 -> 115 us, 4 M vertices 1272 -> 282 us,
@@ -55,7 +55,15 @@ constexpr uint32_t kNoParent = 0xffffffffu;
 constexpr int kGridNoHubs = 128;
 constexpr int kHubLanes = 64;  // lanes per step of the hub pass
 constexpr int kLevelsPerGraph = 4;
-constexpr int kLevelsFirst = 4;  // wide levels of the first replay: what power-law graphs need
+// Wide levels of the first replay: what power-law graphs need.  A level that
+// is not needed costs 6-7 us, a second replay with its wait 60.  Below 2^18
+// edges the one-workgroup levels leave at most three (4096 vertices, 97K edges
+// 98 -> 92 us; 1100 to 10,000 vertices 89-103 -> 83-97; with two, 8000 vertices
+// go from 100 to 136), above it the fourth is needed.  Graphs without hubs
+// have tens of levels: with fewer in the first replay a lattice of 20,000
+// vertices goes from 275 us to 305.
+constexpr int kLevelsFirst = 4, kLevelsFirstSmall = 3;
+constexpr int64_t kSmallEdges = int64_t(1) << 18;
 
 struct BfsState {
   unsigned count[2];      // frontier sizes (double buffered by q)
@@ -688,7 +696,8 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
   key = mix_key(mix_key(mix_key(key, cap), B.hub), hubs ? 1u : 0u);
   uint32_t replays = 0, slots = 0;
   for (;;) {
-    const int nl = replays == 0 ? kLevelsFirst : kLevelsPerGraph;
+    const int first = hubs && g->m < kSmallEdges ? kLevelsFirstSmall : kLevelsFirst;
+    const int nl = replays == 0 ? first : kLevelsPerGraph;
     ktimer.begin();
     g->replay(replays == 0 ? g->bfs_head : g->bfs_batch, key, [&](hipStream_t cs) {
       enqueue_levels(B, hubs, replays == 0, nl, cs);

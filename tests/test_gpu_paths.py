@@ -289,6 +289,32 @@ def test_bfs_narrow_wide_and_pulled_levels(gx, oracle, n, hub_degree, symmetric,
             gx.tune_set(knob, -1)
 
 
+@pytest.mark.parametrize("layers,degree", [(4, 24), (8, 12), (9, 14), (9, 16)])
+def test_bfs_more_wide_levels_than_the_first_replay(gx, oracle, layers, degree):
+    """Layers of 1000 vertices, each with `degree` edges into the next one and
+    a hub: every level is wide, on both sides of the edge count up to which the
+    first replay is shorter (2^18)."""
+    rng = np.random.default_rng(degree)
+    width = 1000
+    n = layers * width + 1
+    u = np.repeat(np.arange((layers - 1) * width), degree)
+    v = (u // width + 1) * width + rng.integers(0, width, len(u))
+    heads = np.arange(layers - 1) * width  # each layer's hub, and the source's edges
+    u = np.concatenate([u, np.repeat(heads, width), np.full(width, n - 1)])
+    v = np.concatenate([v, (np.arange(layers - 1)[:, None] * width + width + np.arange(width)).ravel(), np.arange(width)])
+    key = np.unique(np.concatenate([u * n + v, v * n + u]))
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(key // n, minlength=n), out=row[1:])
+    col = (key % n).astype(np.int32)
+    print(f"bfs layers={layers} n={n} m={len(col)}", flush=True)
+    for symmetric in (False, True):  # True pulls the heavy levels
+        G = gx.Graph.from_csr(row, col, symmetric=symmetric)
+        for src in (n - 1, 0, n // 2):
+            exp = oracle.bfs(row, col, src)
+            for _ in range(2):
+                assert np.array_equal(u32(gx.bfs(G, src)[0]), exp)
+
+
 def lattice_csr(rows, cols, whi, seed):
     """Symmetric weighted CSR of a rows x cols lattice with a few long edges."""
     rng = np.random.default_rng(seed)
