@@ -251,16 +251,17 @@ __device__ __forceinline__ TdOp make_td(const Bufs& B, uint32_t (&stage)[kWideWa
 // neighbours itself, four in flight; what is left of longer lists is walked by
 // the wavefront together, one list after another, so that an unreached hub does
 // not hold a wavefront for as many steps as it has neighbours.
-constexpr int kPullSerial = 32;
+constexpr uint32_t kPullSerial = 32;
 
 __device__ __forceinline__ bool pull_scan(const int32_t* __restrict__ col, const uint32_t* __restrict__ front,
                                           int32_t begin, int32_t end, uint32_t& who) {
   bool hit = false;
-  const int32_t stop = min(end, begin + kPullSerial);
-  for (int32_t e = begin; e < stop && !hit; e += 4) {
+  const uint32_t len = static_cast<uint32_t>(end - begin);
+  const uint32_t serial = min(len, kPullSerial);
+  for (uint32_t i = 0; i < serial && !hit; i += 4) {
     uint32_t u[4], w[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) u[k] = static_cast<uint32_t>(col[min(e + k, end - 1)]);
+    for (int k = 0; k < 4; ++k) u[k] = static_cast<uint32_t>(col[list_edge(begin, i + k, len)]);
 #pragma unroll
     for (int k = 0; k < 4; ++k) w[k] = front[u[k] >> 5];
 #pragma unroll
@@ -270,14 +271,14 @@ __device__ __forceinline__ bool pull_scan(const int32_t* __restrict__ col, const
         who = u[k];
       }
   }
-  uint64_t rest = __ballot(!hit && stop < end);
+  uint64_t rest = __ballot(!hit && serial < len);
   while (rest) {
     const int i = __ffsll(static_cast<unsigned long long>(rest)) - 1;
     rest &= rest - 1;
-    const int32_t b = __builtin_amdgcn_readlane(stop, i), last = __builtin_amdgcn_readlane(end, i);
-    for (int32_t e = b; e < last; e += kWave) {
-      const int32_t mine = e + static_cast<int32_t>(lane_id());
-      const uint32_t u = static_cast<uint32_t>(col[min(mine, last - 1)]);
+    const int32_t b = __builtin_amdgcn_readlane(begin, i);
+    const uint32_t n = __builtin_amdgcn_readlane(len, i);
+    for (uint32_t j = kPullSerial; j < n; j += kWave) {
+      const uint32_t u = static_cast<uint32_t>(col[list_edge(b, j + lane_id(), n)]);
       const uint64_t in = __ballot((front[u >> 5] >> (u & 31)) & 1u);
       if (in) {
         const uint32_t first = __builtin_amdgcn_readlane(u, __ffsll(static_cast<unsigned long long>(in)) - 1);

@@ -46,6 +46,14 @@ __device__ __forceinline__ bool wave_append(bool pred, T item, T* queue, unsigne
   return true;
 }
 
+// Edge ids are int32 and go up to 2^31 - 1, so the end of a list plus a
+// wavefront's lanes may lie outside their range.  Loops over a list therefore
+// count positions from its first edge (unsigned: a length plus a step fits).
+// Edge at position i of a list of `len` >= 1 edges, the last one beyond its end.
+__host__ __device__ __forceinline__ int32_t list_edge(int32_t begin, uint32_t i, uint32_t len) {
+  return begin + static_cast<int32_t>(i < len ? i : len - 1);
+}
+
 template <class T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
