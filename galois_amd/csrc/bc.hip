@@ -226,7 +226,7 @@ constexpr int kVisitGrid = 512;
 
 struct ChunkTable {
   uint32_t* vtx;     // owning vertex
-  int32_t* begin;    // first edge (end = min(begin + chunk, row[vtx + 1]))
+  int32_t* begin;    // first edge (chunk_len(begin, row[vtx + 1], chunk) of them)
   uint8_t* whole;    // 1 when the chunk is the vertex's whole adjacency
   int64_t count;
   uint32_t* multi;   // vertices with more than one chunk
@@ -254,9 +254,9 @@ __global__ void chunk_fill_kernel(const int32_t* __restrict__ row, int64_t n, in
     const int32_t b = row[v], e = row[v + 1];
     uint32_t k = first[v];
     const uint8_t w = (e - b) <= chunk ? 1 : 0;
-    for (int32_t x = b; x < e; x += chunk, ++k) {
+    for (int64_t x = b; x < e; x += chunk, ++k) {
       vtx[k] = static_cast<uint32_t>(v);
-      begin[k] = x;
+      begin[k] = static_cast<int32_t>(x);
       whole[k] = w;
     }
   }
@@ -478,15 +478,15 @@ __global__ void __launch_bounds__(kBlock) bcb_forward_kernel(
     const uint64_t need = lanes & ~vis[goff + v];
     if (need == 0) continue;
     const int32_t eb = T.begin[c];
-    const int32_t ee = min(eb + T.chunk, trow[v + 1]);
+    const uint32_t len = chunk_len(eb, trow[v + 1], T.chunk);
     uint64_t acc_mask = 0;
     float sig = 0.f;
-    for (int32_t e0 = eb; e0 < ee; e0 += kWave) {
-      const int32_t e = e0 + static_cast<int32_t>(lane);
+    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+      const uint32_t j = j0 + lane;
       uint32_t u = 0;
       uint64_t f = 0;
-      if (e < ee) {
-        u = static_cast<uint32_t>(tcol[e]);
+      if (j < len) {
+        u = static_cast<uint32_t>(tcol[eb + static_cast<int32_t>(j)]);
         f = FL[goff + u] & need;
       }
       uint64_t act = __ballot(f != 0);
@@ -563,14 +563,14 @@ __global__ void __launch_bounds__(kBlock) bcb_backward_kernel(
     const uint64_t mine = FL[goff + v];
     if (mine == 0) continue;
     const int32_t eb = T.begin[c];
-    const int32_t ee = min(eb + T.chunk, row[v + 1]);
+    const uint32_t len = chunk_len(eb, row[v + 1], T.chunk);
     double acc = 0.0;
-    for (int32_t e0 = eb; e0 < ee; e0 += kWave) {
-      const int32_t e = e0 + static_cast<int32_t>(lane);
+    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+      const uint32_t j = j0 + lane;
       uint32_t w = 0;
       uint64_t f = 0;
-      if (e < ee) {
-        w = static_cast<uint32_t>(col[e]);
+      if (j < len) {
+        w = static_cast<uint32_t>(col[eb + static_cast<int32_t>(j)]);
         f = FL1[goff + w] & mine;
       }
       uint64_t act = __ballot(f != 0);

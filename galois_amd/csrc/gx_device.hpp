@@ -54,6 +54,11 @@ __host__ __device__ __forceinline__ int32_t list_edge(int32_t begin, uint32_t i,
   return begin + static_cast<int32_t>(i < len ? i : len - 1);
 }
 
+// Edges of the chunk that starts at `begin` in a list that ends at `end`.
+__host__ __device__ __forceinline__ uint32_t chunk_len(int32_t begin, int32_t end, int chunk) {
+  return static_cast<uint32_t>(end - begin < chunk ? end - begin : chunk);
+}
+
 template <class T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll

@@ -508,8 +508,10 @@ __global__ void __launch_bounds__(kBlock) bc_backward_kernel(const int32_t* __re
     const uint32_t u = q[i];
     double sum = 0.0;
     unsigned found = 0;
-    for (int32_t e = row[u] + static_cast<int32_t>(lane); e < row[u + 1]; e += kWave) {
-      const uint32_t v = static_cast<uint32_t>(col[e]);
+    const int32_t begin = row[u];
+    const uint32_t deg = static_cast<uint32_t>(row[u + 1] - begin);
+    for (uint32_t j = lane; j < deg; j += kWave) {
+      const uint32_t v = static_cast<uint32_t>(col[begin + static_cast<int32_t>(j)]);
       if (len[v] == r + 1) {
         sum += (1.0 + static_cast<double>(__uint_as_float(dep[v]))) / nsp[v];
         found = 1;

@@ -179,7 +179,8 @@ __global__ void __launch_bounds__(kBlock) sb_relax_kernel(BBufs B) {
     const int64_t my = base + lane * nwaves;
     uint64_t mp = 0;
     uint32_t mrow = 0, mrow_hi = 0, mg = 0;  // group * n + vertex, group
-    int32_t mb = 0, me = 0;
+    int32_t mb = 0;
+    uint32_t mlen = 0;
     unsigned mfirst = 0;
     if (my < items) {
       mg = static_cast<uint32_t>(my / B.nchunks);
@@ -191,7 +192,7 @@ __global__ void __launch_bounds__(kBlock) sb_relax_kernel(BBufs B) {
       mrow_hi = static_cast<uint32_t>(r >> 32);
       if (mp) {
         mb = B.cbegin[mc];
-        me = min(mb + kEdgeChunk, B.row[mu + 1]);
+        mlen = chunk_len(mb, B.row[mu + 1], kEdgeChunk);
         mfirst = mb == B.row[mu];
       }
     }
@@ -205,9 +206,10 @@ __global__ void __launch_bounds__(kBlock) sb_relax_kernel(BBufs B) {
       live &= live - 1;
       const int64_t r = (static_cast<int64_t>(__builtin_amdgcn_readlane(mrow_hi, i1)) << 32) |
                         static_cast<uint32_t>(__builtin_amdgcn_readlane(mrow, i1));
-      const int32_t e = __builtin_amdgcn_readlane(mb, i1) + static_cast<int32_t>(lane);
       du1 = dist[r * 64 + lane];
-      if (e < static_cast<int32_t>(__builtin_amdgcn_readlane(me, i1))) {
+      const int32_t eb = __builtin_amdgcn_readlane(mb, i1);
+      if (lane < static_cast<uint32_t>(__builtin_amdgcn_readlane(mlen, i1))) {
+        const int32_t e = eb + static_cast<int32_t>(lane);
         col1 = static_cast<uint32_t>(B.col[e]);
         w1 = B.w[e];
       }
@@ -221,7 +223,8 @@ __global__ void __launch_bounds__(kBlock) sb_relax_kernel(BBufs B) {
       more = live != 0;
       if (more) stage();
       const uint64_t pend = readlane64(mp, i);
-      const int32_t eb = __builtin_amdgcn_readlane(mb, i), ee = __builtin_amdgcn_readlane(me, i);
+      const int32_t eb = __builtin_amdgcn_readlane(mb, i);
+      const uint32_t len = __builtin_amdgcn_readlane(mlen, i);
       const int64_t goff = static_cast<uint32_t>(__builtin_amdgcn_readlane(mg, i)) * B.n;
       const uint64_t act = __ballot(((pend >> lane) & 1ull) && du < limit);
       const bool on = (act >> lane) & 1ull;
@@ -236,16 +239,14 @@ __global__ void __launch_bounds__(kBlock) sb_relax_kernel(BBufs B) {
         pushed += on;
       }
       if (act == 0) continue;
-      if (on) edges += static_cast<unsigned>(ee - eb);
-      for (int32_t e0 = eb; e0 < ee; e0 += kWave) {
-        if (e0 != eb) {
-          const int32_t e = e0 + static_cast<int32_t>(lane);
-          if (e < ee) {
-            cv = static_cast<uint32_t>(B.col[e]);
-            cw = B.w[e];
-          }
+      if (on) edges += len;
+      for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+        if (j0 != 0 && j0 + lane < len) {
+          const int32_t e = eb + static_cast<int32_t>(j0 + lane);
+          cv = static_cast<uint32_t>(B.col[e]);
+          cw = B.w[e];
         }
-        const int left = min(static_cast<int>(kWave), ee - e0);
+        const int left = static_cast<int>(min(static_cast<uint32_t>(kWave), len - j0));
         for (int k0 = 0; k0 < left; k0 += kUnroll) {
           uint32_t v[kUnroll], dv[kUnroll];
 #pragma unroll

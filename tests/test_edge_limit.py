@@ -1,7 +1,8 @@
 """Edge ids are int32 and a graph may hold up to 2^31 - 1 edges, so that the
 last lists end where an id plus a wavefront's lanes no longer fits.  The loops
-that walk such a list (the pulled BFS levels) are restated here with the helper
-they use, in a host build of the header; no GPU."""
+that walk such a list (the pulled BFS levels, the chunks of the batched sweeps)
+are restated here with the helpers they use, in a host build of the header;
+no GPU."""
 from __future__ import annotations
 
 import shutil
@@ -19,7 +20,7 @@ SRC = r'''
 #include <cstdio>
 #include <vector>
 #include "gx_device.hpp"
-using gx::list_edge;
+using gx::chunk_len; using gx::list_edge;
 constexpr int32_t kLast = INT32_MAX;  // one past the last edge of the largest graph
 
 // Every edge of [begin, end) seen at least once and none outside: at most
@@ -50,12 +51,27 @@ int main() {
       for (uint32_t j = 32; j < n; j += 64)
         for (uint32_t lane = 0; lane < 64; ++lane) scan.at(list_edge(begin, j + lane, n));
       if (!scan.ok()) ++wrong;
+      // The list cut into chunks, every chunk walked 64 edges at a time.
+      for (int chunk : {64, 256, 4096}) {
+        Seen walk(begin, end);
+        for (int64_t x = begin; x < end; x += chunk) {
+          const int32_t b = static_cast<int32_t>(x);
+          const uint32_t c = chunk_len(b, end, chunk);
+          if (c == 0 || c > static_cast<uint32_t>(chunk)) ++wrong;
+          for (uint32_t j0 = 0; j0 < c; j0 += 64)
+            for (uint32_t lane = 0; lane < 64; ++lane)
+              if (j0 + lane < c) walk.at(b + static_cast<int32_t>(j0 + lane));
+        }
+        if (!walk.ok()) ++wrong;
+        for (int h : walk.hits) if (h != 1) ++wrong;
+      }
     }
   }
   // One list of every edge: the position after the last step still fits.
   const uint32_t all = static_cast<uint32_t>(kLast);
   const uint32_t last_step = 32 + (all - 33) / 64 * 64;
   if (last_step + 64 < last_step || list_edge(0, last_step + 63, all) != kLast - 1) ++wrong;
+  if (chunk_len(0, kLast, 4096) != 4096u || chunk_len(kLast - 1, kLast, 256) != 1u) ++wrong;
   std::printf("%ld\n", wrong);
   return 0;
 }
