@@ -47,7 +47,7 @@ class gx_stats(C.Structure):
 class gx_pb_layout_info(C.Structure):
     _fields_ = [(name, C.c_int64) for name in ("bins", "groups", "pieces", "tasks", "sliced_bins", "jobs_long",
                                                 "jobs_mid", "jobs_short", "task_edges")] + [
-        ("built", C.c_int32), ("reserved", C.c_int32)]
+        ("built", C.c_int32), ("slice_edges", C.c_int32)]
 
     def as_dict(self) -> dict:
         return {name: getattr(self, name) for name, _ in self._fields_ if name != "reserved"}

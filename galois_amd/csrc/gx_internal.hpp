@@ -130,7 +130,8 @@ struct PbLayout {
   bool ready = false;
   int64_t nbins = 0, ngroups = 0, npieces = 0, ntasks = 0, nmulti = 0;
   int64_t njobs[3] = {0, 0, 0};  // long, mid, short jobs
-  int64_t task_entries = 0;      // slice size (edges) the tasks were cut with
+  int64_t task_limit = 0;        // value of "pr.task_edges" the layout was built under
+  int64_t task_entries = 0;      // slice size (edges) the tasks were cut with, at most task_limit
   int64_t nonzero = 0;           // vertices with out-edges: degree-order ids [0, nonzero)
   DevBuf gsrc16, dst16, vals, pieces, jobs, tasks, multi, gacc;
 };

@@ -582,7 +582,8 @@ extern "C" gx_status gx_pagerank_layout_info(const gx_graph* g, gx_pb_layout_inf
     info->jobs_long = L.njobs[0];
     info->jobs_mid = L.njobs[1];
     info->jobs_short = L.njobs[2];
-    info->task_edges = L.task_entries;
+    info->task_edges = L.task_limit;
+    info->slice_edges = static_cast<int32_t>(L.task_entries);
   }
   GX_API_END
 }

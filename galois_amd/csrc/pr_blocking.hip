@@ -481,7 +481,8 @@ void build_layout(gx_graph* g) {
   L.npieces = static_cast<int64_t>(pieces.size());
   L.ntasks = static_cast<int64_t>(tv.size());
   L.nmulti = static_cast<int64_t>(multi.size());
-  L.task_entries = task_limit;
+  L.task_limit = task_limit;
+  L.task_entries = static_cast<int64_t>(task_entries);
   {
     DevBuf nz;
     nz.ensure(8);

@@ -344,13 +344,15 @@ gx_status gx_pagerank_pull(gx_graph* g, double alpha, double tol,
  * on (built by the first such call and kept with the graph; all zero
  * before): destination bins (= source chunks) of 16384 vertices, (source,
  * bin) groups, phase-1 pieces, phase-2 tasks, bins summed in slices, phase-2
- * jobs per length class, and the slice size in edges it was built with
- * ("pr.task_edges").  No reference counterpart. */
+ * jobs per length class, the value of "pr.task_edges" it was built under
+ * (task_edges) and the slice size in edges its bins were cut with
+ * (slice_edges: the same when the knob was set, else at most that, see the
+ * knob).  No reference counterpart. */
 typedef struct gx_pb_layout_info {
   int64_t bins, groups, pieces, tasks, sliced_bins;
   int64_t jobs_long, jobs_mid, jobs_short;
   int64_t task_edges;
-  int32_t built, reserved;
+  int32_t built, slice_edges;
 } gx_pb_layout_info;
 gx_status gx_pagerank_layout_info(const gx_graph* g, gx_pb_layout_info* info);
 

@@ -1,0 +1,51 @@
+"""Dispatch rules and knobs on the GPU: what a call reports about the path it
+took, paths that the default rules leave to larger graphs, and inputs in orders
+and of values that a path's layout could mistake."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gpu_paths import weighted_csr
+
+pytestmark = pytest.mark.gpu
+
+
+class knobs:
+    """Knobs set for a block."""
+
+    def __init__(self, gx, **values):
+        self.gx, self.values = gx, {k.replace("__", "."): v for k, v in values.items()}
+
+    def __enter__(self):
+        for k, v in self.values.items():
+            self.gx.tune_set(k, v)
+
+    def __exit__(self, *exc):
+        for k in self.values:
+            self.gx.tune_set(k, -1)
+
+
+@pytest.mark.parametrize("n,m", [(700, 3000), (40000, 1000000), (16384, 2400000), (300000, 4000000)])
+def test_layout_reports_its_slices(gx, n, m):
+    """task_edges is the knob's value for the layout, slice_edges what its bins
+    were cut with: as many as the knob says when it is set, m / 160 within
+    [2^13, the default] otherwise.  A slice holds at most 511 edges more, and a
+    bin is cut if and only if it holds more edges than a slice."""
+    row, col, _ = weighted_csr(n, m, n, 1)
+    m = len(col)
+    print(f"layout n={n} m={m}", flush=True)
+    for edges in (-1, 1 << 12, 1 << 13, 1 << 19, 1 << 30):
+        G = gx.Graph.from_csr(row, col)
+        with knobs(gx, pr__blocking=1, pr__task_edges=edges):
+            gx.pagerank(G, tol=0.0, max_iter=1)
+        info = gx.pagerank_layout_info(G)
+        assert info["task_edges"] == (edges if edges > 0 else 1 << 19)
+        assert info["slice_edges"] == (edges if edges > 0 else min(1 << 19, max(m // 160, 1 << 13)))
+        assert info["tasks"] * (info["slice_edges"] + 511) >= m
+        # A bin is 16384 destinations of the degree order.
+        order = np.lexsort((np.arange(n), -np.diff(row)))
+        rank = np.empty(n, np.int64)
+        rank[order] = np.arange(n)
+        heavy = np.bincount(rank[col] // 16384, minlength=info["bins"])
+        assert info["sliced_bins"] == int((heavy > info["slice_edges"]).sum())
