@@ -21,7 +21,8 @@ Knobs and candidates:
   sssp.max_merge       most delta buckets one SSSP phase may cover
   sssp.hub_refine      SSSP hub steps: 0 = hubs expanded in the step that
                        admits them, r > 0 = deferred and expanded 2^(r-1)
-                       distances per hub step
+                       distances per hub step, -1 = the default, whose slices
+                       follow the number of hubs
   bc.chunk             batched BC: edges per work item, the degree-bin boundary
                        between whole-adjacency items and split ones
   bc.grid              batched BC: workgroups of each level sweep
@@ -40,7 +41,7 @@ CANDIDATES: dict[str, list[int]] = {
     "pr.blocking": [1, 0],
     "pr.hot_sources": [0, 1 << 17, 1 << 18, 1 << 19, 1 << 20, 1 << 21],
     "sssp.max_merge": [1, 16, 64, 256, 1024],
-    "sssp.hub_refine": [0, 1, 2, 3],
+    "sssp.hub_refine": [-1, 0, 1, 2, 3],
     "bc.chunk": [64, 128, 256, 512, 1024],
     "bc.grid": [2048, 4096, 8192, 16384],
 }

@@ -108,10 +108,11 @@ constexpr int kHubSelectGrid = 128;
 constexpr unsigned long long kMergeLow = 1ull << 15;
 constexpr unsigned long long kMergeHigh = 1ull << 18;
 
-// A hub step's slice of distances (sssp.hub_refine) doubles when the step
-// expanded few hubs and halves when it expanded many: a step costs 20 us however
-// few hubs it has.  With weights to 60000 fixed slices of one distance took 90 ms
-// on RMAT-22, these 8 (2^8 and 2^12 to 2^14 and 2^18 within 1% of each other).
+// While sssp.hub_refine is not set, a hub step's slice of distances doubles when
+// the step expanded few hubs and halves when it expanded many: a step costs 20 us
+// however few hubs it has.  With weights to 60000 fixed slices of one distance took
+// 90 ms on RMAT-22, these 8 (2^8 and 2^12 to 2^14 and 2^18 within 1% of each
+// other).  A set knob's slices stay as they are.
 constexpr unsigned kHubsFew = 1u << 10, kHubsMany = 1u << 14;
 
 enum Mode : unsigned { kIdle = 0, kRelax = 1, kAdvance = 2, kHubs = 3 };
@@ -140,6 +141,7 @@ struct SsspState {
   uint32_t hub_min_next;   // the same over the hubs a hub step keeps
   uint32_t hub_limit;      // a hub step expands the pending hubs at or below this distance
   uint32_t hub_span;       // a hub step's slice of distances
+  unsigned hub_adapt;      // hub_span follows the hubs of a step
   unsigned hub_step;       // this step selects and expands pending hubs
   uint32_t near_min;       // smallest distance in the near queue the step reads
   uint32_t near_min_next;  // the same for the near queue the step fills
@@ -198,7 +200,7 @@ __global__ void sssp_init_kernel(uint32_t* __restrict__ dist, uint32_t* __restri
 
 __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint32_t* nearq0, uint32_t src,
                                   uint32_t* dist, unsigned max_width,
-                                  uint32_t hub_span) {
+                                  uint32_t hub_span, unsigned hub_adapt) {
   for (int i = threadIdx.x; i < 2 * kWideGrid; i += blockDim.x) tally[i] = 0;
   if (threadIdx.x == 0) {
     S->dist_out = dist;
@@ -222,6 +224,7 @@ __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint3
     S->hub_kept = 0;
     S->hub_min = S->hub_min_next = S->hub_limit = 0xffffffffu;
     S->hub_span = hub_span;
+    S->hub_adapt = hub_adapt;
     S->hub_step = 0;
     S->near_min = 0;  // the source
     S->near_min_next = 0xffffffffu;
@@ -242,7 +245,7 @@ __global__ void sssp_reset_kernel(SsspState* S, unsigned long long* tally, uint3
 __device__ __forceinline__ void close_step(SsspState* S) {
   if (S->hub_step) {
     S->hq ^= 1;
-    if (S->hub_span != 0) {
+    if (S->hub_adapt) {
       if (S->hub_expand < kHubsFew && S->hub_span < (1u << 30)) S->hub_span *= 2;
       else if (S->hub_expand > kHubsMany && S->hub_span > 1) S->hub_span /= 2;
     }
@@ -922,7 +925,8 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   sssp_init_kernel<<<grid_for(n, kBlock, 4096), kBlock, 0, s>>>(B.dist, B.stamp, B.done, B.hubmark, n,
                                                                  run_src);
   GX_LAUNCHED("sssp_init_kernel");
-  sssp_reset_kernel<<<1, kBlock, 0, s>>>(B.S, B.tally, B.nearq[0], run_src, B.dist, max_width, B.hub_span);
+  sssp_reset_kernel<<<1, kBlock, 0, s>>>(B.S, B.tally, B.nearq[0], run_src, B.dist, max_width, B.hub_span,
+                                      B.hub_span != 0 && !tune_is_set("sssp.hub_refine") ? 1u : 0u);
   GX_LAUNCHED("sssp_reset_kernel");
   uint64_t key = 0;
   for (const void* p : {(const void*)B.row, (const void*)B.col, (const void*)B.w,

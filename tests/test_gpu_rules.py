@@ -6,7 +6,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_gpu_paths import weighted_csr
+from test_gpu_paths import u32, weighted_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,36 @@ def test_layout_reports_its_slices(gx, n, m):
         rank[order] = np.arange(n)
         heavy = np.bincount(rank[col] // 16384, minlength=info["bins"])
         assert info["sliced_bins"] == int((heavy > info["slice_edges"]).sum())
+
+
+def hub_chain(hubs, degree, step):
+    """Symmetric weighted CSR: vertex 0 joined to `hubs` hubs at distances step,
+    2 * step, ...; each hub joined to `degree` leaves of its own."""
+    n = 1 + hubs + hubs * degree
+    hub = np.arange(1, hubs + 1)
+    u = np.concatenate([np.zeros(hubs, np.int64), np.repeat(hub, degree)])
+    v = np.concatenate([hub, np.arange(1 + hubs, n)])
+    w = np.concatenate([step * hub, np.ones(hubs * degree, np.int64)]).astype(np.uint32)
+    u, v, w = np.concatenate([u, v]), np.concatenate([v, u]), np.concatenate([w, w])
+    o = np.lexsort((v, u))
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(u, minlength=n), out=row[1:])
+    return row, v[o].astype(np.int32), w[o]
+
+
+@pytest.mark.parametrize("hubs,degree,step", [(40, 200, 1000), (60, 130, 50000)])
+def test_sssp_set_slices_stay(gx, oracle, hubs, degree, step):
+    """With sssp.hub_refine set, a hub step takes the pending hubs within
+    2^(r - 1) of the nearest one, however few they are: hubs 1000 apart take a
+    step each at r = 1, and one step at r = 32.  One bucket holds them all."""
+    row, col, w = hub_chain(hubs, degree, step)
+    G = gx.Graph.from_csr(row, col, w, symmetric=True)
+    exp = oracle.sssp(row, col, w, 0, 31)
+    steps = {}
+    for r in (0, 1, 32):
+        with knobs(gx, sssp__hub_refine=r):
+            d, st = gx.sssp(G, 0, 31)
+        assert np.array_equal(u32(d), exp)
+        steps[r] = st.iterations
+    print(f"sssp hubs={hubs} steps={steps}", flush=True)
+    assert steps[1] >= hubs and steps[32] < 10 and steps[0] < 10
