@@ -53,13 +53,15 @@ int64_t default_relabel(int64_t n, int64_t) { return n >= (int64_t(1) << 24) ? 1
 // Hubs expanded in distance order, one distance at a time (r = 1), in the
 // relax steps whenever no near item is closer: RMAT-26 SSSP 49.7 -> 39.0 ms
 // (1.84 -> 1.10 relaxations per edge; two distances 39.8 ms).  Each extra step
-// costs about 20 us whatever the graph, so on smaller graphs the number of edges
-// decides.  RMAT graphs, weights to 255: 94M edges 3.19 ms without and 3.85 with
-// it, 130M edges 4.31 and 3.77 (weights to 20: 2.58 and 2.42, to 1000: 5.9 and
-// 6.1).  The line is drawn between the two, at 7 * 2^24 edges.
-int64_t default_hub_refine(int64_t n, int64_t m) {
-  return n >= (int64_t(1) << 24) || m >= (int64_t(7) << 24) ? 1 : 0;
-}
+// costs about 20 us whatever the graph, and below 2^24 vertices they do not pay.
+// 2^22 vertices, ms without slices and with them, weights to 20, 255 and 1000:
+//   RMAT        104M edges  2.59 2.66   4.01 4.16   5.27 6.39
+//               128M        2.50 2.85   4.18 4.23   5.90 5.93
+//               159M        3.49 2.76   4.67 4.39   6.75 6.98
+//   flatter     109M        3.93 4.67   6.22 8.03   7.17 11.1
+//   (.45, .22)  134M        4.51 6.20   7.52 8.11   6.66 10.6
+//               167M        5.54 7.53   8.57 8.53   7.20 10.2
+int64_t default_hub_refine(int64_t n, int64_t) { return n >= (int64_t(1) << 24) ? 1 : 0; }
 int64_t default_batch_width(int64_t, int64_t) { return 64; }
 int64_t default_bc_grid(int64_t, int64_t) { return 256 * 32; }
 struct Knob {

@@ -893,13 +893,7 @@ extern "C" gx_status gx_sssp_delta(gx_graph* g, uint32_t src, uint32_t shift, ui
   B.cap = cap;
   B.hub_off = g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(cap));
   B.hub = hub_degree();
-  int64_t refine = tune_effective("sssp.hub_refine", n, g->m);
-  // Wide buckets hold many slices of a weight range, and each slice is a step:
-  // RMAT-22 with 2^13 and weights to 1000 5.8 ms without slices and 8.1 with
-  // them, to 255 4.2 and 4.2, to 20 2.6 and 2.4 (2^6 and 2^8, to 255: 4.3 and
-  // 3.8).  The default leaves them out there; on the largest graphs they pay
-  // whatever the buckets.
-  if (!tune_is_set("sssp.hub_refine") && n < (int64_t(1) << 24) && shift > 8) refine = 0;
+  const int64_t refine = tune_effective("sssp.hub_refine", n, g->m);
   B.defer = static_cast<uint32_t>(tune_effective("sssp.defer_hubs", n, g->m)) | (refine > 0 ? 1u : 0u);
   B.hub_span = refine > 0 ? 1u << std::min<int64_t>(refine - 1, 31) : 0u;
   const bool hubs = max_degree(g) > static_cast<int64_t>(B.hub);

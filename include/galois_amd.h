@@ -145,10 +145,10 @@ void gx_set_profiling(int on);
  *                          order and most are expanded once; 0 = off;
  *                          hub selection joins a relax step whenever no near
  *                          item is closer than the hubs it takes; default 1
- *                          (one distance at a time) from 2^24 vertices or
- *                          7 * 2^24 edges on, else 0; range [0, 32]; while
- *                          not set, the slice doubles after steps of few hubs
- *                          and halves again after steps of many
+ *                          (one distance at a time) from 2^24 vertices on,
+ *                          else 0; range [0, 32]; while not set, the slice
+ *                          doubles after steps of few hubs and halves again
+ *                          after steps of many
  *   "sssp.batch_width"     gx_sssp_batched: buckets per phase, shared by
  *                          the 64 sources of a wavefront; 0 = adaptive as
  *                          gx_sssp_delta's phases; default 64
