@@ -647,14 +647,16 @@ def main() -> int:
     #  pull: 4m column ids + 4(n+1) row offsets + 4n y (read once) + 4n x_old +
     #    4n out-degrees + 8n (x', y' written).
     algo_bytes = 4 * m + 4 * (n + 1) + 12 * n
-    blocked = gx.tune_get("pr.blocking") != 0
+    # The sweep that ran: the layout is built by the first solve that takes it
+    # (a tuned value of 0 is set, and a solve below the size rule builds none).
+    blocked = gx.tune_get("pr.blocking") != 0 and bool(gx.pagerank_layout_info(G))
     sweep = "blocked" if blocked else "pull"
     sweep_ms = sweep_ms_total / max(sweeps, 1)
     if blocked:
         kname = ("propagation-blocked sweep: pb::gather_kernel<float> + pb::accum_kernel<PbFin> "
                  "+ pb::multi_kernel<PbFin> (sliced bins)")
     else:
-        kname = ("pull sweep: rs::sweep_kernel<float,HOT,PrSrc,PrFin> + rs::span_finalize_kernel")
+        kname = ("pull sweep: rs::sweep_kernel<float,PrSrc,PrFin> + rs::span_finalize_kernel")
     achieved = algo_bytes / (sweep_ms * 1e-3) / 1e9
     design_rate = design_bytes / (sweep_ms * 1e-3) / 1e9
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",

@@ -62,7 +62,8 @@ DEFAULT_CACHE = Path(os.environ.get("XDG_CACHE_HOME", Path.home() / ".cache")) /
 
 def signature(gx, G, algo: str, args: dict | None = None) -> str:
     """Coarse workload key: algorithm, device, log2 n, log2 avg/max degree,
-    symmetry, and the arguments that pick a different kernel (precision)."""
+    symmetry, and the arguments that pick a different kernel or that the best
+    values depend on (precision, bucket shift, source groups)."""
     import torch
     row, _, _ = G.to_host() if G.m < (1 << 24) else (None, None, None)
     if row is not None:
@@ -74,6 +75,8 @@ def signature(gx, G, algo: str, args: dict | None = None) -> str:
     sym = bool(G.flags & 1)
     a = args or {}
     variant = a.get("precision", "fp32") if algo == "pagerank" else ""
+    if algo == "sssp":  # how many hub slices a bucket holds depends on its width
+        variant = f"shift={a.get('shift', 6)}"
     if algo == "bc":  # a batch's group count shapes the sweeps
         variant = f"groups={(len(a.get('sources', [0])) + 63) // 64}"
     return json.dumps([algo, dev, round(math.log2(max(G.n, 1))), round(math.log2(max(G.m / max(G.n, 1), 1))),

@@ -167,8 +167,11 @@ void gx_set_profiling(int on);
  *                          default 8192, range [256, 65536]
  * Unknown keys and out-of-range values are GX_ERR_INVALID.
  * gx_tune_get returns the value set (-1 when unset); gx_tune_effective the
- * value an entry point uses on a graph of n vertices and m edges: the value
- * set, else the built-in default for that size.  A slice may exceed
+ * value set, else the built-in default for a graph of n vertices and m edges.
+ * An entry point uses that value, but for two rules that hold while the knob is
+ * not set and are stated with it: FP32 solves of fewer than 2^21 edges pull
+ * ("pr.blocking"; gx_pagerank_layout_info's `built` stays 0), and smaller graphs
+ * are cut finer ("pr.task_edges"; its `slice_edges`).  A slice may exceed
  * "pr.task_edges" by up to 511 edges: it is closed at the first job that
  * reaches the limit, and a job holds at most 512 edges. */
 gx_status gx_tune_set(const char* key, int64_t value);
