@@ -544,12 +544,18 @@ __device__ __forceinline__ void relax_step(const Bufs& B, Stage& sn, Stage& sf) 
 // other workgroups find, which costs some expansions at distances that are not
 // final yet.
 // On graphs with hubs, whose shorter paths local rounds run ahead of, only the
-// smallest steps of small graphs have them: unit weights in wide buckets,
-// 4096 vertices 258 -> 245 us with up to 2048 items (328 with three rounds),
-// 1 M vertices 699 -> 729; weights to 255, 4096 vertices 652 -> 414 us, 100,000
-// 1012 -> 974.
+// smallest steps (up to 2048 items; with three rounds instead of two unit weights
+// on 4096 vertices take 328 us) of small graphs have them.  RMAT graphs, us
+// without local rounds and with them, weights to 255 in buckets of 2^6 and 2^13,
+// unit weights, weights to 60000 in buckets of 2^13:
+//   0.10M edges  574 425   387 384   242 243   622 610
+//   0.20M        635 499   449 463   259 252   694 677
+//   0.43M        684 524   479 495   272 267   730 723
+//   0.99M        841 827   647 640   315 289   1298 1283
+//   1.82M        894 880   652 689   290 304   1143 1157
+//   3.73M        969 991   691 751   338 350   1210 1250
 constexpr unsigned kLocalMaxHubs = 1u << 11;
-constexpr int64_t kLocalHubEdges = int64_t(1) << 22;
+constexpr int64_t kLocalHubEdges = int64_t(1) << 20;
 constexpr unsigned kLocalMax = 1u << 16;  // near items: at most one batch per workgroup
 // Rounds: a lattice of 2048 x 2048 takes 3.54 ms with one, 2.84 with 2, 2.87
 // with 8, 3.10 with 16, one of 300,000 vertices 1.52, 0.96, 0.59 and 0.56.
