@@ -212,6 +212,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
     P.npieces = L.npieces;
     P.ntiles = L.ntiles;
     P.ngroups = L.ngroups;
+    P.nruns = L.nruns;
     P.nbins = L.nbins;
     P.bin_rows = L.bin_rows;
     return P;
@@ -361,6 +362,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   exclusive_scan_u32(cut, cut, ng + int64_t(1), s);
   uint32_t nr = 0;
   read_bytes(g, &nr, cut + ng, 4);
+  L.nruns = nr;
   uint64_t* rkey = reinterpret_cast<uint64_t*>(wb);
   uint64_t* rsorted = reinterpret_cast<uint64_t*>(wd);
   L.row16.ensure(static_cast<size_t>(ng) * 2);

@@ -77,7 +77,7 @@ struct Plan {
   const uint16_t* row16;     // per group: row in its bin
   const uint2* runs;         // per bin, in chunk order: first group, length (at most kWave)
   const Bin* bins;           // nbins, most runs first
-  int64_t npieces, ntiles, ngroups, nbins;
+  int64_t npieces, ntiles, ngroups, nruns, nbins;
   int bin_rows;              // most rows of a bin (LDS sums)
 };
 

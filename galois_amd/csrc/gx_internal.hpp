@@ -141,7 +141,7 @@ struct PbLayout {
 struct BlockSums {
   bool ready = false;
   int shift = 0, bin_rows = 0;
-  int64_t npieces = 0, ntiles = 0, ngroups = 0, nbins = 0;
+  int64_t npieces = 0, ntiles = 0, ngroups = 0, nruns = 0, nbins = 0;
   DevBuf pieces, idx16, eid, tile_grp, row16, runs, bins;
 };
 

@@ -542,11 +542,15 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
     // hot/cold split).  Blocked: per row x and the out-degree read by phase 1,
     // x_old read and x' written by the finaliser (3R + 4); 2 bytes of
     // destination id per edge; per group a 2-byte source id, the
-    // contribution written and read back; 12 bytes per phase-2 job.
+    // contribution written and read back; 12 bytes per phase-2 job.  Blocked row
+    // sums: per row as the pull; 2 bytes of index per edge, tiles padded; per
+    // group the partial sum written and read back and its 2-byte row; 8 bytes
+    // per run.
     const int64_t R = sizeof(Real), m = g->m;
     const int64_t njobs = L.njobs[0] + L.njobs[1] + L.njobs[2];
     st->main_kernel_bytes = static_cast<uint64_t>(
-        blocked ? 2 * m + (2 + 2 * R) * L.ngroups + (3 * R + 4) * n + 12 * njobs
+        sums      ? 2 * S.ntiles * bs::kTile + (2 + 2 * R) * S.ngroups + 8 * S.nruns + (4 * R + 4) * n
+        : blocked ? 2 * m + (2 + 2 * R) * L.ngroups + (3 * R + 4) * n + 12 * njobs
                 : 4 * m + (hot > 0 ? 2 : 1) * 4 * (n + 1) + (4 * R + 4) * n + (hot > 0 ? 2 * R * n : 0));
   }
 }

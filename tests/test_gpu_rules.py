@@ -82,3 +82,45 @@ def test_sssp_set_slices_stay(gx, oracle, hubs, degree, step):
         steps[r] = st.iterations
     print(f"sssp hubs={hubs} steps={steps}", flush=True)
     assert steps[1] >= hubs and steps[32] < 10 and steps[0] < 10
+
+
+def groups_of(row, col, shift, range_edges=2048):
+    """(row, chunk of 2^shift sources) groups of the degree-ordered transpose, cut
+    where a wavefront's range of edges ends inside a chunk."""
+    n = len(row) - 1
+    deg = np.diff(row)
+    rank = np.empty(n, np.int64)
+    rank[np.lexsort((np.arange(n), -deg))] = np.arange(n)
+    u, v = rank[np.repeat(np.arange(n), deg)], rank[col]
+    chunk = u >> shift
+    o = np.lexsort((v, chunk))
+    chunk, v = chunk[o], v[o]
+    first = np.searchsorted(chunk, np.arange(chunk.max() + 2))
+    at = np.arange(len(chunk)) - first[chunk]
+    new = np.ones(len(chunk), bool)
+    new[1:] = (chunk[1:] != chunk[:-1]) | (v[1:] != v[:-1]) | (at[1:] % range_edges == 0)
+    tiles = int(sum(-(-c // 512) for c in np.diff(first)))
+    return int(new.sum()), tiles
+
+
+@pytest.mark.parametrize("n,m", [(600011, 9000000), (1 << 19, 8500000)])
+def test_fp64_pull_states_the_bytes_of_the_path_it_took(gx, n, m):
+    """main_kernel_bytes of an FP64 sweep: blocked sums from 2^23 edges on (two
+    bytes per edge position, 18 per group, eight per run of at most 64 groups, 36
+    per row), the row sweep with the hot split."""
+    rng = np.random.default_rng(n)
+    key = np.unique(rng.integers(0, n, m) * n + np.minimum(rng.integers(0, n, m), rng.integers(0, n, m)))
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(key // n, minlength=n), out=row[1:])
+    col = (key % n).astype(np.int32)
+    m = len(col)
+    assert m >= 1 << 23
+    G = gx.Graph.from_csr(row, col)
+    st = gx.pagerank(G, tol=0.0, max_iter=2, precision="fp64")[1]
+    groups, tiles = groups_of(row, col, 13)
+    fixed = 2 * 512 * tiles + 18 * groups + 36 * n
+    print(f"bytes n={n} m={m} groups={groups} fixed={fixed} stated={st.main_kernel_bytes}", flush=True)
+    assert fixed + 8 * -(-groups // 64) <= st.main_kernel_bytes <= fixed + 8 * groups
+    with knobs(gx, pr__hot_sources=1000):
+        st = gx.pagerank(G, tol=0.0, max_iter=2, precision="fp64")[1]
+    assert st.main_kernel_bytes == 4 * m + 8 * (n + 1) + 36 * n + 16 * n
