@@ -665,8 +665,10 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
     B.narrow_max = kNarrowEdges;
     B.batch = kBatchMax;
   }
-  // Symmetric graphs with hubs pull their heavy levels (level_begin).
-  if (hubs && (g->flags & GX_GRAPH_SYMMETRIC)) {
+  // Symmetric graphs with hubs pull their heavy levels (level_begin): the lists
+  // then stand for the in-edges, which a push does not ask of them, so the first
+  // search looks whether they do.
+  if (hubs && (g->flags & GX_GRAPH_SYMMETRIC) && edges_paired(g)) {
     B.front = g->scratch<uint64_t>(WS_BITMAP1, (n + 63) / 64);
     B.pull_min = static_cast<uint64_t>(n) / 4;
   }

@@ -17,6 +17,7 @@
 #include <memory>
 
 
+#include "frontier.hpp"
 #include "gx_device.hpp"
 #include "gx_internal.hpp"
 
@@ -87,6 +88,72 @@ int64_t max_degree(gx_graph* g) {
   }
   g->max_deg = mx;
   return g->max_deg;
+}
+
+// Sum over the edges of a 64-bit hash of the unordered pair, added upwards (u <
+// v) and taken off downwards: zero when the edges come in pairs, and otherwise
+// with a probability of 2^-64.  Read once per
+// graph: 130M edges 0.7 ms, 7.7M 0.06.
+struct PairOp {
+  const int32_t* __restrict__ col;
+  uint64_t sum = 0;
+  template <int U>
+  __device__ __forceinline__ void run(const bool (&valid)[U], const uint32_t (&u)[U], const int32_t (&e)[U]) {
+    uint32_t v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = valid[k] ? static_cast<uint32_t>(col[e[k]]) : u[k];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const uint64_t h = mix64((static_cast<uint64_t>(min(u[k], v[k])) << 32) | max(u[k], v[k]));
+      if (u[k] != v[k]) sum += u[k] < v[k] ? h : 0 - h;
+    }
+  }
+  __device__ __forceinline__ void after_step() {}
+  __device__ __forceinline__ void finish(unsigned long long* out) {
+    __shared__ unsigned long long s_sum[kWideWaves];
+    unsigned long long total;
+    waves_exclusive_sum<kWideBlock>(wave_sum(static_cast<unsigned long long>(sum)), s_sum, &total);
+    if (threadIdx.x == 0 && total) atomicAdd(out, total);
+  }
+};
+
+struct PairState {
+  unsigned long long sum;
+  unsigned hub_count, overflow;
+};
+constexpr uint32_t kPairHub = 256;  // longer lists are spread over the grid
+
+__global__ void __launch_bounds__(kWideBlock) pair_sum_kernel(const int32_t* __restrict__ row, PairOp op, int64_t n,
+                                                              uint32_t* __restrict__ hubq, PairState* S) {
+  expand_queue<kWideBlock, PairOp, false, kWideEdges>(row, nullptr, static_cast<unsigned>(n), kPairHub, hubq,
+                                                      &S->hub_count, static_cast<unsigned>(n), &S->overflow, op);
+  op.finish(&S->sum);
+}
+
+__global__ void __launch_bounds__(kWideBlock) pair_hubs_kernel(const int32_t* __restrict__ row, PairOp op, int64_t n,
+                                                               const uint32_t* __restrict__ hubq,
+                                                               const uint32_t* __restrict__ hub_off, PairState* S) {
+  expand_hubs<kWideBlock, PairOp, kWideBlock, kWideEdges>(row, hubq, S->hub_count, static_cast<unsigned>(n), hub_off,
+                                                          op);
+  op.finish(&S->sum);
+}
+
+bool edges_paired(gx_graph* g) {
+  if (g->paired < 0) {
+    hipStream_t s = g->stream;
+    PairState* S = g->scratch<PairState>(WS_REDUCE, 1);
+    uint32_t* hubq = g->scratch<uint32_t>(WS_Q2, g->n);
+    uint32_t* hub_off = g->scratch<uint32_t>(WS_HUBOFF, hub_off_words(g->n));
+    fill<uint32_t>(reinterpret_cast<uint32_t*>(S), 0u, sizeof(PairState) / 4, s);
+    if (g->m > 0) {
+      pair_sum_kernel<<<kWideGrid, kWideBlock, 0, s>>>(g->row, PairOp{g->col}, g->n, hubq, S);
+      launch_hub_offsets<kWideBlock * kWideEdges>(g->row, hubq, &S->hub_count, static_cast<unsigned>(g->n), hub_off, s);
+      pair_hubs_kernel<<<kWideGrid, kWideBlock, 0, s>>>(g->row, PairOp{g->col}, g->n, hubq, hub_off, S);
+      GX_LAUNCHED("pair_sum_kernel");
+    }
+    g->paired = read_scalar(g, &S->sum) == 0 ? 1 : 0;
+  }
+  return g->paired == 1;
 }
 
 void sort_keys_u64(const uint64_t* in, uint64_t* out, int64_t count, int end_bit, hipStream_t s) {

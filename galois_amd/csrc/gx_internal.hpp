@@ -213,6 +213,7 @@ struct gx_graph {
   gx::DevBuf outdeg_buf;  // uint32 out-degree (for transpose-based PR)
   bool has_outdeg = false;
   int64_t max_deg = -1;  // largest out-degree, computed on demand (gx::max_degree)
+  int paired = -1;       // whether every edge has its reverse, on demand (gx::edges_paired)
   gx::PullPlan pull_plan;            // degree-ordered transpose (PageRank pull)
   gx::PullPlan csc_plan, csr_plan;   // plain transpose / CSR (weighted PageRank and adjoint)
   gx::BlockSums csc_sums[2], csr_sums[2];  // the same sums in blocks, FP32 and FP64 (weighted PageRank and adjoint)
@@ -363,6 +364,9 @@ void edge_sources(const int32_t* row, int64_t n, int64_t m, uint32_t* src, hipSt
 void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s);
 // Largest out-degree of the graph (one reduction, then cached).
 int64_t max_degree(gx_graph* g);
+// Whether every edge (u, v) has its reverse (v, u), as often (one pass over the
+// edges, then cached).
+bool edges_paired(gx_graph* g);
 // Scans and radix sort of the build path (sort.hip): sum scan (exclusive),
 // max scan (inclusive), both may run in place; stable ascending LSD radix
 // sort of count < 2^32 keys over bits [0, end_bit) with optional uint32

@@ -6,7 +6,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_gpu_paths import u32, weighted_csr
+from test_gpu_paths import random_csr, u32, weighted_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -82,6 +82,53 @@ def test_sssp_set_slices_stay(gx, oracle, hubs, degree, step):
         steps[r] = st.iterations
     print(f"sssp hubs={hubs} steps={steps}", flush=True)
     assert steps[1] >= hubs and steps[32] < 10 and steps[0] < 10
+
+
+@pytest.mark.parametrize("n,m,missing", [(2000, 30000, 0), (2000, 30000, 1), (20001, 400000, 1), (20001, 400000, None)])
+def test_bfs_does_not_take_the_symmetric_flag_on_trust(gx, oracle, n, m, missing):
+    """Levels follow the edges as they are, also where a graph that is said to be
+    symmetric lacks reverse edges (`missing` of every vertex but the last, or all
+    of them): a pulled level would not see the edge that has no reverse."""
+    row, col = random_csr(n, m, n, symmetric=missing is not None, shuffle_hubs=True)
+    if missing:  # the last neighbour of every vertex goes
+        src = np.repeat(np.arange(n), np.diff(row))
+        keep = np.ones(len(col), bool)
+        full = np.flatnonzero(np.diff(row) > 1)[:-1]
+        keep[row[full + 1] - 1] = False
+        src, col = src[keep], col[keep]
+        row = np.zeros(n + 1, np.int32)
+        np.cumsum(np.bincount(src, minlength=n), out=row[1:])
+    for flag in (True, False):
+        G = gx.Graph.from_csr(row, col, symmetric=flag)
+        for src in (0, n // 3, int(np.argmax(np.diff(row)))):
+            print(f"bfs n={n} m={len(col)} missing={missing} flag={flag} src={src}", flush=True)
+            assert np.array_equal(u32(gx.bfs(G, src)[0]), oracle.bfs(row, col, src)), (flag, src)
+
+
+def test_bfs_lists_with_repeated_edges(gx, oracle):
+    """Repeated and unsorted adjacency entries: a symmetric graph whose edges come
+    twice (heavy levels pulled), and one whose reverses come once."""
+    n = 20001
+    row, col = random_csr(n, 200000, 5, order="random", shuffle_hubs=True)
+    src = np.repeat(np.arange(n), np.diff(row))
+    for again in (np.ones(len(col), bool), src < col):
+        u, v = np.concatenate([src, src[again]]), np.concatenate([col, col[again]])
+        o = np.lexsort((np.random.default_rng(6).random(len(u)), u))
+        u, v = u[o], v[o].astype(np.int32)
+        r = np.zeros(n + 1, np.int32)
+        np.cumsum(np.bincount(u, minlength=n), out=r[1:])
+        G = gx.Graph.from_csr(r, v, symmetric=True)
+        for s in (0, n - 1, int(np.argmax(np.diff(r)))):
+            exp = oracle.bfs(r, v, s)
+            assert np.array_equal(u32(gx.bfs(G, s)[0]), exp)
+            assert np.array_equal(u32(gx.bfs_do(G, s)[0]), exp)
+        assert np.array_equal(u32(gx.connected_components(G)[0]), oracle.cc(r, v))
+        w = np.random.default_rng(7).integers(1, 200, len(v)).astype(np.uint32)
+        W = gx.Graph.from_csr(r, v, w)
+        for shift in (0, 6, 13):
+            assert np.array_equal(u32(gx.sssp(W, 3, shift)[0]), oracle.sssp(r, v, w, 3, 6))
+        got = u32(gx.sssp_batched(W, [3, 17], 6)[0])
+        assert np.array_equal(got[0], oracle.sssp(r, v, w, 3, 6)) and np.array_equal(got[1], oracle.sssp(r, v, w, 17, 6))
 
 
 def groups_of(row, col, shift, range_edges=2048):
