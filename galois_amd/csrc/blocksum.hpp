@@ -89,6 +89,23 @@ bool pays(int64_t n, int64_t m);
 Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t* perm, int64_t n, int64_t m,
            int shift, bool weighted, BlockSums& cache);
 
+// Runs `prepare` (build and the scratch that goes with it); false, with nothing
+// left of the layout, where device memory does not hold them: the build works in
+// 32 bytes an edge, where the row sweep's plan takes one.  The sums then go
+// through the row sweep.
+template <class F>
+bool fits(BlockSums& cache, F prepare) {
+  try {
+    prepare();
+    return true;
+  } catch (const Error& e) {
+    if (e.code != GX_ERR_ALLOC) throw;
+  }
+  (void)hipGetLastError();  // the failed allocation is dealt with
+  cache = BlockSums{};
+  return false;
+}
+
 // wt[p] = w[eid[p]] (0 where padded).
 void layout_weights(const Plan& P, const float* w, float* wt, hipStream_t s);
 

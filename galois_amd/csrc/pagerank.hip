@@ -417,12 +417,17 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   // here is 20 to 40 sweeps, so that the layout has to pay for itself sooner
   // than in a training loop: 4.1M edges 1.08 -> 0.80 ms a solve, but the first
   // one 4.1 -> 6.3 ms; 20.6M edges 4.13 -> 2.04 ms, the first 9.4 -> 9.6 ms.
-  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && g->m >= (int64_t(1) << 23) && bs::pays(n, g->m);
   rs::RowPlan P{}, PA{};
   bs::Plan S{};
+  Real* partial = nullptr;
+  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && g->m >= (int64_t(1) << 23) && bs::pays(n, g->m) &&
+                    bs::fits(D.sums, [&] {
+                      S = bs::build(g, D.trow.as<int32_t>(), D.tcol.as<int32_t>(), nullptr, n, g->m,
+                                    bs::Shape<Real>::kShift, false, D.sums);
+                      partial = g->scratch<Real>(WS_BC_SIGMA, S.ngroups);
+                    });
   if (sums) {
-    S = bs::build(g, D.trow.as<int32_t>(), D.tcol.as<int32_t>(), nullptr, n, g->m, bs::Shape<Real>::kShift, false,
-                  D.sums);
+    // S
   } else if (blocked) {
     pb::build_layout(g);
     D.pb.vals.ensure(D.pb.ngroups * sizeof(Real));  // grows once for FP64 contributions
@@ -448,7 +453,6 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   double* part_resid = parts;
   double* part_dang = parts + nparts;
   double* carry = blocked || sums ? nullptr : g->scratch<double>(WS_V2, 2 * P.nchunks);
-  Real* partial = sums ? g->scratch<Real>(WS_BC_SIGMA, S.ngroups) : nullptr;
   PrState* state = g->scratch<PrState>(WS_COUNTERS, 1);
   PrState* host = static_cast<PrState*>(g->host_pinned(sizeof(PrState)));
 

@@ -340,16 +340,19 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
   const int64_t n = g->n, m = g->m;
   hipStream_t s = g->stream;
   build_transpose(g);
-  const bool blocked = bs::pays(n, m);
+  bs::Plan L{};
+  float* wl = nullptr;
+  Real* partial = nullptr;
+  const bool blocked = bs::pays(n, m) && bs::fits(g->csc_sums[sizeof(Real) == 8], [&] {
+                         L = bs::build(g, g->trow(), g->tcol(), g->tperm(), n, m, bs::Shape<Real>::kShift, true,
+                                       g->csc_sums[sizeof(Real) == 8]);
+                         wl = g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile);
+                         partial = g->scratch<Real>(WS_BC_SIGMA, L.ngroups);
+                       });
   const rs::RowPlan P = blocked ? rs::RowPlan{} : rs::build_plan(g, g->trow(), g->tcol(), n, m, g->csc_plan);
-  const bs::Plan L = blocked ? bs::build(g, g->trow(), g->tcol(), g->tperm(), n, m, bs::Shape<Real>::kShift, true,
-                                         g->csc_sums[sizeof(Real) == 8])
-                             : bs::Plan{};
   const rs::RowPlan W = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);  // row sums of the weights
   Real* inv_s = g->scratch<Real>(WS_V4, n);
   Real* wt = blocked ? nullptr : g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
-  float* wl = blocked ? g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile) : nullptr;
-  Real* partial = blocked ? g->scratch<Real>(WS_BC_SIGMA, L.ngroups) : nullptr;
   Real* xb = g->scratch<Real>(WS_V0, 2 * n);
   Real* yb = g->scratch<Real>(WS_V1, 2 * n);
   Real* xs[2] = {xb, xb + n};
@@ -404,13 +407,17 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   const int64_t n = g->n, m = g->m;
   hipStream_t s = g->stream;
   const rs::RowPlan P = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);
-  const bool blocked = bs::pays(n, m);
-  const bs::Plan L =
-      blocked ? bs::build(g, g->row, g->col, nullptr, n, m, bs::Shape<Real>::kShift, true, g->csr_sums[sizeof(Real) == 8]) : bs::Plan{};
+  bs::Plan L{};
+  float* wl = nullptr;
+  Real* partial = nullptr;
+  const bool blocked = bs::pays(n, m) && bs::fits(g->csr_sums[sizeof(Real) == 8], [&] {
+                         L = bs::build(g, g->row, g->col, nullptr, n, m, bs::Shape<Real>::kShift, true,
+                                       g->csr_sums[sizeof(Real) == 8]);
+                         wl = g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile);
+                         partial = g->scratch<Real>(WS_BC_SIGMA, L.ngroups);
+                       });
   Real* inv_s = g->scratch<Real>(WS_V4, n);
   Real* wr = blocked ? nullptr : g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
-  float* wl = blocked ? g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile) : nullptr;
-  Real* partial = blocked ? g->scratch<Real>(WS_BC_SIGMA, L.ngroups) : nullptr;
   Real* lb = g->scratch<Real>(WS_V0, 2 * n);
   Real* pl = g->scratch<Real>(WS_V1, n);
   Real* lam[2] = {lb, lb + n};

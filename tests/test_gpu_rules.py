@@ -171,3 +171,43 @@ def test_fp64_pull_states_the_bytes_of_the_path_it_took(gx, n, m):
     with knobs(gx, pr__hot_sources=1000):
         st = gx.pagerank(G, tol=0.0, max_iter=2, precision="fp64")[1]
     assert st.main_kernel_bytes == 4 * m + 8 * (n + 1) + 36 * n + 16 * n
+
+
+def test_sums_without_room_for_the_blocked_layout(gx):
+    """Where device memory holds the row sweep but not the layout of the blocked
+    sums (32 bytes of working memory an edge), a solve takes the row sweep instead
+    of failing, and the layout once there is room again."""
+    import torch
+    G = gx.Graph.rmat(20, 16, symmetric=False, weights="lognormal")
+    n, m = G.n, G.m
+    assert m >= 1 << 23
+    alone = gx.Graph.rmat(20, 16, symmetric=False, weights="lognormal")
+    w = torch.from_numpy(alone.to_host()[2]).cuda()
+    t = torch.full((n,), 1.0 / n, device="cuda")
+    c = torch.linspace(-1, 1, n, device="cuda")
+
+    def solve(H):
+        a = gx.pagerank(H, tol=0.0, max_iter=5, precision="fp64")[0]
+        x = gx.pagerank_weighted(H, w, t, tol=0.0, max_iter=5)[0]
+        return (a, x, *gx.pagerank_adjoint(H, w, x, c, tol=0.0, max_iter=5)[:2])
+
+    exp = [v.cpu().numpy() for v in solve(alone)]
+    alone.free()
+    # What both paths need: the degree order, the transpose, their vectors.
+    with knobs(gx, pr__blocking=0):
+        gx.pagerank(G, tol=0.0, max_iter=1)
+    G.build_transpose()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = 28 * m  # the layouts want more, the row sweeps with their outputs about 16 m
+    free, _ = torch.cuda.mem_get_info()
+    hold = torch.empty(free - room, dtype=torch.uint8, device="cuda")
+    print(f"m={m} free={free} held={free - room}", flush=True)
+    got = [v.cpu().numpy() for v in solve(G)]
+    del hold
+    torch.cuda.empty_cache()
+    again = [v.cpu().numpy() for v in solve(G)]
+    for a, b, e in zip(got, again, exp):
+        rel = 1e-12 if e.dtype == np.float64 else 1e-5
+        assert np.abs(a - e).max() <= rel * np.abs(e).max()
+        assert np.array_equal(b, e)
