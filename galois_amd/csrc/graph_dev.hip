@@ -61,8 +61,8 @@ static void fill(T* p, T v, int64_t n, hipStream_t s) {
   GX_LAUNCHED("fill_kernel");
 }
 
-void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s) {
-  scan_u32_sum(in, out, count, s);
+void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s, uint32_t* tmp) {
+  scan_u32_sum(in, out, count, s, tmp);
 }
 
 __global__ void max_degree_kernel(const int32_t* __restrict__ row, int64_t n, unsigned* __restrict__ out) {
@@ -384,12 +384,12 @@ void ensure_outdeg(gx_graph* g) {
 }
 
 // Source vertex of every CSR edge (uint32[m]) into `src`.
-void edge_sources(const int32_t* row, int64_t n, int64_t m, uint32_t* src, hipStream_t s) {
+void edge_sources(const int32_t* row, int64_t n, int64_t m, uint32_t* src, hipStream_t s, uint32_t* tmp) {
   if (m == 0) return;
   fill<uint32_t>(src, 0u, m, s);
   row_heads_kernel<<<grid_for(n, 256, 1 << 16), 256, 0, s>>>(row, src, n);
   GX_LAUNCHED("row_heads_kernel");
-  inclusive_max_scan_u32(src, src, m, s);
+  inclusive_max_scan_u32(src, src, m, s, tmp);
 }
 
 void build_transpose(gx_graph* g) {

@@ -142,7 +142,8 @@ struct BlockSums {
   bool ready = false;
   int shift = 0, bin_rows = 0;
   int64_t npieces = 0, ntiles = 0, ngroups = 0, nruns = 0, nbins = 0;
-  DevBuf pieces, idx16, eid, tile_grp, row16, runs, bins;
+  bool weighted = false;
+  DevBuf edges, groups;  // idx16 | eid | tile_grp | pieces, and runs | bins | row16
 };
 
 struct DegreeOrder {
@@ -359,9 +360,10 @@ void build_relabeled(gx_graph* g);     // g->relab (degree-ordered CSR, uint32 w
 // out[v] = in[new_of_old[v]] for v < n (results back to the caller's ids).
 void unpermute_u32(const uint32_t* in, const uint32_t* new_of_old, uint32_t* out, int64_t n, hipStream_t s);
 // Source vertex of every CSR edge into src[m].
-void edge_sources(const int32_t* row, int64_t n, int64_t m, uint32_t* src, hipStream_t s);
+// (tmp as of the scans below, of m items.)
+void edge_sources(const int32_t* row, int64_t n, int64_t m, uint32_t* src, hipStream_t s, uint32_t* tmp = nullptr);
 // Exclusive prefix sum of `count` uint32 values into uint32 `out` (may alias).
-void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s);
+void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s, uint32_t* tmp = nullptr);
 // Largest out-degree of the graph (one reduction, then cached).
 int64_t max_degree(gx_graph* g);
 // Whether every edge (u, v) has its reverse (v, u), as often (one pass over the
@@ -371,15 +373,20 @@ bool edges_paired(gx_graph* g);
 // max scan (inclusive), both may run in place; stable ascending LSD radix
 // sort of count < 2^32 keys over bits [0, end_bit) with optional uint32
 // values carried along (inputs are not changed; in and out must differ).
-void scan_u32_sum(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s);
-void inclusive_max_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s);
+// tmp, where a function takes one: scratch of the caller's (scan_words(count) or
+// sort_words(count) words), with which nothing is allocated and nothing waited for.
+int64_t scan_words(int64_t count);
+int64_t sort_words(int64_t count);
+void scan_u32_sum(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s, uint32_t* tmp = nullptr);
+void inclusive_max_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s, uint32_t* tmp = nullptr);
 void radix_sort_u64(const uint64_t* kin, uint64_t* kout, const uint32_t* vin, uint32_t* vout, int64_t count,
                     int end_bit, hipStream_t s);
 // Ascending radix sort of count keys over bits [0, end_bit) (in is not changed).
+void sort_keys_u64(const uint64_t* in, uint64_t* out, int64_t count, int end_bit, hipStream_t s);
 // The same sort of a's keys with b (as long) as the other buffer: returns the
 // one that holds the result, the other's contents are lost.
-uint64_t* radix_sort_pair_u64(uint64_t* a, uint64_t* b, int64_t count, int end_bit, hipStream_t s);
-void sort_keys_u64(const uint64_t* in, uint64_t* out, int64_t count, int end_bit, hipStream_t s);
+uint64_t* radix_sort_pair_u64(uint64_t* a, uint64_t* b, int64_t count, int end_bit, hipStream_t s,
+                              uint32_t* tmp = nullptr);
 // Out-edge chunks of the CSR: every vertex's adjacency cut into pieces of at
 // most kEdgeChunk edges, (vertex, first edge) per chunk in vertex order;
 // built once per graph and kept with it (bc.hip).

@@ -123,9 +123,10 @@ __global__ void __launch_bounds__(kScanBlock) scan_tile_kernel(const uint32_t* i
 }
 
 // Scan of `count` items of in into out (may alias), exclusive or inclusive,
-// starting at 0.  Tile totals are scanned by the same routine.
+// starting at 0.  Tile totals (tmp: scan_words(count)) are scanned by the same
+// routine.
 template <class Op>
-void scan_u32(const uint32_t* in, uint32_t* out, int64_t count, bool exclusive, Op op, hipStream_t s) {
+void scan_u32(const uint32_t* in, uint32_t* out, int64_t count, bool exclusive, Op op, hipStream_t s, uint32_t* tmp) {
   if (count <= 0) return;
   const int64_t tiles = (count + kScanTile - 1) / kScanTile;
   GX_REQUIRE(tiles < (int64_t(1) << 31), "scan too large");
@@ -137,20 +138,25 @@ void scan_u32(const uint32_t* in, uint32_t* out, int64_t count, bool exclusive, 
     GX_LAUNCHED("scan_tile_kernel");
     return;
   }
-  DevBuf tot;
-  tot.ensure(tiles * 4);
-  scan_reduce_kernel<Op><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, count, tot.as<uint32_t>(), op);
+  scan_reduce_kernel<Op><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, count, tmp, op);
   GX_LAUNCHED("scan_reduce_kernel");
-  scan_u32(tot.as<uint32_t>(), tot.as<uint32_t>(), tiles, true, op, s);
+  scan_u32(tmp, tmp, tiles, true, op, s, tmp + tiles);
   if (exclusive)
-    scan_tile_kernel<Op, true><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, count, tot.as<uint32_t>(),
-                                                                                   out, op);
+    scan_tile_kernel<Op, true><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, count, tmp, out, op);
   else
-    scan_tile_kernel<Op, false><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, count, tot.as<uint32_t>(),
-                                                                                    out, op);
+    scan_tile_kernel<Op, false><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, count, tmp, out, op);
   GX_LAUNCHED("scan_tile_kernel");
-  // `tot` is freed when this returns: wait for the launches that read it
-  GX_HIP(hipStreamSynchronize(s));
+}
+
+// The same with scratch of its own where the caller has none.
+template <class Op>
+void scan_alone(const uint32_t* in, uint32_t* out, int64_t count, bool exclusive, Op op, hipStream_t s,
+                uint32_t* tmp) {
+  const int64_t words = tmp ? 0 : scan_words(count);
+  DevBuf own;
+  if (words > 0) own.ensure(words * 4);
+  scan_u32(in, out, count, exclusive, op, s, tmp ? tmp : own.as<uint32_t>());
+  if (words > 0) GX_HIP(hipStreamSynchronize(s));  // `own` is freed when this returns
 }
 
 // ------------------------------------------------------------ radix sort
@@ -268,12 +274,23 @@ __global__ void __launch_bounds__(kSortBlock) radix_scatter_kernel(const uint64_
 
 }  // namespace
 
-void scan_u32_sum(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s) {
-  scan_u32(in, out, count, true, SumOp{}, s);
+int64_t scan_words(int64_t count) {
+  int64_t words = 0;
+  for (int64_t t = (count + kScanTile - 1) / kScanTile; t > 1; t = (t + kScanTile - 1) / kScanTile) words += t;
+  return words;
 }
 
-void inclusive_max_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s) {
-  scan_u32(in, out, count, false, MaxOp{}, s);
+int64_t sort_words(int64_t count) {
+  const int64_t tiles = (count + kSortTile - 1) / kSortTile;
+  return tiles * kDigits + scan_words(tiles * kDigits);
+}
+
+void scan_u32_sum(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s, uint32_t* tmp) {
+  scan_alone(in, out, count, true, SumOp{}, s, tmp);
+}
+
+void inclusive_max_scan_u32(const uint32_t* in, uint32_t* out, int64_t count, hipStream_t s, uint32_t* tmp) {
+  scan_alone(in, out, count, false, MaxOp{}, s, tmp);
 }
 
 void radix_sort_u64(const uint64_t* kin, uint64_t* kout, const uint32_t* vin, uint32_t* vout, int64_t count,
@@ -293,10 +310,15 @@ void radix_sort_u64(const uint64_t* kin, uint64_t* kout, const uint32_t* vin, ui
   }
   const int64_t tiles = (count + kSortTile - 1) / kSortTile;
   GX_REQUIRE(tiles * kDigits < (int64_t(1) << 32), "sort: too many tiles");
-  DevBuf tk, tv, counts;
-  tk.ensure(count * 8);
-  if (vals) tv.ensure(count * 4);
-  counts.ensure(tiles * kDigits * 4);
+  // One allocation: the other key (and value) buffer of several passes, the
+  // counts with their scan's scratch.
+  const int64_t other = passes > 1 ? count : 0;
+  DevBuf scratch;
+  scratch.ensure(other * (vals ? 12 : 8) + sort_words(count) * 4);
+  uint64_t* const tk = scratch.as<uint64_t>();
+  uint32_t* const tv = reinterpret_cast<uint32_t*>(tk + other);
+  uint32_t* const counts = tv + (vals ? other : 0);
+  uint32_t* const tmp = counts + tiles * kDigits;
   const uint64_t* sk = kin;
   const uint32_t* sv = vin;
   for (int p = 0; p < passes; ++p) {
@@ -304,45 +326,48 @@ void radix_sort_u64(const uint64_t* kin, uint64_t* kout, const uint32_t* vin, ui
     const int bits = std::min(8, end_bit - shift);
     const uint32_t mask = (1u << bits) - 1u;
     const bool to_out = (passes - p) % 2 == 1;  // the last pass writes the output
-    uint64_t* dk = to_out ? kout : tk.as<uint64_t>();
-    uint32_t* dv = vals ? (to_out ? vout : tv.as<uint32_t>()) : nullptr;
-    radix_hist_kernel<<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(sk, count, shift, mask,
-                                                                          counts.as<uint32_t>(), tiles);
+    uint64_t* dk = to_out ? kout : tk;
+    uint32_t* dv = vals ? (to_out ? vout : tv) : nullptr;
+    radix_hist_kernel<<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(sk, count, shift, mask, counts, tiles);
     GX_LAUNCHED("radix_hist_kernel");
-    scan_u32(counts.as<uint32_t>(), counts.as<uint32_t>(), tiles * kDigits, true, SumOp{}, s);
+    scan_u32(counts, counts, tiles * kDigits, true, SumOp{}, s, tmp);
     if (vals)
       radix_scatter_kernel<true><<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(
-          sk, sv, count, shift, mask, counts.as<uint32_t>(), tiles, dk, dv);
+          sk, sv, count, shift, mask, counts, tiles, dk, dv);
     else
       radix_scatter_kernel<false><<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(
-          sk, nullptr, count, shift, mask, counts.as<uint32_t>(), tiles, dk, nullptr);
+          sk, nullptr, count, shift, mask, counts, tiles, dk, nullptr);
     GX_LAUNCHED("radix_scatter_kernel");
     sk = dk;
     sv = dv;
   }
-  GX_HIP(hipStreamSynchronize(s));  // scratch buffers are freed on return
+  GX_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
 }
 
-uint64_t* radix_sort_pair_u64(uint64_t* a, uint64_t* b, int64_t count, int end_bit, hipStream_t s) {
+uint64_t* radix_sort_pair_u64(uint64_t* a, uint64_t* b, int64_t count, int end_bit, hipStream_t s,
+                              uint32_t* counts) {
   GX_REQUIRE(count >= 0 && count < (int64_t(1) << 32), "sort: too many keys");
   GX_REQUIRE(end_bit >= 0 && end_bit <= 64, "sort: bad bit range");
   if (count == 0) return a;
   const int64_t tiles = (count + kSortTile - 1) / kSortTile;
   GX_REQUIRE(tiles * kDigits < (int64_t(1) << 32), "sort: too many tiles");
-  DevBuf counts;
-  counts.ensure(tiles * kDigits * 4);
+  DevBuf own;
+  if (!counts) {
+    own.ensure(sort_words(count) * 4);
+    counts = own.as<uint32_t>();
+  }
+  uint32_t* const tmp = counts + tiles * kDigits;
   for (int shift = 0; shift < end_bit; shift += 8) {
     const uint32_t mask = (1u << std::min(8, end_bit - shift)) - 1u;
-    radix_hist_kernel<<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(a, count, shift, mask,
-                                                                          counts.as<uint32_t>(), tiles);
+    radix_hist_kernel<<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(a, count, shift, mask, counts, tiles);
     GX_LAUNCHED("radix_hist_kernel");
-    scan_u32(counts.as<uint32_t>(), counts.as<uint32_t>(), tiles * kDigits, true, SumOp{}, s);
+    scan_u32(counts, counts, tiles * kDigits, true, SumOp{}, s, tmp);
     radix_scatter_kernel<false><<<static_cast<unsigned>(tiles), kSortBlock, 0, s>>>(
-        a, nullptr, count, shift, mask, counts.as<uint32_t>(), tiles, b, nullptr);
+        a, nullptr, count, shift, mask, counts, tiles, b, nullptr);
     GX_LAUNCHED("radix_scatter_kernel");
     std::swap(a, b);
   }
-  GX_HIP(hipStreamSynchronize(s));  // the counts are freed on return
+  if (own.p) GX_HIP(hipStreamSynchronize(s));  // freed on return
   return a;
 }
 
