@@ -20,6 +20,9 @@ namespace {
 constexpr int kB = 256;
 constexpr double kAvgRun = 16.0;
 constexpr uint32_t kNone = 0xffffffffu;
+// 16: at 64 and 256 a graph without hubs keeps its error (1.06e-16 against 0.67e-16)
+// and the solves take as long.
+constexpr uint32_t kPairRow = 16, kHalveRow = 64;
 constexpr uint32_t kFirst = 1u << 31;  // grow: first group of a wavefront's range
 
 unsigned grid(int64_t n) { return grid_for(n, kB, 16384); }
@@ -169,12 +172,18 @@ __global__ void weights_kernel(const uint32_t* __restrict__ eid, const float* __
   }
 }
 
+// Per block of 2^shift rows: its edges, and those of its longest row.  One
+// wavefront per block.
 __global__ void block_edges_kernel(const int32_t* __restrict__ rowoff, int64_t n, int shift, int64_t nblocks,
-                                   uint32_t* __restrict__ out) {
-  for (int64_t b = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x; b < nblocks;
-       b += static_cast<int64_t>(gridDim.x) * kB) {
+                                   uint2* __restrict__ out) {
+  const int64_t nw = static_cast<int64_t>(gridDim.x) * (kB / kWave);
+  for (int64_t b = blockIdx.x * static_cast<int64_t>(kB / kWave) + threadIdx.x / kWave; b < nblocks; b += nw) {
     const int64_t r0 = b << shift, r1 = std::min<int64_t>(n, (b + 1) << shift);
-    out[b] = static_cast<uint32_t>(rowoff[r1] - rowoff[r0]);
+    uint32_t longest = 0;
+    for (int64_t r = r0 + lane_id(); r < r1; r += kWave)
+      longest = max(longest, static_cast<uint32_t>(rowoff[r + 1] - rowoff[r]));
+    longest = wave_max(longest);
+    if (lane_id() == 0) out[b] = make_uint2(static_cast<uint32_t>(rowoff[r1] - rowoff[r0]), longest);
   }
 }
 
@@ -218,7 +227,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
     P.ngroups = L.ngroups;
     P.nruns = L.nruns;
     P.nbins = L.nbins;
-    P.bin_rows = L.bin_rows;
+    P.lds_sums = L.lds_sums;
     return P;
   };
   if (L.ready && L.shift == shift) return view();
@@ -235,7 +244,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   const size_t area_a = (m + 2) * 8, area_b = (m + 2) * 8, area_c = (m + 2) * 4, area_d = most_tiles * kTile * 8,
                area_e = (m + 2) * 4;
   const int64_t most_blocks = n / 512 + 1, most_bins = n / 16 + most_blocks + 1;
-  const size_t tables = 2 * (nchunks + 1) * 4 + most_tiles + 9 * most_blocks + 8 * (most_bins + 1) + 16 * 256;
+  const size_t tables = 2 * (nchunks + 1) * 4 + most_tiles + 13 * most_blocks + 8 * (most_bins + 1) + 16 * 256;
   const size_t scratch = std::max(sort_words(m), scan_words(m + 2)) * 4;
   DevBuf work;
   work.ensure(up(area_a) + up(area_b) + up(area_c) + up(area_d) + up(area_e) + up(scratch) + tables);
@@ -270,7 +279,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   // its workgroup and at most 32 (64K edges, against which the staging of the
   // chunk costs little), and about a thousand pieces spread a graph over the
   // CUs.
-  const int64_t waves = shift == Shape<float>::kShift ? Shape<float>::kBlock / kWave : Shape<double>::kBlock / kWave;
+  constexpr int64_t waves = kGatherBlock / kWave;
   const uint32_t kPieceTiles = static_cast<uint32_t>(
       kRangeTiles * std::min<int64_t>(32, std::max<int64_t>(waves, m / (int64_t(1024) * kRangeTiles * kTile))));
   std::vector<Piece> pieces;
@@ -317,35 +326,47 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   group_kernel<<<grid(nt * int64_t(kWave)), kB, 0, s>>>(idx16, prow, nt, tile_grp, first, grow);
   GX_LAUNCHED("bs::group_kernel");
   // 4. Bins: rows per block so that a run holds about 16 groups (a quarter of
-  // a wavefront's lanes), between 512 and 4096 (4 and 32 KB of LDS sums).
+  // a wavefront's lanes), between 512 and 4096 (4 and 32 KB of LDS sums).  FP64
+  // vectors have two sums a row in bins with rows of more than kPairRow edges, 8 to
+  // 32 KB up to 2048 rows.  With 64 KB for 4096 rows too few wavefronts fit a CU
+  // (RMAT-26 245 ms a solve -> 551), and with 2048 the runs are half as long (418),
+  // so blocks of 4096 rows have them only where they are halved, which one with a
+  // row of more than kHalveRow edges is.
   int bshift = 9;
   while (bshift < 12 && static_cast<double>(ng) * (int64_t(1) << bshift) < kAvgRun * static_cast<double>(nchunks) * n) ++bshift;
   const int64_t nblocks = (n + (int64_t(1) << bshift) - 1) >> bshift;
-  uint32_t* bedges = reinterpret_cast<uint32_t*>(take(nblocks * 4));
-  block_edges_kernel<<<grid(nblocks), kB, 0, s>>>(rowoff, n, bshift, nblocks, bedges);
+  uint2* bedges = reinterpret_cast<uint2*>(take(nblocks * 8));
+  block_edges_kernel<<<grid(nblocks * kWave), kB, 0, s>>>(rowoff, n, bshift, nblocks, bedges);
   GX_LAUNCHED("bs::block_edges_kernel");
-  std::vector<uint32_t> hedges(nblocks), hbin(nblocks);
+  std::vector<uint2> hedges(nblocks);
+  std::vector<uint32_t> hbin(nblocks), brows;
   std::vector<uint8_t> hshift(nblocks);
-  read_bytes(g, hedges.data(), bedges, nblocks * 4);
+  read_bytes(g, hedges.data(), bedges, nblocks * 8);
+  const bool f64 = shift == Shape<double>::kShift;
+  const int lds_sums = f64 && bshift < 12 ? 2 << bshift : 1 << bshift;
   std::vector<uint32_t> brow;
   // A block is halved until its groups (at most its edges, and a row's at most
   // the chunks) are within three times the average or 16 rows are left.
   const double most = 3.0 * std::max(1.0, static_cast<double>(ng) / static_cast<double>(nblocks));
   for (int64_t b = 0; b < nblocks; ++b) {
     int sh = bshift;
-    double w = std::min<double>(hedges[b], static_cast<double>(nchunks) * (int64_t(1) << bshift));
-    while (sh > 4 && w > most) {
+    double w = std::min<double>(hedges[b].x, static_cast<double>(nchunks) * (int64_t(1) << bshift));
+    while (sh > 4 && (w > most || (f64 && hedges[b].y > kHalveRow && (2 << sh) > lds_sums))) {
       w /= 2;
       --sh;
     }
     hbin[b] = static_cast<uint32_t>(brow.size());
     hshift[b] = static_cast<uint8_t>(sh);
     const int64_t r0 = b << bshift, r1 = std::min<int64_t>(n, (b + 1) << bshift);
-    for (int64_t r = r0; r < r1; r += int64_t(1) << sh) brow.push_back(static_cast<uint32_t>(r));
+    const uint32_t pair = f64 && hedges[b].y > kPairRow && (2 << sh) <= lds_sums ? kPair : 0u;
+    for (int64_t r = r0; r < r1; r += int64_t(1) << sh) {
+      brow.push_back(static_cast<uint32_t>(r));
+      brows.push_back(static_cast<uint32_t>(std::min<int64_t>(r1 - r, int64_t(1) << sh)) | pair);
+    }
   }
   L.nbins = static_cast<int64_t>(brow.size());
   brow.push_back(static_cast<uint32_t>(n));
-  L.bin_rows = 1 << bshift;
+  L.lds_sums = lds_sums;
   uint32_t* drow = reinterpret_cast<uint32_t*>(take(brow.size() * 4));
   uint32_t* dbin = reinterpret_cast<uint32_t*>(take(nblocks * 4));
   uint8_t* dshift = reinterpret_cast<uint8_t*>(take(nblocks));
@@ -382,7 +403,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   std::vector<uint32_t> hoffs(L.nbins + 1);
   read_bytes(g, hoffs.data(), boff, hoffs.size() * 4);
   std::vector<Bin> bins(L.nbins);
-  for (int64_t b = 0; b < L.nbins; ++b) bins[b] = Bin{brow[b], brow[b + 1] - brow[b], hoffs[b], hoffs[b + 1]};
+  for (int64_t b = 0; b < L.nbins; ++b) bins[b] = Bin{brow[b], brows[b], hoffs[b], hoffs[b + 1]};
   std::stable_sort(bins.begin(), bins.end(), [](const Bin& a, const Bin& b) { return a.run1 - a.run0 > b.run1 - b.run0; });
   GX_HIP(hipMemcpyAsync(const_cast<Bin*>(P.bins), bins.data(), bins.size() * sizeof(Bin), hipMemcpyHostToDevice, s));
   GX_HIP(hipStreamSynchronize(s));  // the host tables above are read by then

@@ -48,17 +48,18 @@ constexpr int kRangeTiles = 4;           // tiles of one wavefront's range: a gr
 constexpr uint32_t kEnd = 1u << 15;      // idx16 flag: last edge of a group
 constexpr int kSumGrid = 256 * 16;       // most wavefronts of phase 2
 
-// Gathered entries per chunk (64 KB of LDS) and lanes per workgroup of phase 1:
-// with the tiles' group sums both precisions then keep 16 wavefronts on a CU.
+// Gathered entries per chunk: 64 KB of LDS.  With the tiles' group sums (FP64 for
+// both precisions, 64 KB) a CU holds one workgroup of phase 1, 16 wavefronts.
+constexpr int kGatherBlock = 1024;
 template <class Real>
 struct Shape;
 template <>
 struct Shape<float> {
-  static constexpr int kShift = 14, kBlock = 512;
+  static constexpr int kShift = 14;
 };
 template <>
 struct Shape<double> {
-  static constexpr int kShift = 13, kBlock = 1024;
+  static constexpr int kShift = 13;
 };
 
 struct Piece {
@@ -66,8 +67,11 @@ struct Piece {
 };
 
 struct Bin {
-  uint32_t row0, rows, run0, run1;
+  uint32_t row0;
+  uint32_t rows;  // with kPair: a row's sum is kept as two, see sum_kernel
+  uint32_t run0, run1;
 };
+constexpr uint32_t kPair = 1u << 31;
 
 struct Plan {
   const Piece* pieces;
@@ -78,7 +82,7 @@ struct Plan {
   const uint2* runs;         // per bin, in chunk order: first group, length (at most kWave)
   const Bin* bins;           // nbins, most runs first
   int64_t npieces, ntiles, ngroups, nruns, nbins;
-  int bin_rows;              // most rows of a bin (LDS sums)
+  int lds_sums;              // LDS doubles a bin has for its sums
 };
 
 // Whether the layout pays for and can be built for this shape (see blocksum.hip).
@@ -149,22 +153,22 @@ struct TileLoad {
 
 // Phase 1 (see the file comment).  y: n entries.
 template <class Real, bool W>
-__global__ void __launch_bounds__(Shape<Real>::kBlock) gather_kernel(Plan P, const float* __restrict__ wt,
-                                                                     const Real* __restrict__ y, int64_t n,
-                                                                     Real* __restrict__ partial,
-                                                                     const unsigned* __restrict__ skip) {
+__global__ void __launch_bounds__(kGatherBlock) gather_kernel(Plan P, const float* __restrict__ wt,
+                                                              const Real* __restrict__ y, int64_t n,
+                                                              double* __restrict__ partial,
+                                                              const unsigned* __restrict__ skip) {
   if (skip && *skip) return;
-  constexpr int kSpan = 1 << Shape<Real>::kShift, kBlock = Shape<Real>::kBlock, kWaves = kBlock / kWave;
+  constexpr int kSpan = 1 << Shape<Real>::kShift, kWaves = kGatherBlock / kWave;
   __shared__ Real ys[kSpan];
-  __shared__ Real stage[kWaves][kTile];
+  __shared__ double stage[kWaves][kTile];
   const Piece pc = P.pieces[blockIdx.x];
   const int64_t base = static_cast<int64_t>(pc.chunk) * kSpan;
   const int cnt = static_cast<int>(n - base < kSpan ? n - base : kSpan);
-  for (int i = threadIdx.x; i < cnt; i += kBlock) ys[i] = y[base + i];
+  for (int i = threadIdx.x; i < cnt; i += kGatherBlock) ys[i] = y[base + i];
   __syncthreads();
   const int lane = static_cast<int>(lane_id());
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  Real* st = stage[wid];
+  double* st = stage[wid];
   for (int64_t r0 = pc.tile0 + wid * kRangeTiles; r0 < pc.tile1; r0 += kWaves * kRangeTiles) {
     const int64_t r1 = r0 + kRangeTiles < pc.tile1 ? r0 + kRangeTiles : pc.tile1;
     double open = 0;  // sum of the group open at the start of the tile (uniform)
@@ -191,18 +195,19 @@ __global__ void __launch_bounds__(Shape<Real>::kBlock) gather_kernel(Plan P, con
       const uint64_t heads = __ballot(ends != 0);
       const uint64_t upto = heads & (~0ull >> (63 - lane));
       const double seg = rs::wave_seg_scan(tail, upto ? 63 - __builtin_clzll(upto) : 0, lane);
-      double acc = __shfl_up(seg, 1);
-      if (lane == 0) acc = 0;
-      if ((heads & ((1ull << lane) - 1)) == 0) acc += open;
+      double before = __shfl_up(seg, 1);
+      if (lane == 0) before = 0;
+      if ((heads & ((1ull << lane) - 1)) == 0) before += open;
       const double last = __shfl(seg, kWave - 1);
       open = heads ? last : open + last;
       uint32_t slot = wave_exclusive_sum(static_cast<uint32_t>(__popc(ends)), lane);
+      double acc = 0;
 #pragma unroll
       for (int u = 0; u < kItems; ++u) {
         acc += v[u];
         if ((ends >> u) & 1u) {
-          st[slot++] = static_cast<Real>(acc);
-          acc = 0;
+          st[slot++] = before + acc;
+          before = acc = 0;
         }
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -219,29 +224,36 @@ __global__ void __launch_bounds__(Shape<Real>::kBlock) gather_kernel(Plan P, con
 // is a chain of short loads (a run is about half a wavefront's lanes), so 16
 // runs are in flight at a time and the next 64 runs' descriptors are loaded
 // ahead: with 4 in flight it took 2-3 times as long.
-template <class Real, class Fin>
-__global__ void __launch_bounds__(kWave) sum_kernel(Plan P, const Real* __restrict__ partial, Fin fin,
+//
+// PAIRS (FP64 vectors): a row of k partial sums, added one after another, is off
+// by 0.3 * sqrt(k / 3) units of its last place, where a sweep that sums values
+// among themselves first stays near half a unit.  In bins with rows of more than
+// kPairRow edges a row therefore has two sums, and the second collects what the
+// additions to the first round off (Knuth's TwoSum; the LDS addition returns what
+// it was added to), so that the row is rounded once.  Relative L2 errors over 8
+// graphs of 700,000 vertices 1.65e-16 -> 1.34e-16 (gather by gather, 512-lane
+// merge-path tiles: 1.40e-16), 600,000 vertices without hubs 1.06 -> 0.67e-16
+// (0.89); PageRank of 1.5 M vertices 2.07 -> 2.31 ms a
+// solve.
+template <bool PAIRS, class Fin>
+__global__ void __launch_bounds__(kWave) sum_kernel(Plan P, const double* __restrict__ partial, Fin fin,
                                                     double* __restrict__ part0, double* __restrict__ part1,
                                                     const unsigned* __restrict__ skip) {
   if (skip && *skip) return;
   fin.load();
   extern __shared__ double acc[];
   const int lane = static_cast<int>(lane_id());
-  double a0 = 0, a1 = 0;
+  rs::DoubleSum a0, a1;  // a lane meets 64 rows a bin, often of one and the same value
   constexpr int kRuns = 16;
   for (int64_t b = blockIdx.x; b < P.nbins; b += gridDim.x) {
     const Bin bin = P.bins[b];
     const uint32_t row0 = bin.row0, q0 = bin.run0, q1 = bin.run1;
-    const int rows = static_cast<int>(bin.rows);
+    const int rows = static_cast<int>(bin.rows & ~kPair);
+    const bool pair = PAIRS && (bin.rows & kPair);
+    double* const low = acc + rows;  // with pair
     uint2 next{0, 0};
     if (q0 + lane < q1) next = P.runs[q0 + lane];
-    // A halved bin has room for several sums per row, which take the runs in
-    // turn: its rows are those with many partial sums, and fewer additions one
-    // after another round less (FP64 PageRank of 1.5 M vertices, relative L2
-    // error 3.7e-16 with one, 1.2e-16 with these, as gather by gather).
-    int copies = 1;
-    while (2 * copies * rows <= P.bin_rows && copies < kRuns) copies *= 2;
-    for (int i = lane; i < copies * rows; i += kWave) acc[i] = 0;
+    for (int i = lane; i < (pair ? 2 * rows : rows); i += kWave) acc[i] = 0;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     for (uint32_t q = q0; q < q1; q += kWave) {
@@ -251,65 +263,78 @@ __global__ void __launch_bounds__(kWave) sum_kernel(Plan P, const Real* __restri
       const int nr = static_cast<int>(q1 - q < kWave ? q1 - q : kWave);
       for (int i = 0; i < nr; i += kRuns) {
         uint32_t r[kRuns];
-        Real x[kRuns];
+        double x[kRuns];
 #pragma unroll
         for (int k = 0; k < kRuns; ++k) {
           const uint32_t g = __builtin_amdgcn_readlane(mine.x, i + k), len = __builtin_amdgcn_readlane(mine.y, i + k);
           r[k] = 0;
-          x[k] = Real(0);
+          x[k] = 0;
           if (static_cast<uint32_t>(lane) < len) {
             r[k] = P.row16[g + lane];
             x[k] = partial[g + lane];
           }
         }
+        auto in_run = [&](int k) {
+          return static_cast<uint32_t>(lane) < static_cast<uint32_t>(__builtin_amdgcn_readlane(mine.y, i + k));
+        };
+        if (pair) {
+          double was[kRuns];
 #pragma unroll
-        for (int k = 0; k < kRuns; ++k)
-          if (static_cast<uint32_t>(lane) < static_cast<uint32_t>(__builtin_amdgcn_readlane(mine.y, i + k)))
-            atomicAdd(&acc[(k & (copies - 1)) * rows + r[k]], static_cast<double>(x[k]));
+          for (int k = 0; k < kRuns; ++k)
+            if (in_run(k)) was[k] = atomicAdd(&acc[r[k]], x[k]);
+#pragma unroll
+          for (int k = 0; k < kRuns; ++k)
+            if (in_run(k)) {
+              const double t = was[k] + x[k], b = t - was[k];
+              atomicAdd(&low[r[k]], (was[k] - (t - b)) + (x[k] - b));
+            }
+        } else {
+#pragma unroll
+          for (int k = 0; k < kRuns; ++k)
+            if (in_run(k)) atomicAdd(&acc[r[k]], x[k]);
+        }
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    for (int h = copies / 2; h > 0; h /= 2) {
-      for (int i = lane; i < h * rows; i += kWave) acc[i] += acc[i + h * rows];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
     constexpr int kU = 4;
     for (int i = lane; i < rows; i += kU * kWave) {
       typename Fin::Pre pre[kU];
 #pragma unroll
       for (int k = 0; k < kU; ++k)
         if (i + k * kWave < rows) pre[k] = fin.pre(row0 + i + k * kWave);
+      double t0 = 0, t1 = 0;
 #pragma unroll
       for (int k = 0; k < kU; ++k)
-        if (i + k * kWave < rows) fin(row0 + i + k * kWave, acc[i + k * kWave], pre[k], a0, a1);
+        if (const int j = i + k * kWave; j < rows)
+          fin(row0 + j, pair ? rs::DoubleSum{acc[j], low[j]}.value() : acc[j], pre[k], t0, t1);
+      a0.add(t0);
+      a1.add(t1);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  a0 = wave_sum(a0);
-  a1 = wave_sum(a1);
+  const double s0 = wave_sum(a0.value()), s1 = wave_sum(a1.value());
   if (lane == 0) {
-    part0[blockIdx.x] = a0;
-    part1[blockIdx.x] = a1;
+    part0[blockIdx.x] = s0;
+    part1[blockIdx.x] = s1;
   }
 }
 
 // Host: one sweep; wt null: unweighted.  Returns the number of partials
 // written to part0/part1 (at most kSumGrid).
 template <class Real, class Fin>
-int launch(const Plan& P, const float* wt, const Real* y, int64_t n, Real* partial, const Fin& fin,
+int launch(const Plan& P, const float* wt, const Real* y, int64_t n, double* partial, const Fin& fin,
            const unsigned* skip, double* part0, double* part1, hipStream_t s) {
   if (P.npieces > 0) {
     if (wt)
-      gather_kernel<Real, true><<<static_cast<unsigned>(P.npieces), Shape<Real>::kBlock, 0, s>>>(P, wt, y, n, partial, skip);
+      gather_kernel<Real, true><<<static_cast<unsigned>(P.npieces), kGatherBlock, 0, s>>>(P, wt, y, n, partial, skip);
     else
-      gather_kernel<Real, false><<<static_cast<unsigned>(P.npieces), Shape<Real>::kBlock, 0, s>>>(P, wt, y, n, partial, skip);
+      gather_kernel<Real, false><<<static_cast<unsigned>(P.npieces), kGatherBlock, 0, s>>>(P, wt, y, n, partial, skip);
     GX_LAUNCHED("bs::gather_kernel");
   }
   const int grid = static_cast<int>(std::min<int64_t>(P.nbins, kSumGrid));
-  sum_kernel<Real, Fin><<<grid, kWave, P.bin_rows * sizeof(double), s>>>(P, partial, fin, part0, part1, skip);
+  sum_kernel<sizeof(Real) == 8, Fin><<<grid, kWave, P.lds_sums * sizeof(double), s>>>(P, partial, fin, part0, part1, skip);
   GX_LAUNCHED("bs::sum_kernel");
   return grid;
 }

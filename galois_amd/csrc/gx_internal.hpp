@@ -140,7 +140,7 @@ struct PbLayout {
 // 2^shift gathered entries, built once per graph.
 struct BlockSums {
   bool ready = false;
-  int shift = 0, bin_rows = 0;
+  int shift = 0, lds_sums = 0;
   int64_t npieces = 0, ntiles = 0, ngroups = 0, nruns = 0, nbins = 0;
   bool weighted = false;
   DevBuf edges, groups;  // idx16 | eid | tile_grp | pieces, and runs | bins | row16

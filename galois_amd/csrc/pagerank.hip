@@ -61,12 +61,18 @@ struct PrState {
   double base;       // (1-a)/n + a*D/n for the next sweep
   double alpha;
   double tol;
-  double inv_n;
+  double n;
   unsigned converged;
   unsigned iters;
   unsigned final_buf;  // x buffer holding the latest iterate
   unsigned max_iter;
 };
+
+// (1 - a)/n + a*D/n in two roundings: every rank has the same, so that what it is
+// off by adds up over the vertices and the iterations instead of averaging out.
+__device__ __forceinline__ double pr_base(const PrState& s, double dang) {
+  return fma(s.alpha, dang, 1.0 - s.alpha) / s.n;
+}
 
 template <class Real>
 struct PrSrc {
@@ -248,7 +254,7 @@ struct PrClose {
   __device__ __forceinline__ void operator()(double r, double d) const {
     state->resid = r;
     state->dang = d;
-    state->base = (1.0 - state->alpha) * state->inv_n + state->alpha * d * state->inv_n;
+    state->base = pr_base(*state, d);
     state->iters += 1;
     state->final_buf = newest_buf;
     if (r < state->tol || state->iters >= state->max_iter) state->converged = 1;
@@ -261,14 +267,13 @@ __global__ void __launch_bounds__(kBlock) pr_reduce_kernel(PrState* state, const
                                                            unsigned newest_buf) {
   if (state->converged) return;
   __shared__ double red[kBlock / kWave];
-  double r = 0, d = 0;
+  rs::DoubleSum r, d;
   for (int i = threadIdx.x; i < nparts; i += kBlock) {
-    r += part_resid[i];
-    d += part_dang[i];
+    r.add(part_resid[i]);
+    d.add(part_dang[i]);
   }
-  r = block_sum(r, red);
-  d = block_sum(d, red);
-  if (threadIdx.x == 0) PrClose{state, newest_buf}(r, d);
+  const double resid = block_sum(r.value(), red), dang = block_sum(d.value(), red);
+  if (threadIdx.x == 0) PrClose{state, newest_buf}(resid, dang);
 }
 
 // x0 = 1/n, y0 = x0/outdeg; dangling partials.
@@ -290,14 +295,14 @@ __global__ void __launch_bounds__(kBlock) pr_init_kernel(Real* __restrict__ x, R
   if (threadIdx.x == 0) part_dang[blockIdx.x] = dang;
 }
 
-__global__ void pr_state_init_kernel(PrState* s, double alpha, double tol, double inv_n, unsigned max_iter) {
+__global__ void pr_state_init_kernel(PrState* s, double alpha, double tol, double n, unsigned max_iter) {
   if (threadIdx.x == 0) {
     s->resid = 0;
     s->dang = 0;
     s->base = 0;
     s->alpha = alpha;
     s->tol = tol;
-    s->inv_n = inv_n;
+    s->n = n;
     s->converged = 0;
     s->iters = 0;
     s->final_buf = 0;
@@ -313,7 +318,7 @@ __global__ void pr_init_reduce_kernel(PrState* state, const double* __restrict__
   d = block_sum(d, red);
   if (threadIdx.x == 0) {
     state->dang = d;
-    state->base = (1.0 - state->alpha) * state->inv_n + state->alpha * d * state->inv_n;
+    state->base = pr_base(*state, d);
     if (state->max_iter == 0) state->converged = 1;
   }
 }
@@ -419,12 +424,12 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   // one 4.1 -> 6.3 ms; 20.6M edges 4.13 -> 2.04 ms, the first 9.4 -> 9.6 ms.
   rs::RowPlan P{}, PA{};
   bs::Plan S{};
-  Real* partial = nullptr;
+  double* partial = nullptr;
   const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && g->m >= (int64_t(1) << 23) && bs::pays(n, g->m) &&
                     bs::fits(D.sums, [&] {
                       S = bs::build(g, D.trow.as<int32_t>(), D.tcol.as<int32_t>(), nullptr, n, g->m,
                                     bs::Shape<Real>::kShift, false, D.sums);
-                      partial = g->scratch<Real>(WS_BC_SIGMA, S.ngroups);
+                      partial = g->scratch<double>(WS_BC_SIGMA, S.ngroups);
                     });
   if (sums) {
     // S
@@ -459,7 +464,7 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   RegionTimer region(s);
   KernelTimer ktimer(s);
   uint32_t launches = 0;
-  pr_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / static_cast<double>(n), max_iter);
+  pr_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, static_cast<double>(n), max_iter);
   pr_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(x[0], y[0], outdeg, n, part_dang);
   GX_LAUNCHED("pr_init_kernel");
   pr_init_reduce_kernel<<<1, kBlock, 0, s>>>(state, part_dang, kSweepGrid);

@@ -40,7 +40,7 @@ struct AdState {
   double base;       // alpha*D/n (forward) or sum(lambda)/n (adjoint)
   double alpha;
   double tol;
-  double inv_n;
+  double n;
   unsigned converged;
   unsigned iters;
   unsigned final_buf;
@@ -174,7 +174,7 @@ struct AdClose {
   __device__ __forceinline__ void operator()(double r, double a) const {
     state->resid = r;
     state->acc = a;
-    state->base = (mode == 0 ? state->alpha : 1.0) * a * state->inv_n;
+    state->base = (mode == 0 ? state->alpha : 1.0) * a / state->n;
     state->iters += 1;
     state->final_buf = newest_buf;
     if (r < state->tol || state->iters >= state->max_iter) state->converged = 1;
@@ -186,24 +186,23 @@ __global__ void __launch_bounds__(kBlock) ad_reduce_kernel(AdState* state, const
                                                            unsigned newest_buf) {
   if (state->converged) return;
   __shared__ double red[kBlock / kWave];
-  double r = 0, a = 0;
+  rs::DoubleSum r, a;
   for (int i = threadIdx.x; i < nparts; i += kBlock) {
-    r += p0[i];
-    a += p1[i];
+    r.add(p0[i]);
+    a.add(p1[i]);
   }
-  r = block_sum(r, red);
-  a = block_sum(a, red);
-  if (threadIdx.x == 0) AdClose{state, mode, newest_buf}(r, a);
+  const double resid = block_sum(r.value(), red), acc = block_sum(a.value(), red);
+  if (threadIdx.x == 0) AdClose{state, mode, newest_buf}(resid, acc);
 }
 
-__global__ void ad_state_init_kernel(AdState* s, double alpha, double tol, double inv_n, unsigned max_iter) {
+__global__ void ad_state_init_kernel(AdState* s, double alpha, double tol, double n, unsigned max_iter) {
   if (threadIdx.x == 0) {
     s->resid = 0;
     s->acc = 0;
     s->base = 0;
     s->alpha = alpha;
     s->tol = tol;
-    s->inv_n = inv_n;
+    s->n = n;
     s->converged = max_iter == 0 ? 1u : 0u;
     s->iters = 0;
     s->final_buf = 0;
@@ -251,7 +250,7 @@ __global__ void ad_init_reduce_kernel(AdState* state, const double* __restrict__
   a = block_sum(a, red);
   if (threadIdx.x == 0) {
     state->acc = a;
-    state->base = (mode == 0 ? state->alpha : 1.0) * a * state->inv_n;
+    state->base = (mode == 0 ? state->alpha : 1.0) * a / state->n;
   }
 }
 
@@ -342,12 +341,12 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
   build_transpose(g);
   bs::Plan L{};
   float* wl = nullptr;
-  Real* partial = nullptr;
+  double* partial = nullptr;
   const bool blocked = bs::pays(n, m) && bs::fits(g->csc_sums[sizeof(Real) == 8], [&] {
                          L = bs::build(g, g->trow(), g->tcol(), g->tperm(), n, m, bs::Shape<Real>::kShift, true,
                                        g->csc_sums[sizeof(Real) == 8]);
                          wl = g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile);
-                         partial = g->scratch<Real>(WS_BC_SIGMA, L.ngroups);
+                         partial = g->scratch<double>(WS_BC_SIGMA, L.ngroups);
                        });
   const rs::RowPlan P = blocked ? rs::RowPlan{} : rs::build_plan(g, g->trow(), g->tcol(), n, m, g->csc_plan);
   const rs::RowPlan W = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);  // row sums of the weights
@@ -370,7 +369,7 @@ void run_forward(gx_graph* g, const float* w, const float* t, double alpha, doub
     bs::layout_weights(L, w, wl, s);
   else if (m)
     permute_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, g->tperm(), m, wt);
-  ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / n, max_iter);
+  ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, static_cast<double>(n), max_iter);
   fwd_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(xs[0], ys[0], inv_s, n, parts);
   ad_init_reduce_kernel<<<1, kBlock, 0, s>>>(state, parts, kSweepGrid, 0);
   GX_LAUNCHED("forward init");
@@ -409,12 +408,12 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
   const rs::RowPlan P = rs::build_plan(g, g->row, g->col, n, m, g->csr_plan);
   bs::Plan L{};
   float* wl = nullptr;
-  Real* partial = nullptr;
+  double* partial = nullptr;
   const bool blocked = bs::pays(n, m) && bs::fits(g->csr_sums[sizeof(Real) == 8], [&] {
                          L = bs::build(g, g->row, g->col, nullptr, n, m, bs::Shape<Real>::kShift, true,
                                        g->csr_sums[sizeof(Real) == 8]);
                          wl = g->scratch<float>(WS_BC_DELTA, L.ntiles * bs::kTile);
-                         partial = g->scratch<Real>(WS_BC_SIGMA, L.ngroups);
+                         partial = g->scratch<double>(WS_BC_SIGMA, L.ngroups);
                        });
   Real* inv_s = g->scratch<Real>(WS_V4, n);
   Real* wr = blocked ? nullptr : g->scratch<Real>(WS_BC_DELTA, std::max<int64_t>(m, 1));
@@ -437,7 +436,7 @@ void run_adjoint(gx_graph* g, const float* w, const Real* x, const float* c, dou
     bs::layout_weights(L, w, wl, s);
   else if (m)
     convert_weights_kernel<Real><<<grid_for(m, kBlock, 8192), kBlock, 0, s>>>(w, m, wr);
-  ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, 1.0 / n, max_iter);
+  ad_state_init_kernel<<<1, 64, 0, s>>>(state, alpha, tol, static_cast<double>(n), max_iter);
   adj_init_kernel<Real><<<kSweepGrid, kBlock, 0, s>>>(lam[0], c, n, parts);
   ad_init_reduce_kernel<<<1, kBlock, 0, s>>>(state, parts, kSweepGrid, 1);
   GX_LAUNCHED("adjoint init");

@@ -18,8 +18,9 @@
 //  2. Each lane reads its 8 consecutive values and sums what follows its last
 //     row end; a segmented scan of those sums over the lanes (DPP, fixed
 //     order) gives every lane the open sum it continues.
-//  3. The lane walks its values once more from that sum and stores a row sum
-//     to LDS at each row end.
+//  3. The lane walks its values once more and stores a row sum to LDS at each
+//     row end, the first one with the open sum added: values are summed among
+//     themselves before they meet the sum of a long row.
 //  4. Consecutive lanes finalise consecutive rows.
 // The sum left open at a tile's end is carried in a register to the next tile
 // of the chunk.  A row that began in an earlier chunk is not finalised where
@@ -81,6 +82,19 @@ __device__ __forceinline__ double block_sum(double v, double* lds) {
   __syncthreads();
   return r;
 }
+
+// A sum and, in lo, what its additions rounded off (Knuth's TwoSum): a long row's
+// is rounded once, however many parts it has.
+struct DoubleSum {
+  double hi = 0, lo = 0;
+  __device__ __forceinline__ void add(double x) {
+    const double t = hi + x, b = t - hi;
+    lo += (hi - (t - b)) + (x - b);
+    hi = t;
+  }
+  // hi alone where the sum is not finite (lo then means nothing).
+  __device__ __forceinline__ double value() const { return isfinite(lo) ? hi + lo : hi; }
+};
 
 template <class T>
 __device__ __forceinline__ T ld_stream(const T* p) {
@@ -215,21 +229,22 @@ __global__ void __launch_bounds__(kBlock) sweep_kernel(RowPlan P, Src src, Fin f
       const uint64_t heads = __ballot(ends != 0);
       const uint64_t upto = heads & (~0ull >> (63 - lane));
       const double seg = wave_seg_scan(tail, upto ? 63 - __builtin_clzll(upto) : 0, lane);
-      double acc = __shfl_up(seg, 1);
-      if (lane == 0) acc = 0;
-      if ((heads & ((1ull << lane) - 1)) == 0) acc += open;
+      double before = __shfl_up(seg, 1);
+      if (lane == 0) before = 0;
+      if ((heads & ((1ull << lane) - 1)) == 0) before += open;
       const double last = __shfl(seg, kWave - 1);
       open = heads ? last : open + last;
       // Row sums (the values are in registers: the LDS area is free).
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
       uint32_t slot = info >> 8;
+      double acc = 0;
 #pragma unroll
       for (int u = 0; u < kItems; ++u) {
         acc += static_cast<double>(v[u]);
         if ((ends >> u) & 1u) {
-          sh.sum[slot++] = acc;
-          acc = 0;
+          sh.sum[slot++] = before + acc;
+          before = acc = 0;
         }
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -282,20 +297,28 @@ __device__ __forceinline__ void finalize_spans(const RowPlan& P, const Fin& fin,
     const uint32_t first = spans ? P.span_first[c] : 0u;
     const double head = spans ? carry[c] : 0.0;
     const typename Fin::Pre pre = spans ? fin.pre(r) : typename Fin::Pre{};
-    double sum = 0;
+    DoubleSum sum;
     // Short spans by their own lane, long ones by the whole wavefront.
     constexpr int kAlone = 8;
     if (spans && c - first <= kAlone)
-      for (int64_t t = first; t < c; ++t) sum += carry[P.nchunks + t];
+      for (int64_t t = first; t < c; ++t) sum.add(carry[P.nchunks + t]);
     for (uint64_t todo = __ballot(spans && c - first > kAlone); todo; todo &= todo - 1) {
       const int i = __ffsll(static_cast<unsigned long long>(todo)) - 1;
       const int64_t f = __shfl(first, i), e = b + i;
-      double s = 0;
-      for (int64_t t = f + lane; t < e; t += kWave) s += carry[P.nchunks + t];
-      s = wave_sum(s);
+      DoubleSum s;
+      for (int64_t t = f + lane; t < e; t += kWave) s.add(carry[P.nchunks + t]);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        const double oh = __shfl_xor(s.hi, off), ol = __shfl_xor(s.lo, off);
+        s.add(oh);
+        s.lo += ol;
+      }
       if (lane == i) sum = s;
     }
-    if (spans) fin(r, sum + head, pre, a0, a1);
+    if (spans) {
+      sum.add(head);
+      fin(r, sum.value(), pre, a0, a1);
+    }
   }
 }
 

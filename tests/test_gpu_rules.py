@@ -211,3 +211,95 @@ def test_sums_without_room_for_the_blocked_layout(gx):
         rel = 1e-12 if e.dtype == np.float64 else 1e-5
         assert np.abs(a - e).max() <= rel * np.abs(e).max()
         assert np.array_equal(b, e)
+
+
+def two_out(n, dest, rng):
+    """Every vertex with two weighted out-edges: one to dest[v], one to a random
+    vertex (none is dangling; no vertex twice in a list)."""
+    other = rng.integers(0, n, n)
+    other = np.where(other == dest, (other + 1) % n, other)
+    lo, hi = np.minimum(dest, other), np.maximum(dest, other)
+    col = np.stack([lo, hi], 1).ravel().astype(np.int32)
+    return np.arange(0, 2 * n + 1, 2, dtype=np.int32), col, (rng.random(2 * n) + 0.5).astype(np.float32)
+
+
+def ulps(got, row, col, w, rows):
+    """How far the values of `rows` after one iteration with alpha = 1/2 and no
+    teleport are from half the exact row sum, in units of the last place: the
+    iteration starts from the rounded 1 / n, halving is exact."""
+    n = len(row) - 1
+    src = np.repeat(np.arange(n), np.diff(row))
+    wl = w.astype(np.longdouble)
+    terms = np.longdouble(got.dtype.type(1.0 / n)) * wl / np.add.reduceat(wl, row[:-1])[src]
+    keep = np.flatnonzero(np.isin(col, rows))
+    keep = keep[np.argsort(col[keep], kind="stable")]
+    at = np.searchsorted(col[keep], rows)
+    exact = np.add.reduceat(terms[keep], at) / 2
+    return np.abs(got[rows].astype(np.longdouble) - exact) / np.spacing(got[rows]).astype(np.longdouble)
+
+
+@pytest.mark.parametrize("n,hubs", [(300007, 60), (1900003, 64), (1900003, 500), (1900003, 6000)])
+def test_long_rows_are_rounded_once_in_fp64(gx, n, hubs):
+    """Rows with hundreds to thousands of terms, spread over the tiles of the row
+    sweep (fewer than 7 * 2^19 edges) or the chunks of the blocked sums: the sum is
+    within half a unit of the last place of the exact one, and the parts' own
+    roundings (each at a small share of the row: 0.09 units in all, four times
+    that at most)."""
+    import torch
+    rng = np.random.default_rng(hubs)
+    rows = np.sort(rng.choice(n, hubs, replace=False))
+    row, col, w = two_out(n, rows[np.arange(n) % hubs], rng)
+    G = gx.Graph.from_csr(row, col, w)
+    t = torch.zeros(n, device="cuda")
+    x, _ = gx.pagerank_weighted(G, torch.from_numpy(w).cuda(), t, alpha=0.5, tol=0.0, max_iter=1, precision="fp64")
+    off = ulps(x.cpu().numpy(), row, col, w, rows)
+    print(f"ulps n={n} hubs={hubs} mean {float(off.mean()):.3f} max {float(off.max()):.3f}", flush=True)
+    assert off.max() <= 0.86
+
+
+def test_rows_of_two_parts_are_rounded_once_in_fp32(gx):
+    """FP32 rows whose terms lie in two chunks of the blocked sums: a part is not
+    rounded to FP32 before it is added (0.5 units each, at half of the row), so
+    that the row is within half a unit and the terms' own roundings (200 terms of
+    0.4 units: 0.03 of the row's, four times that at most)."""
+    import torch
+    rng = np.random.default_rng(3)
+    n = 116 * 16384
+    v = np.arange(n)
+    dest = (v >> 15) * 163 + np.minimum((v & 16383) // 100, 162)
+    row, col, w = two_out(n, dest, rng)
+    G = gx.Graph.from_csr(row, col, w)
+    x, _ = gx.pagerank_weighted(G, torch.from_numpy(w).cuda(), torch.zeros(n, device="cuda"), alpha=0.5, tol=0.0,
+                                max_iter=1)
+    off = ulps(x.cpu().numpy(), row, col, w, np.unique(dest))
+    print(f"ulps fp32 rows={len(off)} mean {float(off.mean()):.3f} max {float(off.max()):.3f}", flush=True)
+    assert off.max() <= 0.65
+
+
+def test_dangling_mass_of_equal_ranks_in_fp64(gx):
+    """Two million vertices without edges have one rank, v' = (1 + k v) / 2n with k
+    of them and alpha = 1/2 (halving and n = 2^21 are exact).  Equal addends round
+    alike, so a mass added up one by one is off by several units whatever the
+    number of lanes; here it is off by at most one (a workgroup's part is rounded
+    once, the parts are added pairwise but for four in a row), and the rank by half
+    of that and half a unit of its own, plus the half of what the iteration before
+    left: two units at most."""
+    from fractions import Fraction
+    rng = np.random.default_rng(9)
+    n, busy = 1 << 21, 100003
+    key = np.unique(rng.integers(0, busy, 9500000) * busy + rng.integers(0, busy, 9500000))
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(key // busy, minlength=n), out=row[1:])
+    col = (key % busy).astype(np.int32)
+    assert len(col) >= 1 << 23 and np.diff(row)[:busy].min() > 0
+    G = gx.Graph.from_csr(row, col)
+    v = Fraction(1, n)
+    worst = 0.0
+    for k in range(1, 9):
+        v = (1 + (n - busy) * v) / (2 * n)
+        x = gx.pagerank(G, alpha=0.5, tol=0.0, max_iter=k, precision="fp64")[0].cpu().numpy()[busy:]
+        assert np.all(x == x[0])
+        off = abs(Fraction(float(x[0])) - v) / Fraction(float(np.spacing(x[0])))
+        worst = max(worst, float(off))
+        print(f"dangling k={k} off by {float(off):.3f} units", flush=True)
+    assert worst <= 2.0
