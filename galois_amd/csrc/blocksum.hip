@@ -5,8 +5,8 @@
 //  2. Each chunk starts on a tile; every position gets its in-chunk index with
 //     the group-end flag, its row and (weighted) its edge id.
 //  3. Group ends counted per tile and scanned; every group gets its row.
-//  4. Bins: blocks of bin_rows rows, halved while they hold many groups, so that
-//     no wavefront of phase 2 sums much more than the others.
+//  4. Bins: blocks of rows, halved while they hold many groups, so that no
+//     wavefront of phase 2 sums much more than the others.
 //  5. Run starts marked and scanned, the runs sorted stably by bin.
 #include <algorithm>
 #include <vector>
@@ -19,6 +19,7 @@ namespace {
 
 constexpr int kB = 256;
 constexpr double kAvgRun = 16.0;
+constexpr int64_t kMinBins = 1024;  // bins that keep phase 2 busy: a wavefront each
 constexpr uint32_t kNone = 0xffffffffu;
 // 16: at 64 and 256 a graph without hubs keeps its error (1.06e-16 against 0.67e-16)
 // and the solves take as long.
@@ -195,12 +196,21 @@ int bits_for(uint64_t v) {  // bits that hold 0 .. v - 1
 
 }  // namespace
 
-// From 2M edges on: below, too few pieces keep the CUs busy.  Forward and
-// adjoint (FP32) / FP64 pull, row sweep against blocks: 1.1M edges 2.7 ms
-// against 4.6; 2.1M edges 0.66 ms against 0.63; 3.2M edges 5.4 ms against 4.1;
-// 4.1M edges 1.08 ms against 0.80; 20.6M edges 4.13 ms against 2.04; 67M edges
-// 75.0 ms against 30.7.
-bool pays(int64_t n, int64_t m) { return m >= (int64_t(1) << 21) && n >= (int64_t(1) << 15) && m < (int64_t(1) << 31); }
+// From 7 * 2^19 edges and 2^15 rows on.  Forward and adjoint in FP32 (FP64), ms, row
+// sweep against blocks, and the first call on a graph, which builds both layouts:
+//   n       m      again                     first
+//   160000  2.56M  3.65 3.76 (3.97 4.00)     5.3 8.0 (6.2 9.0)
+//   200000  3.20M  4.81 3.83 (5.36 4.46)     7.3 8.1 (8.4 8.9)
+//   230000  3.68M  5.81 4.31 (5.99 4.96)     8.7 8.9 (9.2 10.1)
+//   270000  4.32M  6.26 4.55 (6.27 5.26)     9.4 9.3 (10.1 10.3)
+//    65536  13.1M  11.3 5.7                  14.3 11.3
+//   1000000 12.0M  14.0 9.2                  17.4 16.4
+//    16384  4.10M  4.44 3.52                 7.1 8.2
+//    32768  3.28M  4.24 3.27                 6.1 7.4
+//     8192  3.28M  4.02 4.39                 5.9 8.5
+bool pays(int64_t n, int64_t m) {
+  return m >= (int64_t(7) << 19) && n >= (int64_t(1) << 15) && m < (int64_t(1) << 31);
+}
 
 void layout_weights(const Plan& P, const float* w, float* wt, hipStream_t s) {
   weights_kernel<<<grid(P.ntiles * kTile), kB, 0, s>>>(P.eid, w, P.ntiles * kTile, wt);
@@ -243,7 +253,7 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   const int64_t most_tiles = (m + kTile - 1) / kTile + nchunks;
   const size_t area_a = (m + 2) * 8, area_b = (m + 2) * 8, area_c = (m + 2) * 4, area_d = most_tiles * kTile * 8,
                area_e = (m + 2) * 4;
-  const int64_t most_blocks = n / 512 + 1, most_bins = n / 16 + most_blocks + 1;
+  const int64_t most_blocks = n / 16 + 1, most_bins = n / 16 + most_blocks + 1;
   const size_t tables = 2 * (nchunks + 1) * 4 + most_tiles + 13 * most_blocks + 8 * (most_bins + 1) + 16 * 256;
   const size_t scratch = std::max(sort_words(m), scan_words(m + 2)) * 4;
   DevBuf work;
@@ -326,14 +336,21 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   group_kernel<<<grid(nt * int64_t(kWave)), kB, 0, s>>>(idx16, prow, nt, tile_grp, first, grow);
   GX_LAUNCHED("bs::group_kernel");
   // 4. Bins: rows per block so that a run holds about 16 groups (a quarter of
-  // a wavefront's lanes), between 512 and 4096 (4 and 32 KB of LDS sums).  FP64
+  // a wavefront's lanes), between 512 and 4096 (4 and 32 KB of LDS sums); where that
+  // makes fewer than kMinBins bins, as few as 16 while the runs are as long (32768
+  // vertices, 10.0M edges, FP64: 3.10 ms a solve with 64 bins, 1.47 with 512,
+  // 1.14 with 1024).  FP64
   // vectors have two sums a row in bins with rows of more than kPairRow edges, 8 to
   // 32 KB up to 2048 rows.  With 64 KB for 4096 rows too few wavefronts fit a CU
   // (RMAT-26 245 ms a solve -> 551), and with 2048 the runs are half as long (418),
   // so blocks of 4096 rows have them only where they are halved, which one with a
   // row of more than kHalveRow edges is.
+  auto avg_run = [&](int shift) {
+    return static_cast<double>(ng) * static_cast<double>(int64_t(1) << shift) / (static_cast<double>(nchunks) * n);
+  };
   int bshift = 9;
-  while (bshift < 12 && static_cast<double>(ng) * (int64_t(1) << bshift) < kAvgRun * static_cast<double>(nchunks) * n) ++bshift;
+  while (bshift < 12 && avg_run(bshift) < kAvgRun) ++bshift;
+  while (bshift > 4 && (n >> bshift) < kMinBins && avg_run(bshift - 1) >= kAvgRun) --bshift;
   const int64_t nblocks = (n + (int64_t(1) << bshift) - 1) >> bshift;
   uint2* bedges = reinterpret_cast<uint2*>(take(nblocks * 8));
   block_edges_kernel<<<grid(nblocks * kWave), kB, 0, s>>>(rowoff, n, bshift, nblocks, bedges);

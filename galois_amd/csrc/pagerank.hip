@@ -420,12 +420,20 @@ static void run_pull(gx_graph* g, double alpha, double tol, uint32_t max_iter, R
   const int64_t hot = blocked ? 0 : hot_sources(n, sizeof(Real));
   // FP64 in one pass: the deterministic sums in blocks where they pay.  A solve
   // here is 20 to 40 sweeps, so that the layout has to pay for itself sooner
-  // than in a training loop: 4.1M edges 1.08 -> 0.80 ms a solve, but the first
-  // one 4.1 -> 6.3 ms; 20.6M edges 4.13 -> 2.04 ms, the first 9.4 -> 9.6 ms.
+  // than in a training loop, and below 2^19 vertices the gathered vector stays in
+  // an XCD's L2.  Row sweep against blocks, ms a solve, and the first one:
+  //   n       m      again        first
+  //    65536  16.0M  1.60 1.66    4.3 5.5
+  //   131072  27.1M  2.37 1.85    6.0 7.2
+  //   262144  13.7M  1.35 1.33    4.5 5.5
+  //   600000   8.1M  1.82 1.37    5.8 6.6
+  //   800000  11.4M  2.30 1.76    6.6 6.9
+  //   1000000 28.1M  3.64 2.38    9.1 9.9
   rs::RowPlan P{}, PA{};
   bs::Plan S{};
   double* partial = nullptr;
-  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && g->m >= (int64_t(1) << 23) && bs::pays(n, g->m) &&
+  const bool sums = !blocked && hot == 0 && sizeof(Real) == 8 && g->m >= (int64_t(1) << 23) &&
+                    n >= (int64_t(1) << 19) && bs::pays(n, g->m) &&
                     bs::fits(D.sums, [&] {
                       S = bs::build(g, D.trow.as<int32_t>(), D.tcol.as<int32_t>(), nullptr, n, g->m,
                                     bs::Shape<Real>::kShift, false, D.sums);

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from test_gpu_paths import random_csr, u32, weighted_csr
+from test_gpu_paths import test_row_sweep_shapes as row_sweep_shapes
 
 pytestmark = pytest.mark.gpu
 
@@ -150,11 +151,11 @@ def groups_of(row, col, shift, range_edges=2048):
     return int(new.sum()), tiles
 
 
-@pytest.mark.parametrize("n,m", [(600011, 9000000), (1 << 19, 8500000)])
+@pytest.mark.parametrize("n,m", [(600011, 9000000), (1 << 19, 8500000), (40000, 9500000)])
 def test_fp64_pull_states_the_bytes_of_the_path_it_took(gx, n, m):
-    """main_kernel_bytes of an FP64 sweep: blocked sums from 2^23 edges on (two
-    bytes per edge position, 18 per group, eight per run of at most 64 groups, 36
-    per row), the row sweep with the hot split."""
+    """main_kernel_bytes of an FP64 sweep: blocked sums from 2^23 edges and 2^19
+    vertices on (two bytes per edge position, 18 per group, eight per run of at most
+    64 groups, 36 per row), the row sweep on fewer vertices and with the hot split."""
     rng = np.random.default_rng(n)
     key = np.unique(rng.integers(0, n, m) * n + np.minimum(rng.integers(0, n, m), rng.integers(0, n, m)))
     row = np.zeros(n + 1, np.int32)
@@ -167,6 +168,9 @@ def test_fp64_pull_states_the_bytes_of_the_path_it_took(gx, n, m):
     groups, tiles = groups_of(row, col, 13)
     fixed = 2 * 512 * tiles + 18 * groups + 36 * n
     print(f"bytes n={n} m={m} groups={groups} fixed={fixed} stated={st.main_kernel_bytes}", flush=True)
+    if n < 1 << 19:
+        assert st.main_kernel_bytes == 4 * m + 4 * (n + 1) + 36 * n
+        return
     assert fixed + 8 * -(-groups // 64) <= st.main_kernel_bytes <= fixed + 8 * groups
     with knobs(gx, pr__hot_sources=1000):
         st = gx.pagerank(G, tol=0.0, max_iter=2, precision="fp64")[1]
@@ -274,6 +278,17 @@ def test_rows_of_two_parts_are_rounded_once_in_fp32(gx):
     off = ulps(x.cpu().numpy(), row, col, w, np.unique(dest))
     print(f"ulps fp32 rows={len(off)} mean {float(off.mean()):.3f} max {float(off.max()):.3f}", flush=True)
     assert off.max() <= 0.65
+
+
+# The blocked sums' side of the size rule (7 * 2^19 edges, 2^15 rows): few chunks and
+# many, rows with edges in every chunk and over many of a wavefront's ranges, mostly
+# empty rows, a last chunk of one vertex, few rows with many edges (small bins).
+@pytest.mark.parametrize("n,m,hubs", [(32768, 3900000, 0), (65537, 7800000, 2), (1 << 20, 6000000, 1),
+                                      (200000, 9000000, 0)])
+def test_blocked_sums_shapes(gx, n, m, hubs):
+    """As the row sweep's shapes, with the same tolerances."""
+    assert len(weighted_csr(n, m, n + m, hubs)[1]) >= 7 << 19
+    row_sweep_shapes(gx, n, m, hubs)
 
 
 def test_dangling_mass_of_equal_ranks_in_fp64(gx):
