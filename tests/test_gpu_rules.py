@@ -132,6 +132,60 @@ def test_bfs_lists_with_repeated_edges(gx, oracle):
         assert np.array_equal(got[0], oracle.sssp(r, v, w, 3, 6)) and np.array_equal(got[1], oracle.sssp(r, v, w, 17, 6))
 
 
+def blocked_shapes():
+    """A source with 600K out-edges (one chunk in several phase-1 pieces), a
+    destination with 600K in-edges (its bin cut into slices), one vertex past a 16K
+    chunk boundary, a band of vertices without edges, dangling vertices."""
+    rng = np.random.default_rng(23)
+    n = 5 * 16384 + 16385
+    k = 600000
+    src = np.concatenate([np.full(k, 70000), rng.integers(0, n, k), rng.integers(0, 16384, 200000)])
+    dst = np.concatenate([rng.integers(0, n, k), np.full(k, 3), rng.integers(0, n, 200000)])
+    quiet = (src >= 32768) & (src < 49152) | (dst >= 32768) & (dst < 49152)
+    src, dst = np.append(src[~quiet], n - 1), np.append(dst[~quiet], 0)
+    key = np.unique(src[src != dst] * n + dst[src != dst])
+    row = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(key // n, minlength=n), out=row[1:])
+    return row, (key % n).astype(np.int32)
+
+
+@pytest.mark.parametrize("edges", [-1, 1 << 12, 1 << 30])
+@pytest.mark.parametrize("shape", ["tables", "rmat16", "rmat20", "one chunk"])
+def test_blocked_fp32_sweep(gx, oracle, shape, edges):
+    """The propagation-blocked FP32 sweep where the default rule would pull (the
+    knob is set): 1e-6 in L1 of the FP64 oracle, bit for bit the same again, on a
+    second handle and however its bins are cut.  Sums are exact, so that only a
+    lost or doubled contribution could differ."""
+    if shape == "tables":
+        row, col = blocked_shapes()
+    elif shape == "one chunk":
+        row, col, _ = weighted_csr(16384, 50000, 2, 1)
+    else:
+        row, col, _ = gx.Graph.rmat(int(shape[4:]), 16, symmetric=False).to_host()
+    print(f"blocked {shape} n={len(row) - 1} m={len(col)} task_edges={edges}", flush=True)
+    exp, it, _ = oracle.pagerank(row, col, tol=1e-10, max_iter=200, threads=8)
+    got = []
+    with knobs(gx, pr__blocking=1):
+        A = gx.Graph.from_csr(row, col)
+        got.append(gx.pagerank(A, tol=1e-10, max_iter=200)[0].cpu().numpy())
+        assert gx.pagerank_layout_info(A)["tasks"] > 0  # the blocked sweep ran
+        with knobs(gx, pr__task_edges=edges):
+            B = gx.Graph.from_csr(row, col)
+            for _ in range(2):
+                got.append(gx.pagerank(B, tol=1e-10, max_iter=200)[0].cpu().numpy())
+        info = gx.pagerank_layout_info(B)
+        assert info["tasks"] > 0 and (edges != 1 << 30 or info["sliced_bins"] == 0)
+        assert edges != 1 << 12 or shape == "one chunk" or info["sliced_bins"] > 0
+    assert np.abs(got[0].astype(np.float64) - exp).sum() < 1e-6
+    for x in got[1:]:
+        assert np.array_equal(got[0], x)
+    with knobs(gx, pr__blocking=0):  # the pull agrees to rounding, on a graph without a layout
+        C = gx.Graph.from_csr(row, col)
+        pulled = gx.pagerank(C, tol=1e-10, max_iter=200)[0].cpu().numpy()
+        assert gx.pagerank_layout_info(C) == {}
+    assert np.abs(pulled.astype(np.float64) - exp).sum() < 1e-6
+
+
 def groups_of(row, col, shift, range_edges=2048):
     """(row, chunk of 2^shift sources) groups of the degree-ordered transpose, cut
     where a wavefront's range of edges ends inside a chunk."""
@@ -175,6 +229,84 @@ def test_fp64_pull_states_the_bytes_of_the_path_it_took(gx, n, m):
     with knobs(gx, pr__hot_sources=1000):
         st = gx.pagerank(G, tol=0.0, max_iter=2, precision="fp64")[1]
     assert st.main_kernel_bytes == 4 * m + 8 * (n + 1) + 36 * n + 16 * n
+
+
+def one_step(row, col, w, t, c, alpha):
+    """One forward iteration from 1/n and, from c, one adjoint iteration with the
+    gradients, in FP64 numpy with its infinities and NaNs; beside each value the
+    sum of its terms' magnitudes, and how far the worst row's weights cancel."""
+    n = len(row) - 1
+    src = np.repeat(np.arange(n), np.diff(row))
+    w = w.astype(np.float64)
+
+    def rows(at, vals):
+        out = np.zeros(n)
+        np.add.at(out, at, vals)
+        return out
+
+    def step(w, t, c, inv, none, sign):
+        x0 = np.full(n, 1.0 / n)
+        x = (1 - alpha) * t + alpha * x0[none].sum() / n + alpha * rows(col, (x0 * inv)[src] * w)
+
+        def below(lam):
+            return np.where(none, lam.sum() / n, rows(src, lam[col] * w) * inv)
+
+        lam = c + alpha * below(c)
+        return x, alpha * t[src] * (lam[col] + sign * below(lam)[src]) * inv[src], (1 - alpha) * lam
+
+    with np.errstate(all="ignore"):
+        s = rows(src, w)
+        inv = np.where(s > 0, 1.0 / np.where(s > 0, s, 1.0), 0.0)
+        none = inv == 0
+        cancel = (rows(src, np.abs(w)) * inv)[~none].max()
+        return step(w, t, c, inv, none, -1), step(np.abs(w), t, np.abs(c), inv, none, 1), cancel
+
+
+@pytest.mark.parametrize("n,m", [(5000, 40000), (32768, 3900000), (100003, 3900000)])
+@pytest.mark.parametrize("values", ["signs", "scales", "not finite"])
+@pytest.mark.parametrize("order", ["ascending", "random", "repeated"])
+def test_row_sums_of_any_values_and_orders(gx, n, m, values, order):
+    """The row sweep and the blocked sums on adjacency lists in any order and with
+    repeated entries, on sums of either sign, of scales far apart, with infinities
+    and NaNs in some rows: FP64 as numpy's to 1e-12 of the terms' magnitudes (times
+    the worst cancellation in a row's weight sum), and not finite in exactly the
+    same places."""
+    import torch
+    rng = np.random.default_rng(n + len(order))
+    row, col, w = weighted_csr(n, m, n, 1 if n < 10000 else 0)
+    if order != "ascending":
+        src = np.repeat(np.arange(n), np.diff(row))
+        if order == "repeated":
+            again = rng.random(len(col)) < 0.2
+            src, col, w = (np.concatenate([a, a[again]]) for a in (src, col, w))
+        o = np.lexsort((rng.random(len(src)), src))
+        src, col, w = src[o], col[o], w[o]
+        row = np.zeros(n + 1, np.int32)
+        np.cumsum(np.bincount(src, minlength=n), out=row[1:])
+    t = (rng.random(n) / n).astype(np.float32)
+    c = rng.standard_normal(n).astype(np.float32)
+    if values == "signs":
+        w[rng.random(len(w)) < 0.1] *= -0.5  # a row whose sum is not positive counts as dangling
+    elif values == "scales":
+        w = np.exp2(rng.integers(-40, 40, len(w))).astype(np.float32)
+        c *= np.exp2(rng.integers(-30, 30, n)).astype(np.float32)
+    else:
+        w[rng.integers(0, len(w), 5)] = [np.inf, np.nan, np.inf, np.nan, np.inf]
+        c[rng.integers(0, n, 3)] = [np.inf, -np.inf, np.nan]
+    print(f"row sums n={n} m={len(col)} {values} {order}", flush=True)
+    G = gx.Graph.from_csr(row, col, w)
+    ww, tt, cc = (torch.from_numpy(a).cuda() for a in (w, t, c))
+    x, _ = gx.pagerank_weighted(G, ww, tt, alpha=0.5, tol=0.0, max_iter=1, precision="fp64")
+    gw, gt, _ = gx.pagerank_adjoint(G, ww, tt.double(), cc, alpha=0.5, tol=0.0, max_iter=1, precision="fp64")
+    got = [a.cpu().numpy() for a in (x, gw, gt)]
+    ref, size, cancel = one_step(row, col, w, t.astype(np.float64), c.astype(np.float64), 0.5)
+    for name, a, b, mag in zip(("x", "grad_w", "grad_t"), got, ref, size):
+        assert np.array_equal(np.isnan(a), np.isnan(b)), name
+        inf = np.isinf(b)
+        assert np.array_equal(np.isinf(a), inf) and np.array_equal(a[inf], b[inf]), name
+        ok = np.isfinite(b) & np.isfinite(mag)
+        # At most 2^20 FP64 roundings of the terms, and of the inverse row sums.
+        assert np.abs(a[ok] - b[ok]).max() <= 1e-12 * cancel * mag[ok].max(), name
 
 
 def test_sums_without_room_for_the_blocked_layout(gx):
