@@ -43,7 +43,6 @@ struct KcoreCounters {
   unsigned rounds;
   unsigned long long items;
   unsigned long long alive;
-  unsigned long long edges;
   unsigned hot_count;
 };
 __global__ void kcore_reset_kernel(KcoreCounters* c) {
@@ -57,7 +56,6 @@ __global__ void kcore_reset_kernel(KcoreCounters* c) {
     c->rounds = 0;
     c->items = 0;
     c->alive = 0;
-    c->edges = 0;
     c->hot_count = 0;
   }
 }
@@ -457,10 +455,8 @@ extern "C" gx_status gx_kcore(gx_graph* g, uint32_t k, uint32_t* degree, uint8_t
   launches += slots * (hubs ? 4 : 2) + 2 * replays;
   const uint32_t rounds = host->rounds;
   const uint64_t items = host->items;
-  uint64_t edges = 0;
   double ms = region.stop();
   if (alive_count) *alive_count = host->alive;
-  (void)edges;
   if (st) {
     std::memset(st, 0, sizeof(*st));
     st->iterations = rounds;
