@@ -652,8 +652,9 @@ extern "C" gx_status gx_bfs(gx_graph* g, uint32_t src, uint32_t* level, gx_stats
   const unsigned cap = static_cast<unsigned>(n);
   // Visited bitmap from 2^25 vertices on: below that the 4-byte level array
   // (<= 128 MB) stays cache-resident and the bitmap's clear and atomics cost
-  // more than they save (RMAT-18 0.455 -> 0.52 ms, RMAT-22 2.03 -> 2.21 ms
-  // with it; RMAT-26 33.9 -> 24.7 ms).
+  // more than they save.  Directed RMAT graphs of 2^24, 2^25 and 2^26 vertices
+  // without it and with it: 3.03 3.20, 6.35 5.99, 12.97 11.08 ms.  Where levels
+  // are pulled, which read the levels, it costs: symmetric RMAT-26 2.35 3.05 ms.
   const int64_t words = (n + 31) / 32;
   const bool use_vis = tune_effective("bfs.visited_bitmap", n, g->m) != 0;
   uint32_t* vis = use_vis ? g->scratch<uint32_t>(WS_BITMAP0, words) : nullptr;

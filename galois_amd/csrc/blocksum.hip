@@ -248,8 +248,9 @@ Plan build(gx_graph* g, const int32_t* rowoff, const int32_t* col, const int32_t
   const int64_t nchunks = (n + (int64_t(1) << shift) - 1) >> shift;
   // Working memory, allocated and freed once (both wait, 0.1 ms and more each; with
   // the layout's parts, the scans' and the sorts' scratch one by one, the first FP64
-  // solve of 700,000 vertices, 13.8M edges, took 8.0 ms, 7.0 this way): five areas used again as the steps go on.  No more groups and runs than
-  // edges; every chunk pads its last tile.
+  // solve of 700,000 vertices, 13.8M edges, took 8.0 ms, 7.0 this way): five areas
+  // used again as the steps go on.  No more groups and runs than edges; every chunk
+  // pads its last tile.
   const int64_t most_tiles = (m + kTile - 1) / kTile + nchunks;
   const size_t area_a = (m + 2) * 8, area_b = (m + 2) * 8, area_c = (m + 2) * 4, area_d = most_tiles * kTile * 8,
                area_e = (m + 2) * 4;

@@ -46,9 +46,16 @@ int64_t default_visited_bitmap(int64_t n, int64_t) { return n >= (int64_t(1) << 
 int64_t default_max_merge(int64_t, int64_t) { return 256; }
 int64_t default_bc_chunk(int64_t, int64_t) { return kEdgeChunk; }
 int64_t default_off(int64_t, int64_t) { return 0; }
-// The degree-ordered copy pays from 2^24 vertices on (RMAT-26 SSSP 72.6 ->
-// 49.5 ms, BFS 17.2 -> 15.5 ms); on RMAT-18 BFS it cost 0.41 -> 0.44 ms and
-// on RMAT-22 SSSP nothing changed.
+// The degree-ordered copy is made by a graph's first search, which takes that
+// long (RMAT-18 0.7 -> 3.5 ms, RMAT-22 1.6 -> 18, 24 5.6 -> 400).  Symmetric RMAT
+// graphs, ms without it and with it:
+//                          2^22           2^24          2^26 vertices
+//   BFS                  0.279 0.227    0.92 0.72     4.06 3.04
+//   direction-optimising 0.273 0.242    0.81 0.47     2.28 1.29
+//   SSSP                 4.13  4.02    11.1  10.1    48.8  34.4
+//   k-core               0.423 0.342    1.28 0.98     3.81 3.16
+// It is made from 2^24 vertices on, for graphs that are searched often.  On 2^22
+// it takes what 140 searches or more give back.
 int64_t default_relabel(int64_t n, int64_t) { return n >= (int64_t(1) << 24) ? 1 : 0; }
 // Hubs expanded in distance order, one distance at a time (r = 1), in the
 // relax steps whenever no near item is closer: RMAT-26 SSSP 49.7 -> 39.0 ms

@@ -272,10 +272,10 @@ int64_t tune_effective(const char* key, int64_t n, int64_t m);
 bool tune_is_set(const char* key);  // a value has been chosen for the knob
 // Default of "pr.task_edges": m / 1024 within [2^19, 2^20].
 int64_t pr_task_edges_default(int64_t n, int64_t m);
-// Degree above which a frontier vertex is expanded by the whole grid.
-// Frontier vertices of higher degree are expanded by the whole grid (default
-// 128: a workgroup batch of 256 frontier vertices then holds at most 32K
-// edges, so short power-law frontiers still spread over the grid).
+// Degree above which a frontier vertex is expanded by the whole grid (default
+// 128: a workgroup takes at most 256 frontier vertices at a time on graphs with
+// hubs, 32K edges, so short power-law frontiers still spread over the grid; on
+// graphs without it takes up to 1024).
 inline uint32_t hub_degree() { return static_cast<uint32_t>(tune_effective("frontier.hub_degree", 0, 0)); }
 
 // Accumulates the device time of the launches of one kernel with HIP events

@@ -46,7 +46,8 @@
 //    inside a bucket is expanded once per drain rather than once per
 //    improvement.  With sssp.hub_refine a step expands only the pending
 //    hubs within a distance slice above the smallest pending hub distance
-//    (one distance by default) and keeps the rest pending, so hubs go out
+//    (2^(r - 1); while the knob is not set one distance at first, then as many
+//    as the hubs per step call for) and keeps the rest pending, so hubs go out
 //    nearly in distance order, almost all at their final distance, and a
 //    hub's hundreds of thousands of edges are relaxed about once instead
 //    of once per improvement (RMAT-26: 1.84 -> 1.10 relaxations per edge).

@@ -131,7 +131,7 @@ void gx_set_profiling(int on);
  *                          default uses it from 2^25 vertices on
  *   "sssp.max_merge"       gx_sssp_delta: most consecutive buckets one
  *                          phase may cover (a phase merges buckets while the
- *                          previous one admitted fewer than 2^14 items);
+ *                          previous one had fewer than 2^15 items);
  *                          1 = one bucket per phase as in the reference's
  *                          OBIM order; default 256, range [1, 2^16]
  *   "sssp.defer_hubs"      gx_sssp_delta: 1 = hubs admitted in a relax step
