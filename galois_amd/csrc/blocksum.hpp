@@ -13,9 +13,10 @@
 //           chunk, then its wavefronts stream the edges (2 bytes of index per
 //           edge, bit 15 set on the last edge of a group; 4 bytes of weight
 //           where there are weights), add each group's products in FP64 and
-//           write one partial sum per group in layout order.
+//           write one FP64 partial sum per group in layout order.
 //   phase 2 (sum_kernel) one wavefront per bin adds the bin's runs, in chunk
-//           order, to FP64 sums in LDS and finalises the bin's rows.
+//           order, to FP64 sums in LDS (for FP64 vectors with what the additions
+//           round off) and finalises the bin's rows.
 //
 // Every order is fixed: a group is summed by one wavefront front to back, and
 // a row's partial sums are added by one wavefront, whose LDS additions are
@@ -23,14 +24,15 @@
 // results are bit-reproducible run to run without exact sums, for any sign,
 // scale, infinity or NaN.
 //
-// Bytes per sweep: 2 per edge (6 with weights), 2R + 2 per group (R the size
-// of a partial sum: FP32 or FP64 as the vector), R + what the finaliser reads
-// and writes per row.
+// Bytes per sweep: 2 per edge (6 with weights), 18 per group (a partial sum
+// written and read, its row), 8 per run, R (the size of a vector's entry) + what
+// the finaliser reads and writes per row.
 //
-// Bound: phase 1 by memory (67M edges with weights, FP32: 0.50 GB in 130 us, 3.9
-// TB/s), phase 2 by the latency of its short runs (25M groups: 85-100 us).  One
-// such sweep took 510-555 us gather by gather; 20.6M edges in FP64 156 us, 38 +
-// 40 us here.
+// Bound: phase 1 by memory (67M edges with weights, FP32: 0.60 GB in 147 us, 4.1
+// TB/s), phase 2 by the latency of its short runs (25M groups: 110-114 us).  One
+// such sweep takes 510-555 us by the row sweep; 20.6M edges in FP64 156 us, 38 +
+// 49 us here.  With FP32 partial sums for FP32 vectors, each rounded, the phases
+// took 122 and 77-91 us; with one sum a row for FP64 vectors phase 2 took 40.
 #pragma once
 
 #include <algorithm>
