@@ -69,6 +69,15 @@ int64_t default_relabel(int64_t n, int64_t) { return n >= (int64_t(1) << 24) ? 1
 //   (.45, .22)  134M        4.51 6.20   7.52 8.11   6.66 10.6
 //               167M        5.54 7.53   8.57 8.53   7.20 10.2
 int64_t default_hub_refine(int64_t n, int64_t) { return n >= (int64_t(1) << 24) ? 1 : 0; }
+// Batched SSSP, 64 sources, buckets of 2^6, ms a call at 1, 4, 16 and 64 buckets per
+// phase and with adaptive phases: fewer rounds make up for the repeated pushes of
+// a wide phase, the more so the more buckets the weights span.
+//   RMAT-20         weights to 255     13.36  9.46  9.27  9.28   13.34
+//                             60000      229   118  78.7  48.5     195
+//   100K vertices                255    4.13  2.47  2.35  2.43    4.13
+//                             60000     64.3  28.5  16.1  7.83    23.1
+//   lattice, 2^18                255    12.5  6.63  4.97  4.52    10.9
+//                             60000      616   193  69.0  27.8    40.4
 int64_t default_batch_width(int64_t, int64_t) { return 64; }
 int64_t default_bc_grid(int64_t, int64_t) { return 256 * 32; }
 struct Knob {

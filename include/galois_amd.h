@@ -116,8 +116,9 @@ void gx_set_profiling(int on);
  *                          also for FP64 (FP64 atomic row sums, order
  *                          dependent in the last bit), 0 = pull sweep for
  *                          both (FP64 row sums; FP64 solves of 2^23 edges and
- *                          2^19 vertices or more sum in blocks); while not set, FP32 solves of
- *                          fewer than 2^21 edges pull as well
+ *                          2^19 vertices or more sum in blocks); while not
+ *                          set, FP32 solves of fewer than 2^21 edges pull as
+ *                          well
  *   "pr.task_edges"        propagation-blocked sweep: a destination bin
  *                          with more in-edges than this is summed by
  *                          several workgroups (slices) that meet in a
